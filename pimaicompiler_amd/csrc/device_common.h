@@ -11,6 +11,7 @@ typedef _Float16 half_t;
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 half8_any_t __attribute__((ext_vector_type(8), aligned(2)));  // eight halves at any address an fp16 may have
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
 static constexpr int kWave = 64;
@@ -54,6 +55,17 @@ __device__ __forceinline__ half8_t load_weight(const half8_t* p)
         return *p;
     else
         return __builtin_nontemporal_load(p);
+}
+// The same wherever the eight halves lie: still one 16-byte load (the hardware takes any address), which touches one line
+// more than an aligned one where it straddles two.
+template <bool KEEP>
+__device__ __forceinline__ half8_t load_weight_any(const half_t* p)
+{
+    const half8_any_t* q = reinterpret_cast<const half8_any_t*>(p);
+    if constexpr (KEEP)
+        return *q;
+    else
+        return __builtin_nontemporal_load(q);
 }
 
 // DPP controls (gfx9 encoding).

@@ -27,8 +27,10 @@ namespace pimhip
 // keeps U chunks per row in flight: R*U independent 16-byte weight loads per lane per iteration.
 // ---------------------------------------------------------------------------------------------
 // SPLIT: x is the concatenation of two vectors that lie apart (x: the first split_chunks 16-byte pieces, x2: the rest);
-// compiled out of every other instance.  KEEP: the weight is read with plain loads (load_weight).
-template <int R, int U, int WAVES, int KS, bool SPLIT = false, bool KEEP = false>
+// compiled out of every other instance.  KEEP: the weight is read with plain loads (load_weight).  ANY: rows, x and K need
+// not be multiples of 16 bytes; the same 16-byte loads at whatever address the row has, and the K % 8 columns behind the
+// last whole piece one per lane.
+template <int R, int U, int WAVES, int KS, bool SPLIT = false, bool KEEP = false, bool ANY = false>
 __device__ __forceinline__ void gemv_mv_f16_body(const half_t* __restrict__ W, const half_t* __restrict__ x,
                                                  const half_t* __restrict__ bias, half_t* __restrict__ y, int N,
                                                  int K, long ldw, int relu, int block,
@@ -45,17 +47,28 @@ __device__ __forceinline__ void gemv_mv_f16_body(const half_t* __restrict__ W, c
     const long row0 = ((long)block * RG + rg) * R;
 
     float acc[R];
-    const half8_t* wrow[R];
+    const half_t* wrow[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         acc[r] = 0.0f;
         long row = row0 + r;
         if (row > N - 1) row = N - 1;  // out-of-range rows re-read the last row and are never stored
-        wrow[r] = reinterpret_cast<const half8_t*>(W + row * ldw);
+        wrow[r] = W + row * ldw;
+        if constexpr (ANY) {
+            const int k = (K & ~7) + lane;
+            if (ks == 0 && k < K) acc[r] = (float)wrow[r][k] * (float)x[k];
+        }
     }
     const half8_t* xv = reinterpret_cast<const half8_t*>(x);
     const half8_t* xv2 = SPLIT ? reinterpret_cast<const half8_t*>(x2) - split_chunks : nullptr;  // (indexed from split_chunks on)
-    auto x_at = [&](int c) { return (SPLIT && c >= split_chunks) ? xv2[c] : xv[c]; };
+    auto x_at = [&](int c) -> half8_t {
+        if constexpr (ANY) return load_weight_any<true>(x + 8 * (long)c);
+        return (SPLIT && c >= split_chunks) ? xv2[c] : xv[c];
+    };
+    auto w_at = [&](const half_t* row, int c) -> half8_t {
+        if constexpr (ANY) return load_weight_any<KEEP>(row + 8 * (long)c);
+        return load_weight<KEEP>(reinterpret_cast<const half8_t*>(row) + c);
+    };
     const int nchunks = K >> 3;
     constexpr int STEP = 64 * KS;
 
@@ -67,7 +80,7 @@ __device__ __forceinline__ void gemv_mv_f16_body(const half_t* __restrict__ W, c
 #pragma unroll
         for (int u = 0; u < U; ++u) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) wr[r][u] = load_weight<KEEP>(wrow[r] + c + u * STEP);
+            for (int r = 0; r < R; ++r) wr[r][u] = w_at(wrow[r], c + u * STEP);
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) xr[u] = x_at(c + u * STEP);
@@ -81,7 +94,7 @@ __device__ __forceinline__ void gemv_mv_f16_body(const half_t* __restrict__ W, c
     for (; c < nchunks; c += STEP) {
         half8_t wr[R];
 #pragma unroll
-        for (int r = 0; r < R; ++r) wr[r] = load_weight<KEEP>(wrow[r] + c);
+        for (int r = 0; r < R; ++r) wr[r] = w_at(wrow[r], c);
         const half8_t xr = x_at(c);
 #pragma unroll
         for (int r = 0; r < R; ++r) acc[r] = dot8(wr[r], xr, acc[r]);
@@ -143,6 +156,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_mv_keep_f16_kernel(const half
     gemv_mv_f16_body<R, U, WAVES, KS, false, true>(W, x, bias, y, N, K, ldw, relu, blockIdx.x);
 }
 
+// The same for rows at any address and of any length (K % 8, the row pitch % 8 or an operand's address not those of whole
+// 16-byte pieces).  A straddling load touches one line in eight more than an aligned one, which is what is left to the
+// aligned kernel's rate: 11624 x 4967 21.3 us (5.4 TB/s; with one wavefront per row and 2-byte loads 76 us), 2049 x 2055
+// 8.8 -> 3.0 us, 512 x 1345 4.0 -> 2.1, 40 x 14833 27 -> 2.9.
+template <int R, int U, int WAVES, int KS, bool KEEP>
+__global__ __launch_bounds__(WAVES * 64) void gemv_mv_any_f16_kernel(const half_t* __restrict__ W,
+                                                                     const half_t* __restrict__ x,
+                                                                     const half_t* __restrict__ bias,
+                                                                     half_t* __restrict__ y, int N, int K, long ldw,
+                                                                     int relu)
+{
+    gemv_mv_f16_body<R, U, WAVES, KS, false, KEEP, true>(W, x, bias, y, N, K, ldw, relu, blockIdx.x);
+}
+
 // y = act(W . cat(x1, x2) + bias) without the concatenation: the second operand of the RNNT joint network's first layer
 // is cat(encoder frame, prediction), which the reference either materialises or splits the product over
 // (compiler/source/frontend/optimizer/remove_cat_for_addmm.cpp:46-191: two dependent launches).
@@ -189,28 +216,6 @@ __global__ __launch_bounds__(kGemvGroupThreads) void gemv_mv_f16_group_kernel(Ge
         gemv_mv_f16_body<2, 4, 4, 4, false, KEEP>(g.W[i], g.x[i], g.bias[i], g.y[i], g.N[i], g.K[i], (long)g.K[i], g.relu[i], block);
     else
         gemv_mv_f16_body<2, 2, 4, 2, false, KEEP>(g.W[i], g.x[i], g.bias[i], g.y[i], g.N[i], g.K[i], (long)g.K[i], g.relu[i], block);
-}
-
-// MV order, any K / leading dimension / alignment: one wavefront per row, 2-byte loads.
-template <int WAVES>
-__global__ __launch_bounds__(WAVES * 64) void gemv_mv_f16_generic_kernel(const half_t* __restrict__ W,
-                                                                         const half_t* __restrict__ x,
-                                                                         const half_t* __restrict__ bias,
-                                                                         half_t* __restrict__ y, int N, int K,
-                                                                         long ldw, int relu)
-{
-    const int lane = threadIdx.x & 63;
-    const long row = (long)blockIdx.x * WAVES + (threadIdx.x >> 6);
-    if (row >= N) return;
-    const half_t* w = W + row * ldw;
-    float acc = 0.0f;
-    for (int k = lane; k < K; k += 64) acc = fmaf((float)w[k], (float)x[k], acc);
-    acc = wave_sum(acc);
-    if (lane == 0) {
-        if (bias) acc += (float)bias[row];
-        if (relu) acc = relu_f32(acc);
-        y[row] = (half_t)acc;
-    }
 }
 
 // ---------------------------------------------------------------------------------------------
