@@ -128,39 +128,53 @@ int get_static_workspace(DeviceState* st, hipStream_t stream, size_t partial_ele
 int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bias, const GemvOuts& outs, int64_t K,
             int64_t N, int64_t lda, int relu, hipStream_t s, bool static_ws = false)
 {
-    bool vec_ok = (N % 8 == 0) && (lda % 8 == 0) && aligned16(A);
-    for (int o = 0; o < outs.count; ++o) vec_ok = vec_ok && aligned16(outs.y[o]);
-    if (!vec_ok) {
+    // The one-column-per-lane kernel where no eight columns exist, and for the smallest products: up to 4096 weights it takes
+    // 1.8 us against 2.3-2.5 us for the kernel below (two barriers more); 672 x 104 already 3.7 against 2.3.
+    if (N < 8 || N * K <= 4096) {
         const int grid = (int)((N + 63) / 64);
         gemv_vm_f16_generic_kernel<<<grid, 64 * kVmGenericWaves, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu);
         return PIMHIP_OK;
     }
-    // Measured on MI355X: 128-column blocks (16 lanes per weight row, 4 rows per wavefront and load) with 8 loads in
-    // flight per lane are fastest for every shape tried; a cross-block reduction costs 1 to 2 us, so K is sliced
-    // only as far as needed for roughly one block per CU (64 blocks for a weight of a few MB), and not at all for
-    // weights of up to 256 KB.
-    constexpr int WAVES = 4, U = 8, LPR = 16;
-    constexpr int GROUPS = WAVES * (64 / LPR);
-    const int col_blocks = (int)((N + LPR * 8 - 1) / (LPR * 8));
+    // Block width: 64 columns (8 lanes per weight row) while the weight is small, so that more blocks share it: 2048 x 2048
+    // 3.5 us against 4.2 with 128 columns, 12896 x 84 4.0 against 6.7.  128 columns for a weight past kKeepCachedBytes, whose
+    // stream is the bound: 4096 x 4096 7.7 us against 8.2 with 64, 1024 x 32000 11.2 against 13.7.
     const int64_t weight_bytes = K * N * (int64_t)sizeof(half_t);
+    const bool large = weight_bytes > (int64_t)kKeepCachedBytes;
+    const int lanes_per_row = large ? 16 : 8;
+    const int cols = 8 * lanes_per_row, row_groups = kVmWaves * 64 / lanes_per_row;
+    const int col_blocks = (int)((N + cols - 1) / cols);
+    // Rows that do not start on a 128-byte line make neighbouring column blocks share lines: they go to one XCD then, whose
+    // L2 hands the shared line to both (1024 x 31999: 11.6 us against 16.4), and the weight is read with plain loads.  Where
+    // no line is shared the same order costs (4096 x 4096 7.9 -> 9.9 us: eight fronts instead of one).
+    const int by_xcd = col_blocks >= 16 && (lda % 64 != 0 || (reinterpret_cast<uintptr_t>(A) & 127u) != 0);
+    // Slices of K: about a block per CU for a large weight, 64 blocks for a small one, but a cross-block sum costs 1 to 2 us
+    // and grows with the slices: none up to 512 rows (272 x 2357: 3.1 us, two slices 3.6) and at most sqrt(K / 40) of them
+    // (12896 rows, 84 columns: 4.0 us with 17, 4.9 with 64).
     int64_t target = weight_bytes / 65536;
     if (target < 64) target = 64;
     if (target > st->num_cus) target = st->num_cus;
     int slices = (int)((target + col_blocks / 2) / col_blocks);  // rounded: 250 column blocks on 256 CUs are not sliced
-    const int max_slices = (int)((K + 31) / 32);
-    if (slices > max_slices) slices = max_slices;
-    if (weight_bytes <= 256 * 1024) slices = 1;
+    if (K <= 512) slices = 1;
+    while (slices > 1 && (int64_t)slices * slices * 40 > K) --slices;
     if (slices < 1) slices = 1;
-    int k_per_slice = (int)((K + slices - 1) / slices);
-    k_per_slice = (k_per_slice + GROUPS - 1) / GROUPS * GROUPS;
-    if (k_per_slice < GROUPS) k_per_slice = GROUPS;  // K == 0: one empty slice, y = act(bias)
-    slices = (int)((K + k_per_slice - 1) / k_per_slice);
-    if (slices < 1) slices = 1;
+    // Small weights and operands of no whole 16-byte pieces run without a workspace where they cannot have one (the static
+    // scratch array is too small, or a graph is being recorded before the stream has its workspace), in one slice.
+    const bool can_do_without = weight_bytes <= 256 * 1024 || (N % 8 != 0) || (lda % 8 != 0) || !aligned16(A) || !aligned16(outs.y[0]);
+    int k_per_slice = 0;
+    auto cut = [&]() {
+        k_per_slice = (int)((K + slices - 1) / slices);
+        k_per_slice = (k_per_slice + row_groups - 1) / row_groups * row_groups;
+        if (k_per_slice < row_groups) k_per_slice = row_groups;  // K == 0: one empty slice, y = act(bias)
+        slices = (int)((K + k_per_slice - 1) / k_per_slice);
+        if (slices < 1) slices = 1;
+    };
+    if (static_ws && can_do_without && (size_t)(slices - 1) * (size_t)N > kStaticScratchFloats) slices = 1;
+    cut();
     float* partial = nullptr;
     unsigned int* status = nullptr;
     unsigned int* poison = nullptr;
     if (slices > 1) {
-        // Records of all slices but the last: partial[slice][N].
+        // Words of all slices but the last: partial[slice][N].
         const size_t partial_elems = (size_t)(slices - 1) * (size_t)N;
         int rc;
         if (static_ws) {
@@ -172,13 +186,18 @@ int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bia
                 partial = ws->partial;
                 status = ws->status_dev;
                 poison = ws->poison;
+            } else if (rc == PIMHIP_ERR_UNSUPPORTED && can_do_without) {
+                rc = PIMHIP_OK;
+                slices = 1;
+                cut();
             }
         }
         if (rc != PIMHIP_OK) return rc;
     }
-    dim3 grid(col_blocks, slices);
-    gemv_vm_f16_kernel<WAVES, U, LPR><<<grid, WAVES * 64, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu,
-                                                                    k_per_slice, partial, status, poison, st->vm_spin_limit);
+    const dim3 grid(by_xcd ? (col_blocks + 7) / 8 * 8 : col_blocks, slices);
+    auto kernel = !large ? gemv_vm_f16_kernel<8, true> : by_xcd ? gemv_vm_f16_kernel<16, true> : gemv_vm_f16_kernel<16, false>;
+    kernel<<<grid, kVmWaves * 64, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu, k_per_slice, partial, status, poison,
+                                          st->vm_spin_limit, by_xcd);
     return PIMHIP_OK;
 }
 

@@ -13,6 +13,8 @@
 // the final reduction.
 #pragma once
 
+#include <type_traits>
+
 #include "device_common.h"
 
 namespace pimhip
@@ -219,22 +221,32 @@ __global__ __launch_bounds__(kGemvGroupThreads) void gemv_mv_f16_group_kernel(Ge
 }
 
 // ---------------------------------------------------------------------------------------------
-// VM order, vector path.  Requirements: N % 8 == 0, lda % 8 == 0, A 16-byte aligned.
-//
-// A block owns CW = 8 * LPR adjacent outputs and a slice [k_begin, k_end) of the reduction.  LPR lanes (8 columns,
-// one 16-byte load each) cover the block's part of one weight row, so a wavefront reads 64 / LPR rows per load
-// instruction and the block's wavefronts interleave over the rows of the slice, U loads in flight per lane.
+// VM order, N >= 8.  A block owns 8 * LPR adjacent outputs and a slice [k_begin, k_end) of the reduction.  LPR lanes (8
+// columns, one 16-byte load each) cover the block's part of one weight row, so a wavefront reads 64 / LPR rows per load
+// instruction and the block's eight wavefronts interleave over the rows of the slice, four loads in flight per lane.  The row
+// groups' sums meet in LDS; from there on a thread stands for one column, 512 / (8 LPR) threads ("parts") per column.
 // gridDim.y slices cover K.  With one slice the block finishes the outputs itself.  With several, the blocks of all
-// slices but the last store their CW partial sums (fp32) as 32-byte records in `partial[slice][N]` and exit; the blocks
-// of the LAST slice add the records to their own sums, in an order that depends on the slice index only (so the result
-// is the same in every run), and apply the epilogue.
+// slices but the last store their partial sums (fp32) in `partial[slice][N]` and exit; the blocks of the LAST slice add
+// them to their own sums, in an order that depends on the slice index only (so the result is the same in every run), and
+// apply the epilogue.
 //
-// A record that has not arrived yet holds kVmEmpty in every word (the bit pattern 0xffffffff: a NaN that no sum of
-// products of fp16 values can be, since arithmetic yields the canonical NaN or the widened payload of an fp16 NaN), so
-// the reducing block polls each record until none of its words is kVmEmpty, adds it and writes kVmEmpty back for the
-// next launch.  Records travel with device-scope (sc1) stores and loads; there is no fence (a device-scope fence writes
-// back and invalidates the XCD's whole L2, once per block) and no ticket counter (store, acknowledgement, atomic,
-// loads would be three trips through the memory side after the last block's arithmetic; polling is one).
+// Rows may lie at any address: a 16-byte load takes what address the row has, and the lane with the last N % 8 columns reads
+// the row's last eight and keeps its own.
+//
+// What bounds it: the stream for a large weight (bytes in flight: eight wavefronts of four loads beat four of eight by 15 %,
+// blocks of 16 wavefronts and 8 loads lose again), for a small one the chain launch, rows, LDS, cross-block words, store.  The
+// group sums are spread over all threads (one thread per column adding all of them took 0.2-0.4 us more).  Measured on
+// MI355X in graph replays against one block of 256 threads per 128 columns, records of 32 bytes and a kernel of 2-byte loads
+// for everything not aligned: 4096 x 4096 9.3 -> 7.7 us, 4096 x 16384 22.4 -> 21.2, 16384 x 4096 24.4 -> 22.7, 1024 x 32000
+// 12.0 -> 11.2, 1024 x 1024 4.7 -> 3.2; odd sizes: 1024 x 31999 22.1 -> 11.6 us, 4046 x 9937 27.3 -> 14.9, 4951 x 1301
+// 30 -> 6.7, 12896 x 84 71 -> 4.0, 1252 x 54 6.5 -> 3.2.
+//
+// A word that has not arrived yet holds kVmEmpty (the bit pattern 0xffffffff: a NaN that no sum of products of fp16 values
+// can be, since arithmetic yields the canonical NaN or the widened payload of an fp16 NaN), so a reducing thread polls
+// each of its column's words until it is something else, adds it and writes kVmEmpty back for the next launch.  Words travel
+// with device-scope (sc1) stores and loads; there is no fence (a device-scope fence writes back and invalidates the XCD's
+// whole L2, once per block) and no ticket counter (store, acknowledgement, atomic, loads would be three trips through the
+// memory side after the last block's arithmetic; polling is one).
 //
 // What the scheme assumes of the dispatcher, and what it does not: the producers never wait for anything, so each of
 // them finishes whatever else occupies the GPU, in any dispatch order; results never depend on the order.  That the
@@ -243,12 +255,12 @@ __global__ __launch_bounds__(kGemvGroupThreads) void gemv_mv_f16_group_kernel(Ge
 // XCD's reducing blocks (the last slice), and a reducing block on one XCD waits at most for the other XCDs to get
 // through the producers dealt to them.  When other work holds CUs of one XCD (a resident sequence kernel on another
 // stream) that wait grows by as much as that XCD is held up.  It is bounded all the same: after `spin_limit` polls
-// of one record (none at all with a limit of 0, which is how a test forces the condition from the host), or one second,
-// the lane gives up on the record and computes that slice's sums for its eight columns itself, with the producer's own
-// order of operations, so the result has the bits it would have had.  The record may still arrive later and would then
-// sit in the workspace as if it belonged to the next launch: the lane raises *poison (a device word the reducing blocks
-// of every launch look at) and *status (for the host), and until the host has refilled the records and cleared both,
-// reducing blocks do not look at records at all and compute every slice themselves: slow, but right.
+// of one word (none at all with a limit of 0, which is how a test forces the condition from the host), or one second,
+// the thread gives up on the word and computes that slice's sum for its column itself, with the producer's own
+// order of operations, so the result has the bits it would have had.  The word may still arrive later and would then
+// sit in the workspace as if it belonged to the next launch: the thread raises *poison (a device word the reducing blocks
+// of every launch look at) and *status (for the host), and until the host has refilled the words and cleared both,
+// reducing blocks do not look at them at all and compute every slice themselves: slow, but right.
 // ---------------------------------------------------------------------------------------------
 // Destinations of a VM product: the same result is stored to `count` buffers (the GNMT attention context goes
 // straight into three concatenation buffers, runtime/source/executor/op_executor/aten_ops_executor.cpp:694-737).
@@ -258,44 +270,34 @@ struct GemvOuts {
     int count;
 };
 
-// 32 contiguous bytes written at device scope (partial sums cross CUs and XCDs).
-__device__ __forceinline__ void store32_device_scope(float* p, const float (&v)[8])
-{
-    const float4_t lo = {v[0], v[1], v[2], v[3]}, hi = {v[4], v[5], v[6], v[7]};
-    asm volatile("global_store_dwordx4 %0, %1, off sc1\n\tglobal_store_dwordx4 %0, %2, off offset:16 sc1" : : "v"(p), "v"(lo), "v"(hi) : "memory");
-}
-// One 32-byte record of partial sums read at device scope (both halves issued together, one wait).
-__device__ __forceinline__ void load32_device_scope_one(const float* p, float4_t& lo, float4_t& hi)
-{
-    asm volatile("global_load_dwordx4 %0, %2, off sc1\n\tglobal_load_dwordx4 %1, %2, off offset:16 sc1\n\ts_waitcnt vmcnt(0)"
-                 : "=&v"(lo), "=&v"(hi)
-                 : "v"(p)
-                 : "memory");
-}
+static constexpr int kVmWaves = 8;
+static constexpr int kVmLoads = 4;  // 16-byte loads in flight per lane
 
-
-template <int WAVES, int U, int LPR>
-__global__ __launch_bounds__(WAVES * 64) void gemv_vm_f16_kernel(const half_t* __restrict__ x,
+// LPR: lanes per weight row.  KEEP: the weight is read with plain loads (load_weight).
+template <int LPR, bool KEEP>
+__global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t* __restrict__ x,
                                                                  const half_t* __restrict__ A,
                                                                  const half_t* __restrict__ bias,
                                                                  GemvOuts outs, int K, int N, long lda,
                                                                  int relu, int k_per_slice, float* partial,
                                                                  unsigned int* status, unsigned int* poison,
-                                                                 unsigned int spin_limit)
+                                                                 unsigned int spin_limit, int by_xcd)
 {
-    static_assert(LPR == 16 || LPR == 32 || LPR == 64, "lanes per weight row");
-    constexpr int RPW = 64 / LPR;          // rows per wavefront and load instruction
-    constexpr int GROUPS = WAVES * RPW;    // row groups per block = LDS rows of the reduction
-    constexpr int STEP = GROUPS;           // rows between consecutive loads of one lane
-    __shared__ float red[GROUPS][8][LPR];
+    constexpr int U = kVmLoads;
+    constexpr int kVmCols = 8 * LPR;
+    constexpr int GROUPS = kVmWaves * (64 / LPR);     // row groups per block = LDS rows of the reduction = rows between loads of a lane
+    constexpr int PARTS = kVmWaves * 64 / kVmCols;    // threads per column when the slices' sums are collected
+    __shared__ __align__(16) float red[GROUPS][kVmCols];
+    __shared__ float parts[PARTS][kVmCols];
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
     const int cg = lane % LPR;             // which 8 columns of the block
-    const int grp = wave * RPW + lane / LPR;
-    const long col0 = ((long)blockIdx.x * LPR + cg) * 8;
-    const bool col_ok = col0 < N;
+    const int grp = tid / LPR;
+    const int bx = by_xcd ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
+    const long base = (long)bx * kVmCols;
+    if (base >= N) return;  // (a grid that goes by XCD is rounded up to whole eights)
+    const long col0 = base + cg * 8;
     const int k_begin = blockIdx.y * k_per_slice;
     const int k_end = min(K, k_begin + k_per_slice);
 
@@ -307,151 +309,145 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_vm_f16_kernel(const half_t* _
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
 
-    if (col_ok) {
-        const half_t* a = A + col0;
-        int k = k_begin + grp;
-        for (; k + (U - 1) * STEP < k_end; k += U * STEP) {
+    const bool whole = col0 + 8 <= N;
+    if (col0 < N) {
+        const half_t* a = A + (whole ? col0 : (long)N - 8);
+        auto take = [&](int k, auto last) __attribute__((always_inline)) {
             half8_t ar[U];
             float xr[U];
+            // (rows past the slice re-read its last one and count as zeros: all of a trip's loads are in flight together)
+            auto row = [&](int u) { return last ? min(k + u * GROUPS, k_end - 1) : k + u * GROUPS; };
 #pragma unroll
-            for (int u = 0; u < U; ++u)
-                ar[u] = load_stream(reinterpret_cast<const half8_t*>(a + (long)(k + u * STEP) * lda));
+            for (int u = 0; u < U; ++u) ar[u] = load_weight_any<KEEP>(a + (long)row(u) * lda);
 #pragma unroll
-            for (int u = 0; u < U; ++u) xr[u] = (float)x[k + u * STEP];
+            for (int u = 0; u < U; ++u) xr[u] = (float)x[row(u)];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
+                if (last && k + u * GROUPS >= k_end) {
+                    xr[u] = 0.0f;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) ar[u][j] = (half_t)0.0f;
+                }
 #pragma unroll
                 for (int j = 0; j < 8; ++j) acc[j] = fmaf((float)ar[u][j], xr[u], acc[j]);
             }
-        }
-        for (; k < k_end; k += STEP) {
-            const half8_t ar = load_stream(reinterpret_cast<const half8_t*>(a + (long)k * lda));
-            const float xr = (float)x[k];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[j] = fmaf((float)ar[j], xr, acc[j]);
-        }
+        };
+        int k = k_begin + grp;
+        for (; k + (U - 1) * GROUPS < k_end; k += U * GROUPS) take(k, std::false_type{});
+        if (k < k_end) take(k, std::true_type{});
     }
-
-    // Combine the GROUPS partial sums of each column in LDS, in group order; lanes tid < LPR end up with the block's result.
+    if (whole || col0 >= N) {
+        *reinterpret_cast<float4_t*>(&red[grp][cg * 8]) = float4_t{acc[0], acc[1], acc[2], acc[3]};
+        *reinterpret_cast<float4_t*>(&red[grp][cg * 8 + 4]) = float4_t{acc[4], acc[5], acc[6], acc[7]};
+    } else {
+        const int first = (int)(N - 8 - base);  // where the loaded columns lie in the block (before its start if it has fewer than eight)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) red[grp][j][cg] = acc[j];
+        for (int j = 0; j < 8; ++j)
+            if (first + j >= cg * 8) red[grp][first + j] = acc[j];
+    }
     __syncthreads();
-    const bool finisher = tid < LPR && col_ok;  // tid < LPR: cg == tid, grp == 0
-    if (tid < LPR) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            float v = red[0][j][cg];
-#pragma unroll
-            for (int g = 1; g < GROUPS; ++g) v += red[g][j][cg];
-            acc[j] = v;
-        }
-    }
 
-    auto epilogue_store = [&](const float (&v)[8]) {
-        half8_t out;
+    // From here on a thread stands for one column.
+    const int c = tid % kVmCols;
+    const int part = tid / kVmCols;
+    const long col = base + c;
+    const bool mine = col < N;
+    // Part p adds the groups p, p + PARTS, .. in that order, then the parts are added in order.
+    {
+        float v = red[part][c];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            float r = v[j];
-            if (bias) r += (float)bias[col0 + j];
-            if (relu) r = relu_f32(r);
-            out[j] = (half_t)r;
-        }
-        for (int o = 0; o < outs.count; ++o) *reinterpret_cast<half8_t*>(outs.y[o] + col0) = out;
+        for (int i = 1; i < GROUPS / PARTS; ++i) v += red[part + i * PARTS][c];
+        parts[part][c] = v;
+    }
+    __syncthreads();
+    auto total = [&]() {
+        float v = parts[0][c];
+#pragma unroll
+        for (int q = 1; q < PARTS; ++q) v += parts[q][c];
+        return v;
+    };
+    const float own = part == 0 ? total() : 0.0f;
+    auto finish = [&](float r) {
+        if (bias) r += (float)bias[col];
+        if (relu) r = relu_f32(r);
+        const half_t out = (half_t)r;
+        for (int o = 0; o < outs.count; ++o) outs.y[o][col] = out;
     };
 
     const int nslices = gridDim.y;
     if (nslices == 1) {
-        if (finisher) epilogue_store(acc);
+        if (part == 0 && mine) finish(own);
         return;
     }
-
     const int last = nslices - 1;
     if ((int)blockIdx.y != last) {
-        if (finisher) store32_device_scope(partial + (long)blockIdx.y * N + col0, acc);
+        if (part == 0 && mine)
+            __hip_atomic_store(reinterpret_cast<unsigned int*>(partial) + (long)blockIdx.y * N + col, __builtin_bit_cast(unsigned int, own),
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return;
     }
-    float own[8];
+    // Part p adds the words of slices p, p + PARTS, ... < last in that order, kVmAhead of them asked for together.
+    constexpr int kVmAhead = 4;
+    float sum = 0.0f;
+    if (mine) {
+        unsigned int* words = reinterpret_cast<unsigned int*>(partial) + col;
+        for (int s0 = part; s0 < last; s0 += kVmAhead * PARTS) {
+            unsigned int w[kVmAhead];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        own[j] = acc[j];  // meaningful in the finisher lanes
-        acc[j] = 0.0f;
-    }
-    // Row group g adds the records of slices g, g + GROUPS, ... < last in that order.
-    if (col_ok) {
-        for (int sl = grp; sl < last; sl += GROUPS) {
-            float* rec = partial + (long)sl * N + col0;
-            float4_t lo, hi;
-            unsigned int spins = 0;
-            unsigned long long t_first = 0ull;
-            bool have = false;
-            while (poisoned == 0u) {
-                if (spins > 0u && (spins & 255u) == 0u && wait_clock_expired(spins, t_first)) spins = 0xffffffffu;  // gives up below
-                if (spins++ >= spin_limit) {
-                    __hip_atomic_store(poison, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    break;
-                }
-                load32_device_scope_one(rec, lo, hi);
-                bool ok = true;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    ok = ok && __builtin_bit_cast(unsigned int, lo[j]) != kVmEmpty && __builtin_bit_cast(unsigned int, hi[j]) != kVmEmpty;
-                if (ok) {
-                    have = true;
-                    break;
-                }
+            for (int q = 0; q < kVmAhead; ++q) {
+                w[q] = kVmEmpty;
+                const int sl = s0 + q * PARTS;
+                if (sl < last && poisoned == 0u && spin_limit > 0u)
+                    w[q] = __hip_atomic_load(words + (long)sl * N, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            if (have) {
-                const float e = __builtin_bit_cast(float, kVmEmpty);
-                const float empty[8] = {e, e, e, e, e, e, e, e};
-                store32_device_scope(rec, empty);
-            } else {
-                // Slice sl's sums for these eight columns, as its own block makes them: every row group's rows in ascending
-                // order, then the groups in order.
-                const half_t* a = A + col0;
-                const int ks_begin = sl * k_per_slice, ks_end = min(K, ks_begin + k_per_slice);
-                float v[8];
-                for (int g = 0; g < GROUPS; ++g) {
-                    float part[8];
 #pragma unroll
-                    for (int j = 0; j < 8; ++j) part[j] = 0.0f;
-                    for (int k = ks_begin + g; k < ks_end; k += STEP) {
-                        const half8_t ar = *reinterpret_cast<const half8_t*>(a + (long)k * lda);
-                        const float xr = (float)x[k];
-#pragma unroll
-                        for (int j = 0; j < 8; ++j) part[j] = fmaf((float)ar[j], xr, part[j]);
+            for (int q = 0; q < kVmAhead; ++q) {
+                const int sl = s0 + q * PARTS;
+                if (sl >= last) break;
+                unsigned int spins = 0;
+                unsigned long long t_first = 0ull;
+                while (w[q] == kVmEmpty && poisoned == 0u) {
+                    if (spins > 0u && (spins & 255u) == 0u && wait_clock_expired(spins, t_first)) spins = 0xffffffffu;  // gives up below
+                    if (spins++ >= spin_limit) {
+                        __hip_atomic_store(poison, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(status, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        break;
                     }
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) v[j] = g == 0 ? part[j] : v[j] + part[j];
+                    w[q] = __hip_atomic_load(words + (long)sl * N, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
-                lo = float4_t{v[0], v[1], v[2], v[3]};
-                hi = float4_t{v[4], v[5], v[6], v[7]};
-            }
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                acc[j] += lo[j];
-                acc[4 + j] += hi[j];
+                float v;
+                if (w[q] != kVmEmpty) {
+                    v = __builtin_bit_cast(float, w[q]);
+                    __hip_atomic_store(words + (long)sl * N, kVmEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                } else {
+                    // Slice sl's sum for this column, as its own block makes it: every row group's rows in ascending order, the
+                    // groups of a part in order, then the parts.
+                    const int ks_begin = sl * k_per_slice, ks_end = min(K, ks_begin + k_per_slice);
+                    v = 0.0f;
+#pragma unroll 1
+                    for (int q2 = 0; q2 < PARTS; ++q2) {
+                        float pv = 0.0f;
+#pragma unroll 1
+                        for (int g = q2; g < GROUPS; g += PARTS) {
+                            float gv = 0.0f;
+#pragma unroll 1
+                            for (int k = ks_begin + g; k < ks_end; k += GROUPS) gv = fmaf((float)A[(long)k * lda + col], (float)x[k], gv);
+                            pv = g == q2 ? gv : pv + gv;
+                        }
+                        v = q2 == 0 ? pv : v + pv;
+                    }
+                }
+                sum += v;
             }
         }
     }
-    __syncthreads();  // the first lanes have read `red` above before it is written again
-#pragma unroll
-    for (int j = 0; j < 8; ++j) red[grp][j][cg] = acc[j];
+    __syncthreads();  // `parts` has been read above before it is written again
+    parts[part][c] = sum;
     __syncthreads();
-    if (finisher) {
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            v[j] = red[0][j][cg];
-#pragma unroll
-            for (int g = 1; g < GROUPS; ++g) v[j] += red[g][j][cg];
-            v[j] += own[j];
-        }
-        epilogue_store(v);
-    }
+    if (part == 0 && mine) finish(total() + own);
 }
 
-// VM order, any N / leading dimension / alignment: 2-byte loads.  A block of 16 wavefronts owns 64 adjacent output
+// VM order, fewer than eight columns, or very few weights: 2-byte loads.  A block of 16 wavefronts owns 64 adjacent output
 // columns (one per lane); wavefront g takes the rows g, g + 16, ... and the sixteen partial sums meet in LDS.
 static constexpr int kVmGenericWaves = 16;
 __global__ __launch_bounds__(64 * kVmGenericWaves) void gemv_vm_f16_generic_kernel(const half_t* __restrict__ x,

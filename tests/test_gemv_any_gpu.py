@@ -1,4 +1,5 @@
-"""GEMV operands of any size and address: rows that are no whole 16-byte pieces.  Reference: the float64 product.  Tolerance per output: half an ulp of fp16
+"""GEMV operands of any size and address: rows that are no whole 16-byte pieces in both weight orders, and the I_X_W kernel at
+the edges of its blocks, row groups and slices.  Reference: the float64 product.  Tolerance per output: half an ulp of fp16
 (2^-11 of the value, 2^-25 below the normal range) for the one rounding, and (in + 1) * 2^-24 times the sum of the products'
 magnitudes for any order of fp32 sums."""
 import pytest
@@ -49,3 +50,61 @@ def test_rows_of_any_length_at_any_address(ops, out_w, in_w, off_w, off_x, pitch
     b = torch.randn(out_w, generator=g).half().to(DEV)
     for bias, relu in ((b, True), (None, False)):
         check(call(L.PIMHIP_W_X_I, W, x, bias, in_w, out_w, ld, relu, off_w), W[:, :in_w], x, bias, relu)
+
+
+@pytest.mark.parametrize("in_w,out_w,off,pitch", [
+    (1, 8, 0, 0), (600, 7, 0, 0), (600, 8, 0, 0), (600, 9, 1, 0), (513, 63, 0, 0), (512, 64, 0, 0), (513, 64, 0, 3), (513, 65, 0, 0),
+    (520, 71, 3, 0), (700, 128, 0, 8), (2305, 129, 0, 0), (8, 4096, 0, 0), (31, 4097, 0, 0), (1025, 1031, 5, 0), (12896, 84, 0, 0),
+    (1500, 2000, 0, 0), (1000, 17000, 0, 0), (3001, 3001, 0, 0), (4101, 2056, 1, 0)])   # the last three: more than 16 MB
+def test_i_x_w_at_the_edges_of_blocks_row_groups_and_slices(ops, in_w, out_w, off, pitch):
+    from pimaicompiler_amd import _lib as L
+    g = torch.Generator().manual_seed(in_w * 3 + out_w)
+    ld = out_w + pitch
+    A = at_offset((0.1 * torch.randn(in_w, ld, generator=g)).half(), off)
+    x = at_offset(torch.randn(in_w, generator=g).half(), off)
+    b = torch.randn(out_w, generator=g).half().to(DEV)
+    w = A[:, :out_w].t()
+    y = call(L.PIMHIP_I_X_W, A, x, b, in_w, out_w, ld, True, off)
+    check(y, w, x, b, True)
+    for _ in range(3):                                     # a fixed order of sums: the same bits in every launch
+        assert torch.equal(call(L.PIMHIP_I_X_W, A, x, b, in_w, out_w, ld, True, off), y)
+    # reducing blocks that do not wait make the missing sums themselves, with the producers' bits
+    torch.cuda.synchronize()
+    ops.set_gemv_spin_limit(0)
+    try:
+        alone = call(L.PIMHIP_I_X_W, A, x, b, in_w, out_w, ld, True, off)
+        torch.cuda.synchronize()
+    finally:
+        ops.set_gemv_spin_limit(1 << 22)
+    assert torch.equal(alone, y)
+    assert torch.equal(call(L.PIMHIP_I_X_W, A, x, b, in_w, out_w, ld, True, off), y)   # (puts the workspace back in order)
+    torch.cuda.synchronize()
+
+
+def test_an_odd_product_is_recorded_on_a_stream_without_a_workspace(ops):
+    """Operands that need no workspace in one slice run so where the stream cannot get one: inside a capture on a fresh
+    stream, and through the entry point that never allocates."""
+    from pimaicompiler_amd import _lib as L
+    lib = L.load()
+    g = torch.Generator().manual_seed(4)
+    k, n = 1500, 2001
+    A, x = (0.1 * torch.randn(k, n, generator=g)).half().to(DEV), torch.randn(k, generator=g).half().to(DEV)
+    y = torch.empty(n, dtype=torch.float16, device=DEV)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        assert lib.pimhip_execute_gemv(y.data_ptr(), x.data_ptr(), A.data_ptr(), None, k, n, 0, L.PIMHIP_ACT_NONE, L.PIMHIP_I_X_W,
+                                       torch.cuda.current_stream().cuda_stream) == 0
+    for _ in range(3):
+        y.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        check(y, A.t(), x, None, False)
+    k, n = 9000, 30001                                      # more partial sums than the static scratch array holds
+    A, x = (0.1 * torch.randn(k, n, generator=g)).half().to(DEV), torch.randn(k, generator=g).half().to(DEV)
+    y = torch.empty(n, dtype=torch.float16, device=DEV)
+    assert lib.pimhip_execute_gemv_static(y.data_ptr(), x.data_ptr(), A.data_ptr(), None, k, n, 0, L.PIMHIP_ACT_NONE, L.PIMHIP_I_X_W,
+                                          torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    check(y, A.t(), x, None, False)
