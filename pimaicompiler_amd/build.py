@@ -71,8 +71,8 @@ ROCM_HOME = os.environ.get("ROCM_HOME") or os.environ.get("ROCM_PATH") or "/opt/
 
 
 def build_aten_ops(verbose=True):
-    """The C++ operator bodies with the reference's signatures (cpp/aten_ops_pimhip.cpp) plus their pybind module,
-    compiled with g++ against this image's LibTorch and linked to libpimhip.so next to it."""
+    """The C++ operator bodies with the reference's signatures (cpp/aten_ops_pimhip.cpp) plus their pybind module and the native
+    per-call path of ops.py (cpp/ops_fastcall.cpp), compiled with g++ against this image's LibTorch and linked to libpimhip.so next to it."""
     import sysconfig
 
     from torch.utils import cpp_extension as ce
@@ -85,8 +85,8 @@ def build_aten_ops(verbose=True):
     # c10/hip/HIPStream.h (torch's current stream) pulls in the HIP runtime API headers; host compiler only.
     cmd += ["-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", f"-I{ROCM_HOME}/include"]
     cmd += [f"-I{p}" for p in ce.include_paths()] + [f"-I{sysconfig.get_paths()['include']}"]
-    cmd += [os.path.join(cpp, "aten_ops_pimhip.cpp"), os.path.join(cpp, "aten_ops_pybind.cpp"), "-o", ATEN_LIB_PATH]
-    cmd += [f"-L{p}" for p in ce.library_paths()] + ["-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_python"]
+    cmd += [os.path.join(cpp, f) for f in ("aten_ops_pimhip.cpp", "aten_ops_pybind.cpp", "ops_fastcall.cpp")] + ["-o", ATEN_LIB_PATH]
+    cmd += [f"-L{p}" for p in ce.library_paths()] + ["-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu", "-ltorch_hip", "-ltorch_python"]
     cmd += [f"-L{PKG_DIR}", "-lpimhip", "-Wl,-rpath,$ORIGIN"] + [f"-Wl,-rpath,{p}" for p in ce.library_paths()]
     if verbose:
         print(" ".join(cmd), flush=True)

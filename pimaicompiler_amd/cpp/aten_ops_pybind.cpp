@@ -1,5 +1,5 @@
 // Python access to the C++ operator bodies of aten_ops_pimhip.cpp, so that the GPU tests can drive the exact code a
-// maintainer of the reference would link.
+// maintainer of the reference would link, and the native per-call path of pimaicompiler_amd.ops (ops_fastcall.cpp).
 #include <torch/extension.h>
 #include <c10/hip/HIPStream.h>
 
@@ -8,12 +8,14 @@
 #include "../../include/pimhip.h"
 #include "aten_ops_pimhip.h"
 #include "custom_ops_pimhip.h"
+#include "ops_fastcall.h"
 
 namespace ops = nn_compiler::runtime::op_executor;
 namespace utils = nn_compiler::runtime::utils;
 
 PYBIND11_MODULE(_aten_ops_pimhip, m)
 {
+    addFastcalls(m.ptr());
     m.def("initialize", &ops::pimhipRuntimeInitialize);
     m.def("deinitialize", &ops::pimhipRuntimeDeinitialize);
     m.def("invalidateLstmPlans", [](std::vector<at::Tensor> params) { return ops::pimhipInvalidateLstmPlans(params); });

@@ -15,6 +15,7 @@ LSTM runs in libpimhip.so.  True matrix-matrix products take the same LibTorch p
 (atenAddmm / atenMatmul, aten_ops.cpp:47-51,362).  Errors are raised as NNRuntimeException
 (runtime/include/executor/utils/utils.h:166-176) instead of being ignored.
 """
+import array
 import collections
 import contextlib
 import ctypes
@@ -43,6 +44,27 @@ def _check(rc):
     if rc != L.PIMHIP_OK:
         msg = L.load().pimhip_last_error().decode("utf-8", "replace")
         raise NNRuntimeException(f"pimhip error {rc}: {msg}")
+
+
+_native_module = None
+
+
+def _native():
+    """The extension module with the per-call path of the operators (cpp/ops_fastcall.cpp): checks, shape dispatch, output
+    tensors and the C ABI call without a Python object per step.  Its functions return None where a call is not the plain
+    case, and the bodies below take it from its start then; an integer is the C ABI's status."""
+    global _native_module
+    if _native_module is None:
+        from . import _aten_ops_pimhip
+        _native_module = _aten_ops_pimhip
+    return _native_module
+
+
+def _result(r):
+    """What a native call returned, its status raised."""
+    if type(r) is int:
+        _check(r)
+    return r
 
 
 _initialized_devices = set()
@@ -82,6 +104,11 @@ def _stream_handle(stream):
     if isinstance(stream, torch.cuda.Stream):
         return stream.cuda_stream
     return int(stream)
+
+
+def _stream_arg(stream):
+    """The stream argument of a native call: None (torch's current stream) or an integer handle."""
+    return None if stream is None else _stream_handle(stream)
 
 
 def gemv_status(stream=None):
@@ -198,6 +225,9 @@ def custom_aten_addmm(act_type, self_tensor, mat1_tensor, mat2_tensor, beta=1, a
 
     VM and MV products ignore beta and alpha exactly as the reference does (aten_ops.cpp:627-628).
     """
+    y = _native().fast_addmm(act_type == "aten::relu", self_tensor, mat1_tensor, mat2_tensor, _stream_arg(stream))
+    if y is not None:
+        return _result(y)
     _require_half_cuda(self_tensor, mat1_tensor, mat2_tensor)
     dim_i0, dim_i1, dim_self = mat1_tensor.dim(), mat2_tensor.dim(), self_tensor.dim()
     s1, s2 = gemm_broadcast(list(mat1_tensor.shape), list(mat2_tensor.shape))
@@ -238,6 +268,9 @@ def custom_aten_addmm(act_type, self_tensor, mat1_tensor, mat2_tensor, beta=1, a
 
 def custom_aten_matmul(self_tensor, other_tensor, stream=None):
     """customAtenMatmul: self . other with the reference's shape dispatch, no bias and no activation."""
+    y = _native().fast_matmul(self_tensor, other_tensor, _stream_arg(stream))
+    if y is not None:
+        return _result(y)
     _require_half_cuda(self_tensor, other_tensor)
     dim_i0, dim_i1 = self_tensor.dim(), other_tensor.dim()
     s1, s2 = gemm_broadcast(list(self_tensor.shape), list(other_tensor.shape))
@@ -302,6 +335,9 @@ def aten_linear(input_tensor, weight, bias=None, act_type="none", stream=None):
     (compiler/source/frontend/optimizer/convert_linear_to_addmm.cpp:50-51, swap_addmm_inputs.cpp:45-97),
     without the two transposes those passes insert.  Inputs with more than one row take the LibTorch passthrough.
     """
+    y = _native().fast_linear(act_type == "aten::relu", input_tensor, weight, bias, _stream_arg(stream))
+    if y is not None:
+        return _result(y)
     _require_half_cuda(input_tensor, weight, bias)
     out_w, in_w = weight.shape
     if input_tensor.numel() != in_w:
@@ -344,6 +380,10 @@ def execute_gemv_group(inputs, weights, biases=None, act_types=None, stream=None
     Replaces executeMultiStream's one-stream-per-GEMV issue
     (runtime/source/executor/op_executor/stream_ops_executor.cpp:27-50).  Returns the list of outputs.
     """
+    outs = _native().fast_group(list(inputs), list(weights), list(biases) if biases is not None else None,
+                                tuple(_act_code(a) for a in act_types) if act_types is not None else None, _stream_arg(stream))
+    if outs is not None:
+        return _result(outs)
     lib = L.load()
     n = len(weights)
     if len(inputs) != n:
@@ -455,6 +495,9 @@ def _custom_add_dims_ok(t1, t2):
 
 def input_projection(x, w, bias=None, stream=None):
     """out[T, N] fp32 = x[T, K] . w[N, K]^T + bias[N] (fp32) on the matrix cores."""
+    out = _native().fast_projection(x, w, bias, w.size(0), False, _stream_arg(stream))
+    if out is not None:
+        return _result(out)
     lib = L.load()
     _require_half_cuda(x, w)
     _ensure_init(w)
@@ -489,6 +532,9 @@ def pack_projection_weight(w, stream=None):
 
 def input_projection_packed(x, packed, n_out, bias=None, stream=None):
     """input_projection with a weight from pack_projection_weight; the same bits, less LDS traffic."""
+    out = _native().fast_projection(x, packed, bias, n_out, True, _stream_arg(stream))
+    if out is not None:
+        return _result(out)
     lib = L.load()
     _require_half_cuda(x, packed)
     x = x.contiguous()
@@ -551,6 +597,7 @@ class LstmPlan:
                                            int(self.num_dirs == 2), self.input_size, self.hidden, self.max_seq_len,
                                            _stream_handle(stream)))
         self._handle = handle
+        self.first_residual_layer = None
         self._finalizer = weakref.finalize(self, LstmPlan._destroy, handle.value)
 
     @staticmethod
@@ -580,6 +627,7 @@ class LstmPlan:
         """Layers from `first_residual_layer` on return and hand up h + their own input (the GNMT wiring: an aten::lstm and an
         aten::add per layer in the reference); None or >= num_layers switches it off (pimhip_lstm_plan_set_residual)."""
         _check(L.load().pimhip_lstm_plan_set_residual(self._handle, self.num_layers if first_residual_layer is None else int(first_residual_layer)))
+        self.first_residual_layer = first_residual_layer
 
     def set_spin_limit(self, limit):
         _check(L.load().pimhip_lstm_plan_set_spin_limit(self._handle, limit))
@@ -637,6 +685,17 @@ class LstmPlan:
                 with torch.cuda.stream(stream) if stream is not None else contextlib.nullcontext():
                     d.copy_(t)
         return y, hn, cn
+
+
+def _bound_step(native_step, keep):
+    """The callable step(stream=None) of a native bound step; `keep` (its buffers, its plan) lives as long as it does."""
+    issue = _native().issue
+
+    def step(stream=None, _keep=keep):
+        rc = issue(native_step, None if stream is None else _stream_handle(stream))
+        if rc:
+            _check(rc)
+    return step
 
 
 class DecoderPlan:
@@ -731,7 +790,6 @@ class DecoderPlan:
         again: what a decoder loop or a graph capture calls per step.  The context comes from `att` [S], the attention
         weights over the encoder outputs (`enc`, handed to set_encoder here; leave it out when set_encoder has been called
         for this sentence), or from `ctx` [H], a context computed elsewhere."""
-        lib = L.load()
         n, H = self.num_layers, self.hidden
         hn = list(h_prev) if hn is None else list(hn)
         cn = list(c_prev) if cn is None else list(cn)
@@ -758,16 +816,10 @@ class DecoderPlan:
                 raise NNRuntimeException("att needs encoder outputs [len(att), H]: pass enc or call set_encoder first")
         if self.vocab and (logits is None or logits.numel() != self.vocab):
             raise NNRuntimeException(f"logits must have {self.vocab} elements")
-        mk = lambda ts: (ctypes.c_void_p * len(ts))(*[t.data_ptr() if t is not None else None for t in ts])  # noqa: E731
-        a_hp, a_cp, a_hn, a_cn, a_out = mk(h_prev), mk(c_prev), mk(hn), mk(cn), mk(outs)
-        a_ctx = mk(list(ctx_outs)) if ctx_outs else None
-        keep = (vecs, a_hp, a_cp, a_hn, a_cn, a_out, a_ctx)
+        mk = lambda ts: [t.data_ptr() if t is not None else None for t in ts]  # noqa: E731
         ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
-        args = (self._handle, ptr(x), ptr(att), ptr(ctx), a_hp, a_cp, a_hn, a_cn, a_out, a_ctx, len(ctx_outs), ptr(logits))
-
-        def step(stream=None, _keep=keep):
-            _check(lib.pimhip_decoder_step(*args, _stream_handle(stream)))
-        return step
+        return _bound_step(_native().bind_decoder(self._handle.value, ptr(x), ptr(att), ptr(ctx), mk(h_prev), mk(c_prev), mk(hn), mk(cn), mk(outs),
+                                                  mk(ctx_outs), ptr(logits)), (self, vecs))
 
 
 class MoePlan:
@@ -841,7 +893,6 @@ class MoePlan:
     def bind(self, x, y, router_logits=None, expert=None):
         """Fixes the buffers of a step (x, y [d_model] fp16; router_logits [E] fp16 and expert [1] int32 optional) and returns
         a callable step(stream=None): what a serving loop or a graph capture calls per token."""
-        lib = L.load()
         _require_half_cuda(x, y, *([router_logits] if router_logits is not None else []))
         for t in (x, y, router_logits, expert):
             if t is not None and not t.is_contiguous():
@@ -853,11 +904,7 @@ class MoePlan:
         if expert is not None and (expert.dtype != torch.int32 or expert.numel() != 1 or expert.device != x.device):
             raise NNRuntimeException("expert must be one int32 on the device")
         ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
-        args = (self._handle, ptr(x), ptr(y), ptr(router_logits), ptr(expert))
-
-        def step(stream=None, _keep=(x, y, router_logits, expert)):
-            _check(lib.pimhip_moe_ffn_step(*args, _stream_handle(stream)))
-        return step
+        return _bound_step(_native().bind_moe(self._handle.value, ptr(x), ptr(y), ptr(router_logits), ptr(expert)), (self, x, y, router_logits, expert))
 
     def forward(self, x, stream=None):
         """y, router_logits, expert (device tensors; nothing is read back) for one token x [.., d_model]."""
@@ -884,8 +931,10 @@ _plan_cache = collections.OrderedDict()
 
 
 def _plan_for(params, has_biases, num_layers, bidirectional, seq_len):
-    key = (tuple(p.data_ptr() for p in params), bool(has_biases), int(num_layers), bool(bidirectional))
-    versions = tuple(p._version for p in params)
+    both = _native().lstm_key(params)
+    if both is None:
+        both = (array.array("Q", [p.data_ptr() for p in params]).tobytes(), array.array("I", [p._version for p in params]).tobytes())
+    key, versions = (both[0], bool(has_biases), int(num_layers), bool(bidirectional)), both[1]
     entry = _plan_cache.get(key)
     if entry is not None and entry[2] != versions:
         del _plan_cache[key]
@@ -910,7 +959,7 @@ def invalidate_lstm_plans(params=None):
         _plan_cache.clear()
         return n
     ptrs = {p.data_ptr() for p in params}
-    stale = [k for k in _plan_cache if ptrs.intersection(k[0])]
+    stale = [k for k, entry in _plan_cache.items() if ptrs.intersection(p.data_ptr() for p in entry[1])]
     for k in stale:
         del _plan_cache[k]
     return len(stale)
@@ -941,7 +990,13 @@ def aten_lstm1(input, hx, params, has_biases, num_layers, dropout, train, bidire
     T = input.size(1) if batch_first else input.size(0)
     h0, c0 = hx[0], hx[1]
     plan = _plan_for(list(params), has_biases, num_layers, bidirectional, T)
-    plan.set_residual(first_residual_layer)  # (a cached plan serves calls with and without: set on every call)
+    if plan.first_residual_layer != first_residual_layer:  # (a cached plan serves calls with and without)
+        plan.set_residual(first_residual_layer)
+    if out is None:
+        r = _native().fast_lstm(plan._handle.value, input, h0, c0, plan.input_size, num_layers * plan.num_dirs, plan.hidden, plan.num_dirs,
+                                bool(batch_first), _stream_arg(stream))
+        if r is not None:
+            return _result(r)
     y, hn, cn = plan.forward(input.reshape(T, input.size(2)), h0, c0, stream, out=out)
     D, H = plan.num_dirs, plan.hidden
     seq = y.view(1, T, D * H) if batch_first else y.view(T, 1, D * H)
@@ -1037,7 +1092,6 @@ class RnntPlan:
         """Fixes the buffers of a step and returns a callable step(stream=None): what a decoding loop or a graph capture calls.
         x [I], h_prev / c_prev / hn / cn [L, H], f [F], logits [V], joint_hidden [J] or None; with run_prediction False (the
         step after a blank) x, c_prev, hn, cn may be None."""
-        lib = L.load()
         given = [t for t in (x, h_prev, c_prev, f, hn, cn, logits, joint_hidden) if t is not None]
         _require_half_cuda(*given)
         for t in given:
@@ -1050,12 +1104,8 @@ class RnntPlan:
             if t is not None and t.numel() != n:
                 raise NNRuntimeException(f"{name} must have {n} elements")
         ptr = lambda t: t.data_ptr() if t is not None else None  # noqa: E731
-        args = (self._handle, ptr(x), ptr(h_prev), ptr(c_prev), ptr(f), ptr(hn), ptr(cn), ptr(logits), ptr(joint_hidden),
-                int(bool(run_prediction)))
-
-        def step(stream=None, _keep=tuple(given)):
-            _check(lib.pimhip_rnnt_step(*args, _stream_handle(stream)))
-        return step
+        return _bound_step(_native().bind_rnnt(self._handle.value, ptr(x), ptr(h_prev), ptr(c_prev), ptr(f), ptr(hn), ptr(cn), ptr(logits),
+                                               ptr(joint_hidden), bool(run_prediction)), (self, given))
 
     def greedy_decode(self, enc, embedding, x0, blank, max_symbols_per_frame=30, max_symbols=None, h0=None, c0=None,
                       run_prediction_first=True, stream=None):
