@@ -73,6 +73,7 @@ static constexpr int kDppQuadXor1 = 0xB1;     // quad_perm:[1,0,3,2]
 static constexpr int kDppQuadXor2 = 0x4E;     // quad_perm:[2,3,0,1]
 static constexpr int kDppRowHalfMirror = 0x141;
 static constexpr int kDppRowMirror = 0x140;
+static constexpr int kDppRowRor8 = 0x128;     // row_ror:8
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_f32(float v)
@@ -80,13 +81,15 @@ __device__ __forceinline__ float dpp_f32(float v)
     return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
 }
 
-// Sum over the 64 lanes of a wavefront; every lane returns the total.
-__device__ __forceinline__ float wave_sum(float v)
+template <int CTRL>
+__device__ __forceinline__ unsigned int dpp_u32(unsigned int v)
 {
-    v += dpp_f32<kDppQuadXor1>(v);
-    v += dpp_f32<kDppQuadXor2>(v);
-    v += dpp_f32<kDppRowHalfMirror>(v);
-    v += dpp_f32<kDppRowMirror>(v);
+    return (unsigned int)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, true);
+}
+
+// Sum over the four rows of 16 lanes: every lane l returns the total of the lanes equal to l modulo 16.
+__device__ __forceinline__ float wave_sum_rows(float v)
+{
     // The two steps across rows of 16 lanes: v_permlane16_swap a, b exchanges rows 1 and 3 of a with rows 0 and 2 of b,
     // v_permlane32_swap a, b the upper 32 lanes of a with the lower 32 of b; with a == b == v on entry, a + b is the
     // pairwise sum in every lane.  (No trip through the LDS crossbar, which the generic shuffle takes.)
@@ -101,6 +104,16 @@ __device__ __forceinline__ float wave_sum(float v)
         v = a + b;
     }
     return v;
+}
+
+// Sum over the 64 lanes of a wavefront; every lane returns the total.
+__device__ __forceinline__ float wave_sum(float v)
+{
+    v += dpp_f32<kDppQuadXor1>(v);
+    v += dpp_f32<kDppQuadXor2>(v);
+    v += dpp_f32<kDppRowHalfMirror>(v);
+    v += dpp_f32<kDppRowMirror>(v);
+    return wave_sum_rows(v);
 }
 
 // The XCD a wavefront runs on: HW_REG_XCC_ID (hardware register 20), bits 3:0.  The probe that reports the placement of a

@@ -123,32 +123,80 @@ __device__ __forceinline__ void store8_plain(void* p, unsigned long long v)
     asm volatile("global_store_dwordx2 %0, %1, off" : : "v"(p), "v"(w) : "memory");
 }
 
-// The 16-bit values that lanes 0, 16, 32 and 48 hold, as one 64-bit word in lane 0 (other lanes: unspecified).
-// v_permlane16_swap with both operands alike leaves lane 16's value beside lane 0's and lane 48's beside lane 32's;
-// v_permlane32_swap then brings the upper pair down.
-__device__ __forceinline__ unsigned long long pack_row_heads(unsigned int v16)
+// The 16-bit values that quads 0 .. 3 of a row of 16 lanes hold (one per quad, in all its lanes), as one 64-bit word in lane 0 of
+// the row: quad 1 is quad 0's mirror within half the row, quads 2 and 3 lie half a row further.
+__device__ __forceinline__ unsigned long long pack_quads(unsigned int v16)
 {
-    unsigned int a = v16, b = v16;
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-    const unsigned int x = a | (b << 16);
-    unsigned int c = x, d = x;
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(c), "+v"(d));
-    return (unsigned long long)c | ((unsigned long long)d << 32);
+    const unsigned int lo = v16 | (dpp_u32<kDppRowHalfMirror>(v16) << 16);
+    return (unsigned long long)lo | ((unsigned long long)dpp_u32<kDppRowRor8>(lo) << 32);
 }
 
-// acc[g], one partial sum per lane and gate, for the unit of this row of 16 lanes: returns, in every lane l, the sum over
-// the 16 lanes of the row of gate ((l >> 2) & 3).  Each stage halves the number of values a lane holds and doubles the
-// lanes they are summed over: mirrored lanes of the row (l ^ 15), mirrored lanes of half a row (l ^ 7), the quad.
-__device__ __forceinline__ float row16_transpose_sum4(const float (&acc)[4], int lane)
+// ---- the step's matrix-vector product on v_smfmac_f32_16x16x64_f16 ----
+// D[16 x 16] += A[16 x 64, two of every four columns present] . B[64 x 16]: the weights are the dense operand, 64 columns of
+// the wavefront's 16 gate rows per instruction, and h is the sparse one.  A row of A holds only half of the 64 columns, but
+// which half is the row's own choice: even rows name columns 0, 1 of every four, odd rows columns 2, 3, so the two rows of a
+// pair together multiply all 64 columns by h, and their two results add up to the dot product.  A matrix instruction thus
+// takes 1024 weights in 16 cycles where v_dot2 takes 512 and a dense MFMA with h as one of its rows as many (batch 1).
+// One register set of A (eight halves per lane) has eight row pairs and holds 512 values of h; instruction m of the eight
+// that use it reads the weights of pair m's 64 columns, and of its result only rows 2m, 2m + 1 mean anything: eight
+// accumulators, of which each row of 16 lanes keeps the two row pairs it holds.  No sum across the 16 lanes is left to do
+// (column n of D is lane n & 15), and a wavefront reads h from LDS once, 2 KB instead of 8.
+typedef _Float16 half16_t __attribute__((ext_vector_type(16)));
+static constexpr int kXcdFrags = kXcdMaxH / 64;  // 64-column weight fragments of a wavefront's 16 gate rows
+
+// The lanes of the operands (checked on the hardware): lane l of A holds, of row l & 15, the eight present columns among columns
+// 16 (l >> 4) .. + 15; lane l of B holds, of column l & 15, rows 8 (l >> 4) .. + 7 and 32 + 8 (l >> 4) .. + 7.  Which columns of
+// the weight matrix the 64 are is free as long as both operands agree.  A lane of B takes two whole 16-byte pieces of its gate
+// row, 8 m + (l >> 4) and four pieces further; halves 0..3 of a piece then meet the even row of A, halves 4..7 the odd one.
+
+// Lane l's eight values of h in register set s of A: two 8-byte halves of neighbouring pieces.
+__device__ __forceinline__ half8_t xcd_h_operand(const half_t* hb, int s, int lane)
 {
-    const bool b3 = lane & 8, b2 = lane & 4;
-    float v2[2];
+    const half_t* src = hb + (8 * (8 * s + ((lane & 15) >> 1)) + 2 * (lane >> 4)) * 8 + 4 * (lane & 1);
+    return __builtin_shufflevector(*reinterpret_cast<const half4_t*>(src), *reinterpret_cast<const half4_t*>(src + 8), 0, 1, 2, 3, 4, 5, 6, 7);
+}
+
+// Fragment m of the gate row that starts at `row` (lane l's column l & 15 of B).
+__device__ __forceinline__ half16_t xcd_weight_fragment(const half_t* row, int m, int lane, int H, bool ok)
+{
+    half8_t lo, hi;
 #pragma unroll
-    for (int r = 0; r < 2; ++r) v2[r] = (b3 ? acc[2 + r] : acc[r]) + dpp_mov_f32<kDppRowMirror>(b3 ? acc[r] : acc[2 + r]);
-    float v = (b2 ? v2[1] : v2[0]) + dpp_mov_f32<kDppRowHalfMirror>(b2 ? v2[0] : v2[1]);
-    v += dpp_mov_f32<kDppQuadXor1>(v);
-    v += dpp_mov_f32<kDppQuadXor2>(v);
-    return v;
+    for (int e = 0; e < 8; ++e) lo[e] = hi[e] = (half_t)0.0f;
+    const int c0 = (8 * m + (lane >> 4)) * 8, c1 = c0 + 32;
+    if (ok && c0 < H) lo = *reinterpret_cast<const half8_t*>(row + c0);  // H % 8 == 0: a piece is entirely in or out of range
+    if (ok && c1 < H) hi = *reinterpret_cast<const half8_t*>(row + c1);
+    return __builtin_shufflevector(lo, hi, 0, 1, 4, 5, 2, 3, 6, 7, 8, 9, 12, 13, 10, 11, 14, 15);
+}
+
+// The accumulators of a step, cleared where the wavefront has nothing else to do (in front of its wait for h).
+struct XcdSums {
+    float4_t d[8];
+    __device__ __forceinline__ void clear()
+    {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            d[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            asm volatile("" : "+v"(d[j]));
+        }
+    }
+};
+
+// In every lane l: the dot product of gate row l & 15 of the wavefront with hb[0 .. H).
+__device__ __forceinline__ float xcd_matvec(const half16_t (&w)[kXcdFrags], const half_t* hb, XcdSums& acc, int H, int lane)
+{
+    const int index = (lane & 1) ? 0xeeeeeeee : 0x44444444;  // columns 2, 3 / 0, 1 of every four
+    const half8_t h0 = xcd_h_operand(hb, 0, lane), h1 = xcd_h_operand(hb, 1, lane);
+#pragma unroll
+    for (int m = 0; m < kXcdFrags; ++m) {
+        if ((m & 3) == 0 && m * 64 >= H) break;  // (uniform) whole fragments past the hidden state are zeros
+        acc.d[m & 7] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(m < 8 ? h0 : h1, w[m], acc.d[m & 7], index, 0, 0);
+    }
+    // Row r of D lies in register r & 3 of lanes 16 (r >> 2) .. + 15: row group q keeps pairs 2 q (registers 0, 1) and 2 q + 1.
+    float f[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) f[q] = (acc.d[2 * q][0] + acc.d[2 * q][1]) + (acc.d[2 * q + 1][2] + acc.d[2 * q + 1][3]);
+    const float lo = (lane & 16) ? f[1] : f[0], hi = (lane & 16) ? f[3] : f[2];
+    return wave_sum_rows((lane & 32) ? hi : lo);
 }
 
 // PIPE = false: groups that neither feed nor are fed across XCDs (a single layer, the two directions of one); everything
@@ -208,26 +256,19 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     if (tid == 0)
         claimed_before = __hip_atomic_exchange(p.claims + xcd * kXcdMembers + rank, g_base, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-    // ---- weights into registers: gate g (LibTorch order i, f, g, o) of unit u0 + (lane >> 4), column pieces 16 c + (lane & 15)
+    // ---- weights into registers: lane l holds gate l & 3 (LibTorch order i, f, g, o) of unit u0 + ((l >> 2) & 3)
     const int u0 = rank * kXcdUnitsPerBlock + wave * kXcdUnitsPerWave;
     const bool units_ok = u0 < H;  // H % 8 == 0: the four units of a wavefront are all inside or all outside
-    const int cl = lane & 15;
+    const int my_unit = u0 + ((lane >> 2) & 3);
+    const int my_gate = lane & 3;
     const half_t* wsrc = is_proj ? pj.w_ih : ch.w_hh;
-    half8_t w[4][8];
+    half16_t w[kXcdFrags];
     {
         half8_t zero;
 #pragma unroll
         for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                const int col = (16 * c + cl) * 8;
-                const bool ok = units_ok && col < H;
-                const long off = ((long)g * H + (u0 + (lane >> 4))) * H + col;
-                w[g][c] = ok ? *reinterpret_cast<const half8_t*>(wsrc + off) : zero;
-            }
-        }
+        for (int m = 0; m < kXcdFrags; ++m) w[m] = xcd_weight_fragment(wsrc + ((long)my_gate * H + my_unit) * H, m, lane, H, units_ok);
         for (int i = tid; i < 2 * kXcdMaxH / 8; i += kXcdThreads) reinterpret_cast<half8_t*>(&hbuf[0][0])[i] = zero;
     }
     if (tid == 0 && claimed_before == g_base) {
@@ -238,9 +279,6 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     }
     __syncthreads();
 
-    // After the reduction lane l holds gate (l >> 2) & 3 of unit l >> 4.
-    const int my_unit = u0 + (lane >> 4);
-    const int my_gate = (lane >> 2) & 3;
     const int uc = units_ok ? my_unit : H - 1;
     // Lanes 0..31 of wavefronts 0..3 fetch piece 32 w + lane of an h vector: 8 fp16 = columns 8 q .. 8 q + 7.  (The other
     // wavefronts never poll: they are the ones that talk to other XCDs, and a wavefront's loads come back in order.)
@@ -288,6 +326,8 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         }
         for (int t = 0; t < T; ++t) {
             half_t* hb = hbuf[t & 1];
+            XcdSums acc;
+            acc.clear();
             if (polls) {
                 const unsigned long long* src = reinterpret_cast<const unsigned long long*>(pj.seq_in + (long)t * H + piece * 8);
                 if (!(filled16(lo) && filled16(hi))) {
@@ -309,17 +349,9 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
                 lo = __hip_atomic_load(nxt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 hi = __hip_atomic_load(nxt + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                if (c * 128 >= H) break;
-                const half8_t hv = *reinterpret_cast<const half8_t*>(hb + (16 * c + cl) * 8);
-#pragma unroll
-                for (int g = 0; g < 4; ++g) acc[g] = dot8(w[g][c], hv, acc[g]);
-            }
-            const float v = row16_transpose_sum4(acc, lane) + bias;
+            const float v = xcd_matvec(w, hb, acc, H, lane) + bias;
             if (dead) return;  // rows made from a stale h must not reach the recurrence: it will make its own
-            if (units_ok && (lane & 3) == 0)
+            if (units_ok && lane < 16)
                 __hip_atomic_store(reinterpret_cast<unsigned int*>(dst + (long)t * 4 * H), __builtin_bit_cast(unsigned int, v), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -387,7 +419,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     const unsigned int* xp_mine = reinterpret_cast<const unsigned int*>(ch.xproj + (long)my_gate * H + uc);  // + t * 4H
     const bool fetcher = wave >= 4;
     const unsigned int* xp_other =
-        reinterpret_cast<const unsigned int*>(ch.xproj + (long)my_gate * H + min(max(u0 - 16, 0) + (lane >> 4), H - 1));  // wavefront w - 4's
+        reinterpret_cast<const unsigned int*>(ch.xproj + (long)my_gate * H + min(max(u0 - 16, 0) + ((lane >> 2) & 3), H - 1));  // wavefront w - 4's
     auto xp_bits_at = [&](int t) { return __hip_atomic_load(xp_mine + (long)t * 4 * H, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     auto wait_xp = [&](int t) {
         unsigned int bits = 0xffffffffu;
@@ -405,12 +437,14 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     } else {
         // Let the P group get kXcdLag steps ahead, then take the first two rows.
         (void)wait_xp(min(kXcdLag, T - 1));
-        reinterpret_cast<unsigned int&>(xring[wave][0][my_gate][lane >> 4]) = wait_xp(0);
-        reinterpret_cast<unsigned int&>(xring[wave][1][my_gate][lane >> 4]) = wait_xp(min(1, T - 1));
+        reinterpret_cast<unsigned int&>(xring[wave][0][my_gate][(lane >> 2) & 3]) = wait_xp(0);
+        reinterpret_cast<unsigned int&>(xring[wave][1][my_gate][(lane >> 2) & 3]) = wait_xp(min(1, T - 1));
     }
 
     for (int s = 0; s < T; ++s) {
         half_t* hb = hbuf[s & 1];
+        XcdSums acc;
+        acc.clear();
         if (!polled) {
             // steps s + 16 .. s + 31 are fetched when step s starts a half, and written over the half that has just been
             // used up one step later (this wavefront's poll in between has waited for them)
@@ -418,8 +452,8 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             if ((s & 15) == 1 && s > 1) deposit_xp(((s >> 4) & 1) ^ 1, xp_next);
         } else if (fetcher && s >= 1 && s + 1 < T) {
             // loaded during step s - 1; read (by this wavefront and by wavefront w - 4) after the barrier of step s + 1
-            reinterpret_cast<unsigned int&>(xring[wave][(s + 1) & 31][my_gate][lane >> 4]) = xp_ahead;
-            reinterpret_cast<unsigned int&>(xring[wave - 4][(s + 1) & 31][my_gate][lane >> 4]) = xp_ahead_other;
+            reinterpret_cast<unsigned int&>(xring[wave][(s + 1) & 31][my_gate][(lane >> 2) & 3]) = xp_ahead;
+            reinterpret_cast<unsigned int&>(xring[wave - 4][(s + 1) & 31][my_gate][(lane >> 2) & 3]) = xp_ahead_other;
         }
         if (sums && s > 0) in_ring[(s - 1) & 1][lane & 31] = in_ahead;  // read after this step's barrier
         // ---- 1. h of the previous step into LDS
@@ -462,54 +496,33 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             if (s > 0 && !dead) emit_sum(s - 1);
         }
 
-        // ---- 2. the four gate rows of this row of lanes' unit
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            if (c * 128 >= H) break;  // (uniform) column pieces 16 c .. 16 c + 15 lie past the hidden state
-            const half8_t hv = *reinterpret_cast<const half8_t*>(hb + (16 * c + cl) * 8);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) acc[g] = dot8(w[g][c], hv, acc[g]);
-        }
-        unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][lane >> 4]);
+        // ---- 2. the wavefront's 16 gate rows
+        const float dot = xcd_matvec(w, hb, acc, H, lane);
+        unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][(lane >> 2) & 3]);
         if (polled && xp_bits == 0xffffffffu) xp_bits = wait_xp(s);  // the P group had not got there when it was fetched
-        const float a = row16_transpose_sum4(acc, lane) + __builtin_bit_cast(float, xp_bits);
+        const float a = dot + __builtin_bit_cast(float, xp_bits);
         const int t = rev ? (T - 1 - s) : s;
 
-        // Every lane activates its own gate; a lane of gate 0 then finds gate f in its mirror within half the row (l ^ 7),
-        // gate o in its mirror within the row (l ^ 15) and gate g in the mirror of that one (l ^ 8).  (The other lanes
-        // combine the gates in another order; their c and h are never used.)
+        // Every lane activates its own gate; the quad's four lanes (one unit) then share them and all make the unit's c and h.
         const bool is_g = my_gate == 2;
         const float sg = fast_sigmoid_f32(is_g ? 2.0f * a : a);
         const float act = is_g ? 2.0f * sg - 1.0f : sg;
-        const float g_i = act;
-        const float g_f = dpp_mov_f32<kDppRowHalfMirror>(act);
-        const float g_o = dpp_mov_f32<kDppRowMirror>(act);
-        const float g_g = dpp_mov_f32<kDppRowMirror>(g_f);
+        const float g_i = dpp_mov_f32<0x00>(act);  // quad_perm broadcasts of lanes 0, 1, 2, 3 of the quad
+        const float g_f = dpp_mov_f32<0x55>(act);
+        const float g_g = dpp_mov_f32<0xAA>(act);
+        const float g_o = dpp_mov_f32<0xFF>(act);
         const float c_new = g_f * c_reg + g_i * g_g;
         const bool h_is_number = (c_new == c_new) && (g_o == g_o);
         const half_t h = (half_t)(g_o * (2.0f * fast_sigmoid_f32(2.0f * c_new) - 1.0f));
         c_reg = c_new;
 
-        // ---- 3. the wavefront's four h values: lanes 0, 16, 32, 48 hold them; lane 0 stores y and publishes
+        // ---- 3. the wavefront's four h values: a quad each; lane 0 stores y and publishes
         const unsigned int hb16 = (unsigned int)__builtin_bit_cast(unsigned short, h);
         const unsigned int pb16 = h_is_number ? hb16 : 0u;       // a NaN cannot carry the flag: it is exchanged as 0, y keeps it
         const unsigned int sb16 = h_is_number ? hb16 : 0x7e00u;  // and goes to the layer above in its canonical form
-        unsigned long long yw = 0ull, pw = 0ull, sw = 0ull;
-        if constexpr (PIPE || RES) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                yw |= (unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)hb16, 16 * i) << (16 * i);
-                pw |= (unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)pb16, 16 * i) << (16 * i);
-                if (emits) sw |= (unsigned long long)(unsigned int)__builtin_amdgcn_readlane((int)sb16, 16 * i) << (16 * i);
-            }
-        } else {
-            // Independent recurrences (a single layer, the two directions of a layer): gathered into lane 0 with two row swaps
-            // each, 3 % of a step faster than eight v_readlane and the scalar shifts behind them.  (The kernel that runs
-            // pipelines of layers keeps the scalar path: there the same change cost 1.5-5 %.)
-            pw = pack_row_heads(pb16);
-            yw = pack_row_heads(hb16);
-        }
+        const unsigned long long pw = pack_quads(pb16);
+        const unsigned long long yw = pack_quads(hb16);
+        const unsigned long long sw = emits ? pack_quads(sb16) : 0ull;
         // (a wavefront one of whose waits gave up after this step's barrier has made its h from stale values: it keeps them
         // to itself, and the group's other members stop at their next wait)
         const bool wave_gave_up = __builtin_amdgcn_ballot_w64(gave_up) != 0ull;
@@ -522,7 +535,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             if (!res && units_ok && ch.y) *reinterpret_cast<unsigned long long*>(ch.y + (long)t * p.y_stride + u0) = yw;
             if (emits) hout[s & 1][wave] = sw;
         }
-        if (s == T - 1 && units_ok && (lane & 15) == 0) {
+        if (s == T - 1 && units_ok && lane < 16 && (lane & 3) == 0) {
             ch.hn[my_unit] = h;
             ch.cn[my_unit] = (half_t)c_new;
         }
