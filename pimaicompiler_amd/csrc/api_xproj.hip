@@ -7,6 +7,49 @@ using namespace pimhip;
 
 namespace pimhip
 {
+namespace
+{
+int tiles_of(int64_t T, int64_t N, int rows) { return (int)((T + rows - 1) / rows * ((N + kXprojTileCols - 1) / kXprojTileCols)); }
+
+// The row tiles per wavefront (MT) of the kernel for many time steps, or 0: the split-K kernels.  Measured on MI355X over T = 50 ..
+// 2048, K = 240 .. 2048, N = 1024 .. 4096 (us, split-K kernel / 64-row / 128-row tiles, plain weights):
+//   64-row tiles in all   128 (T 200, K 1024, N 4096) 9.7 / 8.7 / -    130 (800, 1024, 1280) 10.6 / 9.2 / 12.4   104 (800, 512, 1024) 6.5 / 7.1 / 8.7
+//                         192 (341, 1024, 4096) 12.5 / 9.8 / 13.2      416 (800, 1024, 4096) 24.6 / 17.7 / 14.5  1024 (2048, 1024, 4096) 56 / 37 / 29
+// A block fills a CU, so what counts is how many tiles the busiest CU runs one after another, a 128-row tile taking 1.5 times as
+// long as a 64-row one.  From half as many 64-row tiles as CUs on they win; against packed weights, whose split-K kernel moves
+// half the LDS bytes, from five eighths (128: 8.3 / 8.7, 192: 10.7 / 9.6).
+int tile_rows(int64_t T, int64_t N, int count, bool packed)
+{
+    constexpr int kCus = 256;
+    if ((double)T * (double)N > 1e12) return 0;  // (counts below stay within an int)
+    const int t64 = count * tiles_of(T, N, 64), t128 = count * tiles_of(T, N, 128);
+    if (t64 < (packed ? kCus * 5 / 8 : kCus / 2)) return 0;
+    const int r64 = (t64 + kCus - 1) / kCus, r128 = (t128 + kCus - 1) / kCus;
+    return 2 * r64 <= 3 * r128 ? 2 : 4;
+}
+
+template <bool PACKED>
+void launch_tiles(int mt, int count, float* const* out, const half_t* x, const half_t* const* w, const float* const* bias, int64_t T, int64_t K,
+                  int64_t N, int64_t ldx, int64_t ldw, int ksteps, XprojFill& fill, hipStream_t s)
+{
+    XprojTileProblems pr;
+    memset(&pr, 0, sizeof(pr));
+    for (int p = 0; p < count; ++p) {
+        pr.w[p] = w[p];
+        pr.bias[p] = bias[p];
+        pr.out[p] = out[p];
+    }
+    const unsigned row_blocks = (unsigned)((T + 32 * mt - 1) / (32 * mt));
+    pr.blocks_per_problem = (tiles_of(T, N, 32 * mt) + 7) / 8 * 8;
+    fill.first_block = pr.blocks_per_problem * count;
+    const unsigned grid = (unsigned)fill.first_block + (unsigned)(fill.count > 0 ? fill.blocks : 0);
+    if (mt == 4)
+        input_projection_tile_f16_kernel<PACKED, 4><<<grid, 512, 0, s>>>(x, pr, (int)T, (int)K, (int)N, (long)ldx, (long)ldw, ksteps, (int)row_blocks, fill);
+    else
+        input_projection_tile_f16_kernel<PACKED, 2><<<grid, 512, 0, s>>>(x, pr, (int)T, (int)K, (int)N, (long)ldx, (long)ldw, ksteps, (int)row_blocks, fill);
+}
+}  // namespace
+
 int launch_input_projection(int count, float* const* out, const half_t* x, const half_t* const* w, const float* const* bias,
                             int64_t T, int64_t K, int64_t N, hipStream_t s, int64_t ldx, int64_t ldw)
 {
@@ -24,6 +67,14 @@ int launch_input_projection(int count, float* const* out, const half_t* x, const
         pr.w[p] = w[p];
         pr.bias[p] = bias[p];
         pr.out[p] = out[p];
+    }
+    if (const int mt = tile_rows(T, N, count, false)) {
+        XprojFill none;  // (count 0: no blocks that fill)
+        memset(&none, 0, sizeof(none));
+        launch_tiles<false>(mt, count, out, x, w, bias, T, K, N, ldx, ldw, 0, none, s);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(PIMHIP_ERR_HIP, "input projection launch failed: %s", hipGetErrorString(e));
+        return PIMHIP_OK;
     }
     // 64 time steps per block row.  Measured on MI355X for T = 50, 200, 800 and K = 240, 1024, 2048 (N = 4096): 32-column
     // tiles are fastest as soon as there are two row blocks, 16-column tiles with one (more blocks than CUs either way).
@@ -63,6 +114,12 @@ int launch_input_projection_packed(int count, float* const* out, const half_t* x
         }
         fill.count = n_ones;
         fill.blocks = 128;
+    }
+    if (const int mt = tile_rows(T, N, count, true)) {
+        launch_tiles<true>(mt, count, out, x, wp, bias, T, K, N, K, 0, ksteps, fill, s);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return fail(PIMHIP_ERR_HIP, "input projection launch failed: %s", hipGetErrorString(e));
+        return PIMHIP_OK;
     }
     XprojPackedProblems pr;
     memset(&pr, 0, sizeof(pr));

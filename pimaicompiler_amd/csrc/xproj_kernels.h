@@ -352,6 +352,234 @@ __global__ __launch_bounds__(64 * KS) void input_projection_packed_f16_kernel(co
     }
 }
 
+// ---------------------------------------------------------------------------------------------
+// Many time steps.  The kernels above split K over the wavefronts of a 64 x 32 tile: 12 KB pass through LDS (6 KB PACKED), written
+// and read, for 16 matrix instructions, and a load has one slab of time to arrive; they level off at 13 % of the matrix cores' rate.  Here a block of
+// eight wavefronts owns BM = 32 * MT time steps x 128 columns, a wavefront 16 * MT x 64 of them over half of a slab's 64 columns (two
+// wavefronts per SIMD, and a chain of sums half as long): 4 + MT fragments read for 4 * MT matrix instructions.
+//   - Loads go from memory straight into LDS, four slabs deep, and are counted, not drained (vmcnt): a slab has the time of two
+//     others to arrive.  Staged through registers one slab ahead (two blocks per CU) a slab took 1.0 us, this way 0.53.
+//   - The fragments of the next slab are read while this one is multiplied: 0.43 us.  What is left is LDS (64 KB read and 32 KB
+//     written per slab and CU) and the 0.21 us of matrix instructions taking turns within a barrier's reach.
+//   - An LDS row is 128 bytes, its 16-byte piece c in place c ^ (row & 7), so that eight rows of one piece fall on all banks.  The
+//     weights are the first operand: a lane's four results are neighbours in a row of out (one 16-byte store).
+//   - PACKED: the weights' fragments (pack_w_fragments_kernel) pass through LDS as they are; the same products in the same order.
+//   - Two slabs' products are one chain of sums in the matrix cores and are then added to the total on the vector units: as far
+//     from the exact sum as the kernels above at 64 columns, closer from there on (relative 6.6e-8 against 8.4e-8 at 1024).
+// 800 x 1024 -> 4096, MI355X: 24.6 -> 14.5 us (packed 19.4 -> 14.4), 2048 x 1024 -> 4096 56.2 -> 29.2 (305 -> 590 TFLOP/s).
+// ---------------------------------------------------------------------------------------------
+static constexpr int kXprojTileCols = 128;
+static constexpr int kXprojTileSlab = 64;
+static constexpr int kXprojTileBufs = 4;
+
+struct XprojTileProblems {
+    const half_t* w[2];  // PACKED: in fragment order
+    const float* bias[2];
+    float* out[2];
+    int blocks_per_problem;
+};
+
+// 16 bytes per lane from memory straight into LDS: lane l's at `lds_base` + 16 l (lds_base: the same in all lanes).  Counted by
+// vmcnt; nothing but an explicit wait orders it.
+__device__ __forceinline__ void load_lds16(const half_t* src, unsigned int lds_base)
+{
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_base), "v"(src) : "memory");
+}
+
+template <int N>
+__device__ __forceinline__ void wait_loads_and_barrier()
+{
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
+}
+
+template <bool PACKED, int MT>
+__global__ __launch_bounds__(512) void input_projection_tile_f16_kernel(const half_t* __restrict__ x, XprojTileProblems problems, int T, int K,
+                                                                        int N, long ldx, long ldw, int ksteps, int row_blocks, XprojFill fill)
+{
+    if (fill.count > 0 && (int)blockIdx.x >= fill.first_block) {
+        xproj_fill_ones(fill, (int)blockIdx.x - fill.first_block, 512);
+        return;
+    }
+    typedef float float4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+    constexpr int BM = 32 * MT;
+    constexpr int XP = BM / 64;                   // 16-byte pieces of x per lane and slab
+    constexpr int WP = kXprojTileCols / 64;       // of w
+    constexpr int PER_SLAB = XP + WP;
+    constexpr int W_AT = BM * kXprojTileSlab;     // halves: x rows first, then w
+    constexpr int SLAB_HALVES = (BM + kXprojTileCols) * kXprojTileSlab;
+    constexpr int LDS_HALVES = kXprojTileBufs * SLAB_HALVES;
+    static_assert(LDS_HALVES * 2 >= 8 * (MT / 2) * 4 * 64 * 16, "the partial tiles of the K halves pass through the same memory");
+    __shared__ __align__(16) half_t lds[LDS_HALVES];
+
+    const int problem = blockIdx.x >= (unsigned)problems.blocks_per_problem ? 1 : 0;
+    const int block = blockIdx.x - problem * problems.blocks_per_problem;
+    const half_t* __restrict__ w = problems.w[problem];
+    const float* __restrict__ bias = problems.bias[problem];
+    float* __restrict__ out = problems.out[problem];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave & 1, wn = (wave >> 1) & 1, ks = wave >> 2;
+    const int r16 = lane & 15;
+    const int kq = lane >> 4;
+    // Workgroups go to the eight XCDs round-robin by linear id.  All row blocks of a column tile belong to one XCD, whose L2 then
+    // holds the weights of few column tiles: every eighth column tile where that divides them evenly (the XCDs then write
+    // neighbouring pieces of out's rows at the same time: 29 against 33 us at 2048 x 1024 -> 4096), else one contiguous eighth of
+    // the tiles counted down the columns, so that no XCD has more tiles than the others (1300 x 1024 -> 1280: 13.7 -> 9.9 us).
+    const int col_tiles = (N + kXprojTileCols - 1) / kXprojTileCols;
+    const int xcd = block & 7, local = block >> 3;
+    const int tile = (col_tiles & 7) == 0 ? (local / row_blocks * 8 + xcd) * row_blocks + local % row_blocks
+                                          : xcd * (problems.blocks_per_problem >> 3) + local;
+    if (tile >= row_blocks * col_tiles) return;  // whole block, before any barrier
+    const int n_base = tile / row_blocks * kXprojTileCols;
+    const int t_base = tile % row_blocks * BM;
+
+    // Loads: instruction i of this wavefront brings rows 64 i + 8 wave .. + 7 of the slab, lane l piece (l & 7) ^ (row & 7) of row
+    // 8 wave + (l >> 3).  Rows past T or N duplicate the last one; their results are never stored.
+    const int lrow = 8 * wave + (lane >> 3);
+    const int kpiece = ((lane & 7) ^ (lrow & 7)) * 8;
+    const half_t* src[PER_SLAB];
+#pragma unroll
+    for (int i = 0; i < XP; ++i) src[i] = x + (long)min(t_base + lrow + 64 * i, T - 1) * ldx;
+#pragma unroll
+    for (int i = 0; i < WP; ++i) {
+        if constexpr (PACKED) {  // one fragment (16 rows, 32 columns) per instruction: fragment 8 i + wave of the slab's sixteen, [tile][step]
+            const int ntiles = (N + 63) / 64 * 4;
+            const int f = 8 * i + wave;
+            src[XP + i] = w + (((long)min(n_base / 16 + (f >> 1), ntiles - 1) * ksteps + (f & 1)) * 64 + lane) * 8;
+        } else {
+            src[XP + i] = w + (long)min(n_base + lrow + 64 * i, N - 1) * ldw;
+        }
+    }
+    const int slabs = (K + kXprojTileSlab - 1) / kXprojTileSlab;
+    const unsigned int lds0 = (unsigned int)(size_t)(__attribute__((address_space(3))) half_t*)lds;
+    auto fetch = [&](int slab) __attribute__((always_inline)) {
+        const unsigned int base = lds0 + (unsigned int)((slab % kXprojTileBufs) * SLAB_HALVES * 2) + (unsigned int)wave * 1024u;
+        const int k = slab * kXprojTileSlab + kpiece;
+        const int kc = k < K ? k : 0;  // (what lies past K is replaced by zeros when it is read; slabs past the last one are never read)
+        const int wslab = min(slab, slabs - 1);
+#pragma unroll
+        for (int i = 0; i < XP; ++i) load_lds16(src[i] + kc, base + (unsigned int)(i * 8192));
+#pragma unroll
+        for (int i = 0; i < WP; ++i) load_lds16(src[XP + i] + (PACKED ? (long)wslab * 1024 : (long)kc), base + (unsigned int)(W_AT * 2 + i * 8192));
+    };
+
+    float4_t total[MT][4], part[MT][4];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) total[m][n] = part[m][n] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    half8_t zero;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
+
+    // The fragments of slab s + 1 are read while slab s is multiplied (reads and matrix instructions behind one barrier, all
+    // wavefronts in step, would take turns).
+    half8_t a[2][MT], b[2][4];
+    auto read = [&](int s, int set) __attribute__((always_inline)) {
+        const half_t* base = lds + (s % kXprojTileBufs) * SLAB_HALVES;
+        const int place = ((ks * 4 + kq) ^ (r16 & 7)) * 8;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) a[set][m] = *reinterpret_cast<const half8_t*>(base + ((wm * MT + m) * 16 + r16) * kXprojTileSlab + place);
+#pragma unroll
+        for (int n = 0; n < 4; ++n)
+            b[set][n] = *reinterpret_cast<const half8_t*>(base + W_AT + (PACKED ? ((wn * 4 + n) * 2 + ks) * 512 + lane * 8
+                                                                               : ((wn * 4 + n) * 16 + r16) * kXprojTileSlab + place));
+    };
+    auto mask = [&](int s, int set) __attribute__((always_inline)) {  // K % 8 == 0: a piece is entirely in or out of range
+        const bool ok = s * kXprojTileSlab + (ks * 4 + kq) * 8 < K;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) a[set][m] = ok ? a[set][m] : zero;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) b[set][n] = ok ? b[set][n] : zero;
+    };
+    auto multiply = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) part[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[set][n], a[set][m], part[m][n], 0, 0, 0);
+    };
+#pragma unroll
+    for (int s = 0; s < kXprojTileBufs - 1; ++s) fetch(s);
+    wait_loads_and_barrier<(kXprojTileBufs - 2) * PER_SLAB>();
+    fetch(kXprojTileBufs - 1);
+    read(0, 0);
+    auto add_up = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                total[m][n] += part[m][n];
+                part[m][n] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+            }
+    };
+    auto advance = [&](int s) __attribute__((always_inline)) {  // slab s is there; everybody has read slab s - 1
+        wait_loads_and_barrier<(kXprojTileBufs - 2) * PER_SLAB>();
+        fetch(s + kXprojTileBufs - 1);
+    };
+    int s = 0;
+    for (; s + 2 < slabs; s += 2) {  // (no condition inside: a wait would be sized for the path with the fewest reads in flight)
+        advance(s + 1);
+        read(s + 1, 1);
+        multiply(0);
+        advance(s + 2);
+        read(s + 2, 0);
+        multiply(1);
+        add_up();
+    }
+    const bool ragged = slabs * kXprojTileSlab != K;
+    if (s + 1 < slabs) {
+        advance(s + 1);
+        read(s + 1, 1);
+        multiply(0);
+        if (ragged) mask(s + 1, 1);
+        multiply(1);
+    } else {
+        if (ragged) mask(s, 0);
+        multiply(0);
+    }
+    add_up();
+
+    // The two K halves of a tile: each wavefront hands the other half of its row tiles over and finishes its own.
+    wait_loads_and_barrier<0>();
+    float4_t* red = reinterpret_cast<float4_t*>(lds);  // [wave][MT / 2][4][64]
+#pragma unroll
+    for (int m = 0; m < MT / 2; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) red[((wave * (MT / 2) + m) * 4 + n) * 64 + lane] = ks ? total[m][n] : total[m + MT / 2][n];
+    __syncthreads();
+
+    // Lane (r16, kq) holds columns 4 kq .. + 3 of time step r16 of every 16 x 16 tile.
+    const bool whole = n_base + kXprojTileCols <= N;
+    float4_t bv[4];
+#pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        const int col = n_base + (wn * 4 + n) * 16 + kq * 4;
+        bv[n] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        if (bias && whole) bv[n] = *reinterpret_cast<const float4_any_t*>(bias + col);
+        else if (bias) bv[n] = float4_t{bias[min(col, N - 1)], bias[min(col + 1, N - 1)], bias[min(col + 2, N - 1)], bias[min(col + 3, N - 1)]};
+    }
+#pragma unroll
+    for (int m = 0; m < MT / 2; ++m) {
+        const int t = t_base + (wm * MT + ks * (MT / 2) + m) * 16 + r16;
+        float* o = out + (long)t * N + n_base + wn * 64 + kq * 4;
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const float4_t mine = ks ? total[m + MT / 2][n] : total[m][n];
+            const float4_t v = (mine + red[(((wave ^ 4) * (MT / 2) + m) * 4 + n) * 64 + lane]) + bv[n];
+            if (t >= T) continue;
+            if (whole) {
+                *reinterpret_cast<float4_any_t*>(o + n * 16) = v;
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n_base + (wn * 4 + n) * 16 + kq * 4 + i < N) o[n * 16 + i] = v[i];
+            }
+        }
+    }
+}
+
 // bsum[i] = b_ih[i] + b_hh[i] in fp32 (either may be null, meaning zero).
 __global__ void lstm_bias_sum_kernel(const half_t* __restrict__ b_ih, const half_t* __restrict__ b_hh,
                                      float* __restrict__ bsum, int n)

@@ -620,3 +620,30 @@ def test_input_projection_matches_fp32_matmul(ops, T, K, N):
     got = ops.input_projection_packed(x.to(DEV), packed, N, b.to(DEV))
     assert maxabs(got, want) <= 1e-4 * max(1.0, float(want.abs().max()))
     assert torch.equal(got, ops.input_projection_packed(x.to(DEV), packed, N, b.to(DEV)))
+
+
+# The projection's kernel for many time steps: 64- and 128-row tiles, ragged in every dimension; K of one, two and an odd number of
+# 64-column slabs, with and without a ragged end.
+@pytest.mark.parametrize("T,K,N", [(700, 8, 1500), (641, 64, 1541), (641, 72, 1537), (2049, 128, 601), (900, 200, 2050), (1100, 320, 2304),
+                                   (1601, 1032, 4097)])
+def test_input_projection_of_many_steps(ops, T, K, N):
+    g = torch.Generator().manual_seed(T + K + N)
+    x = torch.randn(T, K, generator=g).half()
+    w = (torch.randn(N, K, generator=g) / math.sqrt(K)).half()
+    b = torch.randn(N, generator=g)
+    want = x.double() @ w.double().t()
+    # every partial sum is below sum |x w|, and at most K / 32 + K / 128 + 8 of them are rounded, one ulp each at most
+    bound = (x.double().abs() @ w.double().abs().t() + b.double().abs()) * (K / 32 + K / 128 + 8) * 2.0 ** -23
+    xd, wd, bd = x.to(DEV), w.to(DEV), b.to(DEV)
+    packed = ops.pack_projection_weight(wd)
+    out = ops.input_projection(xd, wd, bd)
+    for got, bias in ((out, b), (ops.input_projection(xd, wd), None), (ops.input_projection_packed(xd, packed, N, bd), b),
+                      (ops.input_projection_packed(xd, packed, N), None)):
+        err = (got.cpu().double() - (want if bias is None else want + bias.double())).abs()
+        assert bool((err <= bound).all()), float((err / bound).max())
+    # an infinity reaches its own row only: what stands in for rows and columns past the end is multiplied by nothing
+    xi = xd.clone()
+    xi[T - 1, 0] = float("inf")
+    got = ops.input_projection(xi, wd, bd)
+    assert torch.equal(got[: T - 1], out[: T - 1]) and not bool(torch.isfinite(got[T - 1][wd[:, 0] != 0]).any())
+    assert torch.equal(got[: T - 1], ops.input_projection_packed(xi, packed, N, bd)[: T - 1]) == torch.equal(out, ops.input_projection_packed(xd, packed, N, bd))
