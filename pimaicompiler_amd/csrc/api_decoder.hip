@@ -215,16 +215,17 @@ extern "C" int pimhip_decoder_plan_set_encoder(PimHipDecoderPlan* plan, const vo
         PIMHIP_HIP_CHECK(hipMalloc(&plan->cx_proj, sizeof(float) * (size_t)L * cap * 4 * H));
         plan->enc_cap = cap;
     }
+    // out[4H, S] = W_ih[:, H:2H] (4H rows of pitch 2H) . enc[S, H]^T: a gate row's S values are contiguous for the step kernel
+    float* outs[kDecMaxLayers];
+    const half_t* ws[kDecMaxLayers];
+    int count = 0;
     for (int l = 0; l < L; ++l) {
         if (!(l > 0 || plan->first_takes_context)) continue;
-        // out[4H, S] = W_ih[:, H:2H] (4H rows of pitch 2H) . enc[S, H]^T: the kernel's "x" is the weight, its "w" the encoder
-        // outputs, so that a gate row's S values are contiguous for the step kernel
-        float* out = plan->cx_proj + (size_t)l * plan->enc_cap * 4 * H;
-        const half_t* w = (const half_t*)enc;
-        const float* no_bias = nullptr;
-        rc = launch_input_projection(1, &out, plan->w_ih[l] + H, &w, &no_bias, 4 * H, H, enc_len, s, 2 * H, H);
-        if (rc != PIMHIP_OK) return rc;
+        outs[count] = plan->cx_proj + (size_t)l * plan->enc_cap * 4 * H;
+        ws[count++] = plan->w_ih[l] + H;
     }
+    rc = launch_context_projection(count, outs, ws, (const half_t*)enc, 4 * H, H, enc_len, 2 * H, s);
+    if (rc != PIMHIP_OK) return rc;
     plan->enc = (const half_t*)enc;
     plan->enc_len = enc_len;
     return PIMHIP_OK;

@@ -366,7 +366,7 @@ __global__ __launch_bounds__(64 * KS) void input_projection_packed_f16_kernel(co
 //   - PACKED: the weights' fragments (pack_w_fragments_kernel) pass through LDS as they are; the same products in the same order.
 //   - Two slabs' products are one chain of sums in the matrix cores and are then added to the total on the vector units: as far
 //     from the exact sum as the kernels above at 64 columns, closer from there on (relative 6.6e-8 against 8.4e-8 at 1024).
-// 800 x 1024 -> 4096, MI355X: 24.6 -> 14.5 us (packed 19.4 -> 14.4), 2048 x 1024 -> 4096 56.2 -> 29.2 (305 -> 590 TFLOP/s).
+// 800 x 1024 -> 4096, MI355X: 24.6 -> 14.5 us (packed 19.4 -> 14.4), 2048 x 1024 -> 4096 56.2 -> 32.8 (305 -> 520 TFLOP/s).
 // ---------------------------------------------------------------------------------------------
 static constexpr int kXprojTileCols = 128;
 static constexpr int kXprojTileSlab = 64;
@@ -423,14 +423,11 @@ __global__ __launch_bounds__(512) void input_projection_tile_f16_kernel(const ha
     const int wm = wave & 1, wn = (wave >> 1) & 1, ks = wave >> 2;
     const int r16 = lane & 15;
     const int kq = lane >> 4;
-    // Workgroups go to the eight XCDs round-robin by linear id.  All row blocks of a column tile belong to one XCD, whose L2 then
-    // holds the weights of few column tiles: every eighth column tile where that divides them evenly (the XCDs then write
-    // neighbouring pieces of out's rows at the same time: 29 against 33 us at 2048 x 1024 -> 4096), else one contiguous eighth of
-    // the tiles counted down the columns, so that no XCD has more tiles than the others (1300 x 1024 -> 1280: 13.7 -> 9.9 us).
+    // Workgroups go to the eight XCDs round-robin by linear id; each XCD takes one contiguous eighth of the tiles, counted down the
+    // columns: its L2 holds the weights of few column tiles, and no XCD has more tiles than the others (column tiles dealt whole to
+    // the XCDs: 13.7 against 9.9 us at 1300 x 1024 -> 1280, 19 against 17 at 2048 x 240 -> 4096, the same where eight divides them).
     const int col_tiles = (N + kXprojTileCols - 1) / kXprojTileCols;
-    const int xcd = block & 7, local = block >> 3;
-    const int tile = (col_tiles & 7) == 0 ? (local / row_blocks * 8 + xcd) * row_blocks + local % row_blocks
-                                          : xcd * (problems.blocks_per_problem >> 3) + local;
+    const int tile = (block & 7) * (problems.blocks_per_problem >> 3) + (block >> 3);
     if (tile >= row_blocks * col_tiles) return;  // whole block, before any barrier
     const int n_base = tile / row_blocks * kXprojTileCols;
     const int t_base = tile % row_blocks * BM;
@@ -568,13 +565,94 @@ __global__ __launch_bounds__(512) void input_projection_tile_f16_kernel(const ha
         for (int n = 0; n < 4; ++n) {
             const float4_t mine = ks ? total[m + MT / 2][n] : total[m][n];
             const float4_t v = (mine + red[(((wave ^ 4) * (MT / 2) + m) * 4 + n) * 64 + lane]) + bv[n];
-            if (t >= T) continue;
-            if (whole) {
+            if (whole && t_base + BM <= T) {
                 *reinterpret_cast<float4_any_t*>(o + n * 16) = v;
-            } else {
+            } else if (whole) {
+                if (t < T) *reinterpret_cast<float4_any_t*>(o + n * 16) = v;
+            } else if (t < T) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     if (n_base + (wn * 4 + n) * 16 + kq * 4 + i < N) o[n * 16 + i] = v[i];
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Few columns, many weight rows, several weights at once: out_l[row][s] = sum_k w_l[row][k] . enc[s][k], the context columns of a
+// decoder's layers over the S encoder positions of a sentence.  25 MB of weights against 24 KB of enc: a stream, which the kernel
+// at the top of this file ran on the 64 workgroups its 64 x 32 tiles gave it, one launch per layer (3 x 11 us).  Here a block
+// takes 32 rows of one layer, its four wavefronts a quarter of K each (every fourth 32-wide step); a wavefront asks for all
+// its weights at once, straight in fragment order (16 lanes on 16 rows: slow on one CU, but with every CU at it faster than
+// the memory), keeps them in 64 registers and runs over the columns 16 at a time.  Sums in the order of the kernel at the top.
+// ---------------------------------------------------------------------------------------------
+static constexpr int kCtxRows = 32;                        // weight rows per block
+static constexpr int kCtxMaxK = 1024;
+static constexpr int kCtxSteps = kCtxMaxK / 32 / kXprojKSplit;  // 32-wide steps per wavefront
+static constexpr int kCtxMaxLayers = 4;
+
+struct CtxProjProblems {
+    const half_t* w[kCtxMaxLayers];
+    float* out[kCtxMaxLayers];
+};
+
+__global__ __launch_bounds__(256) void context_projection_f16_kernel(const half_t* __restrict__ enc, int S, int K, int N, long ldw,
+                                                                     CtxProjProblems problems)
+{
+    typedef float float4_any_t __attribute__((ext_vector_type(4), aligned(4)));
+    __shared__ __align__(16) float4_t red[2][kXprojKSplit][kCtxRows / 16][64];
+    const int lane = threadIdx.x & 63;
+    const int ks = threadIdx.x >> 6;
+    const int r16 = lane & 15;
+    const int kq = lane >> 4;
+    const int row0 = blockIdx.x * kCtxRows;
+    const half_t* __restrict__ w = problems.w[blockIdx.y];
+    float* __restrict__ out = problems.out[blockIdx.y];
+
+    half8_t zero;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
+    // K % 8 == 0: a piece is entirely in or out of range; rows past N duplicate the last one and are not stored
+    half8_t wf[kCtxRows / 16][kCtxSteps];
+#pragma unroll
+    for (int i = 0; i < kCtxSteps; ++i) {
+        const int k = (i * kXprojKSplit + ks) * 32 + kq * 8;
+#pragma unroll
+        for (int m = 0; m < kCtxRows / 16; ++m)
+            wf[m][i] = k < K ? *reinterpret_cast<const half8_t*>(w + (long)min(row0 + m * 16 + r16, N - 1) * ldw + k) : zero;
+    }
+    for (int s0 = 0, buf = 0; s0 < S; s0 += 16, buf ^= 1) {
+        const half_t* e = enc + (long)min(s0 + r16, S - 1) * K;
+        half8_t ef[kCtxSteps];
+#pragma unroll
+        for (int i = 0; i < kCtxSteps; ++i) {
+            const int k = (i * kXprojKSplit + ks) * 32 + kq * 8;
+            ef[i] = k < K ? *reinterpret_cast<const half8_t*>(e + k) : zero;
+        }
+        float4_t acc[kCtxRows / 16];
+#pragma unroll
+        for (int m = 0; m < kCtxRows / 16; ++m) {
+            acc[m] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int i = 0; i < kCtxSteps; ++i) acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ef[i], wf[m][i], acc[m], 0, 0, 0);
+            red[buf][ks][m][lane] = acc[m];
+        }
+        __syncthreads();  // (the other buffer was last read in front of the previous barrier)
+        if (ks < kCtxRows / 16) {
+            // lane (r16, kq) holds positions s0 + 4 kq .. + 3 of weight row r16 of the tile
+            float4_t v = red[buf][0][ks][lane];
+#pragma unroll
+            for (int q = 1; q < kXprojKSplit; ++q) v += red[buf][q][ks][lane];
+            const int row = row0 + ks * 16 + r16, s = s0 + kq * 4;
+            if (row < N && s < S) {
+                float* o = out + (long)row * S + s;
+                if (s + 3 < S) {
+                    *reinterpret_cast<float4_any_t*>(o) = v;
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (s + i < S) o[i] = v[i];
+                }
             }
         }
     }

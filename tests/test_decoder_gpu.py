@@ -118,6 +118,15 @@ def test_fused_decoder_step_matches_libtorch_cpu(ops, H, in0, L, first_ctx, firs
     check(case, got, want, ctx_given=True)
 
 
+# The context columns of all layers in one launch: sentences around its tiles of 16 positions and its longest, hidden sizes that are not
+# whole tiles of 32 rows and 128 columns.
+@pytest.mark.parametrize("H,L,first_ctx,src_len", [(40, 2, True, 16), (264, 3, False, 17), (136, 4, True, 33), (1024, 2, False, 160),
+                                                   (264, 2, True, 161)])
+def test_context_columns_of_a_sentence(ops, H, L, first_ctx, src_len):
+    case = Case(77 + H + src_len, H, H, L, first_ctx, 9, 0, src_len)
+    check(case, run_fused(ops, case, case.plan(ops), case.x, case.h, case.c), case.cpu_step(case.x, case.h, case.c))
+
+
 def test_one_plan_serves_sentences_of_different_lengths(ops):
     """set_encoder once per sentence: a long sentence after a short one makes the projection buffer grow, a short one after
     it reuses the larger buffer with another row pitch; every step is checked against the CPU."""
