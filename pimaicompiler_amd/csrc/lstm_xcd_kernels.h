@@ -35,12 +35,13 @@
 // path: P_k looks one step ahead while it multiplies, R_k starts a few steps late and from then on finds its rows
 // waiting.  All groups then advance at the rate of one group, L layers in about the time of one.
 //
-// A workgroup has eight wavefronts; wavefront w owns hidden units 32 * rank + 4 * w .. + 3, one per row of 16 lanes:
-// lane l keeps, of the four gate rows of unit l >> 4, the 8-wide column pieces 16 c + (l & 15), c = 0..7, in 128 registers
-// for the whole sequence.  Per step: lanes 0..15 of every wavefront fetch one 16-byte piece of the group's entries into
-// LDS, one barrier, four dot products of 64 columns per lane, a transposing reduction over the 16 lanes of a row that
-// leaves gate g of the unit in lanes 4 g .. 4 g + 3 of the row, the gate arithmetic in the lanes of gate 0, and one
-// 8-byte store of the wavefront's four new h values into the workgroup's entry.
+// A workgroup has eight wavefronts; wavefront w owns hidden units 32 * rank + 4 * w .. + 3, whose 16 gate rows it keeps in 128
+// registers per lane for the whole sequence, as 16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16.  Per step: the first two
+// wavefronts fetch the group's entries into LDS (16 bytes per lane), one barrier, 16 matrix instructions, which leave the four gates of
+// unit (l >> 2) & 3 in the lanes of that quad, the gate arithmetic, and one 8-byte store of the wavefront's four new h values
+// into the workgroup's entry.  What bounds a step (1.30 us at H = 1024, 1.05 at 320, where nearly all of it is this): the
+// store becoming visible in the L2 and the poll that finds it, 0.43 us at best for such a round; 0.21 us are matrix instructions.
+// The products on v_dot2 with a reduction over 16 lanes: 1.49 us (one layer), 1.57 (pipelines of layers).
 #pragma once
 
 #include <type_traits>
@@ -156,16 +157,40 @@ __device__ __forceinline__ half8_t xcd_h_operand(const half_t* hb, int s, int la
     return __builtin_shufflevector(*reinterpret_cast<const half4_t*>(src), *reinterpret_cast<const half4_t*>(src + 8), 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// Fragment m of the gate row that starts at `row` (lane l's column l & 15 of B).
-__device__ __forceinline__ half16_t xcd_weight_fragment(const half_t* row, int m, int lane, int H, bool ok)
+// A wavefront's fragments.  16 lanes on 16 rows, 64 bytes of each, is what a fragment would ask of memory: 3 us per launch slower
+// than whole 256-byte pieces of rows.  So all loads are issued that way (instruction 4 i + j: rows 4 j .. + 3, columns 128 i .. + 127)
+// and each 16 rows x 128 columns then change lanes through 4 KB of LDS of the wavefront's own, 16-byte piece p of row r in place
+// p ^ r.  Row n: gate n & 3 of unit u0 + (n >> 2).
+__device__ __forceinline__ void xcd_load_weights(half16_t (&w)[kXcdFrags], const half_t* src, half_t* stage, int u0, int lane, int H, bool ok)
 {
-    half8_t lo, hi;
+    half8_t zero;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) lo[e] = hi[e] = (half_t)0.0f;
-    const int c0 = (8 * m + (lane >> 4)) * 8, c1 = c0 + 32;
-    if (ok && c0 < H) lo = *reinterpret_cast<const half8_t*>(row + c0);  // H % 8 == 0: a piece is entirely in or out of range
-    if (ok && c1 < H) hi = *reinterpret_cast<const half8_t*>(row + c1);
-    return __builtin_shufflevector(lo, hi, 0, 1, 4, 5, 2, 3, 6, 7, 8, 9, 12, 13, 10, 11, 14, 15);
+    for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
+    half8_t raw[kXcdFrags / 2][4];
+#pragma unroll
+    for (int i = 0; i < kXcdFrags / 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int n = 4 * j + (lane >> 4), col = 128 * i + 8 * (lane & 15);  // H % 8 == 0: a piece is entirely in or out of range
+            raw[i][j] = (ok && col < H) ? *reinterpret_cast<const half8_t*>(src + ((long)(n & 3) * H + u0 + (n >> 2)) * H + col) : zero;
+        }
+    const int n = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < kXcdFrags / 2; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int r = 4 * j + (lane >> 4);
+            *reinterpret_cast<half8_t*>(stage + r * 128 + ((lane & 15) ^ r) * 8) = raw[i][j];
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (one wavefront's LDS accesses stay in order; this keeps the compiler's too)
+#pragma unroll
+        for (int m = 0; m < 2; ++m) {
+            const half8_t lo = *reinterpret_cast<const half8_t*>(stage + n * 128 + ((8 * m + g) ^ n) * 8);
+            const half8_t hi = *reinterpret_cast<const half8_t*>(stage + n * 128 + ((8 * m + 4 + g) ^ n) * 8);
+            w[2 * i + m] = __builtin_shufflevector(lo, hi, 0, 1, 4, 5, 2, 3, 6, 7, 8, 9, 12, 13, 10, 11, 14, 15);
+        }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
 }
 
 // The accumulators of a step, cleared where the wavefront has nothing else to do (in front of its wait for h).
@@ -211,6 +236,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     __shared__ __align__(16) half_t hbuf[2][kXcdMaxH];  // h of the previous step, double buffered by step parity
     __shared__ __align__(16) float xring[kXcdWaves][32][4][4];  // per wavefront: [step & 31][gate][unit] projection terms
     __shared__ __align__(16) unsigned long long hout[2][kXcdWaves];  // the workgroup's 32 new h values, for the layer above
+    __shared__ __align__(16) half_t wstage[kXcdWaves][16 * 128];     // xcd_load_weights
     __shared__ unsigned short in_ring[2][kXcdUnitsPerBlock];        // RES: the layer's own input of the last two steps, for the sums
     // Raised by a wavefront one of whose waits gave up, always in front of a step's barrier, and read by all right behind
     // it: the workgroup then leaves the loop of steps together, publishes nothing more and computes its units by itself.
@@ -267,8 +293,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         half8_t zero;
 #pragma unroll
         for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
-#pragma unroll
-        for (int m = 0; m < kXcdFrags; ++m) w[m] = xcd_weight_fragment(wsrc + ((long)my_gate * H + my_unit) * H, m, lane, H, units_ok);
+        xcd_load_weights(w, wsrc, wstage[wave], u0, lane, H, units_ok);
         for (int i = tid; i < 2 * kXcdMaxH / 8; i += kXcdThreads) reinterpret_cast<half8_t*>(&hbuf[0][0])[i] = zero;
     }
     if (tid == 0 && claimed_before == g_base) {
@@ -280,12 +305,11 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     __syncthreads();
 
     const int uc = units_ok ? my_unit : H - 1;
-    // Lanes 0..31 of wavefronts 0..3 fetch piece 32 w + lane of an h vector: 8 fp16 = columns 8 q .. 8 q + 7.  (The other
-    // wavefronts never poll: they are the ones that talk to other XCDs, and a wavefront's loads come back in order.)
-    // A group that neither feeds nor is fed across XCDs spreads the polls over all eight wavefronts, 16 lanes each.
-    const bool crosses = PIPE && (is_proj || ch.xproj_polled != 0 || ch.seq_out != nullptr || (RES && ch.res_in != nullptr));
-    const int piece = crosses ? wave * 32 + lane : wave * 16 + lane;
-    const bool polls = (crosses ? (wave < 4 && lane < 32) : lane < 16) && piece * 8 < H;
+    // The lanes of wavefronts 0 and 1 fetch piece 64 w + lane of an h vector: 8 fp16 = columns 8 q .. 8 q + 7.  Few wavefronts with
+    // all their lanes: spread over eight of 16 lanes a step takes 1.42 us, over four of 32 1.32, over two 1.31 (H = 1024).  (The
+    // wavefronts that talk to other XCDs, 4 .. 7, never poll: a wavefront's loads come back in order.)
+    const int piece = wave * 64 + lane;
+    const bool polls = wave < 2 && piece * 8 < H;
 
     // One bounded wait: `again` loads and tests; gives up like every wait of this kernel, after spin_limit polls, and
     // also after kXcdWaitTicks of the constant 100 MHz clock, however long a poll takes in the environment the kernel
