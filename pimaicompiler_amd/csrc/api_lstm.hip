@@ -774,38 +774,55 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
         for (int l = 0; l < L; ++l) {
             half_t* layer_out = (l == L - 1) ? (half_t*)y : plan->ybuf[l & 1];
             const int64_t in_w = plan->cells[(size_t)l * D].in_w;
-            for (int d = 0; d < D; ++d) {
-                const int ci = l * D + d;
-                const PimHipLstmPlan::Cell& c = plan->cells[ci];
-                float* xp = plan->xproj + (size_t)d * plan->max_seq_len * 4 * H;
-                half_t* yd = layer_out + (size_t)d * H;
-                const half_t* h0c = h0p + (size_t)ci * H;
-                const half_t* c0c = c0p + (size_t)ci * H;
-                half_t* hnc = hnp + (size_t)ci * H;
-                half_t* cnc = cnp + (size_t)ci * H;
-                if (!fuse_xproj) {
-                    float* outs1[1] = {xp};
-                    const half_t* ws1[1] = {c.w_ih};
-                    const float* bs1[1] = {c.bsum};
-                    rc = launch_input_projection(1, outs1, layer_in, ws1, bs1, T, in_w, 4 * H, s);
-                    if (rc != PIMHIP_OK) return rc;
+            if (!fuse_xproj) {
+                float* outs2[2];
+                const half_t* ws2[2];
+                const float* bs2[2];
+                for (int d = 0; d < D; ++d) {
+                    const PimHipLstmPlan::Cell& c = plan->cells[(size_t)l * D + d];
+                    outs2[d] = plan->xproj + (size_t)d * plan->max_seq_len * 4 * H;
+                    ws2[d] = c.w_ih;
+                    bs2[d] = c.bsum;
                 }
-                float* cst = plan->c_state + (size_t)d * H;
-                const unsigned grid = (unsigned)((H + 3) / 4);
-                // what a step's launch reads: W_hh, and W_ih when the projection is made in the same kernel
-                const int keep = (unsigned long long)(4 * H) * (unsigned long long)(H + (fuse_xproj ? in_w : 0)) * sizeof(half_t) <= kKeepCachedBytes;
-                for (int64_t step = 0; step < T; ++step) {
+                rc = launch_input_projection(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, s);
+                if (rc != PIMHIP_OK) return rc;
+            }
+            const unsigned grid = (unsigned)((H + 3) / 4);
+            // what a step's launch reads: W_hh, and W_ih when the projection is made in the same kernel
+            const int keep = (unsigned long long)D * (unsigned long long)(4 * H) * (unsigned long long)(H + (fuse_xproj ? in_w : 0)) * sizeof(half_t) <= kKeepCachedBytes;
+            LstmStepPair p2;
+            memset(&p2, 0, sizeof(p2));
+            for (int64_t step = 0; step < T; ++step) {
+                const bool last = step == T - 1;
+                for (int d = 0; d < D; ++d) {
+                    const int ci = l * D + d;
+                    const PimHipLstmPlan::Cell& c = plan->cells[ci];
                     const int64_t t = d ? (T - 1 - step) : step;
                     const int64_t tp = d ? (t + 1) : (t - 1);
-                    const half_t* h_prev = (step == 0) ? h0c : (yd + tp * y_stride);
-                    const bool last = step == T - 1;
-                    (keep ? lstm_step_f16_kernel<4, true> : lstm_step_f16_kernel<4, false>)<<<grid, 256, 0, s>>>(
-                        c.w_ih, c.w_hh, c.bsum, fuse_xproj ? nullptr : (xp + t * 4 * H), layer_in + t * in_w, h_prev,
-                        (step == 0) ? c0c : nullptr, cst, yd + t * y_stride, last ? hnc : nullptr, last ? cnc : nullptr,
-                        (int)in_w, (int)H);
+                    half_t* yd = layer_out + (size_t)d * H;
+                    LstmStepDir& sd = p2.dir[d];
+                    sd.w_ih = c.w_ih;
+                    sd.w_hh = c.w_hh;
+                    sd.bsum = c.bsum;
+                    sd.xproj = fuse_xproj ? nullptr : plan->xproj + (size_t)d * plan->max_seq_len * 4 * H + t * 4 * H;
+                    sd.x = layer_in + t * in_w;
+                    sd.h_prev = (step == 0) ? h0p + (size_t)ci * H : (yd + tp * y_stride);
+                    sd.c_in_f16 = (step == 0) ? c0p + (size_t)ci * H : nullptr;
+                    sd.c_state = plan->c_state + (size_t)d * H;
+                    sd.h_out = yd + t * y_stride;
+                    sd.hn_f16 = last ? hnp + (size_t)ci * H : nullptr;
+                    sd.cn_f16 = last ? cnp + (size_t)ci * H : nullptr;
                 }
-                PIMHIP_HIP_CHECK(hipGetLastError());
+                if (D == 2) {
+                    (keep ? lstm_step_pair_f16_kernel<4, true> : lstm_step_pair_f16_kernel<4, false>)<<<dim3(grid, 2), 256, 0, s>>>(p2, (int)in_w, (int)H);
+                } else {
+                    // (plain arguments: the kernel's first instructions have them in registers)
+                    const LstmStepDir& sd = p2.dir[0];
+                    (keep ? lstm_step_f16_kernel<4, true> : lstm_step_f16_kernel<4, false>)<<<grid, 256, 0, s>>>(
+                        sd.w_ih, sd.w_hh, sd.bsum, sd.xproj, sd.x, sd.h_prev, sd.c_in_f16, sd.c_state, sd.h_out, sd.hn_f16, sd.cn_f16, (int)in_w, (int)H);
+                }
             }
+            PIMHIP_HIP_CHECK(hipGetLastError());
             if (residual(l)) {
                 add_input(layer_out, layer_in);
                 PIMHIP_HIP_CHECK(hipGetLastError());

@@ -647,3 +647,22 @@ def test_input_projection_of_many_steps(ops, T, K, N):
     got = ops.input_projection(xi, wd, bd)
     assert torch.equal(got[: T - 1], out[: T - 1]) and not bool(torch.isfinite(got[T - 1][wd[:, 0] != 0]).any())
     assert torch.equal(got[: T - 1], ops.input_projection_packed(xi, packed, N, bd)[: T - 1]) == torch.equal(out, ops.input_projection_packed(xd, packed, N, bd))
+
+
+# One launch for a step of both directions: hidden sizes around its blocks of four units and its 128-column strides; one step (projection in
+# the launch) and three (projection before it).
+@pytest.mark.parametrize("I,H,T", [(8, 8, 1), (24, 72, 1), (520, 1032, 1), (40, 88, 3), (8, 2056, 3)])
+def test_step_of_both_directions_equals_each_alone(ops, I, H, T):
+    params, x, h0, c0 = workloads.lstm_inputs(31 + H, I, H, 1, True, T)
+    dev = [p.to(DEV) for p in params]
+    xd, h0, c0 = x.reshape(T, I).to(DEV), h0.to(DEV), c0.to(DEV)
+    both = ops.LstmPlan(dev, True, 1, True, T)
+    both.set_mode(1)
+    y, hn, cn = both.forward(xd, h0, c0)
+    for d in range(2):
+        one = ops.LstmPlan(dev[4 * d:4 * d + 4], True, 1, False, T)
+        one.set_mode(1)
+        y1, hn1, cn1 = one.forward(xd if d == 0 else xd.flip(0).contiguous(), h0[d:d + 1].contiguous(), c0[d:d + 1].contiguous())
+        y1 = y1.reshape(T, H) if d == 0 else y1.reshape(T, H).flip(0)
+        assert torch.equal(y.reshape(T, 2 * H)[:, d * H:(d + 1) * H], y1)
+        assert torch.equal(hn.reshape(2, H)[d], hn1.reshape(H)) and torch.equal(cn.reshape(2, H)[d], cn1.reshape(H))
