@@ -68,7 +68,8 @@ int launch_input_projection(int count, float* const* out, const half_t* x, const
         pr.bias[p] = bias[p];
         pr.out[p] = out[p];
     }
-    if (const int mt = tile_rows(T, N, count, false)) {
+    // (K == 0, out = bias, stays below: the tiles' loop always has a slab)
+    if (const int mt = K > 0 ? tile_rows(T, N, count, false) : 0) {
         XprojFill none;  // (count 0: no blocks that fill)
         memset(&none, 0, sizeof(none));
         launch_tiles<false>(mt, count, out, x, w, bias, T, K, N, ldx, ldw, 0, none, s);

@@ -649,6 +649,19 @@ def test_input_projection_of_many_steps(ops, T, K, N):
     assert torch.equal(got[: T - 1], ops.input_projection_packed(xi, packed, N, bd)[: T - 1]) == torch.equal(out, ops.input_projection_packed(xd, packed, N, bd))
 
 
+# A reduction of width 0 leaves the bias, also where there are enough time steps for the kernel above (whose loop takes one slab at least).
+def test_input_projection_of_no_columns(ops):
+    import ctypes
+    from pimaicompiler_amd import _lib
+    T, N = 800, 4096
+    some = torch.ones(64, dtype=torch.float16, device=DEV)  # (operands of no elements; the entry point wants addresses)
+    b = torch.arange(N, dtype=torch.float32, device=DEV)
+    out = torch.full((T, N), -1.0, device=DEV)
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert _lib.load().pimhip_input_projection(out.data_ptr(), some.data_ptr(), some.data_ptr(), b.data_ptr(), T, 0, N, stream) == 0
+    assert torch.equal(out, b.expand(T, N))
+
+
 # One launch for a step of both directions: hidden sizes around its blocks of four units and its 128-column strides; one step (projection in
 # the launch) and three (projection before it).
 @pytest.mark.parametrize("I,H,T", [(8, 8, 1), (24, 72, 1), (520, 1032, 1), (40, 88, 3), (8, 2056, 3)])
