@@ -42,6 +42,8 @@
 // into the workgroup's entry.  What bounds a step (1.30 us at H = 1024, 1.05 at 320, where nearly all of it is this): the
 // store becoming visible in the L2 and the poll that finds it, 0.43 us at best for such a round; 0.21 us are matrix instructions.
 // The products on v_dot2 with a reduction over 16 lanes: 1.49 us (one layer), 1.57 (pipelines of layers).
+// Few units are the other way round: up to about 256 the step's chain through the matrix instructions is longer than v_dot2's was
+// (80 steps of both directions of 64 units 84.5 us against 74, of 256 89.7 against 86, of 512 96 against 102).
 #pragma once
 
 #include <type_traits>
@@ -168,15 +170,22 @@ __device__ __forceinline__ void xcd_load_weights(half16_t (&w)[kXcdFrags], const
     for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
     half8_t raw[kXcdFrags / 2][4];
 #pragma unroll
-    for (int i = 0; i < kXcdFrags / 2; ++i)
+    for (int i = 0; i < kXcdFrags / 2; ++i) {
+        if (128 * i >= H) break;  // (uniform)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int n = 4 * j + (lane >> 4), col = 128 * i + 8 * (lane & 15);  // H % 8 == 0: a piece is entirely in or out of range
             raw[i][j] = (ok && col < H) ? *reinterpret_cast<const half8_t*>(src + ((long)(n & 3) * H + u0 + (n >> 2)) * H + col) : zero;
         }
+    }
     const int n = lane & 15, g = lane >> 4;
 #pragma unroll
     for (int i = 0; i < kXcdFrags / 2; ++i) {
+        if (128 * i >= H) {  // (uniform) nothing but zeros: 64 KB per CU and i that need not pass through LDS
+#pragma unroll
+            for (int m = 0; m < 2; ++m) w[2 * i + m] = __builtin_shufflevector(zero, zero, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+            continue;
+        }
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int r = 4 * j + (lane >> 4);
@@ -210,7 +219,15 @@ struct XcdSums {
 __device__ __forceinline__ float xcd_matvec(const half16_t (&w)[kXcdFrags], const half_t* hb, XcdSums& acc, int H, int lane)
 {
     const int index = (lane & 1) ? 0xeeeeeeee : 0x44444444;  // columns 2, 3 / 0, 1 of every four
-    const half8_t h0 = xcd_h_operand(hb, 0, lane), h1 = xcd_h_operand(hb, 1, lane);
+    const half8_t h0 = xcd_h_operand(hb, 0, lane);
+    if (H <= 256) {  // (uniform) four fragments: half the sums and no second operand; the chain is all a step of few units has
+#pragma unroll
+        for (int m = 0; m < 4; ++m) acc.d[m] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(h0, w[m], acc.d[m], index, 0, 0);
+        const float f0 = (acc.d[0][0] + acc.d[0][1]) + (acc.d[1][2] + acc.d[1][3]);
+        const float f1 = (acc.d[2][0] + acc.d[2][1]) + (acc.d[3][2] + acc.d[3][3]);
+        return wave_sum_rows((lane & 32) ? 0.0f : (lane & 16) ? f1 : f0);
+    }
+    const half8_t h1 = xcd_h_operand(hb, 1, lane);
 #pragma unroll
     for (int m = 0; m < kXcdFrags; ++m) {
         if ((m & 3) == 0 && m * 64 >= H) break;  // (uniform) whole fragments past the hidden state are zeros
