@@ -98,8 +98,9 @@ int pimhip_get_gemm_type(const int64_t* self_shape4, const int64_t* other_shape4
  * rounding to fp16 at the store.  As in the reference's VM/MV branches there is no alpha/beta
  * (aten_ops.cpp:627-628).  ld_weight == 0 selects the dense pitch.
  * The I_X_W order splits the reduction over blocks for all but small weights; the blocks exchange partial sums through
- * a per-stream workspace the library allocates on the first such call on a stream (the call synchronises that stream
- * then, and again whenever a later call needs a larger workspace).  Calls that share a stream must not overlap.  Every
+ * a per-stream workspace the library allocates on the first such call on a stream.  It has one size for every product and
+ * is kept until pimhip_deinitialize, so a graph that holds such a product stays valid whatever runs on the stream later.
+ * Calls that share a stream must not overlap.  Every
  * wait inside the kernel is bounded, and one that gives up costs time, not the result: the block computes the missing
  * partial sums itself, in the order their own block would have, so the result has the bits it would have had
  * (pimhip_gemv_fallbacks counts such events; the next I_X_W call on that stream outside a graph capture puts the workspace

@@ -33,8 +33,7 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 
 // ---- per-device state --------------------------------------------------------------------------
 struct SplitWorkspace {
-    float* partial = nullptr;            // [slices][N] fp32 records of the VM kernel; every word kVmEmpty between launches
-    size_t partial_elems = 0;
+    float* partial = nullptr;            // [slices][N] fp32 records of the VM kernel (vm_max_partials words); every word kVmEmpty between launches
     unsigned int* status = nullptr;      // pinned host word the kernel sets when a wait for a record gives up
     unsigned int* status_dev = nullptr;  // the same word as the device addresses it
     unsigned int* poison = nullptr;      // device word set at the same time: until it is cleared, reducing blocks ignore the records

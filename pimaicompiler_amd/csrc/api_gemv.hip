@@ -10,44 +10,43 @@ namespace
 {
 constexpr size_t kStaticScratchFloats = 64 * 1024;  // the array itself is in api_core.hip, where its address is looked up
 
+// The workspace of a stream: one size for every product (vm_max_partials) and kept until pimhip_deinitialize, so that a graph
+// that holds its address stays valid whatever runs on the stream later.
 int get_split_workspace(DeviceState* st, hipStream_t stream, size_t partial_elems, SplitWorkspace** out)
 {
+    if (partial_elems > vm_max_partials(st->num_cus))
+        return fail(PIMHIP_ERR_UNSUPPORTED, "this I_X_W product needs %zu partial sums, a workspace holds %zu", partial_elems, vm_max_partials(st->num_cus));
     std::lock_guard<std::mutex> lock(g_mutex);
     SplitWorkspace& ws = st->workspaces[stream];
     const bool gave_up = ws.status && *ws.status != 0u;
     bool capturing = false;
-    if (!ws.status || ws.partial_elems < partial_elems || gave_up) {
+    if (!ws.partial || gave_up) {
         hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
         PIMHIP_HIP_CHECK(hipStreamIsCapturing(stream, &capture));
         capturing = capture != hipStreamCaptureStatusNone;
         // Allocation, synchronisation and the memset below are not for a graph.
-        if (capturing && (!ws.status || ws.partial_elems < partial_elems))
-            return fail(PIMHIP_ERR_UNSUPPORTED, "this I_X_W product needs its stream's workspace (re)allocated, which a graph must not "
+        if (capturing && !ws.partial)
+            return fail(PIMHIP_ERR_UNSUPPORTED, "this I_X_W product needs its stream's workspace allocated, which a graph must not "
                                                 "record: run it once on this stream before the capture");
     }
     if (!ws.status) {
         PIMHIP_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&ws.status), sizeof(unsigned int), hipHostMallocMapped));
         *ws.status = 0u;
         PIMHIP_HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&ws.status_dev), ws.status, 0));
-        PIMHIP_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&ws.poison), sizeof(unsigned int)));
-        PIMHIP_HIP_CHECK(hipMemsetAsync(ws.poison, 0, sizeof(unsigned int), stream));
     }
+    if (!ws.poison) PIMHIP_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&ws.poison), sizeof(unsigned int)));
     // A reducing block of an earlier product on this stream gave up on a record.  That product's result was completed by
     // the block itself, and the products since have ignored the records (the poison word is up); outside a capture the
     // records are refilled here and both words cleared.  (Inside one the launch goes ahead as it is: right, only slower.)
     const bool recover = gave_up && !capturing;
-    if (ws.partial_elems < partial_elems || recover) {
-        // Work already queued on this stream may still use the old buffer.
-        PIMHIP_HIP_CHECK(hipStreamSynchronize(stream));
-        if (ws.partial_elems < partial_elems) {
-            if (ws.partial) PIMHIP_HIP_CHECK(hipFree(ws.partial));
-            ws.partial = nullptr;
-            ws.partial_elems = 0;
-            PIMHIP_HIP_CHECK(hipMalloc(&ws.partial, partial_elems * sizeof(float)));
-            ws.partial_elems = partial_elems;
-        }
-        PIMHIP_HIP_CHECK(hipMemsetAsync(ws.partial, 0xff, ws.partial_elems * sizeof(float), stream));  // every word kVmEmpty
+    if (!ws.partial || recover) {
+        if (recover) PIMHIP_HIP_CHECK(hipStreamSynchronize(stream));  // queued products still use the records
+        float* partial = ws.partial;
+        const size_t bytes = vm_max_partials(st->num_cus) * sizeof(float);
+        if (!partial) PIMHIP_HIP_CHECK(hipMalloc(&partial, bytes));
+        PIMHIP_HIP_CHECK(hipMemsetAsync(partial, 0xff, bytes, stream));  // every word kVmEmpty
         PIMHIP_HIP_CHECK(hipMemsetAsync(ws.poison, 0, sizeof(unsigned int), stream));
+        ws.partial = partial;
         if (recover) ++ws.gave_up_events;
         *ws.status = 0u;
     }
@@ -135,47 +134,16 @@ int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bia
         gemv_vm_f16_generic_kernel<<<grid, 64 * kVmGenericWaves, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu);
         return PIMHIP_OK;
     }
-    // Block width: 64 columns (8 lanes per weight row) while the weight is small, so that more blocks share it: 2048 x 2048
-    // 3.5 us against 4.2 with 128 columns, 12896 x 84 4.0 against 6.7.  128 columns for a weight past kKeepCachedBytes, whose
-    // stream is the bound: 4096 x 4096 7.7 us against 8.2 with 64, 1024 x 32000 11.2 against 13.7.
-    const int64_t weight_bytes = K * N * (int64_t)sizeof(half_t);
-    const bool large = weight_bytes > (int64_t)kKeepCachedBytes;
-    const int lanes_per_row = large ? 16 : 8;
-    const int cols = 8 * lanes_per_row, row_groups = kVmWaves * 64 / lanes_per_row;
-    const int col_blocks = (int)((N + cols - 1) / cols);
-    // Rows that do not start on a 128-byte line make neighbouring column blocks share lines: they go to one XCD then, whose
-    // L2 hands the shared line to both (1024 x 31999: 11.6 us against 16.4), and the weight is read with plain loads.  Where
-    // no line is shared the same order costs (4096 x 4096 7.9 -> 9.9 us: eight fronts instead of one).
-    const int by_xcd = col_blocks >= 16 && (lda % 64 != 0 || (reinterpret_cast<uintptr_t>(A) & 127u) != 0);
-    // Slices of K: about a block per CU for a large weight, 64 blocks for a small one, but a cross-block sum costs 1 to 2 us
-    // and grows with the slices: none up to 512 rows (272 x 2357: 3.1 us, two slices 3.6) and at most sqrt(K / 40) of them
-    // (12896 rows, 84 columns: 4.0 us with 17, 4.9 with 64).
-    int64_t target = weight_bytes / 65536;
-    if (target < 64) target = 64;
-    if (target > st->num_cus) target = st->num_cus;
-    int slices = (int)((target + col_blocks / 2) / col_blocks);  // rounded: 250 column blocks on 256 CUs are not sliced
-    if (K <= 512) slices = 1;
-    while (slices > 1 && (int64_t)slices * slices * 40 > K) --slices;
-    if (slices < 1) slices = 1;
-    // Small weights and operands of no whole 16-byte pieces run without a workspace where they cannot have one (the static
-    // scratch array is too small, or a graph is being recorded before the stream has its workspace), in one slice.
-    const bool can_do_without = weight_bytes <= 256 * 1024 || (N % 8 != 0) || (lda % 8 != 0) || !aligned16(A) || !aligned16(outs.y[0]);
-    int k_per_slice = 0;
-    auto cut = [&]() {
-        k_per_slice = (int)((K + slices - 1) / slices);
-        k_per_slice = (k_per_slice + row_groups - 1) / row_groups * row_groups;
-        if (k_per_slice < row_groups) k_per_slice = row_groups;  // K == 0: one empty slice, y = act(bias)
-        slices = (int)((K + k_per_slice - 1) / k_per_slice);
-        if (slices < 1) slices = 1;
-    };
-    if (static_ws && can_do_without && (size_t)(slices - 1) * (size_t)N > kStaticScratchFloats) slices = 1;
-    cut();
+    VmPlan plan = vm_plan(K, N, lda, reinterpret_cast<uintptr_t>(A), st->num_cus);
+    // Small weights and operands of no whole 16-byte pieces run without a workspace where they cannot have one (a graph is being
+    // recorded before the stream has its workspace), in one slice.
+    const bool can_do_without = K * N * (int64_t)sizeof(half_t) <= 256 * 1024 || (N % 8 != 0) || (lda % 8 != 0) || !aligned16(A) || !aligned16(outs.y[0]);
     float* partial = nullptr;
     unsigned int* status = nullptr;
     unsigned int* poison = nullptr;
-    if (slices > 1) {
+    if (plan.slices > 1) {
         // Words of all slices but the last: partial[slice][N].
-        const size_t partial_elems = (size_t)(slices - 1) * (size_t)N;
+        const size_t partial_elems = (size_t)(plan.slices - 1) * (size_t)N;
         int rc;
         if (static_ws) {
             rc = get_static_workspace(st, s, partial_elems, &partial, &status, &poison);
@@ -188,16 +156,15 @@ int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bia
                 poison = ws->poison;
             } else if (rc == PIMHIP_ERR_UNSUPPORTED && can_do_without) {
                 rc = PIMHIP_OK;
-                slices = 1;
-                cut();
+                vm_cut(plan, K, 1);
             }
         }
         if (rc != PIMHIP_OK) return rc;
     }
-    const dim3 grid(by_xcd ? (col_blocks + 7) / 8 * 8 : col_blocks, slices);
-    auto kernel = !large ? gemv_vm_f16_kernel<8, true> : by_xcd ? gemv_vm_f16_kernel<16, true> : gemv_vm_f16_kernel<16, false>;
-    kernel<<<grid, kVmWaves * 64, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu, k_per_slice, partial, status, poison,
-                                          st->vm_spin_limit, by_xcd);
+    const dim3 grid(plan.by_xcd ? (plan.col_blocks + 7) / 8 * 8 : plan.col_blocks, plan.slices);
+    auto kernel = plan.lanes_per_row == 8 ? gemv_vm_f16_kernel<8, true> : plan.by_xcd ? gemv_vm_f16_kernel<16, true> : gemv_vm_f16_kernel<16, false>;
+    kernel<<<grid, kVmWaves * 64, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu, plan.rows_per_slice, partial, status, poison,
+                                          st->vm_spin_limit, plan.by_xcd);
     return PIMHIP_OK;
 }
 

@@ -16,6 +16,7 @@
 #include <type_traits>
 
 #include "device_common.h"
+#include "vm_plan.h"
 
 namespace pimhip
 {
@@ -270,7 +271,6 @@ struct GemvOuts {
     int count;
 };
 
-static constexpr int kVmWaves = 8;
 static constexpr int kVmLoads = 4;  // 16-byte loads in flight per lane
 
 // LPR: lanes per weight row.  KEEP: the weight is read with plain loads (load_weight).

@@ -1,0 +1,55 @@
+"""How I_X_W products are cut into slices (csrc/vm_plan.h), compiled for the host: what the exchange of partial sums relies on, over
+sizes at and around the edges of the rule."""
+import itertools
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+DRIVER = r"""
+#include <cstdio>
+#include "vm_plan.h"
+int main()
+{
+    long long K, N, lda, addr;
+    int cus;
+    while (scanf("%lld %lld %lld %lld %d", &K, &N, &lda, &addr, &cus) == 5) {
+        const pimhip::VmPlan p = pimhip::vm_plan(K, N, lda, (uintptr_t)addr, cus);
+        printf("%d %d %d %d %zu\n", p.lanes_per_row, p.col_blocks, p.slices, p.rows_per_slice, pimhip::vm_max_partials(cus));
+    }
+}
+"""
+
+SIZES = (8, 9, 63, 64, 65, 84, 127, 129, 512, 513, 1000, 1023, 2048, 2357, 4096, 4951, 8191, 16384, 30001, 32768, 65535, 200000)
+
+
+@pytest.fixture(scope="module")
+def plans(tmp_path_factory):
+    if shutil.which("g++") is None:
+        pytest.skip("no C++ compiler")
+    d = tmp_path_factory.mktemp("vm_plan")
+    (d / "driver.cpp").write_text(DRIVER)
+    subprocess.run(["g++", "-std=c++17", "-Wall", "-Werror", "-I", os.path.join(ROOT, "pimaicompiler_amd", "csrc"), str(d / "driver.cpp"), "-o",
+                    str(d / "driver")], check=True, capture_output=True)
+
+    def run(cases):
+        text = "\n".join(" ".join(map(str, c)) for c in cases)
+        out = subprocess.run([str(d / "driver")], input=text, check=True, capture_output=True, text=True).stdout
+        return [tuple(map(int, line.split())) for line in out.splitlines()]
+    return run
+
+
+def test_partial_sums_of_every_product_fit_a_workspace_of_one_size(plans):
+    """A workspace never grows, so no recorded graph can be left with the address of a freed one."""
+    cases = [(k, n, n, 0, cus) for k, n, cus in itertools.product((0, 1) + SIZES, SIZES, (32, 64, 256, 304))]
+    sliced = 0
+    for (k, n, _, _, cus), (lanes, blocks, slices, rows, words) in zip(cases, plans(cases)):
+        assert blocks == -(-n // (8 * lanes)) and slices >= 1
+        assert (slices - 1) * rows < max(k, 1) <= max(slices * rows, 1) or k == 0   # the slices cover K, none is empty
+        assert (slices - 1) * n <= words, (k, n, cus)
+        assert words <= 64 * 1024 or cus > 512                                       # the static scratch array holds them as well
+        sliced += slices > 1
+    assert sliced > 100
