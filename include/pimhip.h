@@ -97,9 +97,15 @@ int pimhip_get_gemm_type(const int64_t* self_shape4, const int64_t* other_shape4
  * out[out_w] = act(sum_k weight * in[k] + bias[out_w]); bias may be NULL.  fp32 accumulation, one
  * rounding to fp16 at the store.  As in the reference's VM/MV branches there is no alpha/beta
  * (aten_ops.cpp:627-628).  ld_weight == 0 selects the dense pitch.
- * The I_X_W order splits the reduction over blocks for all but small weights; the blocks exchange partial sums through
- * a per-stream workspace the library allocates on the first such call on a stream.  It has one size for every product and
- * is kept until pimhip_deinitialize, so a graph that holds such a product stays valid whatever runs on the stream later.
+ * The I_X_W order splits the reduction over blocks for all but short reductions; the blocks exchange partial sums.
+ * Weights of at most 256 KB, and operands of no whole 16-byte pieces (out_w or ld_weight no multiple of 8, weight or out not
+ * 16-byte aligned), need no workspace: outside a graph capture the sums go through memory pimhip_initialize has set aside for
+ * such products (32 streams of a GPU; a further stream, and hipStreamPerThread, do without), inside one each block sums all the
+ * slices it needs by itself, in the same order (same bits, up to four times as long where in_w is long).  They allocate and
+ * synchronise nothing and may be replayed beside anything.
+ * All others go through a per-stream workspace the library allocates on the first such call on a stream.  It has one size for
+ * every product and is kept until pimhip_deinitialize, so a graph that holds such a product stays valid whatever runs on the
+ * stream later; replays must not overlap other such products of the stream it was captured on.
  * Calls that share a stream must not overlap.  Every
  * wait inside the kernel is bounded, and one that gives up costs time, not the result: the block computes the missing
  * partial sums itself, in the order their own block would have, so the result has the bits it would have had
@@ -130,8 +136,9 @@ int pimhip_execute_gemv_cat2(void* out, const void* in1, int64_t in1_w, const vo
  * but the partial sums of a sliced I_X_W product go through a 256 KiB array that is part of the library's
  * image on every GPU it runs on, instead of a per-stream workspace: the call allocates, frees and synchronises
  * nothing and records kernels only.  A product that needs more than 65536 partial sums
- * ((slices - 1) * out_w; none that pimhip_execute_gemv slices on a 256-CU part does) is refused with
- * PIMHIP_ERR_UNSUPPORTED.  All calls on one GPU share the array: calls that may overlap there (different streams,
+ * ((slices - 1) * out_w; at most 128 per CU, 32768 on a 256-CU part) is refused with
+ * PIMHIP_ERR_UNSUPPORTED.  The products that need no workspace (pimhip_execute_gemv) do not touch the array; all other calls
+ * on one GPU share it: calls that may overlap there (different streams,
  * or replays of graphs holding such calls) race and must be ordered by the caller.  A wait that gives up is made good
  * inside the launch as in pimhip_execute_gemv; the next call outside a graph capture refills the array (the one case in
  * which this entry point synchronises the stream). */

@@ -2,6 +2,7 @@
 // include/pimhip.h that belongs to no kernel family.
 #include "api_common.h"
 #include "shape_logic.h"
+#include "vm_plan.h"
 
 namespace pimhip
 {
@@ -33,6 +34,42 @@ static __device__ __align__(256) float scratch[kStaticScratchFloats];
 static __device__ unsigned int scratch_poison;
 
 std::map<int, DeviceState> g_devices;
+
+void free_vm_regions(DeviceState& st)
+{
+    if (st.region_partials) hipFree(st.region_partials);
+    if (st.region_poisons) hipFree(st.region_poisons);
+    if (st.region_statuses) hipHostFree(st.region_statuses);
+    st.region_partials = nullptr;
+    st.region_poisons = st.region_statuses = nullptr;
+    for (SplitWorkspace& r : st.regions) r = SplitWorkspace();
+    st.region_of.clear();
+}
+
+// 4 MiB on a part of 256 CUs.  A device that has no room for them does without.
+void allocate_vm_regions(DeviceState& st)
+{
+    const size_t words = vm_max_partials(st.num_cus);
+    unsigned int* statuses_dev = nullptr;
+    if (hipMalloc(&st.region_partials, kVmRegions * words * sizeof(float)) != hipSuccess ||
+        hipMalloc(&st.region_poisons, kVmRegions * sizeof(unsigned int)) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void**>(&st.region_statuses), kVmRegions * sizeof(unsigned int), hipHostMallocMapped) != hipSuccess ||
+        hipHostGetDevicePointer(reinterpret_cast<void**>(&statuses_dev), st.region_statuses, 0) != hipSuccess) {
+        (void)hipGetLastError();
+        free_vm_regions(st);
+        return;
+    }
+    launch_fill_u32(reinterpret_cast<unsigned int*>(st.region_partials), kVmRegions * words, kVmEmpty, nullptr);
+    launch_fill_u32(st.region_poisons, kVmRegions, 0u, nullptr);
+    for (int i = 0; i < kVmRegions; ++i) {
+        SplitWorkspace& r = st.regions[i];
+        r.partial = st.region_partials + i * words;
+        r.poison = st.region_poisons + i;
+        r.status = st.region_statuses + i;
+        r.status_dev = statuses_dev + i;
+        *r.status = 0u;
+    }
+}
 }  // namespace
 
 std::mutex g_mutex;
@@ -122,6 +159,8 @@ extern "C" int pimhip_initialize(int device)
         PIMHIP_HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&st.static_status_dev), st.static_status, 0));
     }
     *st.static_status = 0u;
+    if (!st.region_partials) allocate_vm_regions(st);
+    PIMHIP_HIP_CHECK(hipGetLastError());
     PIMHIP_HIP_CHECK(hipStreamSynchronize(nullptr));
     st.initialized = true;
     return PIMHIP_OK;
@@ -148,6 +187,7 @@ extern "C" int pimhip_deinitialize(void)
             if (w.second.status) hipHostFree(w.second.status);
         }
         kv.second.workspaces.clear();
+        free_vm_regions(kv.second);
         if (kv.second.static_status) hipHostFree(kv.second.static_status);
         if (kv.second.seq_event) hipEventDestroy(kv.second.seq_event);
         kv.second.initialized = false;

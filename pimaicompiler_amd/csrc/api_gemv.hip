@@ -10,6 +10,19 @@ namespace
 {
 constexpr size_t kStaticScratchFloats = 64 * 1024;  // the array itself is in api_core.hip, where its address is looked up
 
+// A reducing block of an earlier product on this stream gave up on a record.  That product's result was completed by the block
+// itself, and the products since have ignored the records (the poison word is up); outside a capture the records are refilled
+// here and both words cleared.  (Inside one the launch goes ahead as it is: right, only slower.)
+int refill_records(DeviceState* st, SplitWorkspace& ws, hipStream_t stream)
+{
+    PIMHIP_HIP_CHECK(hipStreamSynchronize(stream));  // queued products still use the records
+    PIMHIP_HIP_CHECK(hipMemsetAsync(ws.partial, 0xff, vm_max_partials(st->num_cus) * sizeof(float), stream));
+    PIMHIP_HIP_CHECK(hipMemsetAsync(ws.poison, 0, sizeof(unsigned int), stream));
+    ++ws.gave_up_events;
+    *ws.status = 0u;
+    return PIMHIP_OK;
+}
+
 // The workspace of a stream: one size for every product (vm_max_partials) and kept until pimhip_deinitialize, so that a graph
 // that holds its address stays valid whatever runs on the stream later.
 int get_split_workspace(DeviceState* st, hipStream_t stream, size_t partial_elems, SplitWorkspace** out)
@@ -35,20 +48,43 @@ int get_split_workspace(DeviceState* st, hipStream_t stream, size_t partial_elem
         PIMHIP_HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&ws.status_dev), ws.status, 0));
     }
     if (!ws.poison) PIMHIP_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&ws.poison), sizeof(unsigned int)));
-    // A reducing block of an earlier product on this stream gave up on a record.  That product's result was completed by
-    // the block itself, and the products since have ignored the records (the poison word is up); outside a capture the
-    // records are refilled here and both words cleared.  (Inside one the launch goes ahead as it is: right, only slower.)
-    const bool recover = gave_up && !capturing;
-    if (!ws.partial || recover) {
-        if (recover) PIMHIP_HIP_CHECK(hipStreamSynchronize(stream));  // queued products still use the records
-        float* partial = ws.partial;
+    if (!ws.partial) {
+        float* partial = nullptr;
         const size_t bytes = vm_max_partials(st->num_cus) * sizeof(float);
-        if (!partial) PIMHIP_HIP_CHECK(hipMalloc(&partial, bytes));
+        PIMHIP_HIP_CHECK(hipMalloc(&partial, bytes));
         PIMHIP_HIP_CHECK(hipMemsetAsync(partial, 0xff, bytes, stream));  // every word kVmEmpty
         PIMHIP_HIP_CHECK(hipMemsetAsync(ws.poison, 0, sizeof(unsigned int), stream));
         ws.partial = partial;
-        if (recover) ++ws.gave_up_events;
-        *ws.status = 0u;
+    } else if (gave_up && !capturing) {
+        const int rc = refill_records(st, ws, stream);
+        if (rc != PIMHIP_OK) return rc;
+    }
+    *out = &ws;
+    return PIMHIP_OK;
+}
+
+// The region of a stream for the products that need no workspace, null where they have to do without: nothing of it may end up in
+// a graph, and hipStreamPerThread names another stream in every thread.
+int get_region(DeviceState* st, hipStream_t stream, SplitWorkspace** out)
+{
+    *out = nullptr;
+    if (!st->region_partials || stream == hipStreamPerThread) return PIMHIP_OK;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {  // (the null stream while another one is being captured)
+        (void)hipGetLastError();
+        return PIMHIP_OK;
+    }
+    if (capture != hipStreamCaptureStatusNone) return PIMHIP_OK;
+    std::lock_guard<std::mutex> lock(g_mutex);
+    auto it = st->region_of.find(stream);
+    if (it == st->region_of.end()) {
+        if (st->region_of.size() >= (size_t)kVmRegions) return PIMHIP_OK;
+        it = st->region_of.emplace(stream, (int)st->region_of.size()).first;
+    }
+    SplitWorkspace& ws = st->regions[it->second];
+    if (*ws.status != 0u) {
+        const int rc = refill_records(st, ws, stream);
+        if (rc != PIMHIP_OK) return rc;
     }
     *out = &ws;
     return PIMHIP_OK;
@@ -124,6 +160,21 @@ int get_static_workspace(DeviceState* st, hipStream_t stream, size_t partial_ele
     return PIMHIP_OK;
 }
 
+void launch_vm_alone(const half_t* x, const half_t* A, const half_t* bias, const GemvOuts& outs, int64_t K, int64_t N, int64_t lda, int relu,
+                     const VmPlan& plan, hipStream_t s)
+{
+    // Slices at a time, and with them the block's width: blocks half as wide from 4096 rows on, where there are enough slices
+    // (16384 x 84 13.9 -> 12.5 us, 4951 x 9 8.3 -> 6.4; 2048 x 2357 the other way round, 5.7 against 8.1).
+    const int ns = K > 4096 ? 8 : 4;
+    const int cols = 8 * plan.lanes_per_row / ns;
+    const int blocks = (int)((N + cols - 1) / cols);
+    const int by_xcd = blocks >= 16;  // (narrow blocks share the lines of a row)
+    auto kernel = plan.lanes_per_row == 8 ? (ns == 8 ? gemv_vm_alone_f16_kernel<8, 8> : gemv_vm_alone_f16_kernel<8, 4>)
+                                          : (ns == 8 ? gemv_vm_alone_f16_kernel<16, 8> : gemv_vm_alone_f16_kernel<16, 4>);
+    kernel<<<by_xcd ? (blocks + 7) / 8 * 8 : blocks, kVmWaves * 64, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu, plan.rows_per_slice,
+                                                                            plan.slices, by_xcd);
+}
+
 int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bias, const GemvOuts& outs, int64_t K,
             int64_t N, int64_t lda, int relu, hipStream_t s, bool static_ws = false)
 {
@@ -134,32 +185,34 @@ int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bia
         gemv_vm_f16_generic_kernel<<<grid, 64 * kVmGenericWaves, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu);
         return PIMHIP_OK;
     }
-    VmPlan plan = vm_plan(K, N, lda, reinterpret_cast<uintptr_t>(A), st->num_cus);
-    // Small weights and operands of no whole 16-byte pieces run without a workspace where they cannot have one (a graph is being
-    // recorded before the stream has its workspace), in one slice.
-    const bool can_do_without = K * N * (int64_t)sizeof(half_t) <= 256 * 1024 || (N % 8 != 0) || (lda % 8 != 0) || !aligned16(A) || !aligned16(outs.y[0]);
+    uintptr_t results = 0;
+    for (int o = 0; o < outs.count; ++o) results |= reinterpret_cast<uintptr_t>(outs.y[o]);
+    const VmPlan plan = vm_plan(K, N, lda, reinterpret_cast<uintptr_t>(A), results, st->num_cus);
     float* partial = nullptr;
     unsigned int* status = nullptr;
     unsigned int* poison = nullptr;
     if (plan.slices > 1) {
         // Words of all slices but the last: partial[slice][N].
         const size_t partial_elems = (size_t)(plan.slices - 1) * (size_t)N;
-        int rc;
-        if (static_ws) {
+        SplitWorkspace* ws = nullptr;
+        int rc = PIMHIP_OK;
+        if (plan.needs_no_workspace) {
+            if (!static_ws) rc = get_region(st, s, &ws);
+            if (rc == PIMHIP_OK && !ws) {
+                launch_vm_alone(x, A, bias, outs, K, N, lda, relu, plan, s);
+                return PIMHIP_OK;
+            }
+        } else if (static_ws) {
             rc = get_static_workspace(st, s, partial_elems, &partial, &status, &poison);
         } else {
-            SplitWorkspace* ws = nullptr;
             rc = get_split_workspace(st, s, partial_elems, &ws);
-            if (rc == PIMHIP_OK) {
-                partial = ws->partial;
-                status = ws->status_dev;
-                poison = ws->poison;
-            } else if (rc == PIMHIP_ERR_UNSUPPORTED && can_do_without) {
-                rc = PIMHIP_OK;
-                vm_cut(plan, K, 1);
-            }
         }
         if (rc != PIMHIP_OK) return rc;
+        if (ws) {
+            partial = ws->partial;
+            status = ws->status_dev;
+            poison = ws->poison;
+        }
     }
     const dim3 grid(plan.by_xcd ? (plan.col_blocks + 7) / 8 * 8 : plan.col_blocks, plan.slices);
     auto kernel = plan.lanes_per_row == 8 ? gemv_vm_f16_kernel<8, true> : plan.by_xcd ? gemv_vm_f16_kernel<16, true> : gemv_vm_f16_kernel<16, false>;
@@ -282,6 +335,8 @@ extern "C" int pimhip_gemv_status(void* stream, int* gave_up)
     int flags = 0;
     auto it = st->workspaces.find(static_cast<hipStream_t>(stream));
     if (it != st->workspaces.end() && it->second.status && *it->second.status != 0u) flags |= 1;
+    auto region = st->region_of.find(static_cast<hipStream_t>(stream));
+    if (region != st->region_of.end() && *st->regions[region->second].status != 0u) flags |= 1;
     if (st->static_status && *st->static_status != 0u) flags |= 2;
     *gave_up = flags;
     return PIMHIP_OK;
@@ -297,6 +352,8 @@ extern "C" int pimhip_gemv_fallbacks(void* stream, uint64_t* events)
     uint64_t n = st->static_gave_up_events + ((st->static_status && *st->static_status != 0u) ? 1u : 0u);
     auto it = st->workspaces.find(static_cast<hipStream_t>(stream));
     if (it != st->workspaces.end()) n += it->second.gave_up_events + ((it->second.status && *it->second.status != 0u) ? 1u : 0u);
+    auto region = st->region_of.find(static_cast<hipStream_t>(stream));
+    if (region != st->region_of.end()) n += st->regions[region->second].gave_up_events + (*st->regions[region->second].status != 0u ? 1u : 0u);
     *events = n;
     return PIMHIP_OK;
 }

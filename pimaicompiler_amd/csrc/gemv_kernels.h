@@ -273,6 +273,50 @@ struct GemvOuts {
 
 static constexpr int kVmLoads = 4;  // 16-byte loads in flight per lane
 
+// acc[j] += A[k][j] * x[k] for k, k + GROUPS, .. < k_end, `a` at the lane's eight columns of row 0.
+template <bool KEEP, int GROUPS>
+__device__ __forceinline__ void vm_sum_rows(float (&acc)[8], const half_t* a, long lda, const half_t* __restrict__ x, int k, int k_end)
+{
+    constexpr int U = kVmLoads;
+    auto take = [&](int k, auto last) __attribute__((always_inline)) {
+        half8_t ar[U];
+        float xr[U];
+        // (rows past the slice re-read its last one and count as zeros: all of a trip's loads are in flight together)
+        auto row = [&](int u) { return last ? min(k + u * GROUPS, k_end - 1) : k + u * GROUPS; };
+#pragma unroll
+        for (int u = 0; u < U; ++u) ar[u] = load_weight_any<KEEP>(a + (long)row(u) * lda);
+#pragma unroll
+        for (int u = 0; u < U; ++u) xr[u] = (float)x[row(u)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (last && k + u * GROUPS >= k_end) {
+                xr[u] = 0.0f;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) ar[u][j] = (half_t)0.0f;
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc[j] = fmaf((float)ar[u][j], xr[u], acc[j]);
+        }
+    };
+    for (; k + (U - 1) * GROUPS < k_end; k += U * GROUPS) take(k, std::false_type{});
+    if (k < k_end) take(k, std::true_type{});
+}
+
+// A row group's eight sums into its row of LDS; the lane with the last N % 8 columns has read the eight before N.
+__device__ __forceinline__ void vm_put_sums(float* row, const float (&acc)[8], int cg, long base, int N)
+{
+    const long col0 = base + cg * 8;
+    if (col0 + 8 <= N || col0 >= N) {
+        *reinterpret_cast<float4_t*>(row + cg * 8) = float4_t{acc[0], acc[1], acc[2], acc[3]};
+        *reinterpret_cast<float4_t*>(row + cg * 8 + 4) = float4_t{acc[4], acc[5], acc[6], acc[7]};
+    } else {
+        const int first = (int)(N - 8 - base);  // where the loaded columns lie in the block (before its start if it has fewer than eight)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (first + j >= cg * 8) row[first + j] = acc[j];
+    }
+}
+
 // LPR: lanes per weight row.  KEEP: the weight is read with plain loads (load_weight).
 template <int LPR, bool KEEP>
 __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t* __restrict__ x,
@@ -283,7 +327,6 @@ __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t
                                                                  unsigned int* status, unsigned int* poison,
                                                                  unsigned int spin_limit, int by_xcd)
 {
-    constexpr int U = kVmLoads;
     constexpr int kVmCols = 8 * LPR;
     constexpr int GROUPS = kVmWaves * (64 / LPR);     // row groups per block = LDS rows of the reduction = rows between loads of a lane
     constexpr int PARTS = kVmWaves * 64 / kVmCols;    // threads per column when the slices' sums are collected
@@ -309,42 +352,8 @@ __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
 
-    const bool whole = col0 + 8 <= N;
-    if (col0 < N) {
-        const half_t* a = A + (whole ? col0 : (long)N - 8);
-        auto take = [&](int k, auto last) __attribute__((always_inline)) {
-            half8_t ar[U];
-            float xr[U];
-            // (rows past the slice re-read its last one and count as zeros: all of a trip's loads are in flight together)
-            auto row = [&](int u) { return last ? min(k + u * GROUPS, k_end - 1) : k + u * GROUPS; };
-#pragma unroll
-            for (int u = 0; u < U; ++u) ar[u] = load_weight_any<KEEP>(a + (long)row(u) * lda);
-#pragma unroll
-            for (int u = 0; u < U; ++u) xr[u] = (float)x[row(u)];
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (last && k + u * GROUPS >= k_end) {
-                    xr[u] = 0.0f;
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) ar[u][j] = (half_t)0.0f;
-                }
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[j] = fmaf((float)ar[u][j], xr[u], acc[j]);
-            }
-        };
-        int k = k_begin + grp;
-        for (; k + (U - 1) * GROUPS < k_end; k += U * GROUPS) take(k, std::false_type{});
-        if (k < k_end) take(k, std::true_type{});
-    }
-    if (whole || col0 >= N) {
-        *reinterpret_cast<float4_t*>(&red[grp][cg * 8]) = float4_t{acc[0], acc[1], acc[2], acc[3]};
-        *reinterpret_cast<float4_t*>(&red[grp][cg * 8 + 4]) = float4_t{acc[4], acc[5], acc[6], acc[7]};
-    } else {
-        const int first = (int)(N - 8 - base);  // where the loaded columns lie in the block (before its start if it has fewer than eight)
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (first + j >= cg * 8) red[grp][first + j] = acc[j];
-    }
+    if (col0 < N) vm_sum_rows<KEEP, GROUPS>(acc, A + (col0 + 8 <= N ? col0 : (long)N - 8), lda, x, k_begin + grp, k_end);
+    vm_put_sums(red[grp], acc, cg, base, N);
     __syncthreads();
 
     // From here on a thread stands for one column.
@@ -445,6 +454,74 @@ __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t
     parts[part][c] = sum;
     __syncthreads();
     if (part == 0 && mine) finish(total() + own);
+}
+
+// The product of gemv_vm_f16_kernel<LPR> in the same slices, with the same sums in the same order (the same bits), by blocks that
+// exchange nothing: a block owns 8 LPR / NS columns and takes NS slices at a time, NS * GROUPS row groups of LPR / NS lanes.  For
+// products that use no workspace where another caller could be using it too (vm_plan.h): recorded into a graph, through the
+// static entry point, on a stream without a region.  What bounds it: a block reads a line of every row, however few of its
+// columns it owns, and the lines of one CU do not come faster than one in 2 to 4 clocks.  MI355X, us, sliced / this one (and with
+// the whole width in a block): VM_ALONE_FIGURES
+template <int LPR, int NS>
+__global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_alone_f16_kernel(const half_t* __restrict__ x, const half_t* __restrict__ A,
+                                                                       const half_t* __restrict__ bias, GemvOuts outs, int K, int N, long lda,
+                                                                       int relu, int k_per_slice, int nslices, int by_xcd)
+{
+    constexpr int GROUPS = kVmWaves * (64 / LPR);
+    constexpr int PARTS = kVmWaves * 8 / LPR;
+    constexpr int LANES = LPR / NS;
+    constexpr int COLS = 8 * LANES;
+    static_assert(NS * PARTS * COLS == kVmWaves * 64, "one thread per slice, part and column");
+    __shared__ __align__(16) float red[NS][GROUPS][COLS];
+    __shared__ float parts[NS][PARTS][COLS];
+    __shared__ float sums[PARTS][COLS];  // of the slices p, p + PARTS, ..: kept by the thread that finishes the column
+
+    const int tid = threadIdx.x;
+    const int cg = tid % LANES, worker = tid / LANES;
+    const int bx = by_xcd ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
+    const long base = (long)bx * COLS;
+    if (base >= N) return;  // (whole blocks)
+    const long col0 = base + cg * 8;
+    const half_t* a = A + (col0 + 8 <= N ? col0 : (long)N - 8);
+    const int c = tid % COLS, part = tid / COLS % PARTS, ps = tid / (COLS * PARTS);
+    if (tid < COLS) {
+#pragma unroll
+        for (int p = 0; p < PARTS; ++p) sums[p][c] = 0.0f;
+    }
+    float own = 0.0f;  // the last slice's sum
+    for (int s0 = 0; s0 < nslices; s0 += NS) {
+        const int s = s0 + worker / GROUPS, grp = worker % GROUPS;
+        float acc[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+        if (s < nslices && col0 < N) vm_sum_rows<true, GROUPS>(acc, a, lda, x, s * k_per_slice + grp, min(K, (s + 1) * k_per_slice));
+        vm_put_sums(red[worker / GROUPS][grp], acc, cg, base, N);
+        __syncthreads();
+        float v = red[ps][part][c];
+#pragma unroll
+        for (int i = 1; i < GROUPS / PARTS; ++i) v += red[ps][part + i * PARTS][c];
+        parts[ps][part][c] = v;
+        __syncthreads();  // (`parts` is read below before the next trip's first barrier, and written again behind it)
+        if (tid < COLS) {
+#pragma unroll
+            for (int i = 0; i < NS; ++i) {
+                float t = parts[i][0][c];
+#pragma unroll
+                for (int q = 1; q < PARTS; ++q) t += parts[i][q][c];
+                if (s0 + i == nslices - 1) own = t;
+                else if (s0 + i < nslices) sums[(s0 + i) % PARTS][c] += t;
+            }
+        }
+    }
+    if (tid < COLS && base + c < N) {
+        float r = sums[0][c];
+#pragma unroll
+        for (int q = 1; q < PARTS; ++q) r += sums[q][c];
+        r += own;
+        if (bias) r += (float)bias[base + c];
+        if (relu) r = relu_f32(r);
+        for (int o = 0; o < outs.count; ++o) outs.y[o][base + c] = (half_t)r;
+    }
 }
 
 // VM order, fewer than eight columns, or very few weights: 2-byte loads.  A block of 16 wavefronts owns 64 adjacent output

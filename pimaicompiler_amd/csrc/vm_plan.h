@@ -16,27 +16,28 @@ struct VmPlan {
     int by_xcd;           // neighbouring column blocks go to one XCD
     int slices;           // of the reduction; the partial sums of all but the last are exchanged in (slices - 1) * N words
     int rows_per_slice;
+    // The product's partial sums never meet those of another caller: it has words of its own where the stream has a region for
+    // it, and runs without any elsewhere (vm_needs_no_workspace).
+    bool needs_no_workspace;
 };
+
+// Weights of at most this many bytes, and operands of no whole 16-byte pieces, touch no workspace a caller would have to order
+// replays of a graph, or calls of the static entry point, against.
+static constexpr int64_t kVmSmallWeightBytes = 256 * 1024;
+inline bool vm_needs_no_workspace(int64_t K, int64_t N, int64_t lda, uintptr_t weight, uintptr_t results)
+{
+    return K * N * 2 <= kVmSmallWeightBytes || N % 8 != 0 || lda % 8 != 0 || (weight & 15u) != 0 || (results & 15u) != 0;
+}
 
 // The most words the partial sums of any product take: below, (slices - 1) * col_blocks is less than the target, which is at
 // most num_cus, and a column block has at most 128 columns.  A workspace of this size never has to grow.
 inline size_t vm_max_partials(int num_cus) { return (size_t)num_cus * 128; }
 
-inline void vm_cut(VmPlan& p, int64_t K, int slices)
-{
-    const int row_groups = kVmWaves * 64 / p.lanes_per_row;
-    int64_t rows = (K + slices - 1) / slices;
-    rows = (rows + row_groups - 1) / row_groups * row_groups;
-    if (rows < row_groups) rows = row_groups;  // K == 0: one empty slice, y = act(bias)
-    p.rows_per_slice = (int)rows;
-    p.slices = (int)((K + rows - 1) / rows);
-    if (p.slices < 1) p.slices = 1;
-}
-
-// N >= 8 outputs, K rows of pitch lda at address `weight`.
-inline VmPlan vm_plan(int64_t K, int64_t N, int64_t lda, uintptr_t weight, int num_cus)
+// N >= 8 outputs, K rows of pitch lda at address `weight`; `results`: the addresses of all destinations, or-ed.
+inline VmPlan vm_plan(int64_t K, int64_t N, int64_t lda, uintptr_t weight, uintptr_t results, int num_cus)
 {
     VmPlan p;
+    p.needs_no_workspace = vm_needs_no_workspace(K, N, lda, weight, results);
     // Block width: 64 columns (8 lanes per weight row) while the weight is small, so that more blocks share it: 2048 x 2048
     // 3.5 us against 4.2 with 128 columns, 12896 x 84 4.0 against 6.7.  128 columns for a weight past kVmLargeWeightBytes, whose
     // stream is the bound: 4096 x 4096 7.7 us against 8.2 with 64, 1024 x 32000 11.2 against 13.7.
@@ -57,7 +58,14 @@ inline VmPlan vm_plan(int64_t K, int64_t N, int64_t lda, uintptr_t weight, int n
     int slices = (int)((target + p.col_blocks / 2) / p.col_blocks);  // rounded: 250 column blocks on 256 CUs are not sliced
     if (K <= 512) slices = 1;
     while (slices > 1 && (int64_t)slices * slices * 40 > K) --slices;
-    vm_cut(p, K, slices < 1 ? 1 : slices);
+    if (slices < 1) slices = 1;
+    const int row_groups = kVmWaves * 64 / p.lanes_per_row;
+    int64_t rows = (K + slices - 1) / slices;
+    rows = (rows + row_groups - 1) / row_groups * row_groups;
+    if (rows < row_groups) rows = row_groups;  // K == 0: one empty slice, y = act(bias)
+    p.rows_per_slice = (int)rows;
+    p.slices = (int)((K + rows - 1) / rows);
+    if (p.slices < 1) p.slices = 1;
     return p;
 }
 }  // namespace pimhip

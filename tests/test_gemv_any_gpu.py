@@ -81,33 +81,72 @@ def test_i_x_w_at_the_edges_of_blocks_row_groups_and_slices(ops, in_w, out_w, of
     torch.cuda.synchronize()
 
 
-def test_an_odd_product_is_recorded_on_a_stream_without_a_workspace(ops):
-    """Operands that need no workspace in one slice run so where the stream cannot get one: inside a capture on a fresh
-    stream, and through the entry point that never allocates."""
+PER_THREAD_STREAM = 2   # hipStreamPerThread
+
+
+@pytest.mark.parametrize("in_w,out_w,off,pitch", [
+    (520, 9, 0, 0), (1024, 64, 0, 0), (8192, 8, 0, 0), (1000, 33, 1, 0), (1500, 2001, 0, 0), (4951, 1301, 3, 0), (12896, 84, 0, 0), (16384, 257, 0, 5),
+    (2048, 1024, 0, 4), (2100, 4001, 0, 0), (9000, 2001, 0, 7)])   # the last two: more than 16 MB, and one of them in several slices
+def test_small_and_odd_products_have_the_same_bits_wherever_they_run(ops, in_w, out_w, off, pitch):
+    """Products that need no workspace: the same sums in the same order on a stream with a region, on one without, inside a capture on
+    a stream that has never run one, in every replay beside other work of the capture stream, and through the static entry point."""
     from pimaicompiler_amd import _lib as L
     lib = L.load()
-    g = torch.Generator().manual_seed(4)
-    k, n = 1500, 2001
-    A, x = (0.1 * torch.randn(k, n, generator=g)).half().to(DEV), torch.randn(k, generator=g).half().to(DEV)
-    y = torch.empty(n, dtype=torch.float16, device=DEV)
+    g = torch.Generator().manual_seed(in_w + out_w)
+    ld = out_w + pitch
+    A = at_offset((0.1 * torch.randn(in_w, ld, generator=g)).half(), off)
+    x = at_offset(torch.randn(in_w, generator=g).half(), off)
+    b = torch.randn(out_w, generator=g).half().to(DEV)
+    eager = call(L.PIMHIP_I_X_W, A, x, b, in_w, out_w, ld, True, off)
+    check(eager, A[:, :out_w].t(), x, b, True)
+    y = torch.empty(out_w, dtype=torch.float16, device=DEV)
+
+    def launch(fn, stream):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        assert fn(y.data_ptr(), x.data_ptr(), A.data_ptr(), b.data_ptr(), in_w, out_w, ld, L.PIMHIP_ACT_RELU, L.PIMHIP_I_X_W, stream) == 0
+        torch.cuda.synchronize()
+        return y
+    main = torch.cuda.current_stream()
+    assert torch.equal(launch(lib.pimhip_execute_gemv_static, main.cuda_stream), eager)
+    assert torch.equal(launch(lib.pimhip_execute_gemv, PER_THREAD_STREAM), eager)
+    side = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    side.wait_stream(main)
+    with torch.cuda.graph(graph, stream=side):
+        assert lib.pimhip_execute_gemv(y.data_ptr(), x.data_ptr(), A.data_ptr(), b.data_ptr(), in_w, out_w, ld, L.PIMHIP_ACT_RELU, L.PIMHIP_I_X_W,
+                                       torch.cuda.current_stream().cuda_stream) == 0
+    others = [torch.empty(out_w, dtype=torch.float16, device=DEV) for _ in range(8)]
+    for _ in range(3):
+        y.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for o in others:                                   # on the capture stream, while the graph is replayed on another one
+            assert lib.pimhip_execute_gemv(o.data_ptr(), x.data_ptr(), A.data_ptr(), b.data_ptr(), in_w, out_w, ld, L.PIMHIP_ACT_RELU,
+                                           L.PIMHIP_I_X_W, side.cuda_stream) == 0
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, eager) and all(torch.equal(o, eager) for o in others)
+
+
+def test_a_product_with_one_odd_destination_needs_no_workspace(ops):
+    """Several destinations: one that is not 16-byte aligned is enough."""
+    g = torch.Generator().manual_seed(6)
+    k, n = 2048, 512
+    A, x = (0.1 * torch.randn(1, k, n, generator=g)).half().to(DEV), torch.randn(1, 1, k, generator=g).half().to(DEV)
+    buf = torch.zeros(2, n + 8, dtype=torch.float16, device=DEV)
+    outs = [buf[0, :n], buf[1, 1:n + 1]]
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     graph = torch.cuda.CUDAGraph()
-    with torch.cuda.graph(graph, stream=side):
-        assert lib.pimhip_execute_gemv(y.data_ptr(), x.data_ptr(), A.data_ptr(), None, k, n, 0, L.PIMHIP_ACT_NONE, L.PIMHIP_I_X_W,
-                                       torch.cuda.current_stream().cuda_stream) == 0
+    with torch.cuda.graph(graph, stream=side):            # (refused if it needed the stream's workspace)
+        ops.aten_bmm(x, A, outs=outs)
     for _ in range(3):
-        y.fill_(float("nan"))
+        buf.zero_()
         graph.replay()
         torch.cuda.synchronize()
-        check(y, A.t(), x, None, False)
-    k, n = 9000, 30001                                      # more partial sums than the static scratch array holds
-    A, x = (0.1 * torch.randn(k, n, generator=g)).half().to(DEV), torch.randn(k, generator=g).half().to(DEV)
-    y = torch.empty(n, dtype=torch.float16, device=DEV)
-    assert lib.pimhip_execute_gemv_static(y.data_ptr(), x.data_ptr(), A.data_ptr(), None, k, n, 0, L.PIMHIP_ACT_NONE, L.PIMHIP_I_X_W,
-                                          torch.cuda.current_stream().cuda_stream) == 0
-    torch.cuda.synchronize()
-    check(y, A.t(), x, None, False)
+        for o in outs:
+            check(o, A[0].t(), x.view(-1), None, False)
+        assert bool((buf[0, n:] == 0).all()) and float(buf[1, 0]) == 0
 
 
 def test_a_recorded_product_outlives_a_larger_one_on_its_stream(ops):

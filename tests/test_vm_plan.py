@@ -17,8 +17,9 @@ int main()
     long long K, N, lda, addr;
     int cus;
     while (scanf("%lld %lld %lld %lld %d", &K, &N, &lda, &addr, &cus) == 5) {
-        const pimhip::VmPlan p = pimhip::vm_plan(K, N, lda, (uintptr_t)addr, cus);
-        printf("%d %d %d %d %zu\n", p.lanes_per_row, p.col_blocks, p.slices, p.rows_per_slice, pimhip::vm_max_partials(cus));
+        // (the results' address is given in the upper half of the weight's)
+        const pimhip::VmPlan p = pimhip::vm_plan(K, N, lda, (uintptr_t)(addr & 0xffff), (uintptr_t)(addr >> 16), cus);
+        printf("%d %d %d %d %zu %d\n", p.lanes_per_row, p.col_blocks, p.slices, p.rows_per_slice, pimhip::vm_max_partials(cus), (int)p.needs_no_workspace);
     }
 }
 """
@@ -46,10 +47,22 @@ def test_partial_sums_of_every_product_fit_a_workspace_of_one_size(plans):
     """A workspace never grows, so no recorded graph can be left with the address of a freed one."""
     cases = [(k, n, n, 0, cus) for k, n, cus in itertools.product((0, 1) + SIZES, SIZES, (32, 64, 256, 304))]
     sliced = 0
-    for (k, n, _, _, cus), (lanes, blocks, slices, rows, words) in zip(cases, plans(cases)):
+    for (k, n, _, _, cus), (lanes, blocks, slices, rows, words, _) in zip(cases, plans(cases)):
         assert blocks == -(-n // (8 * lanes)) and slices >= 1
         assert (slices - 1) * rows < max(k, 1) <= max(slices * rows, 1) or k == 0   # the slices cover K, none is empty
         assert (slices - 1) * n <= words, (k, n, cus)
         assert words <= 64 * 1024 or cus > 512                                       # the static scratch array holds them as well
         sliced += slices > 1
     assert sliced > 100
+
+
+def test_small_and_odd_products_need_no_workspace(plans):
+    """Weights of at most 256 KB, and operands of no whole 16-byte pieces (sizes, pitch, either address, any destination)."""
+    cases, want = [], []
+    for k, n, pitch, weight, results in itertools.product((513, 1024, 4951), (8, 64, 128, 136, 1301, 2048), (0, 3, 8), (0, 2, 8, 64), (0, 2, 48)):
+        cases.append((k, n, n + pitch, weight | results << 16, 256))
+        want.append(k * n * 2 <= 256 * 1024 or n % 8 != 0 or (n + pitch) % 8 != 0 or weight % 16 != 0 or results % 16 != 0)
+    got = plans(cases)
+    assert [bool(g[5]) for g in got] == want
+    # ... and are cut like any other product of their size, so that their sums do not depend on where the records are
+    assert all(g[2:4] == h[2:4] for g, h in zip(got, plans([(k, n, n, 0, cus) for k, n, _, _, cus in cases])))
