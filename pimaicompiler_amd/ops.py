@@ -569,7 +569,9 @@ class LstmPlan:
         lib = L.load()
         _require_half_cuda(*params)
         _ensure_init(params[0])
-        self.params = [p.contiguous() for p in params]  # keeps the weights alive for the plan's lifetime
+        # Keeps the weights' memory for the plan's lifetime: tensors of its own, which stay where they are when the caller's are
+        # given other memory (`p.data = ...`, Module.half(), Module.to()).
+        self.params = [p.contiguous().detach() for p in params]
         self.has_biases = bool(has_biases)
         self.num_layers = int(num_layers)
         self.num_dirs = 2 if bidirectional else 1
@@ -921,10 +923,11 @@ def _overlap(a, b):
     return a.numel() > 0 and b.numel() > 0 and a0 < b0 + b.numel() * b.element_size() and b0 < a0 + a.numel() * a.element_size()
 
 
-# Plans of aten_lstm1/2 calls, found again by their weights.  An entry keeps the caller's own tensors (so their
-# addresses cannot be reused by other weights while it lives) and their version counters: a plan holds values derived
-# from the weights (b_ih + b_hh, w_ih in matrix-core order, contiguous copies), so an in-place update of a weight makes
-# it stale, and the next call builds a new one.  Updates torch does not count (writes through data_ptr from other
+# Plans of aten_lstm1/2 calls, found again by their weights.  An entry (plan, kept, versions, params) holds the memory of the
+# weights through tensors of its own, `kept`: their addresses, which make the key, cannot be reused by other weights while it
+# lives, also where the caller's tensors `params` have been given other memory since.  And it holds their version counters: a
+# plan has values derived from the weights (b_ih + b_hh, w_ih in matrix-core order, contiguous copies), so an in-place update of a
+# weight makes it stale, and the next call builds a new one.  Updates torch does not count (writes through data_ptr from other
 # libraries) need invalidate_lstm_plans.  At most PLAN_CACHE_MAX plans are kept; the least recently used one goes first.
 PLAN_CACHE_MAX = 64
 _plan_cache = collections.OrderedDict()
@@ -943,7 +946,7 @@ def _plan_for(params, has_biases, num_layers, bidirectional, seq_len):
     if plan is None or plan.max_seq_len < seq_len:
         cap = max(int(seq_len), 2 * plan.max_seq_len if plan is not None else 0, 16)
         plan = LstmPlan(params, has_biases, num_layers, bidirectional, cap)
-        _plan_cache[key] = (plan, list(params), versions)
+        _plan_cache[key] = (plan, [p.detach() for p in params], versions, list(params))
     _plan_cache.move_to_end(key)
     while len(_plan_cache) > PLAN_CACHE_MAX:
         _plan_cache.popitem(last=False)
@@ -959,7 +962,8 @@ def invalidate_lstm_plans(params=None):
         _plan_cache.clear()
         return n
     ptrs = {p.data_ptr() for p in params}
-    stale = [k for k, entry in _plan_cache.items() if ptrs.intersection(p.data_ptr() for p in entry[1])]
+    # (the addresses a plan was built for, and where its tensors are now)
+    stale = [k for k, (_, kept, _, tensors) in _plan_cache.items() if ptrs.intersection(p.data_ptr() for p in kept + tensors)]
     for k in stale:
         del _plan_cache[k]
     return len(stale)
