@@ -130,6 +130,22 @@ __global__ void xcc_map_kernel(unsigned int* out)
     if (threadIdx.x == 0) out[blockIdx.x] = hw_xcc_id();
 }
 
+// Whether the per-XCD kernel multiplies on v_dot2 or on sparse matrix instructions.  The latter take whole groups of 256 columns,
+// v_dot2 of 128, their chain is longer and their weights pass through LDS first (1 to 1.6 us per launch).  Measured on MI355X
+// (graph replays, us per call, v_dot2 / sparse):
+//   one direction or both  64 units, 80 steps 73.8 / 84.5   384 (80) 93.2 / 95.2   512 (20) 31.0 / 31.1 (240) 280 / 271   640 (240) 300 / 312
+//                          768 (80) 115.0 / 115.4 (240) 317 / 315   896 (20) 42.2 / 43.0 (80) 122.6 / 120.9   1024 (10) 31.7 / 32.1 (20) 45.7 / 45.0 (80) 131 / 123
+//   two layers             128 (80) 90 / 94   256 (5) 19.5 / 19.9 (10) 24.9 / 24.8 (80) 100 / 97   640 (10) 30.8 / 32.1 (80) 127 / 123
+//                          1024 (5) 32.9 / 33.8 (10) 40.7 / 39.9 (20) 56.5 / 52.4
+bool xcd_on_dot(int64_t H, int64_t T, bool pipeline)
+{
+    if (pipeline) return H <= 128 || T < (H > 512 && H <= 640 ? 24 : 10);
+    if (H > 896) return T < 16;
+    if (H > 768) return T < 48;
+    if (H > 640) return T < 96;
+    return H <= 384 || H > 512 || T < 32;
+}
+
 // The per-XCD kernel finds its place by the hardware's XCC_ID and relies on two things the hardware does today: ids 0..7,
 // and workgroup b of a launch going to XCD (b + o) % 8 for some start o.  One probe launch of the same grid tells whether
 // this device, as this process sees it (CU masks, partition mode), behaves so; where it does not, the kernel is not offered.
@@ -294,9 +310,12 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
     if (H <= kXcdMaxH && plan->num_cus == kXcdCount * kXcdMembers) {
         int per_cu = 0;
         int per_cu_pipe = 0;
+        int per_cu_dot = 0, per_cu_pipe_dot = 0;
         PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lstm_xcd_f16_kernel<false>, kXcdThreads, 0));
         PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_pipe, lstm_xcd_f16_kernel<true>, kXcdThreads, 0));
-        plan->xcd_ok = per_cu >= 1 && per_cu_pipe >= 1;
+        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_dot, lstm_xcd_dot_f16_kernel<false>, kXcdThreads, 0));
+        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_pipe_dot, lstm_xcd_dot_f16_kernel<true>, kXcdThreads, 0));
+        plan->xcd_ok = per_cu >= 1 && per_cu_pipe >= 1 && per_cu_dot >= 1 && per_cu_pipe_dot >= 1;
         if (plan->xcd_ok) {
             bool rotation = false;
             const int rc_probe = xcd_dispatch_is_a_rotation(kXcdCount * kXcdMembers, s, &rotation);
@@ -304,8 +323,10 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
             plan->xcd_ok = rotation;
         }
         int per_cu_res = 0;
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_res, lstm_xcd_res_f16_kernel, kXcdThreads, 0));
-        plan->xcd_res_ok = plan->xcd_ok && per_cu_res >= 1;
+        int per_cu_res_dot = 0;
+        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_res, lstm_xcd_res_f16_kernel<XcdSparse>, kXcdThreads, 0));
+        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_res_dot, lstm_xcd_res_f16_kernel<XcdDot>, kXcdThreads, 0));
+        plan->xcd_res_ok = plan->xcd_ok && per_cu_res >= 1 && per_cu_res_dot >= 1;
     }
     if (plan->xcd_ok) {
         const size_t words = (size_t)kXcdRegionWords * kXcdMaxChains;
@@ -624,10 +645,10 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             a.H = (int)H;
             a.T = (int)T;
             a.spin_limit = plan->spin_limit;
-            if (any_res)
-                lstm_xcd_res_f16_kernel<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
-            else
-                lstm_xcd_f16_kernel<true><<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
+            const bool dot = xcd_on_dot(H, T, true);
+            auto kernel = any_res ? (dot ? lstm_xcd_res_f16_kernel<XcdDot> : lstm_xcd_res_f16_kernel<XcdSparse>)
+                                  : (dot ? lstm_xcd_dot_f16_kernel<true> : lstm_xcd_f16_kernel<true>);
+            kernel<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
             PIMHIP_HIP_CHECK(hipGetLastError());
             layer_in = group_out;
             l += n;
@@ -671,7 +692,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             a.H = (int)H;
             a.T = (int)T;
             a.spin_limit = plan->spin_limit;
-            lstm_xcd_f16_kernel<false><<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
+            (xcd_on_dot(H, T, false) ? lstm_xcd_dot_f16_kernel<false> : lstm_xcd_f16_kernel<false>)<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
             if (residual(l)) add_input(layer_out, layer_in);
             PIMHIP_HIP_CHECK(hipGetLastError());
             layer_in = layer_out;

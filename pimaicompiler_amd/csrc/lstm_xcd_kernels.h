@@ -36,14 +36,19 @@
 // waiting.  All groups then advance at the rate of one group, L layers in about the time of one.
 //
 // A workgroup has eight wavefronts; wavefront w owns hidden units 32 * rank + 4 * w .. + 3, whose 16 gate rows it keeps in 128
-// registers per lane for the whole sequence, as 16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16.  Per step: the first two
-// wavefronts fetch the group's entries into LDS (16 bytes per lane), one barrier, 16 matrix instructions, which leave the four gates of
-// unit (l >> 2) & 3 in the lanes of that quad, the gate arithmetic, and one 8-byte store of the wavefront's four new h values
-// into the workgroup's entry.  What bounds a step (1.30 us at H = 1024, 1.05 at 320, where nearly all of it is this): the
-// store becoming visible in the L2 and the poll that finds it, 0.43 us at best for such a round; 0.21 us are matrix instructions.
-// The products on v_dot2 with a reduction over 16 lanes: 1.49 us (one layer), 1.57 (pipelines of layers).
-// Few units are the other way round: up to about 256 the step's chain through the matrix instructions is longer than v_dot2's was
-// (80 steps of both directions of 64 units 84.5 us against 74, of 256 89.7 against 86, of 512 96 against 102).
+// registers per lane for the whole sequence.  Per step: the first wavefronts fetch the group's entries into LDS (16 bytes per lane),
+// one barrier, the 16 rows' products with h, the gate arithmetic, and one 8-byte store of the wavefront's four new h values into the
+// workgroup's entry.  What bounds a step: the store becoming visible in the L2 and the poll that finds it, 0.43 us at best
+// for such a round, and a chain of dependent instructions between two rounds.
+// The products come in two kinds, chosen by size and length (xcd_on_dot in api_lstm.hip, with the figures):
+//   XcdSparse  16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16: 0.21 us of matrix instructions at H = 1024; a step 1.30 us
+//              (a single layer; v_dot2 1.49, in pipelines of layers 1.57)
+//   XcdDot     v_dot2 and a transposing reduction over 16 lanes: half the columns per group of instructions that an unused part
+//              of h is skipped in, a shorter chain for few units (64 units 0.85 us a step against 0.98), nothing through LDS at
+//              the start of a launch
+// Against 64 bits the sums are equally far off (rms error over the sum of the products' magnitudes, 64 .. 1024 columns, MI355X): signs
+// mixed 4.7e-9 .. 9.7e-9 on v_dot2 and 3.2e-9 .. 7.9e-9 sparse, all of one sign 3.4e-8 .. 5.2e-8 and 3.5e-8 .. 4.9e-8; an h made
+// from the same previous h differs from its 64-bit value by 2.07e-4 relative with either, the rounding to fp16.
 #pragma once
 
 #include <type_traits>
@@ -126,13 +131,91 @@ __device__ __forceinline__ void store8_plain(void* p, unsigned long long v)
     asm volatile("global_store_dwordx2 %0, %1, off" : : "v"(p), "v"(w) : "memory");
 }
 
-// The 16-bit values that quads 0 .. 3 of a row of 16 lanes hold (one per quad, in all its lanes), as one 64-bit word in lane 0 of
-// the row: quad 1 is quad 0's mirror within half the row, quads 2 and 3 lie half a row further.
-__device__ __forceinline__ unsigned long long pack_quads(unsigned int v16)
-{
-    const unsigned int lo = v16 | (dpp_u32<kDppRowHalfMirror>(v16) << 16);
-    return (unsigned long long)lo | ((unsigned long long)dpp_u32<kDppRowRor8>(lo) << 32);
-}
+// ---- the step's matrix-vector product on v_dot2 ----
+// Row l >> 4 of 16 lanes has the wavefront's unit l >> 4: its lanes keep, of the four gate rows, the 8-wide column pieces
+// 16 c + (l & 15), c = 0 .. 7.  Four dot products of up to 64 columns per lane, then a transposing reduction over the 16 lanes.
+struct XcdDot {
+    half8_t w[4][8];
+
+    static __device__ __forceinline__ int unit(int lane) { return lane >> 4; }
+    static __device__ __forceinline__ int gate(int lane) { return (lane >> 2) & 3; }
+    static __device__ __forceinline__ bool first_of_gate(int lane) { return (lane & 3) == 0; }
+    static __device__ __forceinline__ bool first_of_unit(int lane) { return (lane & 15) == 0; }
+
+    __device__ __forceinline__ void load(const half_t* src, int u0, int, int lane, int H, bool ok)
+    {
+        half8_t zero;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                const int col = (16 * c + (lane & 15)) * 8;  // H % 8 == 0: a piece is entirely in or out of range
+                w[g][c] = (ok && col < H) ? *reinterpret_cast<const half8_t*>(src + ((long)g * H + u0 + (lane >> 4)) * H + col) : zero;
+            }
+        }
+    }
+
+    struct Sums {
+        __device__ __forceinline__ void clear() {}
+    };
+
+    // In every lane: the dot product of its unit's gate row gate(lane) with hb[0 .. H).
+    __device__ __forceinline__ float matvec(const half_t* hb, Sums&, int H, int lane) const
+    {
+        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            if (c * 128 >= H) break;  // (uniform) column pieces 16 c .. 16 c + 15 lie past the hidden state
+            const half8_t hv = *reinterpret_cast<const half8_t*>(hb + (16 * c + (lane & 15)) * 8);
+#pragma unroll
+            for (int g = 0; g < 4; ++g) acc[g] = dot8(w[g][c], hv, acc[g]);
+        }
+        // Each stage halves the number of values a lane holds and doubles the lanes they are summed over: mirrored lanes of
+        // the row (l ^ 15), mirrored lanes of half a row (l ^ 7), the quad.
+        const bool b3 = lane & 8, b2 = lane & 4;
+        float v2[2];
+#pragma unroll
+        for (int r = 0; r < 2; ++r) v2[r] = (b3 ? acc[2 + r] : acc[r]) + dpp_mov_f32<kDppRowMirror>(b3 ? acc[r] : acc[2 + r]);
+        float v = (b2 ? v2[1] : v2[0]) + dpp_mov_f32<kDppRowHalfMirror>(b2 ? v2[0] : v2[1]);
+        v += dpp_mov_f32<kDppQuadXor1>(v);
+        v += dpp_mov_f32<kDppQuadXor2>(v);
+        return v;
+    }
+
+    // The activated gates of a unit, right in the lanes of gate 0: f in the mirror within half the row (l ^ 7), o in the mirror
+    // within the row (l ^ 15), g in the mirror of that one (l ^ 8).  (What the other lanes make of them is never used.)
+    static __device__ __forceinline__ void share(float act, float& i, float& f, float& g, float& o)
+    {
+        i = act;
+        f = dpp_mov_f32<kDppRowHalfMirror>(act);
+        o = dpp_mov_f32<kDppRowMirror>(act);
+        g = dpp_mov_f32<kDppRowMirror>(f);
+    }
+
+    // The four units' 16-bit values, which lanes 0, 16, 32 and 48 hold, as one word in lane 0 (other lanes: unspecified).
+    // v_permlane16_swap with both operands alike leaves lane 16's value beside lane 0's and lane 48's beside lane 32's;
+    // v_permlane32_swap then brings the upper pair down.  (v_readlane and scalar shifts: 1-5 % of a step more.)
+    static __device__ __forceinline__ unsigned long long pack(unsigned int v16)
+    {
+        unsigned int a = v16, b = v16;
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+        const unsigned int x = a | (b << 16);
+        unsigned int c = x, d = x;
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(c), "+v"(d));
+        return (unsigned long long)c | ((unsigned long long)d << 32);
+    }
+
+    // The lanes that fetch a 16-byte piece of h each, and which: all of wavefronts 0 and 1 (16 lanes of each of the eight: up to 6 %
+    // of a step more), or, in pipelines, 32 of the first four (all of two: up to 2 % more for up to 128 units).
+    template <bool PIPE>
+    static __device__ __forceinline__ bool polls(int wave, int lane, int& piece)
+    {
+        piece = PIPE ? wave * 32 + lane : wave * 64 + lane;
+        return PIPE ? (wave < 4 && lane < 32) : wave < 2;
+    }
+};
 
 // ---- the step's matrix-vector product on v_smfmac_f32_16x16x64_f16 ----
 // D[16 x 16] += A[16 x 64, two of every four columns present] . B[64 x 16]: the weights are the dense operand, 64 columns of
@@ -159,87 +242,125 @@ __device__ __forceinline__ half8_t xcd_h_operand(const half_t* hb, int s, int la
     return __builtin_shufflevector(*reinterpret_cast<const half4_t*>(src), *reinterpret_cast<const half4_t*>(src + 8), 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
-// A wavefront's fragments.  16 lanes on 16 rows, 64 bytes of each, is what a fragment would ask of memory: 3 us per launch slower
-// than whole 256-byte pieces of rows.  So all loads are issued that way (instruction 4 i + j: rows 4 j .. + 3, columns 128 i .. + 127)
-// and each 16 rows x 128 columns then change lanes through 4 KB of LDS of the wavefront's own, 16-byte piece p of row r in place
-// p ^ r.  Row n: gate n & 3 of unit u0 + (n >> 2).
-__device__ __forceinline__ void xcd_load_weights(half16_t (&w)[kXcdFrags], const half_t* src, half_t* stage, int u0, int lane, int H, bool ok)
-{
-    half8_t zero;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
-    half8_t raw[kXcdFrags / 2][4];
-#pragma unroll
-    for (int i = 0; i < kXcdFrags / 2; ++i) {
-        if (128 * i >= H) break;  // (uniform)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int n = 4 * j + (lane >> 4), col = 128 * i + 8 * (lane & 15);  // H % 8 == 0: a piece is entirely in or out of range
-            raw[i][j] = (ok && col < H) ? *reinterpret_cast<const half8_t*>(src + ((long)(n & 3) * H + u0 + (n >> 2)) * H + col) : zero;
-        }
-    }
-    const int n = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int i = 0; i < kXcdFrags / 2; ++i) {
-        if (128 * i >= H) {  // (uniform) nothing but zeros: 64 KB per CU and i that need not pass through LDS
-#pragma unroll
-            for (int m = 0; m < 2; ++m) w[2 * i + m] = __builtin_shufflevector(zero, zero, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
-            continue;
-        }
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int r = 4 * j + (lane >> 4);
-            *reinterpret_cast<half8_t*>(stage + r * 128 + ((lane & 15) ^ r) * 8) = raw[i][j];
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (one wavefront's LDS accesses stay in order; this keeps the compiler's too)
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            const half8_t lo = *reinterpret_cast<const half8_t*>(stage + n * 128 + ((8 * m + g) ^ n) * 8);
-            const half8_t hi = *reinterpret_cast<const half8_t*>(stage + n * 128 + ((8 * m + 4 + g) ^ n) * 8);
-            w[2 * i + m] = __builtin_shufflevector(lo, hi, 0, 1, 4, 5, 2, 3, 6, 7, 8, 9, 12, 13, 10, 11, 14, 15);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    }
-}
+struct XcdSparse {
+    half16_t w[kXcdFrags];
 
-// The accumulators of a step, cleared where the wavefront has nothing else to do (in front of its wait for h).
-struct XcdSums {
-    float4_t d[8];
-    __device__ __forceinline__ void clear()
+    // Lane l holds gate l & 3 of unit (l >> 2) & 3, in all four rows of 16 lanes.
+    static __device__ __forceinline__ int unit(int lane) { return (lane >> 2) & 3; }
+    static __device__ __forceinline__ int gate(int lane) { return lane & 3; }
+    static __device__ __forceinline__ bool first_of_gate(int lane) { return lane < 16; }
+    static __device__ __forceinline__ bool first_of_unit(int lane) { return lane < 16 && (lane & 3) == 0; }
+
+    // A wavefront's fragments.  16 lanes on 16 rows, 64 bytes of each, is what a fragment would ask of memory: 3 us per launch slower
+    // than whole 256-byte pieces of rows.  So all loads are issued that way (instruction 4 i + j: rows 4 j .. + 3, columns 128 i .. + 127)
+    // and each 16 rows x 128 columns then change lanes through 4 KB of LDS of the wavefront's own, 16-byte piece p of row r in place
+    // p ^ r.  Row n: gate n & 3 of unit u0 + (n >> 2).
+    __device__ __forceinline__ void load(const half_t* src, int u0, int wave, int lane, int H, bool ok)
     {
+        __shared__ __align__(16) half_t staged[kXcdWaves][16 * 128];
+        half_t* stage = staged[wave];
+        half8_t zero;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            d[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            asm volatile("" : "+v"(d[j]));
+        for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
+        half8_t raw[kXcdFrags / 2][4];
+#pragma unroll
+        for (int i = 0; i < kXcdFrags / 2; ++i) {
+            if (128 * i >= H) break;  // (uniform)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int n = 4 * j + (lane >> 4), col = 128 * i + 8 * (lane & 15);  // H % 8 == 0: a piece is entirely in or out of range
+                raw[i][j] = (ok && col < H) ? *reinterpret_cast<const half8_t*>(src + ((long)(n & 3) * H + u0 + (n >> 2)) * H + col) : zero;
+            }
         }
+        const int n = lane & 15, g = lane >> 4;
+#pragma unroll
+        for (int i = 0; i < kXcdFrags / 2; ++i) {
+            if (128 * i >= H) {  // (uniform) nothing but zeros: 64 KB per CU and i that need not pass through LDS
+#pragma unroll
+                for (int m = 0; m < 2; ++m) w[2 * i + m] = __builtin_shufflevector(zero, zero, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+                continue;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int r = 4 * j + (lane >> 4);
+                *reinterpret_cast<half8_t*>(stage + r * 128 + ((lane & 15) ^ r) * 8) = raw[i][j];
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (one wavefront's LDS accesses stay in order; this keeps the compiler's too)
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                const half8_t lo = *reinterpret_cast<const half8_t*>(stage + n * 128 + ((8 * m + g) ^ n) * 8);
+                const half8_t hi = *reinterpret_cast<const half8_t*>(stage + n * 128 + ((8 * m + 4 + g) ^ n) * 8);
+                w[2 * i + m] = __builtin_shufflevector(lo, hi, 0, 1, 4, 5, 2, 3, 6, 7, 8, 9, 12, 13, 10, 11, 14, 15);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
+    }
+
+    // The accumulators of a step, cleared where the wavefront has nothing else to do (in front of its wait for h).
+    struct Sums {
+        float4_t d[8];
+        __device__ __forceinline__ void clear()
+        {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                d[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                asm volatile("" : "+v"(d[j]));
+            }
+        }
+    };
+
+    // In every lane l: the dot product of gate row l & 15 of the wavefront with hb[0 .. H).
+    __device__ __forceinline__ float matvec(const half_t* hb, Sums& acc, int H, int lane) const
+    {
+        const int index = (lane & 1) ? 0xeeeeeeee : 0x44444444;  // columns 2, 3 / 0, 1 of every four
+        const half8_t h0 = xcd_h_operand(hb, 0, lane);
+        if (H <= 256) {  // (uniform) four fragments: half the sums and no second operand; the chain is all a step of few units has
+#pragma unroll
+            for (int m = 0; m < 4; ++m) acc.d[m] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(h0, w[m], acc.d[m], index, 0, 0);
+            const float f0 = (acc.d[0][0] + acc.d[0][1]) + (acc.d[1][2] + acc.d[1][3]);
+            const float f1 = (acc.d[2][0] + acc.d[2][1]) + (acc.d[3][2] + acc.d[3][3]);
+            return wave_sum_rows((lane & 32) ? 0.0f : (lane & 16) ? f1 : f0);
+        }
+        const half8_t h1 = xcd_h_operand(hb, 1, lane);
+#pragma unroll
+        for (int m = 0; m < kXcdFrags; ++m) {
+            if ((m & 3) == 0 && m * 64 >= H) break;  // (uniform) whole fragments past the hidden state are zeros
+            acc.d[m & 7] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(m < 8 ? h0 : h1, w[m], acc.d[m & 7], index, 0, 0);
+        }
+        // Row r of D lies in register r & 3 of lanes 16 (r >> 2) .. + 15: row group q keeps pairs 2 q (registers 0, 1) and 2 q + 1.
+        float f[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) f[q] = (acc.d[2 * q][0] + acc.d[2 * q][1]) + (acc.d[2 * q + 1][2] + acc.d[2 * q + 1][3]);
+        const float lo = (lane & 16) ? f[1] : f[0], hi = (lane & 16) ? f[3] : f[2];
+        return wave_sum_rows((lane & 32) ? hi : lo);
+    }
+
+    // The activated gates of a unit: the quad's four lanes share them.
+    static __device__ __forceinline__ void share(float act, float& i, float& f, float& g, float& o)
+    {
+        i = dpp_mov_f32<0x00>(act);  // quad_perm broadcasts of lanes 0, 1, 2, 3 of the quad
+        f = dpp_mov_f32<0x55>(act);
+        g = dpp_mov_f32<0xAA>(act);
+        o = dpp_mov_f32<0xFF>(act);
+    }
+
+    // The four units' 16-bit values, one per quad of a row of 16 lanes, as one word in lane 0 of the row: quad 1 is quad 0's mirror
+    // within half the row, quads 2 and 3 lie half a row further.
+    static __device__ __forceinline__ unsigned long long pack(unsigned int v16)
+    {
+        const unsigned int lo = v16 | (dpp_u32<kDppRowHalfMirror>(v16) << 16);
+        return (unsigned long long)lo | ((unsigned long long)dpp_u32<kDppRowRor8>(lo) << 32);
+    }
+
+    // The lanes that fetch a piece of h each: all of wavefronts 0 and 1.  Spread over eight wavefronts of 16 lanes a step takes
+    // 1.42 us, over four of 32 1.32, over two 1.31 (H = 1024).
+    template <bool PIPE>
+    static __device__ __forceinline__ bool polls(int wave, int lane, int& piece)
+    {
+        piece = wave * 64 + lane;
+        return wave < 2;
     }
 };
-
-// In every lane l: the dot product of gate row l & 15 of the wavefront with hb[0 .. H).
-__device__ __forceinline__ float xcd_matvec(const half16_t (&w)[kXcdFrags], const half_t* hb, XcdSums& acc, int H, int lane)
-{
-    const int index = (lane & 1) ? 0xeeeeeeee : 0x44444444;  // columns 2, 3 / 0, 1 of every four
-    const half8_t h0 = xcd_h_operand(hb, 0, lane);
-    if (H <= 256) {  // (uniform) four fragments: half the sums and no second operand; the chain is all a step of few units has
-#pragma unroll
-        for (int m = 0; m < 4; ++m) acc.d[m] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(h0, w[m], acc.d[m], index, 0, 0);
-        const float f0 = (acc.d[0][0] + acc.d[0][1]) + (acc.d[1][2] + acc.d[1][3]);
-        const float f1 = (acc.d[2][0] + acc.d[2][1]) + (acc.d[3][2] + acc.d[3][3]);
-        return wave_sum_rows((lane & 32) ? 0.0f : (lane & 16) ? f1 : f0);
-    }
-    const half8_t h1 = xcd_h_operand(hb, 1, lane);
-#pragma unroll
-    for (int m = 0; m < kXcdFrags; ++m) {
-        if ((m & 3) == 0 && m * 64 >= H) break;  // (uniform) whole fragments past the hidden state are zeros
-        acc.d[m & 7] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(m < 8 ? h0 : h1, w[m], acc.d[m & 7], index, 0, 0);
-    }
-    // Row r of D lies in register r & 3 of lanes 16 (r >> 2) .. + 15: row group q keeps pairs 2 q (registers 0, 1) and 2 q + 1.
-    float f[4];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) f[q] = (acc.d[2 * q][0] + acc.d[2 * q][1]) + (acc.d[2 * q + 1][2] + acc.d[2 * q + 1][3]);
-    const float lo = (lane & 16) ? f[1] : f[0], hi = (lane & 16) ? f[3] : f[2];
-    return wave_sum_rows((lane & 32) ? hi : lo);
-}
 
 // PIPE = false: groups that neither feed nor are fed across XCDs (a single layer, the two directions of one); everything
 // that concerns P groups and the hand-overs is compiled out, which is worth 10 % of a step.
@@ -247,13 +368,12 @@ __device__ __forceinline__ float xcd_matvec(const half16_t (&w)[kXcdFrags], cons
 // that hands the previous step's 32 h values to the layer above adds the layer's own input of that step, which it asked
 // for a step earlier, and stores y from there too (one step late; hn stays h).  Compiled in only for stacks that have such
 // layers.
-template <bool PIPE, bool RES>
+template <bool PIPE, bool RES, class Product>
 __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
 {
     __shared__ __align__(16) half_t hbuf[2][kXcdMaxH];  // h of the previous step, double buffered by step parity
     __shared__ __align__(16) float xring[kXcdWaves][32][4][4];  // per wavefront: [step & 31][gate][unit] projection terms
     __shared__ __align__(16) unsigned long long hout[2][kXcdWaves];  // the workgroup's 32 new h values, for the layer above
-    __shared__ __align__(16) half_t wstage[kXcdWaves][16 * 128];     // xcd_load_weights
     __shared__ unsigned short in_ring[2][kXcdUnitsPerBlock];        // RES: the layer's own input of the last two steps, for the sums
     // Raised by a wavefront one of whose waits gave up, always in front of a step's barrier, and read by all right behind
     // it: the workgroup then leaves the loop of steps together, publishes nothing more and computes its units by itself.
@@ -299,18 +419,18 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     if (tid == 0)
         claimed_before = __hip_atomic_exchange(p.claims + xcd * kXcdMembers + rank, g_base, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-    // ---- weights into registers: lane l holds gate l & 3 (LibTorch order i, f, g, o) of unit u0 + ((l >> 2) & 3)
+    // ---- weights into registers
     const int u0 = rank * kXcdUnitsPerBlock + wave * kXcdUnitsPerWave;
     const bool units_ok = u0 < H;  // H % 8 == 0: the four units of a wavefront are all inside or all outside
-    const int my_unit = u0 + ((lane >> 2) & 3);
-    const int my_gate = lane & 3;
-    const half_t* wsrc = is_proj ? pj.w_ih : ch.w_hh;
-    half16_t w[kXcdFrags];
+    const int unit = Product::unit(lane);  // of the wavefront's four
+    const int my_unit = u0 + unit;
+    const int my_gate = Product::gate(lane);  // (LibTorch order i, f, g, o)
+    Product weights;
+    weights.load(is_proj ? pj.w_ih : ch.w_hh, u0, wave, lane, H, units_ok);
     {
         half8_t zero;
 #pragma unroll
         for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
-        xcd_load_weights(w, wsrc, wstage[wave], u0, lane, H, units_ok);
         for (int i = tid; i < 2 * kXcdMaxH / 8; i += kXcdThreads) reinterpret_cast<half8_t*>(&hbuf[0][0])[i] = zero;
     }
     if (tid == 0 && claimed_before == g_base) {
@@ -322,11 +442,10 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     __syncthreads();
 
     const int uc = units_ok ? my_unit : H - 1;
-    // The lanes of wavefronts 0 and 1 fetch piece 64 w + lane of an h vector: 8 fp16 = columns 8 q .. 8 q + 7.  Few wavefronts with
-    // all their lanes: spread over eight of 16 lanes a step takes 1.42 us, over four of 32 1.32, over two 1.31 (H = 1024).  (The
-    // wavefronts that talk to other XCDs, 4 .. 7, never poll: a wavefront's loads come back in order.)
-    const int piece = wave * 64 + lane;
-    const bool polls = wave < 2 && piece * 8 < H;
+    // Lanes of the first wavefronts fetch one piece of an h vector each: 8 fp16 = columns 8 q .. 8 q + 7.  (The wavefronts that talk
+    // to other XCDs, 4 .. 7, never poll: a wavefront's loads come back in order.)
+    int piece;
+    const bool polls = Product::template polls<PIPE || RES>(wave, lane, piece) && piece * 8 < H;
 
     // One bounded wait: `again` loads and tests; gives up like every wait of this kernel, after spin_limit polls, and
     // also after kXcdWaitTicks of the constant 100 MHz clock, however long a poll takes in the environment the kernel
@@ -367,7 +486,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         }
         for (int t = 0; t < T; ++t) {
             half_t* hb = hbuf[t & 1];
-            XcdSums acc;
+            typename Product::Sums acc;
             acc.clear();
             if (polls) {
                 const unsigned long long* src = reinterpret_cast<const unsigned long long*>(pj.seq_in + (long)t * H + piece * 8);
@@ -390,9 +509,9 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
                 lo = __hip_atomic_load(nxt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 hi = __hip_atomic_load(nxt + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            const float v = xcd_matvec(w, hb, acc, H, lane) + bias;
+            const float v = weights.matvec(hb, acc, H, lane) + bias;
             if (dead) return;  // rows made from a stale h must not reach the recurrence: it will make its own
-            if (units_ok && lane < 16)
+            if (units_ok && Product::first_of_gate(lane))
                 __hip_atomic_store(reinterpret_cast<unsigned int*>(dst + (long)t * 4 * H), __builtin_bit_cast(unsigned int, v), __ATOMIC_RELAXED,
                                    __HIP_MEMORY_SCOPE_AGENT);
         }
@@ -460,7 +579,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     const unsigned int* xp_mine = reinterpret_cast<const unsigned int*>(ch.xproj + (long)my_gate * H + uc);  // + t * 4H
     const bool fetcher = wave >= 4;
     const unsigned int* xp_other =
-        reinterpret_cast<const unsigned int*>(ch.xproj + (long)my_gate * H + min(max(u0 - 16, 0) + ((lane >> 2) & 3), H - 1));  // wavefront w - 4's
+        reinterpret_cast<const unsigned int*>(ch.xproj + (long)my_gate * H + min(max(u0 - 16, 0) + unit, H - 1));  // wavefront w - 4's
     auto xp_bits_at = [&](int t) { return __hip_atomic_load(xp_mine + (long)t * 4 * H, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
     auto wait_xp = [&](int t) {
         unsigned int bits = 0xffffffffu;
@@ -478,13 +597,13 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     } else {
         // Let the P group get kXcdLag steps ahead, then take the first two rows.
         (void)wait_xp(min(kXcdLag, T - 1));
-        reinterpret_cast<unsigned int&>(xring[wave][0][my_gate][(lane >> 2) & 3]) = wait_xp(0);
-        reinterpret_cast<unsigned int&>(xring[wave][1][my_gate][(lane >> 2) & 3]) = wait_xp(min(1, T - 1));
+        reinterpret_cast<unsigned int&>(xring[wave][0][my_gate][unit]) = wait_xp(0);
+        reinterpret_cast<unsigned int&>(xring[wave][1][my_gate][unit]) = wait_xp(min(1, T - 1));
     }
 
     for (int s = 0; s < T; ++s) {
         half_t* hb = hbuf[s & 1];
-        XcdSums acc;
+        typename Product::Sums acc;
         acc.clear();
         if (!polled) {
             // steps s + 16 .. s + 31 are fetched when step s starts a half, and written over the half that has just been
@@ -493,8 +612,8 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             if ((s & 15) == 1 && s > 1) deposit_xp(((s >> 4) & 1) ^ 1, xp_next);
         } else if (fetcher && s >= 1 && s + 1 < T) {
             // loaded during step s - 1; read (by this wavefront and by wavefront w - 4) after the barrier of step s + 1
-            reinterpret_cast<unsigned int&>(xring[wave][(s + 1) & 31][my_gate][(lane >> 2) & 3]) = xp_ahead;
-            reinterpret_cast<unsigned int&>(xring[wave - 4][(s + 1) & 31][my_gate][(lane >> 2) & 3]) = xp_ahead_other;
+            reinterpret_cast<unsigned int&>(xring[wave][(s + 1) & 31][my_gate][unit]) = xp_ahead;
+            reinterpret_cast<unsigned int&>(xring[wave - 4][(s + 1) & 31][my_gate][unit]) = xp_ahead_other;
         }
         if (sums && s > 0) in_ring[(s - 1) & 1][lane & 31] = in_ahead;  // read after this step's barrier
         // ---- 1. h of the previous step into LDS
@@ -538,32 +657,30 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         }
 
         // ---- 2. the wavefront's 16 gate rows
-        const float dot = xcd_matvec(w, hb, acc, H, lane);
-        unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][(lane >> 2) & 3]);
+        const float dot = weights.matvec(hb, acc, H, lane);
+        unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][unit]);
         if (polled && xp_bits == 0xffffffffu) xp_bits = wait_xp(s);  // the P group had not got there when it was fetched
         const float a = dot + __builtin_bit_cast(float, xp_bits);
         const int t = rev ? (T - 1 - s) : s;
 
-        // Every lane activates its own gate; the quad's four lanes (one unit) then share them and all make the unit's c and h.
+        // Every lane activates its own gate; the lanes of a unit then share them.
         const bool is_g = my_gate == 2;
         const float sg = fast_sigmoid_f32(is_g ? 2.0f * a : a);
         const float act = is_g ? 2.0f * sg - 1.0f : sg;
-        const float g_i = dpp_mov_f32<0x00>(act);  // quad_perm broadcasts of lanes 0, 1, 2, 3 of the quad
-        const float g_f = dpp_mov_f32<0x55>(act);
-        const float g_g = dpp_mov_f32<0xAA>(act);
-        const float g_o = dpp_mov_f32<0xFF>(act);
+        float g_i, g_f, g_g, g_o;
+        Product::share(act, g_i, g_f, g_g, g_o);
         const float c_new = g_f * c_reg + g_i * g_g;
         const bool h_is_number = (c_new == c_new) && (g_o == g_o);
         const half_t h = (half_t)(g_o * (2.0f * fast_sigmoid_f32(2.0f * c_new) - 1.0f));
         c_reg = c_new;
 
-        // ---- 3. the wavefront's four h values: a quad each; lane 0 stores y and publishes
+        // ---- 3. the wavefront's four h values: lane 0 stores y and publishes
         const unsigned int hb16 = (unsigned int)__builtin_bit_cast(unsigned short, h);
         const unsigned int pb16 = h_is_number ? hb16 : 0u;       // a NaN cannot carry the flag: it is exchanged as 0, y keeps it
         const unsigned int sb16 = h_is_number ? hb16 : 0x7e00u;  // and goes to the layer above in its canonical form
-        const unsigned long long pw = pack_quads(pb16);
-        const unsigned long long yw = pack_quads(hb16);
-        const unsigned long long sw = emits ? pack_quads(sb16) : 0ull;
+        const unsigned long long pw = Product::pack(pb16);
+        const unsigned long long yw = Product::pack(hb16);
+        const unsigned long long sw = emits ? Product::pack(sb16) : 0ull;
         // (a wavefront one of whose waits gave up after this step's barrier has made its h from stale values: it keeps them
         // to itself, and the group's other members stop at their next wait)
         const bool wave_gave_up = __builtin_amdgcn_ballot_w64(gave_up) != 0ull;
@@ -576,7 +693,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             if (!res && units_ok && ch.y) *reinterpret_cast<unsigned long long*>(ch.y + (long)t * p.y_stride + u0) = yw;
             if (emits) hout[s & 1][wave] = sw;
         }
-        if (s == T - 1 && units_ok && lane < 16 && (lane & 3) == 0) {
+        if (s == T - 1 && units_ok && Product::first_of_unit(lane)) {
             ch.hn[my_unit] = h;
             ch.cn[my_unit] = (half_t)c_new;
         }
@@ -648,13 +765,20 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
 template <bool PIPE>
 __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_f16_kernel(LstmXcdArgs p)
 {
-    lstm_xcd_body<PIPE, false>(p);
+    lstm_xcd_body<PIPE, false, XcdSparse>(p);
+}
+
+template <bool PIPE>
+__global__ __launch_bounds__(kXcdThreads) void lstm_xcd_dot_f16_kernel(LstmXcdArgs p)
+{
+    lstm_xcd_body<PIPE, false, XcdDot>(p);
 }
 
 // The pipeline for stacks that have layers with a residual sum.
+template <class Product>
 __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_res_f16_kernel(LstmXcdArgs p)
 {
-    lstm_xcd_body<true, true>(p);
+    lstm_xcd_body<true, true, Product>(p);
 }
 
 }  // namespace pimhip
