@@ -380,11 +380,15 @@ struct XprojTileProblems {
 };
 
 // 16 bytes per lane from memory straight into LDS: lane l's at `lds_base` + 16 l (lds_base: the same in all lanes).  Counted by
-// vmcnt; nothing but an explicit wait orders it.
+// vmcnt; nothing but an explicit wait orders it.  (The compiler allocates m0 to nothing and sets it in front of each use of its
+// own, but it joins equal settings of m0 where it sees none in between: it is told of this one, and warns that m0 is reserved.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void load_lds16(const half_t* src, unsigned int lds_base)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_base), "v"(src) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" : : "s"(lds_base), "v"(src) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 
 template <int N>
 __device__ __forceinline__ void wait_loads_and_barrier()
