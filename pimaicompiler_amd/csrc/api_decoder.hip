@@ -224,7 +224,7 @@ extern "C" int pimhip_decoder_plan_set_encoder(PimHipDecoderPlan* plan, const vo
         outs[count] = plan->cx_proj + (size_t)l * plan->enc_cap * 4 * H;
         ws[count++] = plan->w_ih[l] + H;
     }
-    rc = launch_context_projection(count, outs, ws, (const half_t*)enc, 4 * H, H, enc_len, 2 * H, s);
+    rc = launch_context_projection(count, outs, ws, (const half_t*)enc, 4 * H, H, enc_len, 2 * H, st->num_cus, s);
     if (rc != PIMHIP_OK) return rc;
     plan->enc = (const half_t*)enc;
     plan->enc_len = enc_len;

@@ -629,10 +629,10 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             const float* bs1[1] = {cf.bsum};
             if (cf.w_ih_packed) {
                 const half_t* ws1[1] = {cf.w_ih_packed};
-                rc = launch_input_projection_packed(1, outs1, layer_in, ws1, bs1, T, cf.in_w, 4 * H, cf.ksteps, s, &seg, 2 * (n - 1));
+                rc = launch_input_projection_packed(1, outs1, layer_in, ws1, bs1, T, cf.in_w, 4 * H, cf.ksteps, st->num_cus, s, &seg, 2 * (n - 1));
             } else {
                 const half_t* ws1[1] = {cf.w_ih};
-                rc = launch_input_projection(1, outs1, layer_in, ws1, bs1, T, cf.in_w, 4 * H, s);
+                rc = launch_input_projection(1, outs1, layer_in, ws1, bs1, T, cf.in_w, 4 * H, st->num_cus, s);
                 launch_fill_segments(seg, 2 * (n - 1), 0xffffffffu, s);
             }
             if (rc != PIMHIP_OK) return rc;
@@ -662,10 +662,10 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             const float* bs2[2] = {c0.bsum, c1.bsum};
             if (c0.w_ih_packed && c1.w_ih_packed) {
                 const half_t* ws2[2] = {c0.w_ih_packed, c1.w_ih_packed};
-                rc = launch_input_projection_packed(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, c0.ksteps, s);
+                rc = launch_input_projection_packed(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, c0.ksteps, st->num_cus, s);
             } else {
                 const half_t* ws2[2] = {c0.w_ih, c1.w_ih};
-                rc = launch_input_projection(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, s);
+                rc = launch_input_projection(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, st->num_cus, s);
             }
             if (rc != PIMHIP_OK) return rc;
             LstmXcdArgs a;
@@ -739,10 +739,10 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
                         const float* bs2[2] = {c.bsum, c2.bsum};
                         if (c.w_ih_packed && c2.w_ih_packed) {
                             const half_t* ws2[2] = {c.w_ih_packed, c2.w_ih_packed};
-                            rc = launch_input_projection_packed(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, c.ksteps, s);
+                            rc = launch_input_projection_packed(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, c.ksteps, st->num_cus, s);
                         } else {
                             const half_t* ws2[2] = {c.w_ih, c2.w_ih};
-                            rc = launch_input_projection(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, s);
+                            rc = launch_input_projection(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, st->num_cus, s);
                         }
                         if (rc != PIMHIP_OK) return rc;
                     }
@@ -805,7 +805,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
                     ws2[d] = c.w_ih;
                     bs2[d] = c.bsum;
                 }
-                rc = launch_input_projection(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, s);
+                rc = launch_input_projection(D, outs2, layer_in, ws2, bs2, T, in_w, 4 * H, st->num_cus, s);
                 if (rc != PIMHIP_OK) return rc;
             }
             const unsigned grid = (unsigned)((H + 3) / 4);

@@ -9,25 +9,6 @@ namespace pimhip
 {
 namespace
 {
-int tiles_of(int64_t T, int64_t N, int rows) { return (int)((T + rows - 1) / rows * ((N + kXprojTileCols - 1) / kXprojTileCols)); }
-
-// The row tiles per wavefront (MT) of the kernel for many time steps, or 0: the split-K kernels.  Measured on MI355X over T = 50 ..
-// 2048, K = 240 .. 2048, N = 1024 .. 4096 (us, split-K kernel / 64-row / 128-row tiles, plain weights):
-//   64-row tiles in all   128 (T 200, K 1024, N 4096) 9.7 / 8.7 / -    130 (800, 1024, 1280) 10.6 / 9.2 / 12.4   104 (800, 512, 1024) 6.5 / 7.1 / 8.7
-//                         192 (341, 1024, 4096) 12.5 / 9.8 / 13.2      416 (800, 1024, 4096) 24.6 / 17.7 / 14.5  1024 (2048, 1024, 4096) 56 / 37 / 29
-// A block fills a CU, so what counts is how many tiles the busiest CU runs one after another, a 128-row tile taking 1.5 times as
-// long as a 64-row one.  From half as many 64-row tiles as CUs on they win; against packed weights, whose split-K kernel moves
-// half the LDS bytes, from five eighths (128: 8.3 / 8.7, 192: 10.7 / 9.6).
-int tile_rows(int64_t T, int64_t N, int count, bool packed)
-{
-    constexpr int kCus = 256;
-    if ((double)T * (double)N > 1e12) return 0;  // (counts below stay within an int)
-    const int t64 = count * tiles_of(T, N, 64), t128 = count * tiles_of(T, N, 128);
-    if (t64 < (packed ? kCus * 5 / 8 : kCus / 2)) return 0;
-    const int r64 = (t64 + kCus - 1) / kCus, r128 = (t128 + kCus - 1) / kCus;
-    return 2 * r64 <= 3 * r128 ? 2 : 4;
-}
-
 template <bool PACKED>
 void launch_tiles(int mt, int count, float* const* out, const half_t* x, const half_t* const* w, const float* const* bias, int64_t T, int64_t K,
                   int64_t N, int64_t ldx, int64_t ldw, int ksteps, XprojFill& fill, hipStream_t s)
@@ -40,7 +21,7 @@ void launch_tiles(int mt, int count, float* const* out, const half_t* x, const h
         pr.out[p] = out[p];
     }
     const unsigned row_blocks = (unsigned)((T + 32 * mt - 1) / (32 * mt));
-    pr.blocks_per_problem = (tiles_of(T, N, 32 * mt) + 7) / 8 * 8;
+    pr.blocks_per_problem = (xproj_tiles(T, N, 32 * mt) + 7) / 8 * 8;
     fill.first_block = pr.blocks_per_problem * count;
     const unsigned grid = (unsigned)fill.first_block + (unsigned)(fill.count > 0 ? fill.blocks : 0);
     if (mt == 4)
@@ -51,7 +32,7 @@ void launch_tiles(int mt, int count, float* const* out, const half_t* x, const h
 }  // namespace
 
 int launch_input_projection(int count, float* const* out, const half_t* x, const half_t* const* w, const float* const* bias,
-                            int64_t T, int64_t K, int64_t N, hipStream_t s, int64_t ldx, int64_t ldw)
+                            int64_t T, int64_t K, int64_t N, int num_cus, hipStream_t s, int64_t ldx, int64_t ldw)
 {
     if (ldx == 0) ldx = K;
     if (ldw == 0) ldw = K;
@@ -69,7 +50,7 @@ int launch_input_projection(int count, float* const* out, const half_t* x, const
         pr.out[p] = out[p];
     }
     // (K == 0, out = bias, stays below: the tiles' loop always has a slab)
-    if (const int mt = K > 0 ? tile_rows(T, N, count, false) : 0) {
+    if (const int mt = K > 0 ? xproj_tile_rows(T, N, count, false, num_cus) : 0) {
         XprojFill none;  // (count 0: no blocks that fill)
         memset(&none, 0, sizeof(none));
         launch_tiles<false>(mt, count, out, x, w, bias, T, K, N, ldx, ldw, 0, none, s);
@@ -95,7 +76,7 @@ int launch_input_projection(int count, float* const* out, const half_t* x, const
 
 // The same with weights in fragment order (pack_w_fragments_kernel); N, K checked by the caller (plan creation).
 int launch_input_projection_packed(int count, float* const* out, const half_t* x, const half_t* const* wp, const float* const* bias,
-                                   int64_t T, int64_t K, int64_t N, int ksteps, hipStream_t s, const FillSegments* ones, int n_ones)
+                                   int64_t T, int64_t K, int64_t N, int ksteps, int num_cus, hipStream_t s, const FillSegments* ones, int n_ones)
 {
     if (T <= 0 || N <= 0) {
         if (ones && n_ones > 0) launch_fill_segments(*ones, n_ones, 0xffffffffu, s);
@@ -116,7 +97,7 @@ int launch_input_projection_packed(int count, float* const* out, const half_t* x
         fill.count = n_ones;
         fill.blocks = 128;
     }
-    if (const int mt = tile_rows(T, N, count, true)) {
+    if (const int mt = xproj_tile_rows(T, N, count, true, num_cus)) {
         launch_tiles<true>(mt, count, out, x, wp, bias, T, K, N, K, 0, ksteps, fill, s);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return fail(PIMHIP_ERR_HIP, "input projection launch failed: %s", hipGetErrorString(e));
@@ -161,7 +142,7 @@ int launch_input_projection_packed(int count, float* const* out, const half_t* x
 
 // out_l[N, S] (fp32) = w_l[N, K] (pitch ldw) . enc[S, K]^T for up to four weights.
 int launch_context_projection(int count, float* const* out, const half_t* const* w, const half_t* enc, int64_t N, int64_t K, int64_t S,
-                              int64_t ldw, hipStream_t s)
+                              int64_t ldw, int num_cus, hipStream_t s)
 {
     // One launch with the weights in registers reads enc from the caches once per 32 weight rows: right for a sentence, and from
     // 200 positions on no faster than a launch per layer.  Measured on MI355X, us of set_encoder at 12 / 50 / 128 / 200 positions
@@ -173,7 +154,7 @@ int launch_context_projection(int count, float* const* out, const half_t* const*
     if (!here) {
         for (int l = 0; l < count; ++l) {
             const float* no_bias = nullptr;
-            const int rc = launch_input_projection(1, &out[l], w[l], &enc, &no_bias, N, K, S, s, ldw, K);
+            const int rc = launch_input_projection(1, &out[l], w[l], &enc, &no_bias, N, K, S, num_cus, s, ldw, K);
             if (rc != PIMHIP_OK) return rc;
         }
         return PIMHIP_OK;
@@ -220,7 +201,7 @@ extern "C" int pimhip_input_projection(void* out, const void* x, const void* w, 
     float* outs[1] = {(float*)out};
     const half_t* ws[1] = {(const half_t*)w};
     const float* bs[1] = {(const float*)bias};
-    return launch_input_projection(1, outs, (const half_t*)x, ws, bs, seq_len, in_w, n_out, static_cast<hipStream_t>(stream), 0, 0);
+    return launch_input_projection(1, outs, (const half_t*)x, ws, bs, seq_len, in_w, n_out, st->num_cus, static_cast<hipStream_t>(stream), 0, 0);
 }
 
 extern "C" int pimhip_projection_packed_bytes(int64_t in_w, int64_t n_out, uint64_t* bytes)
@@ -266,5 +247,5 @@ extern "C" int pimhip_input_projection_packed(void* out, const void* x, const vo
     float* outs[1] = {(float*)out};
     const half_t* wps[1] = {(const half_t*)packed};
     const float* bs[1] = {(const float*)bias};
-    return launch_input_projection_packed(1, outs, (const half_t*)x, wps, bs, seq_len, in_w, n_out, ksteps, static_cast<hipStream_t>(stream));
+    return launch_input_projection_packed(1, outs, (const half_t*)x, wps, bs, seq_len, in_w, n_out, ksteps, st->num_cus, static_cast<hipStream_t>(stream));
 }

@@ -11,6 +11,7 @@
 #pragma once
 
 #include "device_common.h"
+#include "xproj_plan.h"
 
 namespace pimhip
 {
@@ -368,7 +369,6 @@ __global__ __launch_bounds__(64 * KS) void input_projection_packed_f16_kernel(co
 //     from the exact sum as the kernels above at 64 columns, closer from there on (relative 6.6e-8 against 8.4e-8 at 1024).
 // 800 x 1024 -> 4096, MI355X: 24.6 -> 14.5 us (packed 19.4 -> 14.4), 2048 x 1024 -> 4096 56.2 -> 32.8 (305 -> 520 TFLOP/s).
 // ---------------------------------------------------------------------------------------------
-static constexpr int kXprojTileCols = 128;
 static constexpr int kXprojTileSlab = 64;
 static constexpr int kXprojTileBufs = 4;
 
