@@ -20,6 +20,8 @@ import collections
 import contextlib
 import ctypes
 import enum
+import importlib
+import warnings
 import weakref
 
 import torch
@@ -49,14 +51,52 @@ def _check(rc):
 _native_module = None
 
 
+class _WithoutExtension:
+    """Stands in for the extension module where only libpimhip.so has been built: no call is taken, so the bodies below run all
+    of them, and a bound step goes through ctypes."""
+
+    @staticmethod
+    def _not_taken(*args):
+        return None
+
+    fast_addmm = fast_matmul = fast_linear = fast_group = fast_projection = fast_lstm = lstm_key = _not_taken
+
+    @staticmethod
+    def bind_moe(*args):
+        return L.load().pimhip_moe_ffn_step, args
+
+    @staticmethod
+    def bind_rnnt(*args):
+        return L.load().pimhip_rnnt_step, args[:-1] + (int(args[-1]),)
+
+    @staticmethod
+    def bind_decoder(handle, x, att, ctx, h_prev, c_prev, hn, cn, outs, ctx_outs, logits):
+        mk = lambda ps: (ctypes.c_void_p * len(ps))(*ps)  # noqa: E731
+        return L.load().pimhip_decoder_step, (handle, x, att, ctx, mk(h_prev), mk(c_prev), mk(hn), mk(cn), mk(outs), mk(ctx_outs) if ctx_outs else None,
+                                              len(ctx_outs), logits)
+
+    @staticmethod
+    def issue(step, stream):
+        fn, args = step
+        return fn(*args, _stream_handle(stream))
+
+
 def _native():
     """The extension module with the per-call path of the operators (cpp/ops_fastcall.cpp): checks, shape dispatch, output
     tensors and the C ABI call without a Python object per step.  Its functions return None where a call is not the plain
-    case, and the bodies below take it from its start then; an integer is the C ABI's status."""
+    case, and the bodies below take it from its start then; an integer is the C ABI's status.  Where it has not been built the
+    bodies take every call, slower (a warning says so, once)."""
     global _native_module
     if _native_module is None:
-        from . import _aten_ops_pimhip
-        _native_module = _aten_ops_pimhip
+        name = __package__ + "._aten_ops_pimhip"
+        try:
+            _native_module = importlib.import_module(name)
+        except ModuleNotFoundError as e:
+            if e.name != name:
+                raise
+            warnings.warn("pimaicompiler_amd._aten_ops_pimhip has not been built: operators are called through ctypes, which takes "
+                          "13 us and more of host time per call (python -m pimaicompiler_amd.build builds it)", RuntimeWarning, stacklevel=3)
+            _native_module = _WithoutExtension()
     return _native_module
 
 
