@@ -187,7 +187,8 @@ PyObject* group(PyObject*, PyObject* const* args, Py_ssize_t nargs)
         const at::Tensor *x, *w, *b = nullptr;
         if (!tensorOf(PyList_GET_ITEM(args[0], i), x) || !tensorOf(PyList_GET_ITEM(args[1], i), w)) return none();
         if (biases && PyList_GET_ITEM(args[2], i) != Py_None && !tensorOf(PyList_GET_ITEM(args[2], i), b)) return none();
-        if (w->dim() != 2 || x->numel() != w->size(1) || !w->is_contiguous() || !x->is_contiguous() || (b && !b->is_contiguous())) return none();
+        if (w->dim() != 2 || x->numel() != w->size(1) || !w->is_contiguous() || !x->is_contiguous() || (b && (!b->is_contiguous() || b->numel() < w->size(0))))
+            return none();
         in[i] = x->data_ptr();
         weight[i] = w->data_ptr();
         bias[i] = b ? b->data_ptr() : nullptr;

@@ -441,6 +441,9 @@ def execute_gemv_group(inputs, weights, biases=None, act_types=None, stream=None
     for x, w in zip(xs, ws):
         if w.dim() != 2 or x.numel() != w.size(1):
             raise NNRuntimeException("each weight must be [out, in] and each input must have `in` elements")
+    for w, b in zip(ws, bs):
+        if b is not None and b.numel() < w.size(0):
+            raise NNRuntimeException(f"bias has {b.numel()} elements, the GEMV produces {w.size(0)}")
     vp = ctypes.c_void_p * n
     rc = lib.pimhip_execute_gemv_group(
         n, vp(*[o.data_ptr() for o in outs]), vp(*[x.data_ptr() for x in xs]), vp(*[w.data_ptr() for w in ws]),

@@ -119,3 +119,18 @@ def test_what_the_native_path_does_not_take_is_refused_as_before(ops):
         ops.execute_gemv_group([x], [w, w])
     with pytest.raises(ops.NNRuntimeException, match="in_w % 8|multiples of 8|grouped launch"):
         ops.execute_gemv_group([half(1, 20)], [half(8, 20)])
+
+
+def test_a_bias_shorter_than_its_product_is_refused_in_a_group(ops, monkeypatch):
+    xs, ws = [half(1, 24), half(1, 24)], [half(40, 24), half(33, 24)]
+
+    def call(*biases):
+        return lambda: ops.execute_gemv_group(xs, ws, list(biases))
+    same(*both(monkeypatch, call(half(40), half(34))))     # (a longer one's tail is not read)
+    from pimaicompiler_amd import ops as O
+    for module in (O._native(), NoNative(O._native())):
+        monkeypatch.setattr(O, "_native_module", module)
+        with pytest.raises(ops.NNRuntimeException, match="bias has 32 elements, the GEMV produces 33"):
+            call(None, half(32))()
+        with pytest.raises(ops.NNRuntimeException, match="bias has 1 elements, the GEMV produces 40"):
+            call(half(1), half(33))()
