@@ -36,7 +36,18 @@ bool streamOf(PyObject* o, void*& s)
     }
     if (!PyLong_Check(o)) return false;
     s = PyLong_AsVoidPtr(o);
-    return !PyErr_Occurred();
+    if (!PyErr_Occurred()) return true;
+    PyErr_Clear();
+    return false;
+}
+
+// An argument that is no integer of 64 bits is the Python body's to refuse.
+bool intOf(PyObject* o, int64_t& v)
+{
+    v = PyLong_AsLongLong(o);
+    if (v != -1 || !PyErr_Occurred()) return true;
+    PyErr_Clear();
+    return false;
 }
 
 at::Tensor newHalf(at::IntArrayRef shape, const at::Tensor& like)
@@ -214,7 +225,8 @@ PyObject* projection(PyObject*, PyObject* const* args, Py_ssize_t n)
     const at::Tensor *x, *w, *b = nullptr;
     void* stream;
     if (n != 6 || !tensorOf(args[0], x) || !tensorOf(args[1], w) || !streamOf(args[5], stream)) return none();
-    const int64_t n_out = PyLong_AsLongLong(args[3]);
+    int64_t n_out;
+    if (!intOf(args[3], n_out)) return none();
     if (args[2] != Py_None) {
         if (!THPVariable_Check(args[2])) return none();
         b = &THPVariable_Unpack(args[2]);
@@ -276,7 +288,8 @@ PyObject* lstm(PyObject*, PyObject* const* args, Py_ssize_t n)
     void* stream;
     if (n != 10 || !tensorOf(args[1], x) || !tensorOf(args[2], h0) || !tensorOf(args[3], c0) || !streamOf(args[9], stream)) return none();
     PimHipLstmPlan* plan = static_cast<PimHipLstmPlan*>(PyLong_AsVoidPtr(args[0]));
-    const int64_t I = PyLong_AsLongLong(args[4]), LD = PyLong_AsLongLong(args[5]), H = PyLong_AsLongLong(args[6]), D = PyLong_AsLongLong(args[7]);
+    int64_t I, LD, H, D;
+    if (!intOf(args[4], I) || !intOf(args[5], LD) || !intOf(args[6], H) || !intOf(args[7], D)) return none();
     const bool batch_first = PyObject_IsTrue(args[8]) == 1;
     if (!plan || x->dim() != 3 || x->size(batch_first ? 0 : 1) != 1 || x->size(2) != I || h0->numel() != LD * H || c0->numel() != LD * H ||
         !x->is_contiguous() || !h0->is_contiguous() || !c0->is_contiguous())

@@ -134,3 +134,15 @@ def test_a_bias_shorter_than_its_product_is_refused_in_a_group(ops, monkeypatch)
             call(None, half(32))()
         with pytest.raises(ops.NNRuntimeException, match="bias has 1 elements, the GEMV produces 40"):
             call(half(1), half(33))()
+
+
+def test_an_argument_of_the_wrong_kind_reaches_the_python_body(ops, monkeypatch):
+    """... whose exception is the caller's, not a SystemError about one left behind by the native call."""
+    import ctypes
+    x, w = half(5, 24), half(40, 24)
+    packed = ops.pack_projection_weight(w)
+    for n_out in (40.0, 1 << 70):
+        with pytest.raises((ctypes.ArgumentError, TypeError, OverflowError, ops.NNRuntimeException)):
+            ops.input_projection_packed(x, packed, n_out)
+    with pytest.raises((ctypes.ArgumentError, TypeError, ValueError)):
+        ops.aten_linear(x[:1], w, stream="main")
