@@ -574,7 +574,8 @@ def pack_projection_weight(w, stream=None):
 
 
 def input_projection_packed(x, packed, n_out, bias=None, stream=None):
-    """input_projection with a weight from pack_projection_weight; the same bits, less LDS traffic."""
+    """input_projection with a weight from pack_projection_weight: the same products, summed in a fixed order that differs from
+    input_projection's where the two take different kernels."""
     out = _native().fast_projection(x, packed, bias, n_out, True, _stream_arg(stream))
     if out is not None:
         return _result(out)

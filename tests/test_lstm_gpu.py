@@ -646,7 +646,13 @@ def test_input_projection_of_many_steps(ops, T, K, N):
     xi[T - 1, 0] = float("inf")
     got = ops.input_projection(xi, wd, bd)
     assert torch.equal(got[: T - 1], out[: T - 1]) and not bool(torch.isfinite(got[T - 1][wd[:, 0] != 0]).any())
-    assert torch.equal(got[: T - 1], ops.input_projection_packed(xi, packed, N, bd)[: T - 1]) == torch.equal(out, ops.input_projection_packed(xd, packed, N, bd))
+    clean = ops.input_projection_packed(xd, packed, N, bd)
+    got = ops.input_projection_packed(xi, packed, N, bd)
+    assert torch.equal(got[: T - 1], clean[: T - 1]) and not bool(torch.isfinite(got[T - 1][wd[:, 0] != 0]).any())
+    # from five eighths as many 64-row tiles as CUs on both kinds of weights take this kernel, with the same sums in the same order
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    if -(-T // 64) * -(-N // 128) >= cus * 5 // 8:
+        assert torch.equal(clean, out)
 
 
 # A reduction of width 0 leaves the bias, also where there are enough time steps for the kernel above (whose loop takes one slab at least).
