@@ -420,6 +420,7 @@ def execute_gemv_group(inputs, weights, biases=None, act_types=None, stream=None
     Replaces executeMultiStream's one-stream-per-GEMV issue
     (runtime/source/executor/op_executor/stream_ops_executor.cpp:27-50).  Returns the list of outputs.
     """
+    act_types = list(act_types) if act_types is not None else None  # (read twice where the native call does not take it)
     outs = _native().fast_group(list(inputs), list(weights), list(biases) if biases is not None else None,
                                 tuple(_act_code(a) for a in act_types) if act_types is not None else None, _stream_arg(stream))
     if outs is not None:

@@ -146,3 +146,10 @@ def test_an_argument_of_the_wrong_kind_reaches_the_python_body(ops, monkeypatch)
             ops.input_projection_packed(x, packed, n_out)
     with pytest.raises((ctypes.ArgumentError, TypeError, ValueError)):
         ops.aten_linear(x[:1], w, stream="main")
+
+
+def test_activations_of_a_group_from_a_generator(ops, monkeypatch):
+    xs, ws, acts = [half(1, 24), half(1, 24)], [half(40, 24), half(33, 24)], ["none", "aten::relu"]
+    native, body = both(monkeypatch, lambda: ops.execute_gemv_group(xs, ws, None, (a for a in acts)))
+    same(native, body)
+    assert bool((body[1] >= 0).all()) and bool((body[0] < 0).any())
