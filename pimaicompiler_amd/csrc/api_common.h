@@ -47,13 +47,10 @@ struct DeviceState {
     int num_cus = 0;
     std::map<hipStream_t, SplitWorkspace> workspaces;  // one per stream: sibling GEMVs on different streams must not share
     // Records of the products that need no workspace (vm_plan.h), apart from `workspaces` because a graph may hold those: one
-    // region per stream, used by launches issued outside a capture only, handed out in order until there are none left.  All
-    // allocated by pimhip_initialize, so that such a product never allocates.
+    // region per stream, used by launches issued outside a capture only, handed out in order until there are none left.
     std::map<hipStream_t, int> region_of;
-    SplitWorkspace regions[kVmRegions];  // (slices of the three arrays below; empty if there was no memory for them)
-    float* region_partials = nullptr;
-    unsigned int* region_poisons = nullptr;
-    unsigned int* region_statuses = nullptr;
+    SplitWorkspace regions[kVmRegions];
+    int region_count = 0;
     // The persistent LSTM kernel needs all its blocks resident at once.  Two of them issued on different streams could
     // each get part of the GPU and wait for the rest forever, so a launch on another stream than the previous one is
     // ordered after it with an event (nothing is added while one stream is used).

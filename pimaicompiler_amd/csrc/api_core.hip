@@ -35,40 +35,32 @@ static __device__ unsigned int scratch_poison;
 
 std::map<int, DeviceState> g_devices;
 
-void free_vm_regions(DeviceState& st)
-{
-    if (st.region_partials) hipFree(st.region_partials);
-    if (st.region_poisons) hipFree(st.region_poisons);
-    if (st.region_statuses) hipHostFree(st.region_statuses);
-    st.region_partials = nullptr;
-    st.region_poisons = st.region_statuses = nullptr;
-    for (SplitWorkspace& r : st.regions) r = SplitWorkspace();
-    st.region_of.clear();
-}
+// The regions of DeviceState::regions: as above, part of the library's image on every GPU, so that no allocation is made for them.
+constexpr size_t kVmRegionFloats = kVmRegions * (size_t)256 * 128;  // 4 MiB: vm_max_partials of 256 CUs each
+static __device__ __align__(256) float region_records[kVmRegionFloats];
+static __device__ unsigned int region_poisons[kVmRegions];
 
-// 4 MiB on a part of 256 CUs.  A device that has no room for them does without.
-void allocate_vm_regions(DeviceState& st)
+// statuses: kVmRegions pinned host words, and the same as the device addresses them
+int set_up_vm_regions(DeviceState& st, unsigned int* statuses, unsigned int* statuses_dev)
 {
+    void *records = nullptr, *poisons = nullptr;
+    PIMHIP_HIP_CHECK(hipGetSymbolAddress(&records, HIP_SYMBOL(region_records)));
+    PIMHIP_HIP_CHECK(hipGetSymbolAddress(&poisons, HIP_SYMBOL(region_poisons)));
+    launch_fill_u32(static_cast<unsigned int*>(records), kVmRegionFloats, kVmEmpty, nullptr);
+    launch_fill_u32(static_cast<unsigned int*>(poisons), kVmRegions, 0u, nullptr);
     const size_t words = vm_max_partials(st.num_cus);
-    unsigned int* statuses_dev = nullptr;
-    if (hipMalloc(&st.region_partials, kVmRegions * words * sizeof(float)) != hipSuccess ||
-        hipMalloc(&st.region_poisons, kVmRegions * sizeof(unsigned int)) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void**>(&st.region_statuses), kVmRegions * sizeof(unsigned int), hipHostMallocMapped) != hipSuccess ||
-        hipHostGetDevicePointer(reinterpret_cast<void**>(&statuses_dev), st.region_statuses, 0) != hipSuccess) {
-        (void)hipGetLastError();
-        free_vm_regions(st);
-        return;
-    }
-    launch_fill_u32(reinterpret_cast<unsigned int*>(st.region_partials), kVmRegions * words, kVmEmpty, nullptr);
-    launch_fill_u32(st.region_poisons, kVmRegions, 0u, nullptr);
-    for (int i = 0; i < kVmRegions; ++i) {
+    st.region_count = (int)(kVmRegionFloats / words < (size_t)kVmRegions ? kVmRegionFloats / words : (size_t)kVmRegions);
+    st.region_of.clear();
+    for (int i = 0; i < st.region_count; ++i) {
         SplitWorkspace& r = st.regions[i];
-        r.partial = st.region_partials + i * words;
-        r.poison = st.region_poisons + i;
-        r.status = st.region_statuses + i;
+        r = SplitWorkspace();
+        r.partial = static_cast<float*>(records) + i * words;
+        r.poison = static_cast<unsigned int*>(poisons) + i;
+        r.status = statuses + i;
         r.status_dev = statuses_dev + i;
         *r.status = 0u;
     }
+    return PIMHIP_OK;
 }
 }  // namespace
 
@@ -155,11 +147,13 @@ extern "C" int pimhip_initialize(int device)
     launch_fill_u32(st.static_poison, 1, 0u, nullptr);
     PIMHIP_HIP_CHECK(hipGetLastError());
     if (!st.static_status) {
-        PIMHIP_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&st.static_status), sizeof(unsigned int), hipHostMallocMapped));
+        // (one word for the static array, one per region)
+        PIMHIP_HIP_CHECK(hipHostMalloc(reinterpret_cast<void**>(&st.static_status), (1 + kVmRegions) * sizeof(unsigned int), hipHostMallocMapped));
         PIMHIP_HIP_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&st.static_status_dev), st.static_status, 0));
     }
     *st.static_status = 0u;
-    if (!st.region_partials) allocate_vm_regions(st);
+    const int rc = set_up_vm_regions(st, st.static_status + 1, st.static_status_dev + 1);
+    if (rc != PIMHIP_OK) return rc;
     PIMHIP_HIP_CHECK(hipGetLastError());
     PIMHIP_HIP_CHECK(hipStreamSynchronize(nullptr));
     st.initialized = true;
@@ -187,7 +181,6 @@ extern "C" int pimhip_deinitialize(void)
             if (w.second.status) hipHostFree(w.second.status);
         }
         kv.second.workspaces.clear();
-        free_vm_regions(kv.second);
         if (kv.second.static_status) hipHostFree(kv.second.static_status);
         if (kv.second.seq_event) hipEventDestroy(kv.second.seq_event);
         kv.second.initialized = false;

@@ -68,7 +68,7 @@ int get_split_workspace(DeviceState* st, hipStream_t stream, size_t partial_elem
 int get_region(DeviceState* st, hipStream_t stream, SplitWorkspace** out)
 {
     *out = nullptr;
-    if (!st->region_partials || stream == hipStreamPerThread) return PIMHIP_OK;
+    if (stream == hipStreamPerThread) return PIMHIP_OK;
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &capture) != hipSuccess) {  // (the null stream while another one is being captured)
         (void)hipGetLastError();
@@ -78,7 +78,7 @@ int get_region(DeviceState* st, hipStream_t stream, SplitWorkspace** out)
     std::lock_guard<std::mutex> lock(g_mutex);
     auto it = st->region_of.find(stream);
     if (it == st->region_of.end()) {
-        if (st->region_of.size() >= (size_t)kVmRegions) return PIMHIP_OK;
+        if (st->region_of.size() >= (size_t)st->region_count) return PIMHIP_OK;
         it = st->region_of.emplace(stream, (int)st->region_of.size()).first;
     }
     SplitWorkspace& ws = st->regions[it->second];
