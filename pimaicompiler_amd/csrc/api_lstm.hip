@@ -308,25 +308,28 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
     }
     // One recurrence per XCD: the part this is written for has 8 XCDs of 32 CUs, a group is one workgroup per CU of one.
     if (H <= kXcdMaxH && plan->num_cus == kXcdCount * kXcdMembers) {
-        int per_cu = 0;
-        int per_cu_pipe = 0;
-        int per_cu_dot = 0, per_cu_pipe_dot = 0;
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lstm_xcd_f16_kernel<false>, kXcdThreads, 0));
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_pipe, lstm_xcd_f16_kernel<true>, kXcdThreads, 0));
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_dot, lstm_xcd_dot_f16_kernel<false>, kXcdThreads, 0));
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_pipe_dot, lstm_xcd_dot_f16_kernel<true>, kXcdThreads, 0));
-        plan->xcd_ok = per_cu >= 1 && per_cu_pipe >= 1 && per_cu_dot >= 1 && per_cu_pipe_dot >= 1;
+        // (the kernels this plan may launch: a pipeline for a stack of one direction, otherwise independent recurrences)
+        const bool pipeline = D == 1 && num_layers >= 2;
+        auto resident = [&](auto kernel, bool* ok) {
+            int per_cu = 0;
+            const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kXcdThreads, 0);
+            *ok = *ok && per_cu >= 1;
+            return e;
+        };
+        plan->xcd_ok = true;
+        PLAN_HIP_CHECK(resident(pipeline ? lstm_xcd_f16_kernel<true> : lstm_xcd_f16_kernel<false>, &plan->xcd_ok));
+        PLAN_HIP_CHECK(resident(pipeline ? lstm_xcd_dot_f16_kernel<true> : lstm_xcd_dot_f16_kernel<false>, &plan->xcd_ok));
         if (plan->xcd_ok) {
             bool rotation = false;
             const int rc_probe = xcd_dispatch_is_a_rotation(kXcdCount * kXcdMembers, s, &rotation);
             if (rc_probe != PIMHIP_OK) return cleanup_fail(rc_probe);
             plan->xcd_ok = rotation;
         }
-        int per_cu_res = 0;
-        int per_cu_res_dot = 0;
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_res, lstm_xcd_res_f16_kernel<XcdSparse>, kXcdThreads, 0));
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu_res_dot, lstm_xcd_res_f16_kernel<XcdDot>, kXcdThreads, 0));
-        plan->xcd_res_ok = plan->xcd_ok && per_cu_res >= 1 && per_cu_res_dot >= 1;
+        plan->xcd_res_ok = plan->xcd_ok && pipeline;
+        if (pipeline) {
+            PLAN_HIP_CHECK(resident(lstm_xcd_res_f16_kernel<XcdSparse>, &plan->xcd_res_ok));
+            PLAN_HIP_CHECK(resident(lstm_xcd_res_f16_kernel<XcdDot>, &plan->xcd_res_ok));
+        }
     }
     if (plan->xcd_ok) {
         const size_t words = (size_t)kXcdRegionWords * kXcdMaxChains;
