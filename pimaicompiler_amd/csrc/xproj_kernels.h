@@ -366,7 +366,7 @@ __global__ __launch_bounds__(64 * KS) void input_projection_packed_f16_kernel(co
 //     weights are the first operand: a lane's four results are neighbours in a row of out (one 16-byte store).
 //   - PACKED: the weights' fragments (pack_w_fragments_kernel) pass through LDS as they are; the same products in the same order.
 //   - Two slabs' products are one chain of sums in the matrix cores and are then added to the total on the vector units: as far
-//     from the exact sum as the kernels above at 64 columns, closer from there on (relative 6.6e-8 against 8.4e-8 at 1024).
+//     from the exact sum as the kernels above at 64 columns, closer from there on (relative 0.84e-7 against 1.12e-7 at 1024).
 // 800 x 1024 -> 4096, MI355X: 24.6 -> 14.5 us (packed 19.4 -> 14.4), 2048 x 1024 -> 4096 56.2 -> 32.8 (305 -> 520 TFLOP/s).
 // ---------------------------------------------------------------------------------------------
 static constexpr int kXprojTileSlab = 64;
