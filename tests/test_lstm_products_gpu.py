@@ -106,3 +106,29 @@ def test_waits_that_give_up_and_nans_in_both_kinds(ops, H, T, layers, bidir, res
         assert torch.equal(fwd[:at], want[0][:at, :H]) and torch.equal(bwd[at + 1:], want[0][at + 1:, H:])
     else:
         assert bool(torch.isnan(y[at:]).all()) and torch.equal(y[:at], want[0][:at])
+
+
+@pytest.mark.parametrize("H,layers,bidir,short,long", [(512, 1, True, 31, 32), (1024, 1, False, 15, 16), (256, 3, False, 9, 10), (640, 2, False, 23, 24)])
+def test_one_plan_runs_both_kinds_in_turn(ops, H, layers, bidir, short, long):
+    """The two kinds share the exchange, its counters and its slots: sequences on either side of a line in turn, eager and replayed."""
+    params, x, h0, c0 = workloads.lstm_inputs(H, 40, H, layers, bidir, long)
+    xd, h0, c0 = x.reshape(long, 40).to(DEV), h0.to(DEV), c0.to(DEV)
+    want = {T: plan_of(ops, params, layers, bidir, T).forward(xd[:T], h0, c0) for T in (short, long)}
+    plan = plan_of(ops, params, layers, bidir, long)
+    for T in (short, long, long, short, short, long):
+        assert all(torch.equal(a, b) for a, b in zip(plan.forward(xd[:T], h0, c0), want[T]))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=side):
+        one = plan.forward(xd[:long], h0, c0)
+        two = plan.forward(xd[:short], h0, c0)
+    for _ in range(3):
+        for t in (*one, *two):
+            t.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip((*one, *two), (*want[long], *want[short])))
+        assert all(torch.equal(a, b) for a, b in zip(plan.forward(xd[:short], h0, c0), want[short]))
+    plan.status()
+    assert plan.fallbacks() == (0, True)
