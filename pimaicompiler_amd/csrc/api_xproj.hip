@@ -144,12 +144,7 @@ int launch_input_projection_packed(int count, float* const* out, const half_t* x
 int launch_context_projection(int count, float* const* out, const half_t* const* w, const half_t* enc, int64_t N, int64_t K, int64_t S,
                               int64_t ldw, int num_cus, hipStream_t s)
 {
-    // One launch with the weights in registers reads enc from the caches once per 32 weight rows: right for a sentence, and from
-    // 200 positions on no faster than a launch per layer.  Measured on MI355X, us of set_encoder at 12 / 50 / 128 / 200 positions
-    // (launch per layer -> this one): three layers of 1024 33 -> 8.3 / 33.6 -> 12.1 / 38.9 -> 20.9 / 30.6 -> 29.5, two of 512
-    // 10.5 -> 6.8 / 12.3 -> 6.6 / 12.2 -> 8.7 / 12.8 -> 12.4.
-    constexpr int64_t kMostPositions = 160;
-    bool here = S <= kMostPositions && K <= kCtxMaxK && K % 8 == 0 && ldw % 8 == 0 && aligned16(enc) && count <= kCtxMaxLayers;
+    bool here = S <= context_most_positions(count, K) && K <= kCtxMaxK && K % 8 == 0 && ldw % 8 == 0 && aligned16(enc) && count <= kCtxMaxLayers;
     for (int l = 0; here && l < count; ++l) here = aligned16(w[l]);
     if (!here) {
         for (int l = 0; l < count; ++l) {

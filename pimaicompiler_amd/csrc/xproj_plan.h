@@ -24,4 +24,13 @@ inline int xproj_tile_rows(int64_t T, int64_t N, int count, bool packed, int num
     const int r64 = (t64 + num_cus - 1) / num_cus, r128 = (t128 + num_cus - 1) / num_cus;
     return 2 * r64 <= 3 * r128 ? 2 : 4;
 }
+
+// The most encoder positions for which the context columns of `layers` layers are made by one launch with the weights in registers
+// (context_projection_f16_kernel) instead of a launch per layer: it reads enc from the caches once per 32 weight rows, 16 positions
+// at a time, so a block's time grows with the positions, and with one layer there is no launch to save.  Measured on MI355X (us of
+// set_encoder, launch per layer / one launch):
+//   one layer     256 wide at 48 / 80 positions 4.4 / 4.0, 4.5 / 5.2   512 5.6 / 4.9, 5.7 / 6.5   704 at 80 / 117 8.6 / 7.6, 9.0 / 10.3   1024 11.6 / 10.3, 13.7 / 14.0
+//   two layers    256 at 160 / 200 8.5 / 8.3, 8.8 / 9.9   1024 at 128 / 160 26.4 / 15.0, 18.2 / 17.9
+//   three layers  256 at 160 12.6 / 8.4   1024 at 128 / 160 / 200 39.4 / 21.9, 27.0 / 25.6, 30.0 / 30.7
+inline int64_t context_most_positions(int layers, int64_t K) { return layers >= 2 ? 160 : K <= 512 ? 48 : 80; }
 }  // namespace pimhip

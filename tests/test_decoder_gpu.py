@@ -121,7 +121,8 @@ def test_fused_decoder_step_matches_libtorch_cpu(ops, H, in0, L, first_ctx, firs
 # The context columns of all layers in one launch: sentences around its tiles of 16 positions and its longest, hidden sizes that are not
 # whole tiles of 32 rows and 128 columns.
 @pytest.mark.parametrize("H,L,first_ctx,src_len", [(40, 2, True, 16), (264, 3, False, 17), (136, 4, True, 33), (1024, 2, False, 160),
-                                                   (264, 2, True, 161)])
+                                                   (264, 2, True, 161), (264, 2, False, 48), (512, 2, False, 49), (520, 2, False, 80),
+                                                   (704, 2, False, 81), (1024, 3, False, 160)])
 def test_context_columns_of_a_sentence(ops, H, L, first_ctx, src_len):
     case = Case(77 + H + src_len, H, H, L, first_ctx, 9, 0, src_len)
     check(case, run_fused(ops, case, case.plan(ops), case.x, case.h, case.c), case.cpu_step(case.x, case.h, case.c))

@@ -15,7 +15,8 @@ int main()
 {
     long long T, N;
     int count, packed, cus;
-    while (scanf("%lld %lld %d %d %d", &T, &N, &count, &packed, &cus) == 5) printf("%d\n", pimhip::xproj_tile_rows(T, N, count, packed != 0, cus));
+    while (scanf("%lld %lld %d %d %d", &T, &N, &count, &packed, &cus) == 5)
+        printf("%d\n", cus == 0 ? (int)pimhip::context_most_positions(count, T) : pimhip::xproj_tile_rows(T, N, count, packed != 0, cus));
 }
 """
 
@@ -47,3 +48,12 @@ def test_half_the_cus_take_the_tiles_at_half_the_work(rule, packed):
     full = rule([(T, 4096, 1, packed, 256) for T in Ts])
     assert full == rule([(T, 2048, 1, packed, 128) for T in Ts]) == rule([(T, 1024, 1, packed, 64) for T in Ts])
     assert set(full) == {0, 2, 4}
+
+
+def test_one_layers_context_columns_stay_with_the_projection_kernels_for_long_sentences(rule):
+    """(No CUs: the rule for the context columns of `count` layers, T wide.)"""
+    def most(layers, width):
+        return rule([(width, 0, layers, 0, 0)])[0]
+    # (256, 512 wide, one layer: slower from about 60 positions on; 704 and more from about 100)
+    assert most(1, 256) < 58 and most(1, 512) < 64 and 64 <= most(1, 704) < 96 and most(1, 1024) < 96
+    assert all(most(n, h) == 160 for n in (2, 3, 4) for h in (256, 512, 1024))
