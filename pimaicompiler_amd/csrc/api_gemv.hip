@@ -113,8 +113,14 @@ int gemv_mv(const half_t* W, const half_t* x, const half_t* bias, half_t* y, int
     // Measured on MI355X over the (out, in) shapes of the GEMV sweep: long rows want the reduction split
     // over the four wavefronts of a block (more rows of the matrix open at once per CU would thrash DRAM
     // pages), short rows want two rows per wavefront.  Few rows: one row per block so that enough blocks exist.
-    // Rows that are not whole 16-byte pieces take the same shapes (swept as well: nothing faster by more than 2 %).
-    if (N < 1024) {
+    // Rows that are not whole 16-byte pieces take the same shapes (swept as well: nothing faster by more than 2 %), short ones
+    // excepted: up to 128 columns 2-byte loads, up to 512, one trip of one wavefront, no sum across wavefronts (32001 x 257 8.4 ->
+    // 6.4 us, 12000 x 257 3.9 -> 3.5, 300 x 257 the same).
+    if (!whole && K <= 128) {
+        gemv_mv_short_f16_kernel<4><<<(unsigned)((N + 3) / 4), 256, 0, s>>>(W, x, bias, y, (int)N, (int)K, (long)ldw, relu);
+    } else if (!whole && K <= 512) {
+        launch_mv<2, 1, 4, 1>(whole, W, x, bias, y, (int)N, (int)K, (long)ldw, relu, s);
+    } else if (N < 1024) {
         if (K >= 2048)
             launch_mv<1, 4, 4, 4>(whole, W, x, bias, y, (int)N, (int)K, (long)ldw, relu, s);
         else

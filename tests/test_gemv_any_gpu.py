@@ -40,6 +40,8 @@ def check(y, w_out_in, x, b, relu):
 @pytest.mark.parametrize("out_w,in_w,off_w,off_x,pitch", [
     (1, 1, 1, 1, 0), (3, 5, 0, 0, 0), (9, 7, 3, 5, 2), (5, 8, 1, 0, 0), (4, 15, 0, 0, 1), (130, 513, 0, 1, 0), (1023, 2049, 7, 0, 0),
     (1024, 1023, 0, 3, 5), (1025, 1029, 2, 2, 0), (1024, 1024, 1, 0, 0), (1024, 1024, 0, 1, 0), (40, 4103, 0, 0, 0),
+    (1030, 127, 0, 0, 0), (5, 128, 1, 0, 0), (1027, 129, 0, 0, 3), (4099, 257, 3, 1, 0), (1, 505, 0, 0, 0), (1025, 511, 0, 0, 0),
+    (7, 512, 0, 1, 0), (1024, 513, 0, 0, 0),
     (2049, 4099, 5, 1, 0), (1500, 6151, 0, 0, 0)])   # the last two exceed 16 MB or 4096 columns: other launch shapes and loads
 def test_rows_of_any_length_at_any_address(ops, out_w, in_w, off_w, off_x, pitch):
     from pimaicompiler_amd import _lib as L
