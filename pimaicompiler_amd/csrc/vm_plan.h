@@ -51,13 +51,14 @@ inline VmPlan vm_plan(int64_t K, int64_t N, int64_t lda, uintptr_t weight, uintp
     p.by_xcd = p.col_blocks >= 16 && (lda % 64 != 0 || (weight & 127u) != 0);
     // Slices of K: about a block per CU for a large weight, 64 blocks for a small one, but a cross-block sum costs 1 to 2 us
     // and grows with the slices: none up to 512 rows (272 x 2357: 3.1 us, two slices 3.6) and at most sqrt(K / 40) of them
-    // (12896 rows, 84 columns: 4.0 us with 17, 4.9 with 64).
+    // (12896 rows, 84 columns: 4.0 us with 17, 4.9 with 64), for a large weight, which needs the blocks, sqrt(K / 10) (16384 x 1000
+    // 9.9 us with 32, 12.8 with 20; 12000 x 1024 7.7 and 8.9; no limit at all is no faster up to 24000 rows).
     int64_t target = weight_bytes / 65536;
     if (target < 64) target = 64;
     if (target > num_cus) target = num_cus;
     int slices = (int)((target + p.col_blocks / 2) / p.col_blocks);  // rounded: 250 column blocks on 256 CUs are not sliced
     if (K <= 512) slices = 1;
-    while (slices > 1 && (int64_t)slices * slices * 40 > K) --slices;
+    while (slices > 1 && (int64_t)slices * slices * (weight_bytes > kVmLargeWeightBytes ? 10 : 40) > K) --slices;
     if (slices < 1) slices = 1;
     const int row_groups = kVmWaves * 64 / p.lanes_per_row;
     int64_t rows = (K + slices - 1) / slices;

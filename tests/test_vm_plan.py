@@ -56,6 +56,12 @@ def test_partial_sums_of_every_product_fit_a_workspace_of_one_size(plans):
     assert sliced > 100
 
 
+def test_slices_of_a_large_weight_with_few_columns(plans):
+    """A weight past 16 MB is read by about a block per CU, or by as many as sqrt(K / 10) slices give."""
+    got = plans([(16384, 1024, 1024, 0, 256), (12000, 1024, 1024, 0, 256), (16384, 520, 520, 0, 256), (4096, 4096, 4096, 0, 256), (12896, 84, 84, 0, 256)])
+    assert [(g[0], g[2]) for g in got] == [(16, 32), (16, 32), (16, 40), (16, 8), (8, 17)]
+
+
 def test_small_and_odd_products_need_no_workspace(plans):
     """Weights of at most 256 KB, and operands of no whole 16-byte pieces (sizes, pitch, either address, any destination)."""
     cases, want = [], []
