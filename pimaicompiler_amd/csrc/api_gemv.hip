@@ -184,15 +184,18 @@ void launch_vm_alone(const half_t* x, const half_t* A, const half_t* bias, const
 int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bias, const GemvOuts& outs, int64_t K,
             int64_t N, int64_t lda, int relu, hipStream_t s, bool static_ws = false)
 {
-    // The one-column-per-lane kernel where no eight columns exist, and for the smallest products: up to 4096 weights it takes
-    // 1.8 us against 2.3-2.5 us for the kernel below (two barriers more); 672 x 104 already 3.7 against 2.3.
-    if (N < 8 || N * K <= 4096) {
+    uintptr_t results = 0;
+    for (int o = 0; o < outs.count; ++o) results |= reinterpret_cast<uintptr_t>(outs.y[o]);
+    // The one-column-per-lane kernel where no eight columns exist, for the smallest products (up to 4096 weights it takes
+    // 1.8 us against 2.3-2.5 us for the kernel below, two barriers more; 672 x 104 already 3.7 against 2.3) and for few rows of no
+    // whole pieces, a load or two per lane: 64 x 1001 2.5 us against 3.2, 64 x 20001 2.8 / 3.8, 100 x 1001 2.7 / 3.2, at 200 rows 3.0 / 3.2
+    // and, with 20001 columns, 3.7 / 3.6.
+    const bool few_odd_rows = K <= 128 && !vm_whole_pieces(N, lda, reinterpret_cast<uintptr_t>(A), results);
+    if (N < 8 || N * K <= 4096 || few_odd_rows) {
         const int grid = (int)((N + 63) / 64);
         gemv_vm_f16_generic_kernel<<<grid, 64 * kVmGenericWaves, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu);
         return PIMHIP_OK;
     }
-    uintptr_t results = 0;
-    for (int o = 0; o < outs.count; ++o) results |= reinterpret_cast<uintptr_t>(outs.y[o]);
     const VmPlan plan = vm_plan(K, N, lda, reinterpret_cast<uintptr_t>(A), results, st->num_cus);
     float* partial = nullptr;
     unsigned int* status = nullptr;

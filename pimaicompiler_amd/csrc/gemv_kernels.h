@@ -546,7 +546,7 @@ __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_alone_f16_kernel(const 
     }
 }
 
-// VM order, fewer than eight columns, or very few weights: 2-byte loads.  A block of 16 wavefronts owns 64 adjacent output
+// VM order, fewer than eight columns, very few weights, or few rows of no whole pieces: 2-byte loads.  A block of 16 wavefronts owns 64 adjacent output
 // columns (one per lane); wavefront g takes the rows g, g + 16, ... and the sixteen partial sums meet in LDS.
 static constexpr int kVmGenericWaves = 16;
 __global__ __launch_bounds__(64 * kVmGenericWaves) void gemv_vm_f16_generic_kernel(const half_t* __restrict__ x,

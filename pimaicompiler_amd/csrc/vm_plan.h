@@ -24,9 +24,13 @@ struct VmPlan {
 // Weights of at most this many bytes, and operands of no whole 16-byte pieces, touch no workspace a caller would have to order
 // replays of a graph, or calls of the static entry point, against.
 static constexpr int64_t kVmSmallWeightBytes = 256 * 1024;
+inline bool vm_whole_pieces(int64_t N, int64_t lda, uintptr_t weight, uintptr_t results)
+{
+    return N % 8 == 0 && lda % 8 == 0 && (weight & 15u) == 0 && (results & 15u) == 0;
+}
 inline bool vm_needs_no_workspace(int64_t K, int64_t N, int64_t lda, uintptr_t weight, uintptr_t results)
 {
-    return K * N * 2 <= kVmSmallWeightBytes || N % 8 != 0 || lda % 8 != 0 || (weight & 15u) != 0 || (results & 15u) != 0;
+    return K * N * 2 <= kVmSmallWeightBytes || !vm_whole_pieces(N, lda, weight, results);
 }
 
 // The most words the partial sums of any product take: below, (slices - 1) * col_blocks is less than the target, which is at

@@ -55,7 +55,7 @@ def test_rows_of_any_length_at_any_address(ops, out_w, in_w, off_w, off_x, pitch
 
 
 @pytest.mark.parametrize("in_w,out_w,off,pitch", [
-    (1, 8, 0, 0), (600, 7, 0, 0), (600, 8, 0, 0), (600, 9, 1, 0), (513, 63, 0, 0), (512, 64, 0, 0), (513, 64, 0, 3), (513, 65, 0, 0),
+    (1, 8, 0, 0), (128, 257, 0, 0), (129, 257, 0, 0), (127, 64, 3, 0), (128, 1032, 0, 5), (17, 4001, 0, 0), (600, 7, 0, 0), (600, 8, 0, 0), (600, 9, 1, 0), (513, 63, 0, 0), (512, 64, 0, 0), (513, 64, 0, 3), (513, 65, 0, 0),
     (520, 71, 3, 0), (700, 128, 0, 8), (2305, 129, 0, 0), (8, 4096, 0, 0), (31, 4097, 0, 0), (1025, 1031, 5, 0), (12896, 84, 0, 0),
     (1500, 2000, 0, 0), (1000, 17000, 0, 0), (3001, 3001, 0, 0), (4101, 2056, 1, 0)])   # the last three: more than 16 MB
 def test_i_x_w_at_the_edges_of_blocks_row_groups_and_slices(ops, in_w, out_w, off, pitch):
