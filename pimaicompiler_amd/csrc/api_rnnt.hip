@@ -1,6 +1,8 @@
 // The RNN-transducer entry points of the C ABI (include/pimhip.h): one step of the greedy decoding loop (the prediction
 // network's LSTM cells at seq_len 1 and the joint network's two products) in one launch, and the whole loop over an
 // utterance in one launch.
+#include <algorithm>
+
 #include "api_common.h"
 #include "rnnt_greedy_kernels.h"
 
@@ -20,8 +22,9 @@ struct PimHipRnntPlan {
     unsigned long long* hx = nullptr;      // [2][blocks][kRnntEntryWords], all ones = empty
     unsigned int* g_counter = nullptr;     // [blocks][kRnntCounterStride]
     unsigned int* greedy = nullptr;        // what the loop kernel exchanges through, refilled before every launch of it:
-                                           // [kRnntGreedySets][blocks][kRnntEntryWords] 8-byte words (all ones), then
-                                           // seen [blocks][kRnntSeenStride] and solo_owner (zero)
+                                           // entries of kRnntEntryWords 8-byte words (all ones), then
+                                           // seen [greedy_blocks][kRnntSeenStride] and solo_owner (zero)
+    int greedy_teams = 1;                  // teams of symbol blocks in the loop kernel
     bool greedy_resident = false;          // all workgroups of the loop kernel fit on the device together
     unsigned int* abort_flag = nullptr;
     unsigned int* abort_host = nullptr;
@@ -42,9 +45,11 @@ size_t exchange_words32(const PimHipRnntPlan* plan) { return (size_t)2 * plan->b
 size_t greedy_exchange_words32(const PimHipRnntPlan* plan)
 {
     const size_t n_lstm = (size_t)plan->num_layers * (plan->hidden / 8), n_joint = plan->joint_size / 8, n_vocab = (plan->vocab + 7) / 8;
-    return (kRnntGreedyVersions * n_lstm + kRnntGreedyRing * (n_joint + n_vocab)) * kRnntEntryWords * 2;
+    return (kRnntGreedyVersions * n_lstm + kRnntGreedyRing * n_joint + kRnntGreedyLogitRing * n_vocab) * kRnntEntryWords * 2;
 }
-size_t greedy_count_words32(const PimHipRnntPlan* plan) { return (size_t)plan->blocks * kRnntSeenStride + kRnntSeenStride; }
+// Workgroups of the loop kernel: those of a step, and the symbol blocks once for each further team.
+int greedy_blocks(const PimHipRnntPlan* plan) { return plan->blocks + (plan->greedy_teams - 1) * (int)((plan->vocab + 7) / 8); }
+size_t greedy_count_words32(const PimHipRnntPlan* plan) { return (size_t)greedy_blocks(plan) * kRnntSeenStride + kRnntSeenStride; }
 
 int destroy_rnnt_plan_locked(PimHipRnntPlan* plan)
 {
@@ -157,12 +162,17 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
     launch_fill_u32(reinterpret_cast<unsigned int*>(plan->hx), exchange_words32(plan), ~0u, s);
     RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->g_counter), sizeof(unsigned int) * (size_t)plan->blocks * kRnntCounterStride));
     launch_fill_u32(plan->g_counter, (size_t)plan->blocks * kRnntCounterStride, 0u, s);
-    RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->greedy), sizeof(unsigned int) * (greedy_exchange_words32(plan) + greedy_count_words32(plan))));
     {
+        // As many teams of symbol blocks as the CUs that are left take, one workgroup to a CU, up to one for each step that the joint
+        // blocks run ahead (29 symbols, us per blank: 1.02 with one team, 0.87 with eight; 341 frames with 121 symbols: 1222, 1113).
+        const int n_vocab = (int)((vocab + 7) / 8);
+        const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
+        plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);
         int greedy_per_cu = 0;
         RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, rnnt_greedy_f16_kernel, kRnntThreads, 0));
-        plan->greedy_resident = (int64_t)greedy_per_cu * st->num_cus >= blocks;
+        plan->greedy_resident = (int64_t)greedy_per_cu * st->num_cus >= greedy_blocks(plan);
     }
+    RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->greedy), sizeof(unsigned int) * (greedy_exchange_words32(plan) + greedy_count_words32(plan))));
     RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->abort_flag), sizeof(unsigned int)));
     launch_fill_u32(plan->abort_flag, 1, 0u, s);
     RNNT_HIP_CHECK(hipGetLastError());
@@ -353,7 +363,8 @@ extern "C" int pimhip_rnnt_greedy_decode(PimHipRnntPlan* plan, const void* enc, 
     a.result = result;
     a.hx = reinterpret_cast<unsigned long long*>(plan->greedy);
     a.seen = plan->greedy + greedy_exchange_words32(plan);
-    a.solo_owner = a.seen + (size_t)plan->blocks * kRnntSeenStride;
+    a.solo_owner = a.seen + (size_t)greedy_blocks(plan) * kRnntSeenStride;
+    a.teams = plan->greedy_teams;
     a.abort_flag = plan->abort_flag;
     a.abort_host = plan->abort_host_dev;
     a.L = plan->num_layers;
@@ -377,7 +388,7 @@ extern "C" int pimhip_rnnt_greedy_decode(PimHipRnntPlan* plan, const void* enc, 
     // fill kernels, not memsets: the call can be recorded into a HIP graph
     launch_fill_u32(plan->greedy, greedy_exchange_words32(plan), ~0u, s);
     launch_fill_u32(plan->greedy + greedy_exchange_words32(plan), greedy_count_words32(plan), 0u, s);
-    rnnt_greedy_f16_kernel<<<dim3(a.alone ? 1u : (unsigned)plan->blocks), dim3(kRnntThreads), 0, s>>>(a);
+    rnnt_greedy_f16_kernel<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
     PIMHIP_HIP_CHECK(hipGetLastError());
     return PIMHIP_OK;
 }

@@ -22,24 +22,34 @@
 //   * most steps of a real utterance are blanks, after which only the frame changes: the joint blocks do not wait for the
 //     decision but publish the hidden vectors of the next steps as well, up to eight ahead, as if every decision in
 //     between were a blank (the frames' columns are asked for a round earlier and their sums kept), and the symbol blocks
-//     turn every hidden vector that arrives into logits, two per round.  When a symbol is emitted, g gets a new version
-//     and what was computed ahead under the old one is simply never looked at.  A run of blanks then costs what the symbol
-//     blocks' round costs, not two hand-overs per step.
+//     turn every hidden vector that arrives into logits.  When a symbol is emitted, g gets a new version
+//     and what was computed ahead under the old one is simply never looked at;
+//   * the symbol blocks exist several times over, as TEAMS: a symbol block's round (a look at 64 entries, a barrier, its sums, the
+//     publish) takes 2 us however few rows it has, so one set of blocks handles a run of blanks one or two steps a round.  The
+//     CUs that no other role needs hold up to seven further copies of W2's rows, team q takes the steps that are q modulo the
+//     number of teams, and the steps published ahead become logits side by side;
+//   * the joint blocks publish the step that everybody waits for alone and then four steps behind each barrier.
+//
+// Measured on MI355X (one team and two steps a publish before; us per blank / per symbol / an utterance of 341 frames and 121
+// symbols, 2 x 320 units, 512 joint units, 29 symbols): 1.42 / 6.8 / 1395 before, 0.87 / 7.3 / 1113 now; 200 frames and 33 symbols
+// of a 400-word vocabulary (2 x 256 units) 881 -> 478 us.  What bounds it now: a symbol's four hand-overs of 1.0 - 1.3 us, which
+// the traffic of the steps published ahead made 0.1 us longer each, and in a run of blanks the eight steps ahead over the two
+// hand-overs and three roles' rounds that they travel (12 steps ahead: 0.82 us per blank, and 2 % more with one layer).
 //
 // Exchange: 8-byte words of three fp16 values and a 16-bit tag, three words per producing block in a 128-byte entry of its
 // own, written and read with device-scope accesses.  The tag says what the word belongs to: h of a layer carries the
 // version of g (the count of the prediction network's runs), hidden vectors and logits carry the step and the version they
 // were computed under; a word with another tag is "not there yet", so nothing is ever cleared and a stale word cannot be
-// taken for a fresh one.  h lives in four sets by version, hidden vectors and logits in rings of sixteen by step.  A
-// producer may overwrite what is sixteen steps old: for the joint blocks' entries that follows from the order of things
+// taken for a fresh one.  h lives in four sets by version, hidden vectors in a ring of sixteen by step, logits in one of 64.  A
+// producer may overwrite what is a ring old: for the joint blocks' entries that follows from the order of things
 // (they run at most eight steps ahead of decisions that the symbol blocks have already published); the symbol blocks, whom
-// a slow reader could fall sixteen steps behind (nobody waits for the layers' blocks during a run of blanks), look at a
+// a slow reader could fall a ring behind (nobody waits for the layers' blocks during a run of blanks), look at a
 // count that every block keeps of the decisions it has taken in (`seen`) before they reuse an entry.
 //
 // Waiting: a block looks at everything it waits for in one round ("pass"): the words of a vector by the first six
-// wavefronts, the logits of the next four steps by the last two (of one step where there are more than 80 symbols).  What
-// the block cannot go on without is polled until it is there, the rest is looked at once; one barrier ends the round, and
-// a pass can take several decisions at once.
+// wavefronts, the logits of the next steps by the last ones (of four steps by one wavefront with up to 40 symbols, one step by
+// each beyond).  What the block cannot go on without is polled until it is there, the rest is looked at once; one barrier ends the round, and
+// a pass can take several decisions at once: a run of blanks is a run of ones in a ballot.
 //
 // Sums run in the order of the step kernel, c is rounded to fp16 after every run of the prediction network as it is when
 // the state travels between launches: symbols and final state equal, bit for bit, those of a loop of pimhip_rnnt_step
@@ -50,18 +60,30 @@
 // of microseconds per step, the same sums): a wait that gives up costs time, not the result.
 #pragma once
 
+#include <type_traits>
+
 #include "rnnt_kernels.h"
 
 namespace pimhip
 {
 
 constexpr int kRnntGreedyVersions = 4;             // h of a layer: one entry per block and version of g, modulo this
-constexpr int kRnntGreedyRing = 16;                // hidden vectors and logits: one entry per block and step, modulo this
+constexpr int kRnntGreedyRing = 16;                // hidden vectors: one entry per block and step, modulo this
+constexpr int kRnntGreedyLogitRing = 64;           // logits: the same
 constexpr int kRnntGreedyAhead = 8;                // steps the joint network runs ahead of the decisions
-constexpr int kRnntGreedyLook = 4;                 // steps whose logits one pass looks at
+constexpr int kRnntGreedyLook = 8;                 // steps whose logits one pass looks at, at most
+constexpr int kRnntGreedyTeams = 8;                // at most this many teams of symbol blocks, each with the steps of one residue
+constexpr int kRnntGreedyBatch = 4;                // hidden vectors a joint block publishes behind one barrier
 static_assert(kRnntGreedyAhead < kRnntGreedyRing && (kRnntGreedyRing & (kRnntGreedyRing - 1)) == 0, "ring");
-constexpr int kRnntGreedyMaxVocab = 512;           // symbols (the logits of the steps a pass looks at lie in LDS)
-constexpr int kRnntGreedyWideVocab = 10;           // with more symbol blocks than this a pass looks at the logits of one step, not four
+static_assert((kRnntGreedyLogitRing & (kRnntGreedyLogitRing - 1)) == 0 && kRnntGreedyLogitRing <= 128, "a ring's steps differ in their 8-bit tags");
+static_assert(kRnntGreedyLook + kRnntGreedyAhead < kRnntGreedyLogitRing, "a look and what is published ahead of it lie in one ring");
+static_assert(kRnntGreedyLook == kRnntWaves && kRnntGreedyLook == 8, "a wavefront per step");
+static_assert(kRnntGreedyBatch <= kRnntWaves, "a wavefront stores one step's word of a batch");
+constexpr int kRnntGreedyMaxVocab = 512;           // symbols
+constexpr int kRnntGreedyRowVocab = 5;             // up to this many symbol blocks to a team (15 words) a step's logits are a row of 16 lanes'
+constexpr int kRnntGreedyRows = 4;                 // ... and a pass looks at as many steps
+constexpr int kRnntGreedyLaneWords = 3;            // words a lane takes of a step's logits where a wavefront takes them
+static_assert(3 * (kRnntGreedyMaxVocab / 8) <= 64 * kRnntGreedyLaneWords, "a wavefront takes a step's logits");
 constexpr int kRnntGreedyEmbHalfs = 16384;         // embedding rows kept in LDS by the first layer's blocks (32 KB)
 constexpr int kRnntSeenStride = 16;                // 32-bit words between the blocks' `seen` counts
 
@@ -90,6 +112,7 @@ struct RnntGreedyArgs {
     int emb_rows, emb_in_lds;
     int blank, max_symbols, max_per_frame;
     int run_pred_first;        // 0: the first step takes g = h0 of the last layer as it is (decoding goes on after a blank)
+    int teams;                 // teams of symbol blocks: team q has the steps that are q modulo `teams`
     unsigned int spin_limit;
     int alone;                 // the launch is one workgroup that decodes by itself
 };
@@ -144,20 +167,69 @@ __device__ __forceinline__ unsigned int rnnt_max_u32(unsigned int v)
     return v;
 }
 
-// torch.argmax over V fp16 values: the first maximum, a NaN counting as the largest.  Every lane returns it.  One integer
-// maximum over keys: the value's bits made monotonic (-0 as +0, a NaN above everything) in front of the index counted from
-// the top, so that of equal values the first wins.  A lane takes the values lane, lane + 64, ..
+// torch.argmax over fp16 values: the first maximum, a NaN counting as the largest.  One integer maximum over keys: the value's
+// bits made monotonic (-0 as +0, a NaN above everything) in front of the index counted from the top, so that of equal
+// values the first wins.  A key is never 0.
+__device__ __forceinline__ unsigned int rnnt_key(unsigned int bits, int i)
+{
+    if (bits == 0x8000u) bits = 0u;
+    unsigned int order = (bits & 0x8000u) ? (~bits & 0xffffu) : (bits | 0x8000u);
+    if ((bits & 0x7fffu) > 0x7c00u) order = 0xffffu;
+    return (order << 16) | (unsigned int)(0xffff - i);
+}
+
+__device__ __forceinline__ int rnnt_key_index(unsigned int key) { return 0xffff - (int)(key & 0xffffu); }
+
+// The argmax of lg[0 .. V); every lane returns it.  A lane takes the values lane, lane + 64, ..
 __device__ __forceinline__ int rnnt_argmax(const half_t* lg, int V, int lane)
 {
     unsigned int key = 0u;
-    for (int i = lane; i < V; i += 64) {
-        unsigned int bits = __builtin_bit_cast(unsigned short, lg[i]);
-        if (bits == 0x8000u) bits = 0u;
-        unsigned int order = (bits & 0x8000u) ? (~bits & 0xffffu) : (bits | 0x8000u);
-        if ((bits & 0x7fffu) > 0x7c00u) order = 0xffffu;
-        key = max(key, (order << 16) | (unsigned int)(0xffff - i));
+    for (int i = lane; i < V; i += 64) key = max(key, rnnt_key(__builtin_bit_cast(unsigned short, lg[i]), i));
+    return rnnt_key_index(rnnt_max_u32(key));
+}
+
+// The largest key of a word of logits: values 8 prod + 3 part .. + 2 (the third word of a block has two).
+__device__ __forceinline__ unsigned int rnnt_word_key(unsigned long long w, int prod, int part)
+{
+    const int i = 8 * prod + 3 * part;
+    unsigned int key = max(rnnt_key((unsigned int)w & 0xffffu, i), rnnt_key((unsigned int)(w >> 16) & 0xffffu, i + 1));
+    if (part < 2) key = max(key, rnnt_key((unsigned int)(w >> 32) & 0xffffu, i + 2));
+    return key;
+}
+
+// The maximum over a row of 16 lanes; every lane of the row returns it.
+__device__ __forceinline__ unsigned int rnnt_max_row(unsigned int v)
+{
+    v = max(v, rnnt_dpp_u32<kDppQuadXor1>(v));
+    v = max(v, rnnt_dpp_u32<kDppQuadXor2>(v));
+    v = max(v, rnnt_dpp_u32<0x124>(v));
+    return max(v, rnnt_dpp_u32<0x128>(v));
+}
+
+// rnnt_sum of several values at once, stage by stage, in the same order each.
+template <int N>
+__device__ __forceinline__ void rnnt_sums(float (&v)[N])
+{
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<kDppQuadXor1>(v[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<kDppQuadXor2>(v[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<0x124>(v[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<0x128>(v[q]);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        float a = v[q], b = v[q];
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+        v[q] = a + b;
     }
-    return 0xffff - (int)(rnnt_max_u32(key) & 0xffffu);
+#pragma unroll
+    for (int q = 0; q < N; ++q) {
+        float a = v[q], b = v[q];
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+        v[q] = a + b;
+    }
 }
 
 // The whole loop by one workgroup.  LDS: hs [L * H] (h of every layer), cs [L * H], tmp [max(H, J)], lg [V].
@@ -243,11 +315,11 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     typedef unsigned long long u64;
     __shared__ __align__(16) half_t buf0[kRnntMaxVec];                              // the vector a role waits for
     __shared__ __align__(16) half_t own[kRnntMaxH];                                 // a layer's blocks: h of their layer; joint blocks: g
-    __shared__ __align__(16) half_t lgs[2][kRnntGreedyLook][kRnntGreedyMaxVocab];   // the logits of the next steps, alternating per pass
+    __shared__ unsigned int keys[2][kRnntGreedyLook];                               // per pass (alternating): the best key of the next steps' logits, 0: not there
     __shared__ __align__(16) half_t emb[kRnntGreedyEmbHalfs];                       // first layer: the embedding rows and x0 behind them
-    __shared__ __align__(16) unsigned short mine[2][12];                            // this block's eight values, alternating per publish
-    __shared__ int missing[3][3 + kRnntGreedyLook];                                 // per pass (rotating): something of the vector / of step j is not
-                                                                                    // there yet; a wait has given up; something of a second vector is not there
+    __shared__ __align__(16) unsigned short mine[2][kRnntGreedyBatch][12];          // this block's eight values (a joint block's of several steps), alternating per publish
+    __shared__ int missing[3][3];                                                   // per pass (rotating): something of the vector is not there yet; a
+                                                                                    // wait has given up; something of a second vector is not there
     __shared__ int someone_gave_up;
     __shared__ int i_decode_alone;
     __shared__ int min_seen_lds;
@@ -266,8 +338,8 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         someone_gave_up = (p.alone || __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) ? 1 : 0;
         i_decode_alone = 0;
     }
-    if (tid < 3 * (3 + kRnntGreedyLook)) (&missing[0][0])[tid] = 0;
-    if (tid < 24) (&mine[0][0])[tid] = 0;
+    if (tid < 9) (&missing[0][0])[tid] = 0;
+    if (tid < 2 * kRnntGreedyBatch * 12) (&mine[0][0][0])[tid] = 0;
     __syncthreads();
 
     RnntGreedyState s = {0, 0, 0, -1, p.run_pred_first};
@@ -276,34 +348,33 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     bool dead = false;                 // a wait of this block has given up (the same in every thread)
     unsigned long long t_first = 0ull;
 
-    auto running = [&]() { return s.t < p.T && s.emitted < p.max_symbols; };
+    auto running = [&]() __attribute__((always_inline)) { return s.t < p.T && s.emitted < p.max_symbols; };
     // The version of g that the current step's joint network sees: runs of the prediction network started, less one.
-    auto g_version = [&]() { return n_pred + s.run_pred - 1; };
+    auto g_version = [&]() __attribute__((always_inline)) { return n_pred + s.run_pred - 1; };
     auto h_tag = [](int version) { return (unsigned int)(version & 0x7fff); };
     auto step_tag = [](int st, int version) { return (unsigned int)(((version & 0x7f) << 8) | (st & 0xff)); };
-    auto h_entry = [&](int version, int block) { return p.hx + ((long)(version & (kRnntGreedyVersions - 1)) * n_lstm + block) * kRnntEntryWords; };
-    auto hid_entry = [&](int st, int j) {
+    auto h_entry = [&](int version, int block) __attribute__((always_inline)) { return p.hx + ((long)(version & (kRnntGreedyVersions - 1)) * n_lstm + block) * kRnntEntryWords; };
+    auto hid_entry = [&](int st, int j) __attribute__((always_inline)) {
         return p.hx + ((long)kRnntGreedyVersions * n_lstm + (long)(st & (kRnntGreedyRing - 1)) * nwj + j) * kRnntEntryWords;
     };
-    auto lg_entry = [&](int st, int j) {
-        return p.hx + ((long)kRnntGreedyVersions * n_lstm + (long)kRnntGreedyRing * nwj + (long)(st & (kRnntGreedyRing - 1)) * nwv + j) * kRnntEntryWords;
+    auto lg_entry = [&](int st, int j) __attribute__((always_inline)) {
+        return p.hx + ((long)kRnntGreedyVersions * n_lstm + (long)kRnntGreedyRing * nwj + (long)(st & (kRnntGreedyLogitRing - 1)) * nwv + j) * kRnntEntryWords;
     };
 
-    // mine[] of this publish goes out as three 8-byte words of three values and the tag each.
-    auto publish = [&](u64* entry, unsigned int tag) {
-        rnnt_barrier();
-        if (tid < 3) {
-            const unsigned short* m = mine[n_publish & 1u] + 3 * tid;
+    // mine[which] of this publish goes out as three 8-byte words of three values and the tag each, from one wavefront (several
+    // steps of a joint or symbol block: one wavefront each behind the same barrier).
+    auto store_words = [&](int which, u64* entry, unsigned int tag) __attribute__((always_inline)) {
+        if (lane < 3) {
+            const unsigned short* m = mine[n_publish & 1u][which] + 3 * lane;
             const u64 w = (u64)m[0] | ((u64)m[1] << 16) | ((u64)m[2] << 32) | ((u64)tag << 48);
-            __hip_atomic_store(entry + tid, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(entry + lane, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
-        ++n_publish;
     };
-    auto my_values = [&]() { return mine[n_publish & 1u]; };
+    auto my_value = [&](int which) __attribute__((always_inline)) -> unsigned short& { return mine[n_publish & 1u][which][wave]; };
 
     // One 8-byte word: looked at once, or (blocks) polled until it carries `tag` or the wait's limits are reached, in which
     // case the thread raises the abort words and this pass's "gave up" flag.  Returns whether the tag is there.
-    auto fetch = [&](const u64* slot, unsigned int tag, bool blocks, int* miss, u64& w) {
+    auto fetch = [&](const u64* slot, unsigned int tag, bool blocks, int* miss, u64& w) __attribute__((always_inline)) {
         unsigned int spins = 0;
         unsigned long long first = 0ull;
         while (true) {
@@ -321,79 +392,144 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 give_up = true;
             }
             if (give_up) {
-                miss[1 + kRnntGreedyLook] = 1;
+                miss[1] = 1;
                 someone_gave_up = 1;
                 return false;
             }
             if (spins != 0xffffffffu) ++spins;
         }
     };
-    auto unpack = [&](u64 w, half_t* dst, int prod, int part) {
+    auto unpack = [&](u64 w, half_t* dst, int prod, int part) __attribute__((always_inline)) {
         unsigned short* d = reinterpret_cast<unsigned short*>(dst) + 8 * prod + 3 * part;
         d[0] = (unsigned short)w;
         d[1] = (unsigned short)(w >> 16);
         if (part < 2) d[2] = (unsigned short)(w >> 32);
     };
     // One round over everything this block waits for: the 8-byte words of a vector (n_vec producers from `vec`, tagged
-    // vec_tag, values to vec_dst) by the first six wavefronts, and with want_steps the logits of the steps step .. step + 3
-    // under the current version by the last two.  What the block cannot go on without is polled until it is there
-    // (vec_blocks; step_blocks: the logits of `step`), the rest is looked at once.  Returns bit 0: the vector is complete;
-    // bit 1 + j: the logits of step + j are.
-    // A second vector (vec2, looked at once) is taken along where the first leaves threads free; bit 30 says it is complete.
-    auto pass = [&](const u64* vec, int n_vec, unsigned int vec_tag, half_t* vec_dst, bool vec_blocks, bool want_steps, bool step_blocks,
-                    const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr) -> int {
+    // vec_tag, values to vec_dst) by the first six wavefronts, and with look_waves the logits of the steps from `step` on under
+    // the current version by as many of the last wavefronts: one step each, or, where a step's words fit a row of 16 lanes, four
+    // steps by the last one.  The wavefront that takes a step's words makes the argmax of them (its key) right there, so that behind
+    // the barrier nothing but a few keys is left to read.  What the block cannot go on without is polled until it is there
+    // (vec_blocks; step_blocks: the logits of `step`), the rest is looked at once.  Returns bit 0: the vector is complete.
+    // A second vector (vec2, looked at once) is taken along where the first leaves threads free; bit 1 says it is complete.
+    // my_key, n_there: the key of step + lane % 8 in every lane, and how many steps from `step` on are there.
+    // (The wavefronts that poll what a step is waited for with are not those that store: a wavefront's memory operations return
+    // in order, and a device-scope store's acknowledgement takes longer than a poll.)
+    unsigned int my_key = 0u;
+    int n_there = 0;
+    const bool row_per_step = nwv <= kRnntGreedyRowVocab;
+    auto pass = [&](const u64* vec, int n_vec, unsigned int vec_tag, half_t* vec_dst, bool vec_blocks, int look_waves, bool step_blocks,
+                    const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr) __attribute__((always_inline)) -> int {
         int* miss = missing[n_pass % 3u];
         u64 w;
-        if (tid < 384) {
-            for (int i = tid; i < 3 * (n_vec + n_vec2); i += 384) {
-                const bool second = i >= 3 * n_vec;
-                const int i2 = second ? i - 3 * n_vec : i;
-                const int prod = i2 / 3, part = i2 - 3 * prod;
-                if (!second) {
-                    if (fetch(vec + (long)prod * kRnntEntryWords + part, vec_tag, vec_blocks, miss, w))
-                        unpack(w, vec_dst, prod, part);
-                    else
-                        miss[0] = 1;
-                } else {
-                    if (fetch(vec2 + (long)prod * kRnntEntryWords + part, vec2_tag, false, miss, w))
-                        unpack(w, vec2_dst, prod, part);
-                    else
-                        miss[2 + kRnntGreedyLook] = 1;
+        const int look = kRnntWaves - 1 - wave;
+        if (look >= look_waves) {
+            if (tid < 384) {
+                // Where a symbol is on its way and this team's hidden vector is not the next one, one word of it is looked at first.
+                const bool there_yet = !s.run_pred || vec_blocks || n_vec == 0 ||
+                                       (unsigned int)(__hip_atomic_load(vec, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 48) == vec_tag;
+                if (!there_yet) miss[0] = miss[2] = 1;
+                for (int i = tid; there_yet && i < 3 * (n_vec + n_vec2); i += 384) {
+                    const bool second = i >= 3 * n_vec;
+                    const int i2 = second ? i - 3 * n_vec : i;
+                    const int prod = i2 / 3, part = i2 - 3 * prod;
+                    if (!second) {
+                        if (fetch(vec + (long)prod * kRnntEntryWords + part, vec_tag, vec_blocks, miss, w))
+                            unpack(w, vec_dst, prod, part);
+                        else
+                            miss[0] = 1;
+                    } else {
+                        if (fetch(vec2 + (long)prod * kRnntEntryWords + part, vec2_tag, false, miss, w))
+                            unpack(w, vec2_dst, prod, part);
+                        else
+                            miss[2] = 1;
+                    }
                 }
             }
-        } else if (want_steps) {
-            // 32 threads per step for the logits of four steps, or (many symbols) all 128 for those of `step` alone
-            const bool wide = nwv > kRnntGreedyWideVocab;
-            const int per_step = wide ? 128 : 32;
-            const int j = (tid - 384) / per_step, i0 = (tid - 384) - j * per_step;
-            if (wide && tid - 384 < kRnntGreedyLook - 1) miss[2 + (tid - 384)] = 1;
-            for (int i = i0; i < 3 * nwv; i += per_step) {
-                const int prod = i / 3, part = i - 3 * prod;
-                if (fetch(lg_entry(step + j, prod) + part, step_tag(step + j, g_version()), step_blocks && j == 0, miss, w))
-                    unpack(w, lgs[n_pass & 1u][j], prod, part);
-                else
-                    miss[1 + j] = 1;
+        } else if (!row_per_step || look == 0) {
+            // A lane's words of `st`: the one of its place in a row of 16 lanes, or those of its place in the wavefront.
+            constexpr int kN = kRnntGreedyLaneWords;
+            const int version = g_version();
+            u64 v[kN];
+            auto look_at = [&](int st, bool in_row) __attribute__((always_inline)) {
+                bool there = true;
+#pragma unroll
+                for (int n = 0; n < kN; ++n) {
+                    const int i = in_row ? (lane & 15) : lane + 64 * n;
+                    if (i < 3 * nwv && !(in_row && n > 0)) v[n] = __hip_atomic_load(lg_entry(st, i / 3) + i % 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+#pragma unroll
+                for (int n = 0; n < kN; ++n) {
+                    const int i = in_row ? (lane & 15) : lane + 64 * n;
+                    if (i < 3 * nwv && !(in_row && n > 0)) there = there && (unsigned int)(v[n] >> 48) == step_tag(st, version);
+                }
+                return there;
+            };
+            auto best = [&](bool in_row) __attribute__((always_inline)) {
+                unsigned int key = 0u;
+#pragma unroll
+                for (int n = 0; n < kN; ++n) {
+                    const int i = in_row ? (lane & 15) : lane + 64 * n;
+                    if (i < 3 * nwv && !(in_row && n > 0)) key = max(key, rnnt_word_key(v[n], i / 3, i % 3));
+                }
+                return key;
+            };
+            const bool blocks = step_blocks && look == 0;
+            unsigned int spins = 0;
+            unsigned long long first = 0ull;
+            bool there;
+            while (true) {
+                there = look_at(step + (row_per_step ? lane >> 4 : look), row_per_step);
+                if (!blocks || __all(there || (row_per_step && lane >= 16))) break;
+                bool give_up = false;
+                if (spins > 0u && (spins & 255u) == 0u) {
+                    if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
+                    if (wait_clock_expired(spins, first)) spins = 0xffffffffu;
+                }
+                if (spins >= p.spin_limit) {
+                    __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    give_up = true;
+                }
+                if (__any(give_up)) {
+                    miss[1] = 1;
+                    someone_gave_up = 1;
+                    break;
+                }
+                if (spins != 0xffffffffu) ++spins;
+            }
+            if (row_per_step) {
+                const unsigned long long m = __ballot(there);
+                const bool whole = ((m >> (lane & 48)) & 0xffffull) == 0xffffull;
+                const unsigned int key = rnnt_max_row(best(true));
+                if ((lane & 15) == 0) keys[n_pass & 1u][lane >> 4] = whole ? key : 0u;
+            } else {
+                unsigned int key = rnnt_max_u32(best(false));
+                if (!__all(there)) key = 0u;
+                if (lane == 0) keys[n_pass & 1u][look] = key;
             }
         }
         rnnt_barrier();
         int r = (n_vec > 0 && miss[0] == 0) ? 1 : 0;
-        if (want_steps) {
-#pragma unroll
-            for (int j = 0; j < kRnntGreedyLook; ++j)
-                if (miss[1 + j] == 0) r |= 2 << j;
+        if (n_vec2 > 0 && miss[2] == 0) r |= 2;
+        n_there = 0;
+        if (look_waves) {
+            const int looked = row_per_step ? kRnntGreedyRows : look_waves;
+            my_key = keys[n_pass & 1u][lane & (kRnntGreedyLook - 1)];
+            const unsigned int there = (unsigned int)__ballot(my_key != 0u) & ((1u << looked) - 1u);
+            n_there = __builtin_ctz(~there);
         }
-        if (n_vec2 > 0 && miss[2 + kRnntGreedyLook] == 0) r |= 1 << 30;
-        if (miss[1 + kRnntGreedyLook] != 0) dead = true;
+        if (miss[1] != 0) dead = true;
         // the flags of the pass after the next are cleared now: their last readers passed this barrier, their next
         // writers come after the next one
-        if (tid < 3 + kRnntGreedyLook) missing[(n_pass + 2u) % 3u][tid] = 0;
+        if (tid < 3) missing[(n_pass + 2u) % 3u][tid] = 0;
         ++n_pass;
         return r;
     };
     // After a pass that brought nothing: counts, and gives up when the limits are reached.  Everybody learns of it behind the
     // next pass's barrier, through that pass's flags (a word that thread 0 wrote now could be read by some threads of this
     // round and not by others).
-    auto nothing_came = [&]() {
+    auto nothing_came = [&]() __attribute__((always_inline)) {
         if (tid == 0) {
             bool give_up = false;
             if (waited > 0u && (waited & 255u) == 0u) {
@@ -407,46 +543,50 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             }
             if (give_up) {
                 someone_gave_up = 1;
-                missing[n_pass % 3u][1 + kRnntGreedyLook] = 1;
+                missing[n_pass % 3u][1] = 1;
             }
             if (waited != 0xffffffffu) ++waited;
         }
     };
-    auto something_came = [&]() {
+    auto something_came = [&]() __attribute__((always_inline)) {
         if (tid == 0) waited = 0u;
     };
-    // Takes the decisions whose logits a pass found (bits 1.. of mask), in order, up to and including the first that emits a
-    // symbol (what lies behind it was computed for a g that is no longer the current one).  Returns how many.
-    auto take_decisions = [&](int mask) {
-        int taken = 0;
-#pragma unroll
-        for (int j = 0; j < kRnntGreedyLook; ++j) {
-            if (!(mask & (2 << j)) || !running()) break;
-            const int k = rnnt_argmax(lgs[(n_pass - 1u) & 1u][j], p.V, lane);
+    // Takes the decisions whose logits a pass found, in order, up to and including the first that emits a symbol (what lies
+    // behind it was computed for a g that is no longer the current one); a run of blanks in one go.  Returns how many.
+    auto take_decisions = [&]() __attribute__((always_inline)) {
+        if (n_there == 0) return 0;
+        const unsigned int blanks = (unsigned int)__ballot(rnnt_key_index(my_key) == p.blank) & ((1u << kRnntGreedyLook) - 1u);
+        int taken = min(min(n_there, __builtin_ctz(~blanks)), p.T - s.t);
+        if (taken > 0) {
+            n_pred += s.run_pred;
+            s.run_pred = 0;
+            s.frame_syms = 0;
+            s.t += taken;
+            step += taken;
+        }
+        if (taken < n_there && s.t < p.T) {
+            const int k = rnnt_key_index(__builtin_amdgcn_readlane(my_key, taken));
             const int at = s.emitted;
             n_pred += s.run_pred;
             ++step;
             ++taken;
-            if (rnnt_greedy_advance(s, k, p.blank, p.max_per_frame)) {
-                if (b == 0 && tid == 0) p.symbols[at] = k;
-                break;
-            }
+            rnnt_greedy_advance(s, k, p.blank, p.max_per_frame);
+            if (b == 0 && tid == 0) p.symbols[at] = k;
         }
-        if (taken > 0 && tid == 0)
-            __hip_atomic_store(p.seen + (long)kRnntSeenStride * b, (unsigned int)step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (tid == 384) __hip_atomic_store(p.seen + (long)kRnntSeenStride * b, (unsigned int)step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         return taken;
     };
     // Waits for a vector.  Returns false when the block has to leave the loop.
-    auto wait_for_vector = [&](const u64* vec, int n_vec, unsigned int tag, half_t* dst) {
-        pass(vec, n_vec, tag, dst, true, false, false);
+    auto wait_for_vector = [&](const u64* vec, int n_vec, unsigned int tag, half_t* dst) __attribute__((always_inline)) {
+        pass(vec, n_vec, tag, dst, true, 0, false);
         return !dead;
     };
     // Waits until the decision of `step` can be taken, and takes those behind it too if their logits are there already.
     // Returns false when the block has to leave the loop.
-    auto wait_for_decisions = [&]() {
-        const int r = pass(nullptr, 0, 0u, nullptr, false, true, true);
+    auto wait_for_decisions = [&]() __attribute__((always_inline)) {
+        pass(nullptr, 0, 0u, nullptr, false, kRnntWaves, true);
         if (dead) return false;
-        take_decisions(r);
+        take_decisions();
         return true;
     };
 
@@ -491,7 +631,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         __syncthreads();
         // W_hh . h of the layer, summed as soon as h is known
         float a_hh[4];
-        auto sum_hh = [&]() {
+        auto sum_hh = [&]() __attribute__((always_inline)) {
             const half8_t* hv = reinterpret_cast<const half8_t*>(own);
 #pragma unroll
             for (int gt = 0; gt < 4; ++gt) {
@@ -532,8 +672,10 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 c_half = rnnt_round(c_new);
                 const unsigned short bits = rnnt_bits((float)h_new);
                 h_last = __builtin_bit_cast(half_t, bits);
-                if (lane == 0) my_values()[wave] = bits;
-                publish(h_entry(version, b), h_tag(version));
+                if (lane == 0) my_value(0) = bits;
+                rnnt_barrier();
+                if (wave == 6) store_words(0, h_entry(version, b), h_tag(version));
+                ++n_publish;
                 // h of this layer, for W_hh at the next symbol
                 if (!wait_for_vector(h_entry(version, l * nwh), nwh, h_tag(version), own)) {
                     ok = false;
@@ -568,7 +710,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         for (int i = tid; i < H; i += kRnntThreads) own[i] = p.h0 ? p.h0[(long)(p.L - 1) * H + i] : (half_t)0.0f;  // g before the first run
         __syncthreads();
         // this lane's part of the row's sum over a frame (nothing is read for a frame the utterance does not have)
-        auto sum_f = [&](int frame) {
+        auto sum_f = [&](int frame) __attribute__((always_inline)) {
             float a = 0.0f;
             if (frame >= 0 && frame < p.T) {
                 const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)frame * p.F);
@@ -579,29 +721,61 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             return a;
         };
         // The sums over the frames around the current one are kept (per thread, in the LDS that the first layer's blocks
-        // use for the embedding rows): frames [af_lo, af_hi) in slots frame mod 16.  A frame is summed once, ahead of its
+        // use for the embedding rows): frame f in slot f mod 16, those up to af_hi.  A frame is summed once, ahead of its
         // turn, whatever the number of symbols it then emits.
         float* af_ring = reinterpret_cast<float*>(emb) + tid;
         static_assert(kRnntGreedyRing * kRnntThreads * sizeof(float) <= kRnntGreedyEmbHalfs * sizeof(half_t), "the ring of frame sums fits");
-        int af_lo = 0, af_hi = 0;
-        auto frame_keep = [&](int frame, float a) {
-            if (frame != af_hi) af_lo = frame;
-            af_hi = frame + 1;
-            if (af_hi - af_lo > kRnntGreedyRing) af_lo = af_hi - kRnntGreedyRing;
-            af_ring[(frame & (kRnntGreedyRing - 1)) * kRnntThreads] = a;
+        static_assert(kRnntGreedyAhead + 1 <= kRnntGreedyRing, "and holds what a round publishes");
+        int af_hi = 0;
+        auto frame_keep = [&](float a) __attribute__((always_inline)) { af_ring[(af_hi++ & (kRnntGreedyRing - 1)) * kRnntThreads] = a; };
+        // The next frames the ring does not hold yet are asked for in front of a wait and summed behind it (their columns travel
+        // while the symbol blocks work): as many as sixteen pieces per lane hold, the eight that two looks can consume.
+        constexpr int kPieces = 16;
+        static_assert(16 <= kPieces && kPieces % kRnntFC == 0, "eight frames of two pieces, or four of four");
+        const bool short_frames = nfp <= 128;
+        half8_t col[kPieces];
+        int f_first = 0, n_ask = 0;
+        auto ask_frames = [&](auto pieces) __attribute__((always_inline)) {
+            constexpr int kP = decltype(pieces)::value;
+            f_first = af_hi;
+            n_ask = max(0, min(min(kPieces / kP, p.T - f_first), s.t + kRnntGreedyRing - f_first));  // (what the ring still needs stays in it)
+#pragma unroll
+            for (int q = 0; q < kPieces / kP; ++q) {
+#pragma unroll
+                for (int k = 0; k < kP; ++k)
+                    col[q * kP + k] = (q < n_ask && lane + 64 * k < nfp) ? reinterpret_cast<const half8_t*>(p.enc + (long)(f_first + q) * p.F)[lane + 64 * k] : wf[k];
+            }
         };
-        auto frame_sum = [&](int frame) {
-            if (frame >= af_lo && frame < af_hi) return af_ring[(frame & (kRnntGreedyRing - 1)) * kRnntThreads];
-            const float a = sum_f(frame);
-            frame_keep(frame, a);
-            return a;
+        auto keep_frames = [&](auto pieces) __attribute__((always_inline)) {
+            constexpr int kP = decltype(pieces)::value;
+#pragma unroll
+            for (int q = 0; q < kPieces / kP; ++q) {
+                if (q < n_ask) {
+                    float a = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < kP; ++k)
+                        if (lane + 64 * k < nfp) a = dot8(wf[k], col[q * kP + k], a);
+                    frame_keep(a);
+                }
+            }
+        };
+        auto ask = [&]() __attribute__((always_inline)) {
+            if (short_frames) ask_frames(std::integral_constant<int, 2>{});
+            else ask_frames(std::integral_constant<int, 4>{});
+        };
+        auto keep = [&]() __attribute__((always_inline)) {
+            if (short_frames) keep_frames(std::integral_constant<int, 2>{});
+            else keep_frames(std::integral_constant<int, 4>{});
         };
         int have_g = -1;          // the version of g in `own`
         int pub = 0;              // the next step to publish a hidden vector for
-        frame_sum(0);
+        ask();
+        keep();
         bool ok = true;
         while (ok && running()) {
             const int version = g_version();
+            const int end = min(step + kRnntGreedyAhead + 1, step + (p.T - s.t));
+            while (af_hi < s.t + (end - step)) frame_keep(sum_f(af_hi));  // (what was not asked for in time)
             if (version != have_g) {
                 if (!wait_for_vector(h_entry(version, (p.L - 1) * nwh), nwh, h_tag(version), own)) {
                     ok = false;
@@ -611,53 +785,40 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 pub = step;
             }
             if (pub < step) pub = step;
-            // the current step first, then up to kRnntGreedyAhead behind it: two per round while symbols come (the next g is
-            // what matters then), more in a run of blanks, where running ahead is all there is to do
-            const int per_round = s.run_pred ? 2 : 5;
-            for (int i = 0; i < per_round; ++i) {
-                const int frame = s.t + (pub - step);
-                if (frame >= p.T || pub > step + kRnntGreedyAhead) break;
-                const half8_t* gv = reinterpret_cast<const half8_t*>(own);
-                float a = frame_sum(frame);
+            // the current step and up to kRnntGreedyAhead behind it: the first alone behind its barrier, then batches
+            const half8_t* gv = reinterpret_cast<const half8_t*>(own);
+            half8_t gk[kRnntHC];
 #pragma unroll
-                for (int k = 0; k < kRnntHC; ++k)
-                    if (lane + 64 * k < nhp) a = dot8(wg[k], gv[lane + 64 * k], a);
-                a = rnnt_sum(a);
-                if (lane == 0) my_values()[wave] = rnnt_bits(relu_f32(a + bias));
-                publish(hid_entry(pub, jb), step_tag(pub, version));
-                ++pub;
-            }
-            // The next frames the ring does not hold yet are asked for now and summed behind the wait for the decisions (their
-            // columns travel while the symbol blocks work): up to four a round, as many as a round can publish.
-            constexpr int kAsk = 4;
-            static_assert(kRnntGreedyAhead + 1 + kAsk <= kRnntGreedyRing, "the ring holds what is asked for ahead");
-            const int f_first = af_hi;
-            int n_ask = 0;
-            half8_t col[kAsk][kRnntFC];
+            for (int k = 0; k < kRnntHC; ++k) gk[k] = gv[min(lane + 64 * k, nhp - 1)];
+            auto publish_some = [&](auto how_many, int n) __attribute__((always_inline)) {
+                constexpr int kB = decltype(how_many)::value;
+                float a[kB];
 #pragma unroll
-            for (int q = 0; q < kAsk; ++q) {
-                const int f = f_first + q;
-                const bool ask = f < p.T && f <= s.t + kRnntGreedyAhead + kAsk;
-                if (ask) n_ask = q + 1;
+                for (int q = 0; q < kB; ++q) a[q] = af_ring[((s.t + (pub + q - step)) & (kRnntGreedyRing - 1)) * kRnntThreads];
 #pragma unroll
-                for (int k = 0; k < kRnntFC; ++k)
-                    col[q][k] = (ask && lane + 64 * k < nfp) ? reinterpret_cast<const half8_t*>(p.enc + (long)f * p.F)[lane + 64 * k] : wf[k];
-            }
-            ok = wait_for_decisions();
+                for (int q = 0; q < kB; ++q) {
 #pragma unroll
-            for (int q = 0; q < kAsk; ++q) {
-                if (q < n_ask) {
-                    float a = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < kRnntFC; ++k)
-                        if (lane + 64 * k < nfp) a = dot8(wf[k], col[q][k], a);
-                    frame_keep(f_first + q, a);
+                    for (int k = 0; k < kRnntHC; ++k)
+                        if (lane + 64 * k < nhp) a[q] = dot8(wg[k], gk[k], a[q]);
                 }
-            }
+                rnnt_sums(a);
+#pragma unroll
+                for (int q = 0; q < kB; ++q)
+                    if (lane == 0) my_value(q) = rnnt_bits(relu_f32(a[q] + bias));
+                rnnt_barrier();
+                if (wave < n) store_words(wave, hid_entry(pub + wave, jb), step_tag(pub + wave, version));
+                ++n_publish;
+                pub += n;
+            };
+            if (pub == step) publish_some(std::integral_constant<int, 1>{}, 1);
+            while (pub < end) publish_some(std::integral_constant<int, kRnntGreedyBatch>{}, min(kRnntGreedyBatch, end - pub));
+            ask();
+            ok = wait_for_decisions();
+            keep();
         }
     } else if (someone_gave_up == 0) {
         // ---- the joint network's second layer: row v of W2, for every hidden vector that arrives ----
-        const int vb = b - n_lstm - nwj, v = 8 * vb + wave;
+        const int team = (b - n_lstm - nwj) / nwv, vb = (b - n_lstm - nwj) - team * nwv, v = 8 * vb + wave;
         const int njp = p.J >> 3;
         const half8_t* row = reinterpret_cast<const half8_t*>(p.w2 + (long)min(v, p.V - 1) * p.J);
         half8_t wv[kRnntJC];
@@ -667,7 +828,8 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             wv[k] = row[min(lane + 64 * k, njp - 1)];
         }
         const float bias = (lane == 0 && p.b2 && v < p.V) ? (float)p.b2[v] : 0.0f;
-        int pub = 0;              // the next step to publish logits for
+        auto own_step = [&](int st) __attribute__((always_inline)) { return st + (team + p.teams - st % p.teams) % p.teams; };  // the first of this team's from st on
+        int pub = team;           // the next step to publish logits for
         int have_version = g_version();
         int min_seen = 0;         // no block has taken in fewer decisions than this
         bool ok = true;
@@ -675,12 +837,12 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             const int version = g_version();
             if (version != have_version) {
                 have_version = version;
-                pub = step;
+                pub = own_step(step);
             }
-            if (pub < step) pub = step;
+            if (pub < step) pub = own_step(step);
             const int frame = s.t + (pub - step);
             bool want = frame < p.T && pub <= step + kRnntGreedyAhead;
-            if (want && pub - kRnntGreedyRing >= min_seen) {
+            if (want && pub - kRnntGreedyLogitRing >= min_seen) {
                 // The entry for step `pub` still holds step pub - ring: has everybody taken that decision in?
                 if (tid == 0) min_seen_lds = 0x7fffffff;
                 rnnt_barrier();
@@ -688,20 +850,21 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     atomicMin(&min_seen_lds, (int)__hip_atomic_load(p.seen + (long)kRnntSeenStride * tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
                 rnnt_barrier();
                 min_seen = min_seen_lds;
-                want = pub - kRnntGreedyRing < min_seen;
+                want = pub - kRnntGreedyLogitRing < min_seen;
             }
             // the hidden vector of `step` itself is what everybody waits for (no decision can come before it): polled; one
             // of a later step is looked for once per round, between looks at the decisions
-            // and the one behind it is taken along (to the LDS that the first layer's blocks use for the embedding rows)
-            const bool want2 = want && frame + 1 < p.T && pub + 1 <= step + kRnntGreedyAhead && pub + 1 - kRnntGreedyRing < min_seen;
-            const int r = pass(hid_entry(pub, 0), want ? nwj : 0, step_tag(pub, version), buf0, pub == step, true, false,
-                               hid_entry(pub + 1, 0), want2 ? nwj : 0, step_tag(pub + 1, version), emb);
+            // and the team's next one is taken along (to the LDS that the first layer's blocks use for the embedding rows)
+            const int pub2 = pub + p.teams;
+            const bool want2 = want && frame + p.teams < p.T && pub2 <= step + kRnntGreedyAhead && pub2 - kRnntGreedyLogitRing < min_seen;
+            const int r = pass(hid_entry(pub, 0), want ? nwj : 0, step_tag(pub, version), buf0, pub == step, kRnntWaves - 6, false,
+                               hid_entry(pub2, 0), want2 ? nwj : 0, step_tag(pub2, version), emb);
             if (dead) {
                 ok = false;
                 break;
             }
             if (r & 1) {
-                const bool two = (r & (1 << 30)) != 0;
+                const bool two = (r & 2) != 0;
                 const half8_t* in0 = reinterpret_cast<const half8_t*>(buf0);
                 const half8_t* in1 = reinterpret_cast<const half8_t*>(emb);
                 float a0 = 0.0f, a1 = 0.0f;
@@ -714,22 +877,17 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 }
                 a0 = rnnt_sum(a0);
                 if (two) a1 = rnnt_sum(a1);
-                if (lane == 0) {
-                    mine[n_publish & 1u][wave] = v < p.V ? rnnt_bits(a0 + bias) : (unsigned short)0xfc00u;   // (-inf past the last symbol)
-                    if (two) mine[(n_publish + 1u) & 1u][wave] = v < p.V ? rnnt_bits(a1 + bias) : (unsigned short)0xfc00u;
+                if (lane == 0) {  // (-inf past the last symbol)
+                    my_value(0) = v < p.V ? rnnt_bits(a0 + bias) : (unsigned short)0xfc00u;
+                    if (two) my_value(1) = v < p.V ? rnnt_bits(a1 + bias) : (unsigned short)0xfc00u;
                 }
-                // both go out behind one barrier, from two wavefronts
                 rnnt_barrier();
-                const int which = tid >> 6, part = tid & 63;
-                if (part < 3 && which < (two ? 2 : 1)) {
-                    const unsigned short* m = mine[(n_publish + which) & 1u] + 3 * part;
-                    const u64 w = (u64)m[0] | ((u64)m[1] << 16) | ((u64)m[2] << 32) | ((u64)step_tag(pub + which, version) << 48);
-                    __hip_atomic_store(lg_entry(pub + which, vb) + part, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                n_publish += two ? 2u : 1u;
-                pub += two ? 2 : 1;
+                const int which = 6 - wave;
+                if (which >= 0 && which < (two ? 2 : 1)) store_words(which, lg_entry(pub + which * p.teams, vb), step_tag(pub + which * p.teams, version));
+                ++n_publish;
+                pub += (two ? 2 : 1) * p.teams;
             }
-            const int taken = take_decisions(r);
+            const int taken = take_decisions();
             if ((r & 1) || taken > 0)
                 something_came();
             else
@@ -742,7 +900,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     if (someone_gave_up != 0) {
         if (tid == 0) i_decode_alone = (p.alone || atomicCAS(p.solo_owner, 0u, 1u) == 0u) ? 1 : 0;
         __syncthreads();
-        if (i_decode_alone) rnnt_greedy_solo(p, solo_hs, solo_cs, buf0, &lgs[0][0][0]);
+        if (i_decode_alone) rnnt_greedy_solo(p, solo_hs, solo_cs, buf0, own);
         return;
     }
     if (b == 0 && tid == 0) {
