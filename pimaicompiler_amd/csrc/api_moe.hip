@@ -35,6 +35,18 @@ std::vector<PimHipMoePlan*> g_moe_plans;
 constexpr size_t kMoeExchangeWords32 = (size_t)2 * kMoeMaxBlocks * kMoeEntryWords * 2;  // the exchange buffer as 32-bit words
 constexpr unsigned long long kMoeEventsBeforeAlone = 3;  // waits given up before a plan stops exchanging for good
 
+// The kernel whose lanes hold as many pieces of a row as there are, or a few more (the loads have no condition on them).
+auto moe_kernel(int64_t d_model, int64_t d_ff)
+{
+    auto of = [&](auto x_pieces) {
+        constexpr int XC = decltype(x_pieces)::value;
+        return d_ff <= 1024 ? moe_ffn_step_f16_kernel<XC, 2> : d_ff <= 2048 ? moe_ffn_step_f16_kernel<XC, 4>
+               : d_ff <= 3072 ? moe_ffn_step_f16_kernel<XC, 6> : moe_ffn_step_f16_kernel<XC, kMoeFC>;
+    };
+    return d_model <= 512 ? of(std::integral_constant<int, 1>{}) : d_model <= 1024 ? of(std::integral_constant<int, 2>{})
+                                                                                 : of(std::integral_constant<int, kMoeXC>{});
+}
+
 int destroy_moe_plan_locked(PimHipMoePlan* plan)
 {
     if (!plan) return PIMHIP_OK;
@@ -91,7 +103,7 @@ extern "C" int pimhip_moe_plan_create(PimHipMoePlan** plan_out, const void* rout
     if (blocks < blocks_for_w2) blocks = blocks_for_w2;
     const int wpb_final = (nwords + blocks - 1) / blocks;
     int per_cu = 0;
-    PIMHIP_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_ffn_step_f16_kernel, kMoeThreads, 0));
+    PIMHIP_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, moe_kernel(d_model, d_ff), kMoeThreads, 0));
     if ((int64_t)per_cu * st->num_cus < blocks)
         return fail(PIMHIP_ERR_UNSUPPORTED, "the %d workgroups of the one-launch step cannot all be resident on this device", blocks);
     if (!aligned16(router_w)) return fail(PIMHIP_ERR_UNSUPPORTED, "router_w must be 16-byte aligned");
@@ -242,7 +254,8 @@ extern "C" int pimhip_moe_ffn_step(PimHipMoePlan* plan, const void* x, void* y, 
         rc = order_after_previous_sequence_launch(st, s);
         if (rc != PIMHIP_OK) return rc;
     }
-    moe_ffn_step_f16_kernel<<<dim3((unsigned)plan->blocks), dim3(kMoeThreads), 0, s>>>(a.x, a.router_w, a.router_b, a.tables, a.d_model, a.d_ff, a.E, a.act, a);
+    moe_kernel(plan->d_model, plan->d_ff)<<<dim3((unsigned)plan->blocks), dim3(kMoeThreads), 0, s>>>(a.x, a.router_w, a.router_b, a.tables, a.d_model,
+                                                                                                    a.d_ff, a.E, a.act, a);
     PIMHIP_HIP_CHECK(hipGetLastError());
     return PIMHIP_OK;
 }

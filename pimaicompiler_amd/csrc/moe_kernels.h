@@ -20,16 +20,19 @@
 // What bounds the step is not bandwidth (9.4 MB) but a chain of dependent round trips: token and router rows, the expert's
 // W1 rows, the all-to-all of `hidden`, the store of y.  So nothing else may stand in that chain: the launch count (which
 // says which set of exchange slots this launch uses) is a device-scope load and is asked for behind the router's cached
-// loads, not in front of them; the
-// slots of the other set are emptied at the very end; a lane that waits looks at ONE 16-byte word of ONE producer per poll
-// (a poll round over all blocks gets slower with every further load per lane); the row of W2 is asked for right behind
-// the rows of W1 and has arrived when the hidden values have.
+// loads, not in front of them; the rows of W2 are asked for right behind the rows of W1, and the hidden values by wavefronts that
+// hold no row of W2 (a wavefront's loads return in order: a poll behind W2's rows waits for them, 0.7 us where another expert's
+// were cached); what is not waited for, the caller's view of the choice, the slots of the next launch, goes out behind the
+// block's own word, but not at the end: a launch lasts until its last store is acknowledged.
+// Measured on MI355X (8 experts, 768 / 3072, one of 13 tokens in a row; time stamps in block 0): start and router 0.9 us, argmax 0.2
+// (0.36 with the choice stored in front), W1 1.2 (1.5 with W2's rows behind the hidden values and twice as many of them, loaded and
+// dropped by wavefronts without a row), exchange 1.2 - 1.6 (1.7), W2 0.5, end and next launch 1.1 (1.2): 6.4 -> 5.5 us a step.
 //
 // Exchange: hx[2][blocks] entries of 64 bytes, a block's words in the first 16 * wpb bytes.  An empty 8-byte half is all
 // ones, which no four fp16 values written here can be (a NaN is written as 0x7e00).  The two sets alternate by the launch
 // count g (a device word read at the start): a launch uses set g & 1 and marks its own entry of the other set empty for the
-// launch after it.  Where every block publishes a word, block 0 advances the count at its end: it has seen everybody's word
-// by then, so everybody has read the count.  A block that publishes nothing could start so late that it reads the count
+// launch after it.  Where every block publishes a word, block 0 advances the count behind its wait for them: everybody
+// has read the count by then.  A block that publishes nothing could start so late that it reads the count
 // after block 0 has advanced it, and would look into the wrong set; grids with such blocks (d_model > d_ff / 2) keep one copy
 // of the count per block, each in a line of its own, read and advanced by its block (0.3 us slower per step).
 //
@@ -39,6 +42,8 @@
 // starts in that self-sufficient mode (the exchange slots may hold values of the launch that was cut short) until the
 // host has refilled the slots and cleared the word.
 #pragma once
+
+#include <type_traits>
 
 #include "device_common.h"
 
@@ -82,8 +87,43 @@ struct MoeStepArgs {
     int count_stride;                // 0: one launch count, advanced by block 0; kMoeCounterStride: one per block
 };
 
+// The barrier between the phases: this wavefront's LDS traffic done, then s_barrier.  __syncthreads() would also wait until the rows
+// of W2, asked for right behind those of W1, have arrived.
+__device__ __forceinline__ void moe_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The maximum over the four rows of 16 lanes (wave_sum_rows' exchanges).
+__device__ __forceinline__ float wave_max_rows(float v)
+{
+    {
+        float a = v, b = v;
+        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+        v = fmaxf(a, b);
+    }
+    {
+        float a = v, b = v;
+        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
+        v = fmaxf(a, b);
+    }
+    return v;
+}
+
+// Two 16-byte device-scope loads in flight together (load16_device_scope).
+__device__ __forceinline__ void load16_twice_device_scope(const void* p, const void* q, unsigned long long (&v)[4])
+{
+    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+    u32x4 a, b;
+    asm volatile("global_load_dwordx4 %0, %2, off sc1\n\tglobal_load_dwordx4 %1, %3, off sc1\n\ts_waitcnt vmcnt(0)"
+                 : "=&v"(a), "=&v"(b) : "v"(p), "v"(q) : "memory");
+    v[0] = (unsigned long long)a[0] | ((unsigned long long)a[1] << 32);
+    v[1] = (unsigned long long)a[2] | ((unsigned long long)a[3] << 32);
+    v[2] = (unsigned long long)b[0] | ((unsigned long long)b[1] << 32);
+    v[3] = (unsigned long long)b[2] | ((unsigned long long)b[3] << 32);
+}
+
 // What the kernel's first instructions need comes as plain arguments in front of the struct: those arrive in scalar
 // registers with the wavefront (kernel-argument preload) instead of through a load at its start.
+// XC, FC: 16-byte pieces of a W1 / W2 row per lane.
+template <int XC, int FC>
 __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const half_t* x_, const half_t* router_w_, const half_t* router_b_,
                                                                        const half_t* const* tables_, int d_model_, int d_ff_, int E_, int act_,
                                                                        MoeStepArgs p)
@@ -118,18 +158,18 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
     for (int i = tid; i < 4 * p.E; i += kMoeThreads) table_s[i / p.E][i % p.E] = p.tables[i];
 
     // ---- the token, then the router: every block computes all E logits ----
-    half8_t xr[kMoeXC];
+    half8_t xr[XC];
     const half8_t* x8 = reinterpret_cast<const half8_t*>(p.x);
 #pragma unroll
-    for (int k = 0; k < kMoeXC; ++k) xr[k] = (lane + 64 * k < nx) ? x8[lane + 64 * k] : zero8;
+    for (int k = 0; k < XC; ++k) xr[k] = (lane + 64 * k < nx) ? x8[lane + 64 * k] : zero8;
     // (two experts per wavefront and pass: all their loads are in flight together, one round trip for E <= 16)
     for (int e0 = wave; e0 < p.E; e0 += 2 * kMoeWaves) {
         const int e1 = e0 + kMoeWaves;
         const half8_t* w8a = reinterpret_cast<const half8_t*>(p.router_w) + (long)e0 * nx;
         const half8_t* w8b = reinterpret_cast<const half8_t*>(p.router_w) + (long)(e1 < p.E ? e1 : e0) * nx;
-        half8_t ra[kMoeXC], rb[kMoeXC];
+        half8_t ra[XC], rb[XC];
 #pragma unroll
-        for (int k = 0; k < kMoeXC; ++k) {
+        for (int k = 0; k < XC; ++k) {
             if (64 * k >= nx) break;  // (uniform) pieces past the row for every lane
             const int c = min(lane + 64 * k, nx - 1);
             ra[k] = w8a[c];
@@ -137,7 +177,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
         }
         float sa = 0.0f, sb = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kMoeXC; ++k) {
+        for (int k = 0; k < XC; ++k) {
             if (lane + 64 * k < nx) {
                 sa = dot8(ra[k], xr[k], sa);
                 sb = dot8(rb[k], xr[k], sb);
@@ -154,7 +194,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
             }
         }
     }
-    __syncthreads();
+    moe_barrier();
     // argmax over the E <= 64 logits, one per lane: the first maximum; a NaN counts as the largest value, as in at::argmax
     const float mine_l = lane < p.E ? logit_s[lane] : -INFINITY;
     const bool is_nan = mine_l != mine_l;
@@ -164,18 +204,13 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
     bv = fmaxf(bv, dpp_f32<kDppQuadXor2>(bv));
     bv = fmaxf(bv, dpp_f32<kDppRowHalfMirror>(bv));
     bv = fmaxf(bv, dpp_f32<kDppRowMirror>(bv));
-    bv = fmaxf(bv, __shfl_xor(bv, 16, kWave));
-    bv = fmaxf(bv, __shfl_xor(bv, 32, kWave));
+    bv = wave_max_rows(bv);
     const unsigned long long max_mask = __ballot(lane < p.E && mine_l == bv);
     const int best = nan_mask ? __builtin_ctzll(nan_mask) : __builtin_ctzll(max_mask);
     float scale = 1.0f;
     if (p.scale_by_prob) {
         const float ex = lane < p.E ? __expf(mine_l - bv) : 0.0f;
         scale = 1.0f / wave_sum(ex);
-    }
-    if (b == 0) {
-        if (tid == 0 && p.expert) p.expert[0] = best;
-        if (tid < p.E && p.router_logits) p.router_logits[tid] = (half_t)logit_s[tid];
     }
     const half8_t* w1 = reinterpret_cast<const half8_t*>(table_s[0][best]);
     const half_t* b1 = table_s[1][best];
@@ -191,68 +226,87 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
         return bits;
     };
     // This wavefront's row of W2[e]: asked for here, consumed at the end.
-    half8_t w2r[kMoeFC];
+    half8_t w2r[FC];
     const int r2 = b * p.rpb2 + wave;
     const bool has_row2 = wave < p.rpb2 && r2 < p.d_model;
     auto ask_for_w2 = [&]() {
-        const half8_t* src = w2 + (long)min(r2, p.d_model - 1) * nf;  // (a row this wavefront does not own is loaded and dropped)
 #pragma unroll
-        for (int k = 0; k < kMoeFC; ++k) {
-            if (64 * k >= nf) break;  // (uniform) pieces past the row for every lane
-            w2r[k] = load_weight<true>(src + min(lane + 64 * k, nf - 1));
-        }
+        for (int k = 0; k < FC; ++k) w2r[k] = load_weight<true>(w2 + (long)r2 * nf + min(lane + 64 * k, nf - 1));
     };
 
     // The launch count (which set of slots this launch uses) and the abort word are device-scope loads, which take longer
     // than the cached ones above and would hold those up if they stood in front of them (a wavefront's loads return in
     // order).  Asked for here, they travel with the rows of W1 and are needed when the block publishes.
-        const unsigned int g = __hip_atomic_load(p.g_counter + p.count_stride * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned int g = __hip_atomic_load(p.g_counter + p.count_stride * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned int poisoned = __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // ---- hidden = act(W1[e] . x + b1[e]): this block's words (asked for whether or not they will be published) ----
+    // Compiled for wavefronts with and without a row of W2, no load behind a condition: the wait for W1's rows is a wait for a
+    // number of loads that may still be in flight, which the compiler has to know.
     const int row0 = 8 * p.wpb * b + wave * p.wpb;  // this wavefront's first row
-    half8_t w1r[kMoeMaxWordsPerBlock][kMoeXC];
+    auto first_product = [&](auto holds_row2) __attribute__((always_inline)) {
+        half8_t w1r[kMoeMaxWordsPerBlock][XC];
 #pragma unroll
-    for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
-        const int r = min(row0 + min(s, p.wpb - 1), p.d_ff - 1);
+        for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
+            const int r = min(row0 + min(s, p.wpb - 1), p.d_ff - 1);
 #pragma unroll
-        for (int k = 0; k < kMoeXC; ++k) {
-            if (64 * k >= nx) break;
-            w1r[s][k] = load_weight<true>(w1 + (long)r * nx + min(lane + 64 * k, nx - 1));
+            for (int k = 0; k < XC; ++k) w1r[s][k] = load_weight<true>(w1 + (long)r * nx + min(lane + 64 * k, nx - 1));
         }
-    }
+        if constexpr (decltype(holds_row2)::value) ask_for_w2();
+        if (poisoned != 0u) block_poisoned = 1;
 #pragma unroll
-    for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
-        const int r = row0 + s;
-        float a = 0.0f;
+        for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
+            const int r = row0 + s;
+            float a = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kMoeXC; ++k)
-            if (lane + 64 * k < nx) a = dot8(w1r[s][k], xr[k], a);
-        a = wave_sum(a);
-        if (lane == 0 && s < p.wpb) mine[wave * p.wpb + s] = r < p.d_ff ? hidden_bits(a, r) : (unsigned short)0;
-    }
+            for (int k = 0; k < XC; ++k)
+                if (lane + 64 * k < nx) a = dot8(w1r[s][k], xr[k], a);
+            a = wave_sum(a);
+            if (lane == 0 && s < p.wpb) mine[wave * p.wpb + s] = r < p.d_ff ? hidden_bits(a, r) : (unsigned short)0;
+        }
+    };
+    if (has_row2) first_product(std::true_type{});
+    else first_product(std::false_type{});
+    const unsigned int set = __builtin_amdgcn_readfirstlane(g) & 1u;
     // Whether the abort word is up is decided for the block as a whole, through LDS: wavefronts look at it at slightly
     // different times and can see different values when it is raised while the launch starts; they would then disagree
     // about the barriers that follow.  (The flags were set to 0 in front of the barrier behind the router.)
-    if (poisoned != 0u) block_poisoned = 1;
-    __syncthreads();
+    moe_barrier();
     const bool alone = p.alone != 0 || block_poisoned != 0;
-    const unsigned int set = g & 1u;
+    // This block's entry of the other set is empty for the next launch (nobody reads that set during this one).  Stored here and
+    // below by wavefronts that do not poll, not at the end: a launch lasts until its last store has been acknowledged, a
+    // microsecond for a device-scope one.
+    auto empty_other_set = [&]() {
+        if (tid < 2 * kMoeMaxWordsPerBlock)
+            __hip_atomic_store(p.hx + ((long)(set ^ 1u) * nb + b) * kMoeEntryWords + tid, kMoeEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    // What the caller sees of the choice (behind the words the others wait for).
+    auto report_choice = [&]() {
+        if (b != 0) return;
+        if (tid == 0 && p.expert) p.expert[0] = best;
+        if (tid < p.E && p.router_logits) p.router_logits[tid] = (half_t)logit_s[tid];
+    };
     if (!alone) {
         if (tid < p.wpb && b * p.wpb + tid < nf) {
             const unsigned long long* src = reinterpret_cast<const unsigned long long*>(&mine[8 * tid]);
             store16_device_scope(p.hx + ((long)set * nb + b) * kMoeEntryWords + 2 * tid, src[0], src[1]);
         }
-        ask_for_w2();
-        // ---- everybody's hidden values: thread t takes word t ----
-        if (tid < nf) {
-            const unsigned long long* slot = p.hx + ((long)set * nb + tid / p.wpb) * kMoeEntryWords + 2 * (tid % p.wpb);
-            unsigned long long lo = kMoeEmpty, hi = kMoeEmpty;
+        empty_other_set();
+        report_choice();
+        // ---- everybody's hidden values: word t and word t + n_poll by the threads behind the wavefronts that wait for a row of W2 ----
+        const int poll0 = 64 * min(min(p.rpb2, kMoeWaves), kMoeWaves - (nf + 127) / 128);
+        const int n_poll = kMoeThreads - poll0, t0 = tid - poll0;
+        if (t0 >= 0 && t0 < nf) {
+            const bool two = t0 + n_poll < nf;
+            const int t1 = two ? t0 + n_poll : t0;
+            const unsigned long long* slot0 = p.hx + ((long)set * nb + t0 / p.wpb) * kMoeEntryWords + 2 * (t0 % p.wpb);
+            const unsigned long long* slot1 = p.hx + ((long)set * nb + t1 / p.wpb) * kMoeEntryWords + 2 * (t1 % p.wpb);
+            unsigned long long v[4];
             unsigned int spins = 0;
             unsigned long long t_first = 0ull;
             bool gave_up = false;
             while (true) {
-                load16_device_scope(slot, lo, hi);
-                if (lo != kMoeEmpty && hi != kMoeEmpty) break;
+                load16_twice_device_scope(slot0, slot1, v);
+                if (v[0] != kMoeEmpty && v[1] != kMoeEmpty && v[2] != kMoeEmpty && v[3] != kMoeEmpty) break;
                 if (spins > 0u && (spins & 255u) == 0u) {
                     if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) gave_up = true;
                     if (wait_clock_expired(spins, t_first)) spins = 0xffffffffu;  // gives up below
@@ -267,46 +321,49 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
             }
             if (gave_up) someone_gave_up = 1;
             typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-            const u64x2 v = {lo, hi};
-            *reinterpret_cast<u64x2*>(&hidden[8 * tid]) = v;
+            *reinterpret_cast<u64x2*>(&hidden[8 * t0]) = u64x2{v[0], v[1]};
+            if (two) *reinterpret_cast<u64x2*>(&hidden[8 * t1]) = u64x2{v[2], v[3]};
         }
-        __syncthreads();
+        moe_barrier();
     } else {
-        ask_for_w2();
-        __syncthreads();
+        empty_other_set();
+        report_choice();
     }
-    if (alone || someone_gave_up) {
+    // (With one count for all: block 0 has seen everybody's word by now, or makes it late, when it has computed by itself.)
+    auto advance_count = [&]() {
+        if (tid == kMoeThreads - 1 && (b == 0 || p.count_stride != 0))  // (the last wavefront seldom has a row of W2 left to finish)
+            __hip_atomic_store(p.g_counter + p.count_stride * b, g + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    const bool by_itself = alone || someone_gave_up != 0;
+    if (!by_itself) advance_count();
+    if (by_itself) {
         // ---- self-sufficient: every hidden value from W1[e], by this block alone ----
         for (int r = wave; r < p.d_ff; r += kMoeWaves) {
             float a = 0.0f;
 #pragma unroll
-            for (int k = 0; k < kMoeXC; ++k)
+            for (int k = 0; k < XC; ++k)
                 if (lane + 64 * k < nx) a = dot8(w1[(long)r * nx + lane + 64 * k], xr[k], a);
             a = wave_sum(a);
             if (lane == 0) hidden[r] = __builtin_bit_cast(half_t, hidden_bits(a, r));
         }
         __syncthreads();
+        advance_count();
     }
 
     // ---- y = W2[e] . hidden + b2[e] ----
-    {
+    if (has_row2) {
         float a = 0.0f;
 #pragma unroll
-        for (int k = 0; k < kMoeFC; ++k) {
+        for (int k = 0; k < FC; ++k) {
             const int c = lane + 64 * k;
             if (c < nf) a = dot8(w2r[k], *reinterpret_cast<const half8_t*>(&hidden[c * 8]), a);
         }
         a = wave_sum(a);
-        if (lane == 0 && has_row2) {
+        if (lane == 0) {
             if (b2) a += (float)b2[r2];
             p.y[r2] = (half_t)(a * scale);
         }
     }
-    // this block's entry of the other set is empty for the next launch (nobody reads that set during this one)
-    if (tid < 2 * kMoeMaxWordsPerBlock)
-        __hip_atomic_store(p.hx + ((long)(set ^ 1u) * nb + b) * kMoeEntryWords + tid, kMoeEmpty, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (tid == 0 && (b == 0 || p.count_stride != 0))
-        __hip_atomic_store(p.g_counter + p.count_stride * b, g + 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace pimhip
