@@ -103,7 +103,7 @@ void launch_mv(bool whole_pieces, const half_t* W, const half_t* x, const half_t
     const bool keep = (unsigned long long)N * (unsigned long long)K * sizeof(half_t) <= kKeepCachedBytes || (!whole_pieces && K < 4096);
     auto kernel = whole_pieces ? (keep ? gemv_mv_keep_f16_kernel<R, U, WAVES, KS> : gemv_mv_f16_kernel<R, U, WAVES, KS>)
                                : (keep ? gemv_mv_any_f16_kernel<R, U, WAVES, KS, true> : gemv_mv_any_f16_kernel<R, U, WAVES, KS, false>);
-    kernel<<<grid, WAVES * 64, 0, s>>>(W, x, b, y, N, K, ldw, relu);
+    launch_kernel(kernel, dim3((unsigned)grid), WAVES * 64, s, W, x, b, y, N, K, ldw, relu);
 }
 
 int gemv_mv(const half_t* W, const half_t* x, const half_t* bias, half_t* y, int64_t N, int64_t K, int64_t ldw,
@@ -117,7 +117,7 @@ int gemv_mv(const half_t* W, const half_t* x, const half_t* bias, half_t* y, int
     // excepted: up to 128 columns 2-byte loads, up to 512, one trip of one wavefront, no sum across wavefronts (32001 x 257 8.4 ->
     // 6.4 us, 12000 x 257 3.9 -> 3.5, 300 x 257 the same).
     if (!whole && K <= 128) {
-        gemv_mv_short_f16_kernel<4><<<(unsigned)((N + 3) / 4), 256, 0, s>>>(W, x, bias, y, (int)N, (int)K, (long)ldw, relu);
+        launch_kernel(gemv_mv_short_f16_kernel<4>, dim3((unsigned)((N + 3) / 4)), 256, s, W, x, bias, y, (int)N, (int)K, (long)ldw, relu);
     } else if (!whole && K <= 512) {
         launch_mv<2, 1, 4, 1>(whole, W, x, bias, y, (int)N, (int)K, (long)ldw, relu, s);
     } else if (N < 1024) {
@@ -193,7 +193,7 @@ int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bia
     const bool few_odd_rows = K <= 128 && !vm_whole_pieces(N, lda, reinterpret_cast<uintptr_t>(A), results);
     if (N < 8 || N * K <= 4096 || few_odd_rows) {
         const int grid = (int)((N + 63) / 64);
-        gemv_vm_f16_generic_kernel<<<grid, 64 * kVmGenericWaves, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu);
+        launch_kernel(gemv_vm_f16_generic_kernel, dim3((unsigned)grid), 64 * kVmGenericWaves, s, x, A, bias, outs, (int)K, (int)N, (long)lda, relu);
         return PIMHIP_OK;
     }
     const VmPlan plan = vm_plan(K, N, lda, reinterpret_cast<uintptr_t>(A), results, st->num_cus);
@@ -225,8 +225,11 @@ int gemv_vm(DeviceState* st, const half_t* x, const half_t* A, const half_t* bia
     }
     const dim3 grid(plan.by_xcd ? (plan.col_blocks + 7) / 8 * 8 : plan.col_blocks, plan.slices);
     auto kernel = plan.lanes_per_row == 8 ? gemv_vm_f16_kernel<8, true> : plan.by_xcd ? gemv_vm_f16_kernel<16, true> : gemv_vm_f16_kernel<16, false>;
-    kernel<<<grid, kVmWaves * 64, 0, s>>>(x, A, bias, outs, (int)K, (int)N, (long)lda, relu, plan.rows_per_slice, partial, status, poison,
-                                          st->vm_spin_limit, plan.by_xcd);
+    VmDests dests;
+    memcpy(dests.y, outs.y, sizeof(dests.y));
+    const unsigned int flags = (relu ? kVmRelu : 0u) | (plan.by_xcd ? kVmByXcd : 0u) | (unsigned int)outs.count << kVmOutsShift;
+    launch_kernel(kernel, grid, kVmWaves * 64, s, x, A, bias, (long)lda, (int)K, (int)N, plan.rows_per_slice, flags, partial, status, poison,
+                  st->vm_spin_limit, plan.slices, dests);
     return PIMHIP_OK;
 }
 
@@ -311,8 +314,8 @@ extern "C" int pimhip_execute_gemv_cat2(void* out, const void* in1, int64_t in1_
     const int keep = (unsigned long long)out_w * (unsigned long long)K * sizeof(half_t) <= kKeepCachedBytes;
     // (the launch shapes of gemv_mv)
     auto launch = [&](auto kernel, unsigned grid) {
-        kernel<<<grid, 256, 0, s>>>((const half_t*)weight, (const half_t*)in1, (const half_t*)in2, split, (const half_t*)bias, (half_t*)out, N,
-                                    (int)K, (long)ldw, relu);
+        launch_kernel(kernel, dim3(grid), 256, s, (const half_t*)weight, (const half_t*)in1, (const half_t*)in2, split, (const half_t*)bias,
+                      (half_t*)out, N, (int)K, (long)ldw, relu);
     };
     if (out_w < 1024) {
         if (K >= 2048)
@@ -452,6 +455,36 @@ extern "C" int pimhip_execute_dot(void* out, const void* a, const void* b, int64
     return PIMHIP_OK;
 }
 
+namespace
+{
+// One launch for problems [0, count) of arrays that start there; the entries have been checked.
+template <int MAX>
+void launch_group(int count, void* const* outs, const void* const* ins, const void* const* weights, const void* const* biases,
+                  const int64_t* in_ws, const int64_t* out_ws, const int* acts, hipStream_t s)
+{
+    GemvGroupArgs<MAX> g;
+    memset(&g, 0, sizeof(g));
+    int blocks = 0;
+    unsigned long long weight_bytes = 0;
+    for (int i = 0; i < count; ++i) {
+        g.W[i] = (const half_t*)weights[i];
+        g.x[i] = (const half_t*)ins[i];
+        g.bias[i] = biases ? (const half_t*)biases[i] : nullptr;
+        g.y[i] = (half_t*)outs[i];
+        g.N[i] = (int)out_ws[i];
+        g.K[i] = (int)in_ws[i];
+        if (acts && acts[i] == PIMHIP_ACT_RELU) g.relu |= 1u << i;
+        g.block_begin[i] = blocks;
+        weight_bytes += (unsigned long long)out_ws[i] * (unsigned long long)in_ws[i] * sizeof(half_t);
+        const int rows_per_block = gemv_group_rows_per_block((int)in_ws[i]);
+        blocks += ((int)out_ws[i] + rows_per_block - 1) / rows_per_block;
+    }
+    g.count = count;
+    launch_kernel(weight_bytes <= kKeepCachedBytes ? gemv_mv_f16_group_kernel<true, MAX> : gemv_mv_f16_group_kernel<false, MAX>,
+                  dim3((unsigned)blocks), kGemvGroupThreads, s, g);
+}
+}  // namespace
+
 extern "C" int pimhip_execute_gemv_group(int count, void* const* outs, const void* const* ins,
                                          const void* const* weights, const void* const* biases,
                                          const int64_t* in_ws, const int64_t* out_ws, const int* acts, void* stream)
@@ -463,12 +496,9 @@ extern "C" int pimhip_execute_gemv_group(int count, void* const* outs, const voi
     if (count == 0) return PIMHIP_OK;
     if (!outs || !ins || !weights || !in_ws || !out_ws) return fail(PIMHIP_ERR_INVALID_ARGUMENT, "null array argument");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    int done = 0;
-    while (done < count) {
-        GemvGroupArgs g;
-        memset(&g, 0, sizeof(g));
-        int n = 0, blocks = 0;
-        unsigned long long weight_bytes = 0;
+    static_assert(kGemvGroupMax <= 32, "a bit of `relu` per problem");
+    for (int done = 0; done < count;) {
+        int n = 0;
         for (; done + n < count && n < kGemvGroupMax; ++n) {
             const int i = done + n;
             if (!outs[i] || !ins[i] || !weights[i]) return fail(PIMHIP_ERR_INVALID_ARGUMENT, "entry %d has a null pointer", i);
@@ -478,24 +508,9 @@ extern "C" int pimhip_execute_gemv_group(int count, void* const* outs, const voi
                 return fail(PIMHIP_ERR_UNSUPPORTED, "entry %d: grouped launch needs in_w %% 8 == 0 and 16-byte aligned in/weight", i);
             const int a = acts ? acts[i] : PIMHIP_ACT_NONE;
             if (a != PIMHIP_ACT_NONE && a != PIMHIP_ACT_RELU) return fail(PIMHIP_ERR_INVALID_ARGUMENT, "entry %d: unknown activation %d", i, a);
-            g.W[n] = (const half_t*)weights[i];
-            g.x[n] = (const half_t*)ins[i];
-            g.bias[n] = biases ? (const half_t*)biases[i] : nullptr;
-            g.y[n] = (half_t*)outs[i];
-            g.N[n] = (int)out_ws[i];
-            g.K[n] = (int)in_ws[i];
-            g.relu[n] = a == PIMHIP_ACT_RELU;
-            g.block_begin[n] = blocks;
-            weight_bytes += (unsigned long long)out_ws[i] * (unsigned long long)in_ws[i] * sizeof(half_t);
-            const int rows_per_block = gemv_group_rows_per_block((int)in_ws[i]);
-            blocks += ((int)out_ws[i] + rows_per_block - 1) / rows_per_block;
         }
-        g.block_begin[n] = blocks;
-        g.count = n;
-        if (weight_bytes <= kKeepCachedBytes)
-            gemv_mv_f16_group_kernel<true><<<blocks, kGemvGroupThreads, 0, s>>>(g);
-        else
-            gemv_mv_f16_group_kernel<false><<<blocks, kGemvGroupThreads, 0, s>>>(g);
+        (n <= 4 ? launch_group<4> : n <= 8 ? launch_group<8> : launch_group<kGemvGroupMax>)(
+            n, outs + done, ins + done, weights + done, biases ? biases + done : nullptr, in_ws + done, out_ws + done, acts ? acts + done : nullptr, s);
         PIMHIP_HIP_CHECK(hipGetLastError());
         done += n;
     }

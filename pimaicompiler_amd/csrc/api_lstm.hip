@@ -838,12 +838,13 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
                     sd.cn_f16 = last ? cnp + (size_t)ci * H : nullptr;
                 }
                 if (D == 2) {
-                    (keep ? lstm_step_pair_f16_kernel<4, true> : lstm_step_pair_f16_kernel<4, false>)<<<dim3(grid, 2), 256, 0, s>>>(p2, (int)in_w, (int)H);
+                    launch_kernel(keep ? lstm_step_pair_f16_kernel<4, true> : lstm_step_pair_f16_kernel<4, false>, dim3(grid, 2), 256, s, p2, (int)in_w, (int)H);
                 } else {
                     // (plain arguments: the kernel's first instructions have them in registers)
                     const LstmStepDir& sd = p2.dir[0];
-                    (keep ? lstm_step_f16_kernel<4, true> : lstm_step_f16_kernel<4, false>)<<<grid, 256, 0, s>>>(
-                        sd.w_ih, sd.w_hh, sd.bsum, sd.xproj, sd.x, sd.h_prev, sd.c_in_f16, sd.c_state, sd.h_out, sd.hn_f16, sd.cn_f16, (int)in_w, (int)H);
+                    launch_kernel(
+                        keep ? lstm_step_f16_kernel<4, true> : lstm_step_f16_kernel<4, false>, dim3(grid), 256, s, sd.w_ih, sd.w_hh, sd.bsum, sd.xproj,
+                        sd.x, sd.h_prev, sd.c_in_f16, sd.c_state, sd.h_out, sd.hn_f16, sd.cn_f16, (int)in_w, (int)H);
                 }
             }
             PIMHIP_HIP_CHECK(hipGetLastError());

@@ -212,16 +212,20 @@ __global__ __launch_bounds__(WAVES * 64) void gemv_mv_cat2_f16_kernel(const half
 // Several independent MV GEMVs in one launch (sibling projections that the reference issues on separate
 // streams, runtime/source/executor/op_executor/stream_ops_executor.cpp:36-47).  Blocks
 // [block_begin[i], block_begin[i+1]) work on problem i.
+// MAX: as many problems as the arguments have room for.  Arguments for 32 are 1.5 KB, which the host writes and a block's first
+// loads fetch from all over: q, k, v and o of 768 with room for 4 instead: 5.3 -> 5.1 us a call,
+// 6.2 -> 5.75 on a slower host core.
 static constexpr int kGemvGroupMax = 32;
+template <int MAX>
 struct GemvGroupArgs {
-    const half_t* W[kGemvGroupMax];
-    const half_t* x[kGemvGroupMax];
-    const half_t* bias[kGemvGroupMax];
-    half_t* y[kGemvGroupMax];
-    int N[kGemvGroupMax];
-    int K[kGemvGroupMax];
-    int relu[kGemvGroupMax];
-    int block_begin[kGemvGroupMax + 1];
+    const half_t* W[MAX];
+    const half_t* x[MAX];
+    const half_t* bias[MAX];
+    half_t* y[MAX];
+    int N[MAX];
+    int K[MAX];
+    int block_begin[MAX];
+    unsigned int relu;  // a bit per problem
     int count;
 };
 
@@ -231,16 +235,16 @@ static constexpr int kGemvGroupThreads = 256;
 static constexpr int kGemvGroupLongRow = 4096;
 __host__ __device__ inline int gemv_group_rows_per_block(int K) { return K >= kGemvGroupLongRow ? 2 : 4; }
 
-template <bool KEEP>  // the group's weights together are small: plain loads (load_weight)
-__global__ __launch_bounds__(kGemvGroupThreads) void gemv_mv_f16_group_kernel(GemvGroupArgs g)
+template <bool KEEP, int MAX>  // KEEP: the group's weights together are small: plain loads (load_weight)
+__global__ __launch_bounds__(kGemvGroupThreads) void gemv_mv_f16_group_kernel(GemvGroupArgs<MAX> g)
 {
     int i = 0;
     while (i + 1 < g.count && (int)blockIdx.x >= g.block_begin[i + 1]) ++i;
     const int block = (int)blockIdx.x - g.block_begin[i];
     if (g.K[i] >= kGemvGroupLongRow)
-        gemv_mv_f16_body<2, 4, 4, 4, false, KEEP>(g.W[i], g.x[i], g.bias[i], g.y[i], g.N[i], g.K[i], (long)g.K[i], g.relu[i], block);
+        gemv_mv_f16_body<2, 4, 4, 4, false, KEEP>(g.W[i], g.x[i], g.bias[i], g.y[i], g.N[i], g.K[i], (long)g.K[i], (int)(g.relu >> i & 1u), block);
     else
-        gemv_mv_f16_body<2, 2, 4, 2, false, KEEP>(g.W[i], g.x[i], g.bias[i], g.y[i], g.N[i], g.K[i], (long)g.K[i], g.relu[i], block);
+        gemv_mv_f16_body<2, 2, 4, 2, false, KEEP>(g.W[i], g.x[i], g.bias[i], g.y[i], g.N[i], g.K[i], (long)g.K[i], (int)(g.relu >> i & 1u), block);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -293,6 +297,14 @@ struct GemvOuts {
     int count;
 };
 
+// The sliced kernel's: with the count among the flags, all its arguments are 112 bytes (what more costs a launch: launch_kernel),
+// and with them at the end what the first instructions need arrives in scalar registers.
+struct VmDests {
+    half_t* y[kGemvMaxOuts];
+};
+static constexpr unsigned int kVmRelu = 1u, kVmByXcd = 2u;
+static constexpr int kVmOutsShift = 2;
+
 static constexpr int kVmLoads = 4;  // 16-byte loads in flight per lane
 
 // acc[j] += A[k][j] * x[k] for k, k + GROUPS, .. < k_end, `a` at the lane's eight columns of row 0.
@@ -343,12 +355,13 @@ __device__ __forceinline__ void vm_put_sums(float* row, const float (&acc)[8], i
 template <int LPR, bool KEEP>
 __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t* __restrict__ x,
                                                                  const half_t* __restrict__ A,
-                                                                 const half_t* __restrict__ bias,
-                                                                 GemvOuts outs, int K, int N, long lda,
-                                                                 int relu, int k_per_slice, float* partial,
+                                                                 const half_t* __restrict__ bias, long lda, int K, int N,
+                                                                 int k_per_slice, unsigned int flags, float* partial,
                                                                  unsigned int* status, unsigned int* poison,
-                                                                 unsigned int spin_limit, int by_xcd)
+                                                                 unsigned int spin_limit, int nslices, VmDests outs)
 {
+    const bool relu = flags & kVmRelu, by_xcd = flags & kVmByXcd;
+    const int out_count = (int)(flags >> kVmOutsShift);
     constexpr int kVmCols = 8 * LPR;
     constexpr int GROUPS = kVmWaves * (64 / LPR);     // row groups per block = LDS rows of the reduction = rows between loads of a lane
     constexpr int PARTS = kVmWaves * 64 / kVmCols;    // threads per column when the slices' sums are collected
@@ -359,7 +372,9 @@ __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t
     const int lane = tid & 63;
     const int cg = lane % LPR;             // which 8 columns of the block
     const int grp = tid / LPR;
-    const int bx = by_xcd ? (int)((blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3)) : (int)blockIdx.x;
+    // (The launch's own size would come with 256 bytes of further arguments: it is counted here, the slices are an argument.)
+    const int per_xcd = ((N + kVmCols - 1) / kVmCols + 7) >> 3;
+    const int bx = by_xcd ? (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3) : (int)blockIdx.x;
     const long base = (long)bx * kVmCols;
     if (base >= N) return;  // (a grid that goes by XCD is rounded up to whole eights)
     const long col0 = base + cg * 8;
@@ -368,7 +383,7 @@ __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t
 
     // (asked for now by the blocks that will reduce, needed when they start to: it travels behind the block's own rows)
     unsigned int poisoned = 0u;
-    if (gridDim.y > 1 && blockIdx.y == gridDim.y - 1) poisoned = __hip_atomic_load(poison, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (nslices > 1 && (int)blockIdx.y == nslices - 1) poisoned = __hip_atomic_load(poison, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
     float acc[8];
 #pragma unroll
@@ -402,10 +417,9 @@ __global__ __launch_bounds__(kVmWaves * 64) void gemv_vm_f16_kernel(const half_t
         if (bias) r += (float)bias[col];
         if (relu) r = relu_f32(r);
         const half_t out = (half_t)r;
-        for (int o = 0; o < outs.count; ++o) outs.y[o][col] = out;
+        for (int o = 0; o < out_count; ++o) outs.y[o][col] = out;
     };
 
-    const int nslices = gridDim.y;
     if (nslices == 1) {
         if (part == 0 && mine) finish(own);
         return;
