@@ -348,20 +348,19 @@ extern "C" int pimhip_decoder_step(PimHipDecoderPlan* plan, const void* x, const
         if (rc != PIMHIP_OK) return rc;
     }
     const dim3 grid(plan->blocks), block(kDecThreads);
-    if (plan->cls_w) {
-        switch (L) {
-            case 1: decoder_step_f16_kernel<1, true><<<grid, block, 0, s>>>(a); break;
-            case 2: decoder_step_f16_kernel<2, true><<<grid, block, 0, s>>>(a); break;
-            case 3: decoder_step_f16_kernel<3, true><<<grid, block, 0, s>>>(a); break;
-            default: decoder_step_f16_kernel<4, true><<<grid, block, 0, s>>>(a); break;
-        }
-    } else {
-        switch (L) {
-            case 1: decoder_step_f16_kernel<1, false><<<grid, block, 0, s>>>(a); break;
-            case 2: decoder_step_f16_kernel<2, false><<<grid, block, 0, s>>>(a); break;
-            case 3: decoder_step_f16_kernel<3, false><<<grid, block, 0, s>>>(a); break;
-            default: decoder_step_f16_kernel<4, false><<<grid, block, 0, s>>>(a); break;
-        }
+    // What a step reads: W_hh and the input columns of every layer, and the classifier.
+    const unsigned long long bytes = ((unsigned long long)L * 8 * H * H + (unsigned long long)plan->vocab * H) * sizeof(half_t);
+    auto launch = [&](auto layers) {
+        constexpr int kL = decltype(layers)::value;
+        if (!plan->cls_w) decoder_step_f16_kernel<kL, false><<<grid, block, 0, s>>>(a);
+        else if (bytes <= kDecKeptBytes) decoder_step_f16_kernel<kL, true><<<grid, block, 0, s>>>(a);
+        else decoder_step_f16_kernel<kL, true, false><<<grid, block, 0, s>>>(a);
+    };
+    switch (L) {
+        case 1: launch(std::integral_constant<int, 1>{}); break;
+        case 2: launch(std::integral_constant<int, 2>{}); break;
+        case 3: launch(std::integral_constant<int, 3>{}); break;
+        default: launch(std::integral_constant<int, 4>{}); break;
     }
     PIMHIP_HIP_CHECK(hipGetLastError());
     return PIMHIP_OK;

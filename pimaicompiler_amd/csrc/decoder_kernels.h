@@ -283,7 +283,14 @@ __device__ constexpr int cls_groups_after(int k)
     return k <= 2 ? 1 : 0;
 }
 
-template <int L, bool CLS>
+// KEEP: how the layers' rows are read (load_weight); classifier rows are read with plain loads.  A loop of steps reads the same
+// weights every step, and plain loads leave them in the caches until then as long as they fit: us a step on MI355X, non-temporal /
+// plain: 1024 units, four layers with 8000 / 32000 / 64000 classifier rows (84 / 135 / 198 MB) 23.2 / 22.0, 28.1 / 26.7, 37.6 / 36.3;
+// three of 776 with 3001 (34 MB) 15.4 / 13.2; two of 512 with 32000 (41 MB) 17.8 / 14.7.  Past the 256 MB Infinity Cache the
+// layers' rows, which the chain waits for, are better read non-temporally: with 88000 / 100000 /
+// 120000 rows (248, 272, 313 MB) plain 43.7 / 48.4 / 58.9, non-temporal 43.9 / 47.8 / 52.8 (classifier rows too: 45.8 / 50.1 / 56.1).
+static constexpr unsigned long long kDecKeptBytes = 240ull << 20;
+template <int L, bool CLS, bool KEEP = true>
 __global__ __launch_bounds__(kDecThreads) void decoder_step_f16_kernel(DecoderStepArgs p)
 {
     static_assert(L >= 1 && L <= kDecMaxLayers, "layers per step");
@@ -348,26 +355,26 @@ __global__ __launch_bounds__(kDecThreads) void decoder_step_f16_kernel(DecoderSt
         auto issue_a = [&](int k) __attribute__((always_inline)) {
             const DecoderLayerArgs& ly = p.layer[k];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) w_hh[k][v] = load_stream(row_ptr(ly.w_hh, v, H, 0) + chunk);
+            for (int v = 0; v < 4; ++v) w_hh[k][v] = load_weight<KEEP>(row_ptr(ly.w_hh, v, H, 0) + chunk);
             if (ly.takes_ctx) {
                 if (ly.cx_proj) {
 #pragma unroll
                     for (int v = 0; v < 4; ++v) m_cx[k][v] = ly.cx_proj[((long)gate_of_slot[v] * H + jc) * S + min(e_mine, S - 1)];
                 } else {
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) w_cx[k][v] = load_stream(row_ptr(ly.w_ih, v, ly.in_w, H) + chunk);
+                    for (int v = 0; v < 4; ++v) w_cx[k][v] = load_weight<KEEP>(row_ptr(ly.w_ih, v, ly.in_w, H) + chunk);
                 }
             }
             if (k == 0 && x_one_piece) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) w_in[0][v] = load_stream(row_ptr(ly.w_ih, v, ly.in_w, 0) + x_chunk);
+                for (int v = 0; v < 4; ++v) w_in[0][v] = load_weight<KEEP>(row_ptr(ly.w_ih, v, ly.in_w, 0) + x_chunk);
                 if (x_active) xvec = reinterpret_cast<const half8_t*>(p.x)[x_chunk];
             }
         };
         auto issue_d = [&](int k) __attribute__((always_inline)) {
             const DecoderLayerArgs& ly = p.layer[k];
 #pragma unroll
-            for (int v = 0; v < 4; ++v) w_in[k][v] = load_stream(row_ptr(ly.w_ih, v, ly.in_w, 0) + chunk);
+            for (int v = 0; v < 4; ++v) w_in[k][v] = load_weight<KEEP>(row_ptr(ly.w_ih, v, ly.in_w, 0) + chunk);
         };
 
         // The classifier's rows are dealt to the streaming wavefronts of the whole grid four at a time.  A wavefront's first
@@ -386,7 +393,7 @@ __global__ __launch_bounds__(kDecThreads) void decoder_step_f16_kernel(DecoderSt
                     const long row = min(r0 + v, (long)V - 1);
                     const half8_t* wp = reinterpret_cast<const half8_t*>(p.cls_w + row * H);
 #pragma unroll
-                    for (int c = 0; c < CH; ++c) dst[v][c] = load_stream(wp + min(c * 64 + lane, nchunks - 1));
+                    for (int c = 0; c < CH; ++c) dst[v][c] = load_weight<true>(wp + min(c * 64 + lane, nchunks - 1));
                 }
             }
         };
@@ -443,7 +450,7 @@ __global__ __launch_bounds__(kDecThreads) void decoder_step_f16_kernel(DecoderSt
             for (int c = x_begin + lane; c < x_end; c += 64) {
                 half8_t wr[4];
 #pragma unroll
-                for (int v = 0; v < 4; ++v) wr[v] = load_stream(row_ptr(p.layer[0].w_ih, v, p.layer[0].in_w, 0) + c);
+                for (int v = 0; v < 4; ++v) wr[v] = load_weight<KEEP>(row_ptr(p.layer[0].w_ih, v, p.layer[0].in_w, 0) + c);
                 const half8_t xr = xv[c];
 #pragma unroll
                 for (int v = 0; v < 4; ++v) acc[0][v] = dot8(wr[v], xr, acc[0][v]);
