@@ -207,6 +207,8 @@ struct XcdDot {
         return (unsigned long long)c | ((unsigned long long)d << 32);
     }
 
+    static __device__ __forceinline__ int place(int piece) { return piece; }  // where a 16-byte piece of h lies in LDS
+
     // The lanes that fetch a 16-byte piece of h each, and which: all of wavefronts 0 and 1 (16 lanes of each of the eight: up to 6 %
     // of a step more), or, in pipelines, 32 of the first four (all of two: up to 2 % more for up to 128 units).
     template <bool PIPE>
@@ -235,11 +237,18 @@ static constexpr int kXcdFrags = kXcdMaxH / 64;  // 64-column weight fragments o
 // the weight matrix the 64 are is free as long as both operands agree.  A lane of B takes two whole 16-byte pieces of its gate
 // row, 8 m + (l >> 4) and four pieces further; halves 0..3 of a piece then meet the even row of A, halves 4..7 the odd one.
 
+// Where the 16-byte piece p of h lies in LDS.  A read of 8 bytes per lane takes from eight rows of 128 bytes (the row pairs of A) two
+// of four pieces; in their own order four of the rows share their banks, and the eight wavefronts' reads of a step took 512 cycles of
+// the LDS where 128 do.  Rows 2 q, 2 q + 1 have their pieces exchanged by 0, 1, 4 or 5 instead: every half wavefront reads all banks
+// once.  Two layers of 1024, 341 steps 480.6 -> 428.8 us, two directions, 50 steps 82.4 -> 75.0.
+__device__ __forceinline__ int xcd_h_place(int p) { return p ^ ((p >> 4 & 1) | (p >> 5 & 1) << 2); }
+
 // Lane l's eight values of h in register set s of A: two 8-byte halves of neighbouring pieces.
 __device__ __forceinline__ half8_t xcd_h_operand(const half_t* hb, int s, int lane)
 {
-    const half_t* src = hb + (8 * (8 * s + ((lane & 15) >> 1)) + 2 * (lane >> 4)) * 8 + 4 * (lane & 1);
-    return __builtin_shufflevector(*reinterpret_cast<const half4_t*>(src), *reinterpret_cast<const half4_t*>(src + 8), 0, 1, 2, 3, 4, 5, 6, 7);
+    const int row = 8 * s + ((lane & 15) >> 1), lo = xcd_h_place(8 * row + 2 * (lane >> 4));
+    return __builtin_shufflevector(*reinterpret_cast<const half4_t*>(hb + lo * 8 + 4 * (lane & 1)),
+                                   *reinterpret_cast<const half4_t*>(hb + (lo ^ 1) * 8 + 4 * (lane & 1)), 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
 struct XcdSparse {
@@ -351,6 +360,8 @@ struct XcdSparse {
         const unsigned int lo = v16 | (dpp_u32<kDppRowHalfMirror>(v16) << 16);
         return (unsigned long long)lo | ((unsigned long long)dpp_u32<kDppRowRor8>(lo) << 32);
     }
+
+    static __device__ __forceinline__ int place(int piece) { return xcd_h_place(piece); }
 
     // The lanes that fetch a piece of h each: all of wavefronts 0 and 1.  Spread over eight wavefronts of 16 lanes a step takes
     // 1.42 us, over four of 32 1.32, over two 1.31 (H = 1024).
@@ -498,7 +509,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
                 }
                 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
                 const u64x2 both = {lo, hi};
-                *reinterpret_cast<half8_t*>(hb + piece * 8) = __builtin_bit_cast(half8_t, both);
+                *reinterpret_cast<half8_t*>(hb + Product::place(piece) * 8) = __builtin_bit_cast(half8_t, both);
             }
             if (gave_up) block_gave_up = 1;
             lds_barrier();
@@ -636,7 +647,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
                 const u64x2 both = {lo, hi};
                 hv = __builtin_bit_cast(half8_t, both);
             }
-            *reinterpret_cast<half8_t*>(hb + piece * 8) = hv;
+            *reinterpret_cast<half8_t*>(hb + Product::place(piece) * 8) = hv;
         }
         if (gave_up) block_gave_up = 1;
         lds_barrier();
