@@ -211,6 +211,7 @@ struct XcdDot {
 
     // The lanes that fetch a 16-byte piece of h each, and which: all of wavefronts 0 and 1 (16 lanes of each of the eight: up to 6 %
     // of a step more), or, in pipelines, 32 of the first four (all of two: up to 2 % more for up to 128 units).
+    static constexpr int kSumWave = 4;  // makes the residual sums (not one that polls)
     template <bool PIPE>
     static __device__ __forceinline__ bool polls(int wave, int lane, int& piece)
     {
@@ -365,6 +366,10 @@ struct XcdSparse {
 
     // The lanes that fetch a piece of h each: all of wavefronts 0 and 1.  Spread over eight wavefronts of 16 lanes a step takes
     // 1.42 us, over four of 32 1.32, over two 1.31 (H = 1024).
+    // The wavefront that makes the residual sums: one that does not poll and is, of the two on its SIMD, the first through its
+    // products (sums around the upper layers, by wavefront 4 / by this one: three layers of 1024, 50 steps 103 / 99 us, three of 512, 100
+    // steps 148 / 135, two of 136, 100 steps 123 / 118).
+    static constexpr int kSumWave = 2;
     template <bool PIPE>
     static __device__ __forceinline__ bool polls(int wave, int lane, int& piece)
     {
@@ -542,10 +547,10 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         const unsigned long long* src = &hout[se & 1][2 * lane];
         store16_device_scope(ch.seq_out + (long)se * H + rank * kXcdUnitsPerBlock + lane * 8, src[0], src[1]);
     };
-    // With one: lanes 0..31 of wavefront 4, one value each: a handful of instructions per step (eight values in each of
+    // With one: lanes 0..31 of the wavefront that makes the sums, one value each: a handful of instructions per step (eight values in each of
     // four lanes took 0.1 us per step more).
     const int eu = rank * kXcdUnitsPerBlock + (lane & 31);  // the unit an emitting lane handles
-    const bool sums = res && wave == 4 && lane < 32 && eu < H;
+    const bool sums = res && wave == Product::kSumWave && lane < 32 && eu < H;
     // The input of step s is asked for right after that step's barrier, together with the projection rows two steps ahead
     // (it exists: the projection row made from it is in use), parked in LDS at the top of step s + 1 and added after
     // that step's barrier.  Every wavefront drains its loads once per step, so what matters is that the load leaves
