@@ -40,12 +40,11 @@
 // one barrier, the 16 rows' products with h, the gate arithmetic, and one 8-byte store of the wavefront's four new h values into the
 // workgroup's entry.  What bounds a step: the store becoming visible in the L2 and the poll that finds it, 0.43 us at best
 // for such a round, and a chain of dependent instructions between two rounds.
-// The products come in two kinds, chosen by size and length (xcd_on_dot in api_lstm.hip, with the figures):
-//   XcdSparse  16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16: 0.21 us of matrix instructions at H = 1024; a step 1.30 us
-//              (a single layer; v_dot2 1.49, in pipelines of layers 1.57)
-//   XcdDot     v_dot2 and a transposing reduction over 16 lanes: half the columns per group of instructions that an unused part
-//              of h is skipped in, a shorter chain for few units (64 units 0.85 us a step against 0.98), nothing through LDS at
-//              the start of a launch
+// The products come in two kinds:
+//   XcdSparse  16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16: 0.21 us of matrix instructions at H = 1024; a step 1.16 us
+//              for a single layer, 1.18 in pipelines (v_dot2 1.43, 1.64)
+//   XcdDot     v_dot2 and a transposing reduction over 16 lanes: nothing passes through LDS at the start of a launch, which short
+//              sequences of independent recurrences notice (xcd_on_dot in api_lstm.hip has the line and the figures)
 // Against 64 bits the sums are equally far off (rms error over the sum of the products' magnitudes, 64 .. 1024 columns, MI355X): signs
 // mixed 4.7e-9 .. 9.7e-9 on v_dot2 and 3.2e-9 .. 7.9e-9 sparse, all of one sign 3.4e-8 .. 5.2e-8 and 3.5e-8 .. 4.9e-8; an h made
 // from the same previous h differs from its 64-bit value by 2.07e-4 relative with either, the rounding to fp16.
@@ -93,6 +92,10 @@ struct XcdProj {
 
 static constexpr int kXcdRoleProj = 9;  // role values: 0 none, 1 + k recurrence of chain k, kXcdRoleProj + j projection j
 static constexpr unsigned long long kXcdWaitTicks = 100000000ull;  // one second of the 100 MHz clock
+// The wavefront that makes the residual sums: one that does not poll and is, of the two on its SIMD, the first through its products
+// (sums around the upper layers, by wavefront 4 / by this one: three layers of 1024, 50 steps 103 / 99 us, three of 512, 100 steps
+// 148 / 135, two of 136, 100 steps 123 / 118).
+static constexpr int kXcdSumWave = 2;
 static constexpr int kXcdLag = 2;       // steps a recurrence fed by a P group lets that group get ahead before it starts
 
 struct LstmXcdArgs {
@@ -134,7 +137,7 @@ __device__ __forceinline__ void store8_plain(void* p, unsigned long long v)
 // ---- the step's matrix-vector product on v_dot2 ----
 // Row l >> 4 of 16 lanes has the wavefront's unit l >> 4: its lanes keep, of the four gate rows, the 8-wide column pieces
 // 16 c + (l & 15), c = 0 .. 7.  Four dot products of up to 64 columns per lane, then a transposing reduction over the 16 lanes.
-struct XcdDot {
+struct XcdDot {  // (no pipelines: chosen for short sequences of recurrences that are fed by none other)
     half8_t w[4][8];
 
     static __device__ __forceinline__ int unit(int lane) { return lane >> 4; }
@@ -208,16 +211,6 @@ struct XcdDot {
     }
 
     static __device__ __forceinline__ int place(int piece) { return piece; }  // where a 16-byte piece of h lies in LDS
-
-    // The lanes that fetch a 16-byte piece of h each, and which: all of wavefronts 0 and 1 (16 lanes of each of the eight: up to 6 %
-    // of a step more), or, in pipelines, 32 of the first four (all of two: up to 2 % more for up to 128 units).
-    static constexpr int kSumWave = 4;  // makes the residual sums (not one that polls)
-    template <bool PIPE>
-    static __device__ __forceinline__ bool polls(int wave, int lane, int& piece)
-    {
-        piece = PIPE ? wave * 32 + lane : wave * 64 + lane;
-        return PIPE ? (wave < 4 && lane < 32) : wave < 2;
-    }
 };
 
 // ---- the step's matrix-vector product on v_smfmac_f32_16x16x64_f16 ----
@@ -363,19 +356,6 @@ struct XcdSparse {
     }
 
     static __device__ __forceinline__ int place(int piece) { return xcd_h_place(piece); }
-
-    // The lanes that fetch a piece of h each: all of wavefronts 0 and 1.  Spread over eight wavefronts of 16 lanes a step takes
-    // 1.42 us, over four of 32 1.32, over two 1.31 (H = 1024).
-    // The wavefront that makes the residual sums: one that does not poll and is, of the two on its SIMD, the first through its
-    // products (sums around the upper layers, by wavefront 4 / by this one: three layers of 1024, 50 steps 103 / 99 us, three of 512, 100
-    // steps 148 / 135, two of 136, 100 steps 123 / 118).
-    static constexpr int kSumWave = 2;
-    template <bool PIPE>
-    static __device__ __forceinline__ bool polls(int wave, int lane, int& piece)
-    {
-        piece = wave * 64 + lane;
-        return wave < 2;
-    }
 };
 
 // PIPE = false: groups that neither feed nor are fed across XCDs (a single layer, the two directions of one); everything
@@ -458,10 +438,11 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     __syncthreads();
 
     const int uc = units_ok ? my_unit : H - 1;
-    // Lanes of the first wavefronts fetch one piece of an h vector each: 8 fp16 = columns 8 q .. 8 q + 7.  (The wavefronts that talk
+    // All lanes of the first two wavefronts fetch one piece of an h vector each: 8 fp16 = columns 8 q .. 8 q + 7.  Spread over eight
+    // wavefronts of 16 lanes a step of 1024 units took 1.42 us, over four of 32 1.32, over two 1.31.  (The wavefronts that talk
     // to other XCDs, 4 .. 7, never poll: a wavefront's loads come back in order.)
-    int piece;
-    const bool polls = Product::template polls<PIPE || RES>(wave, lane, piece) && piece * 8 < H;
+    const int piece = wave * 64 + lane;
+    const bool polls = wave < 2 && piece * 8 < H;
 
     // One bounded wait: `again` loads and tests; gives up like every wait of this kernel, after spin_limit polls, and
     // also after kXcdWaitTicks of the constant 100 MHz clock, however long a poll takes in the environment the kernel
@@ -550,7 +531,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     // With one: lanes 0..31 of the wavefront that makes the sums, one value each: a handful of instructions per step (eight values in each of
     // four lanes took 0.1 us per step more).
     const int eu = rank * kXcdUnitsPerBlock + (lane & 31);  // the unit an emitting lane handles
-    const bool sums = res && wave == Product::kSumWave && lane < 32 && eu < H;
+    const bool sums = res && wave == kXcdSumWave && lane < 32 && eu < H;
     // The input of step s is asked for right after that step's barrier, together with the projection rows two steps ahead
     // (it exists: the projection row made from it is in use), parked in LDS at the top of step s + 1 and added after
     // that step's barrier.  Every wavefront drains its loads once per step, so what matters is that the load leaves
@@ -784,17 +765,15 @@ __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_f16_kernel(LstmXcdArgs p
     lstm_xcd_body<PIPE, false, XcdSparse>(p);
 }
 
-template <bool PIPE>
 __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_dot_f16_kernel(LstmXcdArgs p)
 {
-    lstm_xcd_body<PIPE, false, XcdDot>(p);
+    lstm_xcd_body<false, false, XcdDot>(p);
 }
 
 // The pipeline for stacks that have layers with a residual sum.
-template <class Product>
 __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_res_f16_kernel(LstmXcdArgs p)
 {
-    lstm_xcd_body<true, true, Product>(p);
+    lstm_xcd_body<true, true, XcdSparse>(p);
 }
 
 }  // namespace pimhip
