@@ -323,7 +323,11 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
     const bool poisoned = __builtin_amdgcn_readfirstlane(__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u;
     if (tid == 0) block_gave_up = poisoned ? 1 : 0;
 
-    // ---- weights into registers: per chain the four gate rows of unit j, columns 16 * lane .. + 15 ----
+    // The 16-byte pieces of a row that a lane has: with 32 columns neighbouring lanes take neighbouring pieces (in one run per lane the
+    // reads of h from LDS met four to a bank: 1424 units, two directions, 98 steps 351 -> 341 us, one layer of 1688, 100 steps 230.5 ->
+    // 228.7), with 16 one run (two to a bank; the other way 2 to 5 % faster with two chains and 1.5 % slower with four).
+    auto piece_of = [&](int c) { return COLS == 32 ? 64 * c + lane : lane * CH + c; };
+    // ---- weights into registers: per chain the four gate rows of unit j ----
     // Accumulator slot v holds gate {i, g, f, o}[v]: the transpose-sum below then leaves gate k in lane k.
     half8_t w_hh[NC][4][CH];
     half8_t w_ih[WAVEFRONT ? NC : 1][4][CH];  // entry 0 unused
@@ -338,7 +342,7 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
             for (int v = 0; v < 4; ++v) {
 #pragma unroll
                 for (int c = 0; c < CH; ++c) {
-                    const int col = lane * COLS + c * 8;
+                    const int col = piece_of(c) * 8;
                     const bool ok = unit_ok && col < H;  // H % 8 == 0: a chunk is entirely inside or outside the row
                     const long off = ((long)gate_of_slot[v] * H + j) * H + col;
                     w_hh[k][v][c] = ok ? *reinterpret_cast<const half8_t*>(p.chain[k].w_hh + off) : zero;
@@ -459,7 +463,7 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
         for (int k = 0; k < NC; ++k) {
             half8_t hv[CH];
 #pragma unroll
-            for (int c = 0; c < CH; ++c) hv[c] = *reinterpret_cast<const half8_t*>(&hb[k][lane * COLS + c * 8]);
+            for (int c = 0; c < CH; ++c) hv[c] = *reinterpret_cast<const half8_t*>(&hb[k][piece_of(c) * 8]);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
                 acc[k][v] = 0.0f;
@@ -471,7 +475,7 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
                 // super-step ago, which is what chain k - 1's buffer holds now.
                 half8_t xv[CH];
 #pragma unroll
-                for (int c = 0; c < CH; ++c) xv[c] = *reinterpret_cast<const half8_t*>(&hb[k - 1][lane * COLS + c * 8]);
+                for (int c = 0; c < CH; ++c) xv[c] = *reinterpret_cast<const half8_t*>(&hb[k - 1][piece_of(c) * 8]);
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
 #pragma unroll
