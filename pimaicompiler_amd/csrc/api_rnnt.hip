@@ -164,7 +164,8 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
     launch_fill_u32(plan->g_counter, (size_t)plan->blocks * kRnntCounterStride, 0u, s);
     {
         // As many teams of symbol blocks as the CUs that are left take, one workgroup to a CU, up to one for each step that the joint
-        // blocks run ahead (29 symbols, us per blank: 1.02 with one team, 0.87 with eight; 341 frames with 121 symbols: 1222, 1113).
+        // blocks run ahead (29 symbols, us per blank: 1.02 with one team, 0.87 with eight; 341 frames with 121 symbols: 1222, 1113; both with the
+        // polls as they were then).
         const int n_vocab = (int)((vocab + 7) / 8);
         const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
         plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);

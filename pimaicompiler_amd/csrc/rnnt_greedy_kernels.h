@@ -31,10 +31,10 @@
 //   * the joint blocks publish the step that everybody waits for alone and then four steps behind each barrier.
 //
 // Measured on MI355X (one team and two steps a publish before; us per blank / per symbol / an utterance of 341 frames and 121
-// symbols, 2 x 320 units, 512 joint units, 29 symbols): 1.42 / 6.8 / 1395 before, 0.87 / 7.3 / 1113 now; 200 frames and 33 symbols
-// of a 400-word vocabulary (2 x 256 units) 881 -> 478 us.  What bounds it now: a symbol's four hand-overs of 1.0 - 1.3 us, which
+// symbols, 2 x 320 units, 512 joint units, 29 symbols): 1.42 / 6.8 / 1395 before, 0.81 / 7.05 / 1056 now; 200 frames and 33 symbols
+// of a 400-word vocabulary (2 x 256 units) 881 -> 450 us.  What bounds it now: a symbol's four hand-overs of 1.0 - 1.3 us, which
 // the traffic of the steps published ahead made 0.1 us longer each, and in a run of blanks the eight steps ahead over the two
-// hand-overs and three roles' rounds that they travel (12 steps ahead: 0.82 us per blank, and 2 % more with one layer).
+// hand-overs and three roles' rounds that they travel (12 steps ahead: 5 % less per blank, and 2 % more with one layer).
 //
 // Exchange: 8-byte words of three fp16 values and a 16-bit tag, three words per producing block in a 128-byte entry of its
 // own, written and read with device-scope accesses.  The tag says what the word belongs to: h of a layer carries the
@@ -447,67 +447,69 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 }
             }
         } else if (!row_per_step || look == 0) {
-            // A lane's words of `st`: the one of its place in a row of 16 lanes, or those of its place in the wavefront.
-            constexpr int kN = kRnntGreedyLaneWords;
-            const int version = g_version();
-            u64 v[kN];
-            auto look_at = [&](int st, bool in_row) __attribute__((always_inline)) {
-                bool there = true;
+            // A lane's words: the one of its place in a row of 16 lanes (of step + row), or those of its place in the wavefront (of
+            // step + look).  Compiled for either, addresses and tags in front of the polls: every instruction of them counts.
+            auto look_at = [&](auto row_c) __attribute__((always_inline)) {
+                constexpr bool kRow = decltype(row_c)::value;
+                constexpr int kN = kRow ? 1 : kRnntGreedyLaneWords;
+                const int st = step + (kRow ? lane >> 4 : look);
+                const unsigned int tag = step_tag(st, g_version());
+                const bool blocks = step_blocks && look == 0;
+                const u64* slot[kN];
+                int prod[kN], part[kN];
+                bool has[kN];
+                u64 v[kN];
 #pragma unroll
                 for (int n = 0; n < kN; ++n) {
-                    const int i = in_row ? (lane & 15) : lane + 64 * n;
-                    if (i < 3 * nwv && !(in_row && n > 0)) v[n] = __hip_atomic_load(lg_entry(st, i / 3) + i % 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    const int i = kRow ? (lane & 15) : lane + 64 * n;
+                    has[n] = i < 3 * nwv;
+                    prod[n] = has[n] ? i / 3 : 0;   // (a lane without a word looks at the first one)
+                    part[n] = has[n] ? i - 3 * prod[n] : 0;
+                    slot[n] = lg_entry(st, prod[n]) + part[n];
                 }
+                unsigned int spins = 0;
+                unsigned long long first = 0ull;
+                bool there;
+                while (true) {
+                    there = true;
 #pragma unroll
-                for (int n = 0; n < kN; ++n) {
-                    const int i = in_row ? (lane & 15) : lane + 64 * n;
-                    if (i < 3 * nwv && !(in_row && n > 0)) there = there && (unsigned int)(v[n] >> 48) == step_tag(st, version);
+                    for (int n = 0; n < kN; ++n) v[n] = __hip_atomic_load(slot[n], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                    for (int n = 0; n < kN; ++n) there = there && (unsigned int)(v[n] >> 48) == tag;
+                    if (!blocks || __all(there || (kRow && lane >= 16))) break;
+                    bool give_up = false;
+                    if (spins > 0u && (spins & 255u) == 0u) {
+                        if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
+                        if (wait_clock_expired(spins, first)) spins = 0xffffffffu;
+                    }
+                    if (spins >= p.spin_limit) {
+                        __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        give_up = true;
+                    }
+                    if (__any(give_up)) {
+                        miss[1] = 1;
+                        someone_gave_up = 1;
+                        break;
+                    }
+                    if (spins != 0xffffffffu) ++spins;
                 }
-                return there;
-            };
-            auto best = [&](bool in_row) __attribute__((always_inline)) {
                 unsigned int key = 0u;
 #pragma unroll
-                for (int n = 0; n < kN; ++n) {
-                    const int i = in_row ? (lane & 15) : lane + 64 * n;
-                    if (i < 3 * nwv && !(in_row && n > 0)) key = max(key, rnnt_word_key(v[n], i / 3, i % 3));
+                for (int n = 0; n < kN; ++n) key = max(key, rnnt_word_key(v[n], prod[n], part[n]));
+                if (kRow) {
+                    const unsigned long long m = __ballot(there);
+                    const bool whole = ((m >> (lane & 48)) & 0xffffull) == 0xffffull;
+                    key = rnnt_max_row(key);
+                    if ((lane & 15) == 0) keys[n_pass & 1u][lane >> 4] = whole ? key : 0u;
+                } else {
+                    key = rnnt_max_u32(key);
+                    if (!__all(there)) key = 0u;
+                    if (lane == 0) keys[n_pass & 1u][look] = key;
                 }
-                return key;
             };
-            const bool blocks = step_blocks && look == 0;
-            unsigned int spins = 0;
-            unsigned long long first = 0ull;
-            bool there;
-            while (true) {
-                there = look_at(step + (row_per_step ? lane >> 4 : look), row_per_step);
-                if (!blocks || __all(there || (row_per_step && lane >= 16))) break;
-                bool give_up = false;
-                if (spins > 0u && (spins & 255u) == 0u) {
-                    if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
-                    if (wait_clock_expired(spins, first)) spins = 0xffffffffu;
-                }
-                if (spins >= p.spin_limit) {
-                    __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                    give_up = true;
-                }
-                if (__any(give_up)) {
-                    miss[1] = 1;
-                    someone_gave_up = 1;
-                    break;
-                }
-                if (spins != 0xffffffffu) ++spins;
-            }
-            if (row_per_step) {
-                const unsigned long long m = __ballot(there);
-                const bool whole = ((m >> (lane & 48)) & 0xffffull) == 0xffffull;
-                const unsigned int key = rnnt_max_row(best(true));
-                if ((lane & 15) == 0) keys[n_pass & 1u][lane >> 4] = whole ? key : 0u;
-            } else {
-                unsigned int key = rnnt_max_u32(best(false));
-                if (!__all(there)) key = 0u;
-                if (lane == 0) keys[n_pass & 1u][look] = key;
-            }
+            if (row_per_step) look_at(std::true_type{});
+            else look_at(std::false_type{});
         }
         rnnt_barrier();
         int r = (n_vec > 0 && miss[0] == 0) ? 1 : 0;
