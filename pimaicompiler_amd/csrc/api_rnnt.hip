@@ -41,6 +41,16 @@ std::vector<PimHipRnntPlan*> g_rnnt_plans;
 
 constexpr unsigned long long kRnntEventsBeforeAlone = 3;  // waits given up before a plan stops exchanging for good
 
+auto greedy_kernel(int64_t vocab)
+{
+    switch (rnnt_greedy_lane_words(vocab)) {
+        case 0: return rnnt_greedy_f16_kernel<0>;
+        case 1: return rnnt_greedy_f16_kernel<1>;
+        case 2: return rnnt_greedy_f16_kernel<2>;
+        default: return rnnt_greedy_f16_kernel<kRnntGreedyLaneWords>;
+    }
+}
+
 size_t exchange_words32(const PimHipRnntPlan* plan) { return (size_t)2 * plan->blocks * kRnntEntryWords * 2; }
 size_t greedy_exchange_words32(const PimHipRnntPlan* plan)
 {
@@ -170,7 +180,7 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
         const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
         plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);
         int greedy_per_cu = 0;
-        RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, rnnt_greedy_f16_kernel, kRnntThreads, 0));
+        RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, greedy_kernel(vocab), kRnntThreads, 0));
         plan->greedy_resident = (int64_t)greedy_per_cu * st->num_cus >= greedy_blocks(plan);
     }
     RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->greedy), sizeof(unsigned int) * (greedy_exchange_words32(plan) + greedy_count_words32(plan))));
@@ -389,7 +399,7 @@ extern "C" int pimhip_rnnt_greedy_decode(PimHipRnntPlan* plan, const void* enc, 
     // fill kernels, not memsets: the call can be recorded into a HIP graph
     launch_fill_u32(plan->greedy, greedy_exchange_words32(plan), ~0u, s);
     launch_fill_u32(plan->greedy + greedy_exchange_words32(plan), greedy_count_words32(plan), 0u, s);
-    rnnt_greedy_f16_kernel<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
+    greedy_kernel(plan->vocab)<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
     PIMHIP_HIP_CHECK(hipGetLastError());
     return PIMHIP_OK;
 }

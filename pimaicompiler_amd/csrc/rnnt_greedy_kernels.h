@@ -82,8 +82,14 @@ static_assert(kRnntGreedyBatch <= kRnntWaves, "a wavefront stores one step's wor
 constexpr int kRnntGreedyMaxVocab = 512;           // symbols
 constexpr int kRnntGreedyRowVocab = 5;             // up to this many symbol blocks to a team (15 words) a step's logits are a row of 16 lanes'
 constexpr int kRnntGreedyRows = 4;                 // ... and a pass looks at as many steps
-constexpr int kRnntGreedyLaneWords = 3;            // words a lane takes of a step's logits where a wavefront takes them
+constexpr int kRnntGreedyLaneWords = 3;            // at most this many words of a step's logits to a lane where a wavefront takes them
 static_assert(3 * (kRnntGreedyMaxVocab / 8) <= 64 * kRnntGreedyLaneWords, "a wavefront takes a step's logits");
+// The kernel for a vocabulary: 0 where a step's words fit a row of 16 lanes, else how many of them a lane of a wavefront takes.
+inline int rnnt_greedy_lane_words(int64_t vocab)
+{
+    const int64_t blocks = (vocab + 7) / 8;
+    return blocks <= kRnntGreedyRowVocab ? 0 : (int)((3 * blocks + 63) / 64);
+}
 constexpr int kRnntGreedyEmbHalfs = 16384;         // embedding rows kept in LDS by the first layer's blocks (32 KB)
 constexpr int kRnntSeenStride = 16;                // 32-bit words between the blocks' `seen` counts
 
@@ -310,6 +316,11 @@ __device__ __forceinline__ void rnnt_greedy_solo(const RnntGreedyArgs& p, half_t
     }
 }
 
+// LANE_WORDS: rnnt_greedy_lane_words.  The loop that polls for logits stands in every hand-over of a decision, so it is compiled for the
+// number of words and nothing else: with three for every vocabulary past 40 symbols and a branch between it and the row's, a
+// transcript of symbols alone took (2 x 320 units, 512 joint units, us a step) 7.29 with 41, 7.54 with 100, 7.58 with 169 and 7.74 with 512
+// symbols, 6.95, 7.21, 7.49 and 7.71 as it is; a run of blanks 1.07, 1.09, 1.11 and 1.28, now 0.94, 0.96, 1.02 and 1.27.
+template <int LANE_WORDS>
 __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const RnntGreedyArgs p)
 {
     typedef unsigned long long u64;
@@ -417,7 +428,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     // in order, and a device-scope store's acknowledgement takes longer than a poll.)
     unsigned int my_key = 0u;
     int n_there = 0;
-    const bool row_per_step = nwv <= kRnntGreedyRowVocab;
+    constexpr bool row_per_step = LANE_WORDS == 0;
     auto pass = [&](const u64* vec, int n_vec, unsigned int vec_tag, half_t* vec_dst, bool vec_blocks, int look_waves, bool step_blocks,
                     const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr) __attribute__((always_inline)) -> int {
         int* miss = missing[n_pass % 3u];
@@ -448,68 +459,64 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             }
         } else if (!row_per_step || look == 0) {
             // A lane's words: the one of its place in a row of 16 lanes (of step + row), or those of its place in the wavefront (of
-            // step + look).  Compiled for either, addresses and tags in front of the polls: every instruction of them counts.
-            auto look_at = [&](auto row_c) __attribute__((always_inline)) {
-                constexpr bool kRow = decltype(row_c)::value;
-                constexpr int kN = kRow ? 1 : kRnntGreedyLaneWords;
-                const int st = step + (kRow ? lane >> 4 : look);
-                const unsigned int tag = step_tag(st, g_version());
-                const bool blocks = step_blocks && look == 0;
-                const u64* slot[kN];
-                int prod[kN], part[kN];
-                bool has[kN];
-                u64 v[kN];
+            // step + look).  Addresses and tags in front of the polls: every instruction of them counts.
+            constexpr bool kRow = row_per_step;
+            constexpr int kN = kRow ? 1 : LANE_WORDS;
+            const int st = step + (kRow ? lane >> 4 : look);
+            const unsigned int tag = step_tag(st, g_version());
+            const bool blocks = step_blocks && look == 0;
+            const u64* slot[kN];
+            int prod[kN], part[kN];
+            bool has[kN];
+            u64 v[kN];
 #pragma unroll
-                for (int n = 0; n < kN; ++n) {
-                    const int i = kRow ? (lane & 15) : lane + 64 * n;
-                    has[n] = i < 3 * nwv;
-                    prod[n] = has[n] ? i / 3 : 0;   // (a lane without a word looks at the first one)
-                    part[n] = has[n] ? i - 3 * prod[n] : 0;
-                    slot[n] = lg_entry(st, prod[n]) + part[n];
+            for (int n = 0; n < kN; ++n) {
+                const int i = kRow ? (lane & 15) : lane + 64 * n;
+                has[n] = i < 3 * nwv;
+                prod[n] = has[n] ? i / 3 : 0;   // (a lane without a word looks at the first one)
+                part[n] = has[n] ? i - 3 * prod[n] : 0;
+                slot[n] = lg_entry(st, prod[n]) + part[n];
+            }
+            unsigned int spins = 0;
+            unsigned long long first = 0ull;
+            bool there;
+            while (true) {
+                there = true;
+#pragma unroll
+                for (int n = 0; n < kN; ++n) v[n] = __hip_atomic_load(slot[n], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                for (int n = 0; n < kN; ++n) there = there && (unsigned int)(v[n] >> 48) == tag;
+                if (!blocks || __all(there || (kRow && lane >= 16))) break;
+                bool give_up = false;
+                if (spins > 0u && (spins & 255u) == 0u) {
+                    if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
+                    if (wait_clock_expired(spins, first)) spins = 0xffffffffu;
                 }
-                unsigned int spins = 0;
-                unsigned long long first = 0ull;
-                bool there;
-                while (true) {
-                    there = true;
-#pragma unroll
-                    for (int n = 0; n < kN; ++n) v[n] = __hip_atomic_load(slot[n], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-#pragma unroll
-                    for (int n = 0; n < kN; ++n) there = there && (unsigned int)(v[n] >> 48) == tag;
-                    if (!blocks || __all(there || (kRow && lane >= 16))) break;
-                    bool give_up = false;
-                    if (spins > 0u && (spins & 255u) == 0u) {
-                        if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
-                        if (wait_clock_expired(spins, first)) spins = 0xffffffffu;
-                    }
-                    if (spins >= p.spin_limit) {
-                        __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                        give_up = true;
-                    }
-                    if (__any(give_up)) {
-                        miss[1] = 1;
-                        someone_gave_up = 1;
-                        break;
-                    }
-                    if (spins != 0xffffffffu) ++spins;
+                if (spins >= p.spin_limit) {
+                    __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                    give_up = true;
                 }
-                unsigned int key = 0u;
-#pragma unroll
-                for (int n = 0; n < kN; ++n) key = max(key, rnnt_word_key(v[n], prod[n], part[n]));
-                if (kRow) {
-                    const unsigned long long m = __ballot(there);
-                    const bool whole = ((m >> (lane & 48)) & 0xffffull) == 0xffffull;
-                    key = rnnt_max_row(key);
-                    if ((lane & 15) == 0) keys[n_pass & 1u][lane >> 4] = whole ? key : 0u;
-                } else {
-                    key = rnnt_max_u32(key);
-                    if (!__all(there)) key = 0u;
-                    if (lane == 0) keys[n_pass & 1u][look] = key;
+                if (__any(give_up)) {
+                    miss[1] = 1;
+                    someone_gave_up = 1;
+                    break;
                 }
-            };
-            if (row_per_step) look_at(std::true_type{});
-            else look_at(std::false_type{});
+                if (spins != 0xffffffffu) ++spins;
+            }
+            unsigned int key = 0u;
+#pragma unroll
+            for (int n = 0; n < kN; ++n) key = max(key, rnnt_word_key(v[n], prod[n], part[n]));
+            if (kRow) {
+                const unsigned long long m = __ballot(there);
+                const bool whole = ((m >> (lane & 48)) & 0xffffull) == 0xffffull;
+                key = rnnt_max_row(key);
+                if ((lane & 15) == 0) keys[n_pass & 1u][lane >> 4] = whole ? key : 0u;
+            } else {
+                key = rnnt_max_u32(key);
+                if (!__all(there)) key = 0u;
+                if (lane == 0) keys[n_pass & 1u][look] = key;
+            }
         }
         rnnt_barrier();
         int r = (n_vec > 0 && miss[0] == 0) ? 1 : 0;

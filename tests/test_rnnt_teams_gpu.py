@@ -28,3 +28,13 @@ def test_teams_of_symbol_blocks_decode_as_single_steps_do(ops, L, I, H, F, J, V,
     plan = ops.RnntPlan(dev(params), True, L, tuple(dev(joint)))
     check(plan.greedy_decode(enc, embedding, x0, blank, max_symbols_per_frame=3),
           loop_driven_from_the_host(plan, enc, embedding, x0, blank, 3, 3 * T))
+
+
+@pytest.mark.parametrize("V", [168, 169, 336, 337])
+def test_words_of_a_step_per_lane(ops, V):
+    """Around the lines between the kernels for one, two and three words of a step's logits to a lane (21 and 42 symbol blocks)."""
+    L, H, F, J, T = 1, 64, 128, 64, 40
+    params, joint, enc, embedding, x0 = model(V, L, H, H, F, J, V, T, V - 1, 0.3)
+    plan = ops.RnntPlan(dev(params), True, L, tuple(dev(joint)))
+    check(plan.greedy_decode(enc, embedding, x0, V - 1, max_symbols_per_frame=3),
+          loop_driven_from_the_host(plan, enc, embedding, x0, V - 1, 3, 3 * T))
