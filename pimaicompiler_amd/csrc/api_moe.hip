@@ -1,5 +1,7 @@
 // The mixture-of-experts feed-forward step of the C ABI (include/pimhip.h): router, choice of the expert and its two
 // products for one token in one launch.
+#include <type_traits>
+
 #include "api_common.h"
 #include "moe_kernels.h"
 

@@ -20,13 +20,14 @@
 // What bounds the step is not bandwidth (9.4 MB) but a chain of dependent round trips: token and router rows, the expert's
 // W1 rows, the all-to-all of `hidden`, the store of y.  So nothing else may stand in that chain: the launch count (which
 // says which set of exchange slots this launch uses) is a device-scope load and is asked for behind the router's cached
-// loads, not in front of them; the rows of W2 are asked for right behind the rows of W1, and the hidden values by wavefronts that
-// hold no row of W2 (a wavefront's loads return in order: a poll behind W2's rows waits for them, 0.7 us where another expert's
-// were cached); what is not waited for, the caller's view of the choice, the slots of the next launch, goes out behind the
-// block's own word, but not at the end: a launch lasts until its last store is acknowledged.
-// Measured on MI355X (8 experts, 768 / 3072, one of 13 tokens in a row; time stamps in block 0): start and router 0.9 us, argmax 0.2
-// (0.36 with the choice stored in front), W1 1.2 (1.5 with W2's rows behind the hidden values and twice as many of them, loaded and
-// dropped by wavefronts without a row), exchange 1.2 - 1.6 (1.7), W2 0.5, end and next launch 1.1 (1.2): 6.4 -> 5.5 us a step.
+// loads, not in front of them; the rows of W2 are asked for once the block's own word is stored, and the hidden values by wavefronts
+// that hold no row of W2 as far as there are enough (a wavefront's loads return in order: a poll behind W2's rows waits for them, 0.7 us
+// where another expert's were cached); what is not waited for, the caller's view of the choice, the slots of the next launch, goes
+// out behind the word too, but not at the end: a launch lasts until its last store is acknowledged.
+// Measured on MI355X (8 experts, 13 tokens in a row from a graph, us a step; in brackets with the rows of W2 right behind those of W1,
+// where the word, which everybody waits for, queues behind up to 64 KB): 256 / 4096 4.57 (4.67), 768 / 1024 4.53 (4.95), 768 / 3072 5.23
+// (5.37), 1024 / 4096 6.41 (6.91), 1792 / 2048 6.64 (7.15), 2048 / 4096 8.91 (9.73).  With every wavefront loading a row of W2, its own or
+// one to drop, and polling behind it: 7.14, 5.38, 6.39, 7.97, 6.99, 9.46.
 //
 // Exchange: hx[2][blocks] entries of 64 bytes, a block's words in the first 16 * wpb bytes.  An empty 8-byte half is all
 // ones, which no four fp16 values written here can be (a NaN is written as 0x7e00).  The two sets alternate by the launch
@@ -42,8 +43,6 @@
 // starts in that self-sufficient mode (the exchange slots may hold values of the launch that was cut short) until the
 // host has refilled the slots and cleared the word.
 #pragma once
-
-#include <type_traits>
 
 #include "device_common.h"
 
@@ -88,7 +87,7 @@ struct MoeStepArgs {
 };
 
 // The barrier between the phases: this wavefront's LDS traffic done, then s_barrier.  __syncthreads() would also wait until the rows
-// of W2, asked for right behind those of W1, have arrived.
+// of W2 have arrived and the stores in front of them are acknowledged.
 __device__ __forceinline__ void moe_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // The maximum over the four rows of 16 lanes (wave_sum_rows' exchanges).
@@ -225,11 +224,12 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
         if (a != a) bits = 0x7e00u;
         return bits;
     };
-    // This wavefront's row of W2[e]: asked for here, consumed at the end.
+    // This wavefront's row of W2[e]: asked for behind the block's word, consumed at the end.
     half8_t w2r[FC];
     const int r2 = b * p.rpb2 + wave;
     const bool has_row2 = wave < p.rpb2 && r2 < p.d_model;
     auto ask_for_w2 = [&]() {
+        if (!has_row2) return;
 #pragma unroll
         for (int k = 0; k < FC; ++k) w2r[k] = load_weight<true>(w2 + (long)r2 * nf + min(lane + 64 * k, nf - 1));
     };
@@ -240,32 +240,25 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
     const unsigned int g = __hip_atomic_load(p.g_counter + p.count_stride * b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned int poisoned = __hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     // ---- hidden = act(W1[e] . x + b1[e]): this block's words (asked for whether or not they will be published) ----
-    // Compiled for wavefronts with and without a row of W2, no load behind a condition: the wait for W1's rows is a wait for a
-    // number of loads that may still be in flight, which the compiler has to know.
     const int row0 = 8 * p.wpb * b + wave * p.wpb;  // this wavefront's first row
-    auto first_product = [&](auto holds_row2) __attribute__((always_inline)) {
-        half8_t w1r[kMoeMaxWordsPerBlock][XC];
+    half8_t w1r[kMoeMaxWordsPerBlock][XC];
 #pragma unroll
-        for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
-            const int r = min(row0 + min(s, p.wpb - 1), p.d_ff - 1);
+    for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
+        const int r = min(row0 + min(s, p.wpb - 1), p.d_ff - 1);
 #pragma unroll
-            for (int k = 0; k < XC; ++k) w1r[s][k] = load_weight<true>(w1 + (long)r * nx + min(lane + 64 * k, nx - 1));
-        }
-        if constexpr (decltype(holds_row2)::value) ask_for_w2();
-        if (poisoned != 0u) block_poisoned = 1;
+        for (int k = 0; k < XC; ++k) w1r[s][k] = load_weight<true>(w1 + (long)r * nx + min(lane + 64 * k, nx - 1));
+    }
+    if (poisoned != 0u) block_poisoned = 1;
 #pragma unroll
-        for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
-            const int r = row0 + s;
-            float a = 0.0f;
+    for (int s = 0; s < kMoeMaxWordsPerBlock; ++s) {
+        const int r = row0 + s;
+        float a = 0.0f;
 #pragma unroll
-            for (int k = 0; k < XC; ++k)
-                if (lane + 64 * k < nx) a = dot8(w1r[s][k], xr[k], a);
-            a = wave_sum(a);
-            if (lane == 0 && s < p.wpb) mine[wave * p.wpb + s] = r < p.d_ff ? hidden_bits(a, r) : (unsigned short)0;
-        }
-    };
-    if (has_row2) first_product(std::true_type{});
-    else first_product(std::false_type{});
+        for (int k = 0; k < XC; ++k)
+            if (lane + 64 * k < nx) a = dot8(w1r[s][k], xr[k], a);
+        a = wave_sum(a);
+        if (lane == 0 && s < p.wpb) mine[wave * p.wpb + s] = r < p.d_ff ? hidden_bits(a, r) : (unsigned short)0;
+    }
     const unsigned int set = __builtin_amdgcn_readfirstlane(g) & 1u;
     // Whether the abort word is up is decided for the block as a whole, through LDS: wavefronts look at it at slightly
     // different times and can see different values when it is raised while the launch starts; they would then disagree
@@ -292,6 +285,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
         }
         empty_other_set();
         report_choice();
+        ask_for_w2();
         // ---- everybody's hidden values: word t and word t + n_poll by the threads behind the wavefronts that wait for a row of W2 ----
         const int poll0 = 64 * min(min(p.rpb2, kMoeWaves), kMoeWaves - (nf + 127) / 128);
         const int n_poll = kMoeThreads - poll0, t0 = tid - poll0;
@@ -328,6 +322,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
     } else {
         empty_other_set();
         report_choice();
+        ask_for_w2();
     }
     // (With one count for all: block 0 has seen everybody's word by now, or makes it late, when it has computed by itself.)
     auto advance_count = [&]() {

@@ -9,8 +9,9 @@ from test_moe_gpu import DEV, TOL, dev, libtorch_cpu, make, maxabs
 pytestmark = pytest.mark.gpu
 
 
+# (1536, 1544 and 1792 / 4096: six and seven rows of the second matrix to a block, more than leave wavefronts enough to poll without one)
 @pytest.mark.parametrize("d_model,d_ff", [(512, 1024), (520, 1032), (1024, 2048), (1032, 2056), (512, 3072), (520, 3080), (2048, 8), (8, 4096),
-                                          (2048, 4096)])
+                                          (2048, 4096), (1536, 4096), (1544, 4096), (1792, 4096)])
 def test_sizes_on_both_sides_of_a_change_of_kernel(ops, d_model, d_ff):
     g, Wr, br, W1, b1, W2, b2 = make(d_model + d_ff, 3, d_model, d_ff, True, scale=0.5 / max(d_model, 64) ** 0.5)
     plan = ops.MoePlan((Wr.to(DEV), br.to(DEV)), dev(W1), dev(W2), dev(b1), dev(b2))
