@@ -2,6 +2,7 @@
 // sums and the classifier in one persistent launch.
 #include "api_common.h"
 #include "decoder_kernels.h"
+#include "decoder_plan.h"
 
 #include <algorithm>
 
@@ -112,10 +113,12 @@ extern "C" int pimhip_decoder_plan_create(PimHipDecoderPlan** plan_out, const vo
     if (classifier_w && !aligned16(classifier_w)) return fail(PIMHIP_ERR_UNSUPPORTED, "the classifier weight is not 16-byte aligned");
 
     const int blocks = (int)((H + kDecUnits - 1) / kDecUnits);
-    int per_cu = 0;
-    PIMHIP_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, decoder_step_f16_kernel<kDecMaxLayers, true>, kDecThreads, 0));
-    if ((int64_t)per_cu * st->num_cus < blocks)
-        return fail(PIMHIP_ERR_UNSUPPORTED, "the %d blocks of the decoder step cannot all be resident on this device", blocks);
+    for (auto kernel : {decoder_step_f16_kernel<kDecMaxLayers, true, true>, decoder_step_f16_kernel<kDecMaxLayers, true, false>}) {
+        int per_cu = 0;
+        PIMHIP_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kDecThreads, 0));
+        if ((int64_t)per_cu * st->num_cus < blocks)
+            return fail(PIMHIP_ERR_UNSUPPORTED, "the %d blocks of the decoder step cannot all be resident on this device", blocks);
+    }
 
     hipStream_t s = static_cast<hipStream_t>(stream);
     int device = -1;
@@ -348,13 +351,12 @@ extern "C" int pimhip_decoder_step(PimHipDecoderPlan* plan, const void* x, const
         if (rc != PIMHIP_OK) return rc;
     }
     const dim3 grid(plan->blocks), block(kDecThreads);
-    // What a step reads: W_hh and the input columns of every layer, and the classifier.
-    const unsigned long long bytes = ((unsigned long long)L * 8 * H * H + (unsigned long long)plan->vocab * H) * sizeof(half_t);
+    const bool keep = dec_rows_stay(L, H, plan->input_size, L - 1 + plan->first_takes_context, ctx_in != nullptr, plan->enc_len, plan->vocab);
     auto launch = [&](auto layers) {
         constexpr int kL = decltype(layers)::value;
-        if (!plan->cls_w) decoder_step_f16_kernel<kL, false><<<grid, block, 0, s>>>(a);
-        else if (bytes <= kDecKeptBytes) decoder_step_f16_kernel<kL, true><<<grid, block, 0, s>>>(a);
-        else decoder_step_f16_kernel<kL, true, false><<<grid, block, 0, s>>>(a);
+        auto kernel = plan->cls_w ? (keep ? decoder_step_f16_kernel<kL, true, true> : decoder_step_f16_kernel<kL, true, false>)
+                                  : (keep ? decoder_step_f16_kernel<kL, false, true> : decoder_step_f16_kernel<kL, false, false>);
+        kernel<<<grid, block, 0, s>>>(a);
     };
     switch (L) {
         case 1: launch(std::integral_constant<int, 1>{}); break;

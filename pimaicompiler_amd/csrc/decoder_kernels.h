@@ -283,14 +283,8 @@ __device__ constexpr int cls_groups_after(int k)
     return k <= 2 ? 1 : 0;
 }
 
-// KEEP: how the layers' rows are read (load_weight); classifier rows are read with plain loads.  A loop of steps reads the same
-// weights every step, and plain loads leave them in the caches until then as long as they fit: us a step on MI355X, non-temporal /
-// plain: 1024 units, four layers with 8000 / 32000 / 64000 classifier rows (84 / 135 / 198 MB) 23.2 / 22.0, 28.1 / 26.7, 37.6 / 36.3;
-// three of 776 with 3001 (34 MB) 15.4 / 13.2; two of 512 with 32000 (41 MB) 17.8 / 14.7.  Past the 256 MB Infinity Cache the
-// layers' rows, which the chain waits for, are better read non-temporally: with 88000 / 100000 /
-// 120000 rows (248, 272, 313 MB) plain 43.7 / 48.4 / 58.9, non-temporal 43.9 / 47.8 / 52.8 (classifier rows too: 45.8 / 50.1 / 56.1).
-static constexpr unsigned long long kDecKeptBytes = 240ull << 20;
-template <int L, bool CLS, bool KEEP = true>
+// KEEP: how the layers' rows are read (load_weight; dec_rows_stay chooses); classifier rows are read with plain loads.
+template <int L, bool CLS, bool KEEP>
 __global__ __launch_bounds__(kDecThreads) void decoder_step_f16_kernel(DecoderStepArgs p)
 {
     static_assert(L >= 1 && L <= kDecMaxLayers, "layers per step");
