@@ -3,6 +3,7 @@
 #include "api_common.h"
 #include "../../include/pimhip_probe.h"
 #include "lstm_kernels.h"
+#include "lstm_plan.h"
 #include "lstm_xcd_kernels.h"
 
 using namespace pimhip;
@@ -128,19 +129,6 @@ namespace
 __global__ void xcc_map_kernel(unsigned int* out)
 {
     if (threadIdx.x == 0) out[blockIdx.x] = hw_xcc_id();
-}
-
-// Whether independent recurrences on XCDs multiply on v_dot2 instead of sparse matrix instructions, whose weights pass through LDS
-// first (1 to 1.6 us per launch) and which win every step: short sequences only, and where sparse fragments are not as good as
-// empty (65 to 256 units) or v_dot2 itself is at its worst.  Pipelines of layers always take the sparse ones.  Measured on MI355X
-// (graph replays, one layer, us per call, v_dot2 / sparse, at 4, 8 and 16 steps):
-//   64 units 12.3 / 12.7, 15.4 / 15.6, 22.2 / 22.2   128 12.2 / 12.2, 15.8 / 15.6   256 13.0 / 12.8, 17.0 / 16.2   320 14.3 / 14.6, 18.6 / 18.4
-//   512 14.3 / 14.8, 19.0 / 18.9   640 16.4 / 17.3, 21.4 / 21.9, 30.9 / 30.5   768 19.2 / 19.6, 24.1 / 24.0   1024 23.5 / 24.0, 29.2 / 28.7, 40.3 / 37.9
-// and at 80 and 200 steps: 64 75.0 / 74.6, 173 / 172   256 86.5 / 76.2, 200 / 174   640 109 / 101, 253 / 231   1024 133 / 114, 305 / 254; two
-// layers 64 86.7 / 83.0   640 124 / 111   1024 159 / 123 (at 4 steps 640 23.9 / 24.4, 1024 32.8 / 31.9).
-bool xcd_on_dot(int64_t H, int64_t T)
-{
-    return (H <= 64 || H > 256) && T < (H > 512 && H <= 640 ? 12 : 8);
 }
 
 // The per-XCD kernel finds its place by the hardware's XCC_ID and relies on two things the hardware does today: ids 0..7,
@@ -315,7 +303,7 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
         };
         plan->xcd_ok = true;
         PLAN_HIP_CHECK(resident(pipeline ? lstm_xcd_f16_kernel<true> : lstm_xcd_f16_kernel<false>, &plan->xcd_ok));
-        if (!pipeline) PLAN_HIP_CHECK(resident(lstm_xcd_dot_f16_kernel, &plan->xcd_ok));
+        PLAN_HIP_CHECK(resident(pipeline ? lstm_xcd_dot_f16_kernel<true> : lstm_xcd_dot_f16_kernel<false>, &plan->xcd_ok));
         if (plan->xcd_ok) {
             bool rotation = false;
             const int rc_probe = xcd_dispatch_is_a_rotation(kXcdCount * kXcdMembers, s, &rotation);
@@ -642,7 +630,8 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             a.H = (int)H;
             a.T = (int)T;
             a.spin_limit = plan->spin_limit;
-            (any_res ? lstm_xcd_res_f16_kernel : lstm_xcd_f16_kernel<true>)<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
+            auto kernel = any_res ? lstm_xcd_res_f16_kernel : xcd_on_dot(H, T, n) ? lstm_xcd_dot_f16_kernel<true> : lstm_xcd_f16_kernel<true>;
+            kernel<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
             PIMHIP_HIP_CHECK(hipGetLastError());
             layer_in = group_out;
             l += n;
@@ -686,7 +675,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             a.H = (int)H;
             a.T = (int)T;
             a.spin_limit = plan->spin_limit;
-            (xcd_on_dot(H, T) ? lstm_xcd_dot_f16_kernel : lstm_xcd_f16_kernel<false>)<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
+            (xcd_on_dot(H, T, 1) ? lstm_xcd_dot_f16_kernel<false> : lstm_xcd_f16_kernel<false>)<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
             if (residual(l)) add_input(layer_out, layer_in);
             PIMHIP_HIP_CHECK(hipGetLastError());
             layer_in = layer_out;

@@ -1,0 +1,34 @@
+// Which kind of products the per-XCD LSTM kernel multiplies with (lstm_xcd_kernels.h): host arithmetic only, so that the lines can be
+// asked for without a GPU.
+#pragma once
+
+#include <stdint.h>
+
+namespace pimhip
+{
+// v_dot2 instead of sparse matrix instructions.  The latter's weights pass through LDS first (1 to 1.6 us per launch), and they take
+// whole fragments of 64 columns in groups of four: v_dot2 is better for short sequences, for fewer than 64 units at any length, and
+// longest for 513 to 656 units, of whose second and third group the sparse fragments are half empty.  From 65 to 256 units one
+// group holds the row and there is nothing to win.  `chained`: the layers a launch runs as a pipeline, 1 for recurrences that are fed by
+// none other; the more there are, the more steps the launch has beside its sequence's.
+// Measured on MI355X (graph replays, time on v_dot2 over time on sparse instructions):
+//   one layer, at 2 / 4 / 6 / 8 / 10 / 16 steps: 64 units 1.00 / 0.95 / 0.99 / 0.99 / 1.01 / 1.01, 128 0.95 / 0.97 / 1.00 / 1.00 / 1.02 / 1.02, 192 1.01 / 1.01 /
+//     1.06 / 1.04 / 1.07 / 1.08, 320 0.97 / 0.97 / 0.99 / 1.02 / 1.04 / 1.06, 512 0.94 / 0.97 / 0.99 / 1.02 / 1.04 / 1.07, 640 0.90 / 0.93 / 0.95 / 0.97 / 0.98 / 1.01,
+//     768 0.94 / 0.97 / 0.99 / 1.02 / 1.02 / 1.05, 1024 0.95 / 0.98 / 1.00 / 1.02 / 1.04 / 1.08; two directions within 0.02 of these
+//   one layer, at 24 / 80 / 200 steps: 8 units 0.97 / 0.95 / 0.95, 32 0.96 / 0.96 / 0.96, 48 0.95 / 0.95 / 0.94, 64 1.00 / 1.01 / 1.01, 128 1.02 / 1.04 / 1.04
+//   two layers, at 2 / 3 / 4 / 6 / 8 steps: 128 1.00 / 1.00 / 1.00 / 0.99 / 1.01, 256 1.01 / 1.02 / 1.03 / 1.04 / 1.05, 512 0.96 / 0.98 / 1.00 / 1.02 / 1.03, 640 0.94 /
+//     0.96 / 0.97 / 0.98 / 1.00, 768 0.98 / 1.00 / 1.00 / 1.01 / 1.03, 1024 0.97 / 0.99 / 1.01 / 1.03 / 1.05; at 24 / 80 / 200: 8 0.97 / 0.98 / 0.98, 48 0.98 / 0.97 /
+//     0.97, 64 1.01 / 1.02 / 1.03
+//   three layers, at 2 / 3 / 4: 512 1.01 / 1.01 / 1.02, 640 0.97 / 1.00 / 1.00, 1024 1.00 / 1.02 / 1.03; at 24 / 80 / 200: 16 0.97 / 0.98 / 0.98, 32 1.06 / 1.13 / 1.15;
+//     four layers, at 2 / 4 / 8: 16 0.98 .. 1.00, 640 1.00 / 1.01 / 1.03
+inline bool xcd_on_dot(int64_t H, int64_t T, int chained)
+{
+    const bool half_empty = H > 512 && H <= 656;
+    if (chained == 1) {
+        if (H <= 64) return H < 64 || T < 24;
+        return H <= 128 ? T < 8 : H > 256 && T < (half_empty ? 11 : 7);
+    }
+    if (chained == 2) return H < 64 || (H > 256 && T < (half_empty ? 7 : 4));
+    return chained == 3 && (H <= 16 || (half_empty && T < 3));
+}
+}  // namespace pimhip

@@ -44,7 +44,7 @@
 //   XcdSparse  16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16: 0.21 us of matrix instructions at H = 1024; a step 1.16 us
 //              for a single layer, 1.18 in pipelines (v_dot2 1.43, 1.64)
 //   XcdDot     v_dot2 and a transposing reduction over 16 lanes: nothing passes through LDS at the start of a launch, which short
-//              sequences of independent recurrences notice (xcd_on_dot in api_lstm.hip has the line and the figures)
+//              sequences notice, and few units leave less of it idle (xcd_on_dot in lstm_plan.h has the lines and the figures)
 // Against 64 bits the sums are equally far off (rms error over the sum of the products' magnitudes, 64 .. 1024 columns, MI355X): signs
 // mixed 4.7e-9 .. 9.7e-9 on v_dot2 and 3.2e-9 .. 7.9e-9 sparse, all of one sign 3.4e-8 .. 5.2e-8 and 3.5e-8 .. 4.9e-8; an h made
 // from the same previous h differs from its 64-bit value by 2.07e-4 relative with either, the rounding to fp16.
@@ -137,7 +137,7 @@ __device__ __forceinline__ void store8_plain(void* p, unsigned long long v)
 // ---- the step's matrix-vector product on v_dot2 ----
 // Row l >> 4 of 16 lanes has the wavefront's unit l >> 4: its lanes keep, of the four gate rows, the 8-wide column pieces
 // 16 c + (l & 15), c = 0 .. 7.  Four dot products of up to 64 columns per lane, then a transposing reduction over the 16 lanes.
-struct XcdDot {  // (no pipelines: chosen for short sequences of recurrences that are fed by none other)
+struct XcdDot {
     half8_t w[4][8];
 
     static __device__ __forceinline__ int unit(int lane) { return lane >> 4; }
@@ -765,9 +765,10 @@ __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_f16_kernel(LstmXcdArgs p
     lstm_xcd_body<PIPE, false, XcdSparse>(p);
 }
 
+template <bool PIPE>
 __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_dot_f16_kernel(LstmXcdArgs p)
 {
-    lstm_xcd_body<false, false, XcdDot>(p);
+    lstm_xcd_body<PIPE, false, XcdDot>(p);
 }
 
 // The pipeline for stacks that have layers with a residual sum.
