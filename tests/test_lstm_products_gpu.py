@@ -1,17 +1,20 @@
-"""The per-XCD recurrence (mode 4) on either side of the lines between its two kinds of products, v_dot2 and sparse matrix
-instructions: sizes around a line in hidden units or steps, whole fragments and ragged ones."""
+"""The per-XCD recurrence (mode 4) with both of its kinds of products, v_dot2 and sparse matrix instructions: whole fragments and ragged
+ones.  Every test asks which kind its size takes (lstm_kinds.py), so that a move of the lines cannot leave one of them untested."""
 import pytest
 import torch
+
+from lstm_kinds import on_dot
 
 from oracle import oracle
 from pimaicompiler_amd import workloads
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-# (hidden size, steps): the second of a pair is across the line from the first
-ONE = [(384, 40), (392, 40), (392, 31), (512, 32), (520, 33), (640, 100), (648, 95), (648, 96), (768, 96), (776, 47), (776, 48), (896, 48), (904, 15),
-       (904, 16), (1024, 16), (8, 12), (256, 20)]
-STACK = [(128, 12), (136, 9), (136, 10), (512, 10), (520, 23), (520, 24), (640, 24), (648, 9), (648, 10), (1024, 10)]
+# (hidden size, steps)
+ONE_SPARSE = [(384, 40), (392, 40), (392, 31), (512, 32), (520, 33), (640, 100), (648, 95), (648, 96), (768, 96), (776, 47), (776, 48), (896, 48), (904, 15),
+              (904, 16), (1024, 16), (256, 20)]
+ONE_DOT = [(8, 12), (56, 40), (64, 7), (128, 7), (392, 6), (512, 4), (520, 10), (640, 10), (776, 6), (904, 5), (1024, 6)]
+STACK_SPARSE = [(128, 12), (136, 9), (136, 10), (512, 10), (520, 23), (520, 24), (640, 24), (648, 9), (648, 10), (1024, 10)]
 
 
 def plan_of(ops, params, layers, bidir, T, res=None):
@@ -23,7 +26,7 @@ def plan_of(ops, params, layers, bidir, T, res=None):
 
 
 @pytest.mark.parametrize("bidir", [False, True])
-@pytest.mark.parametrize("H,T", ONE)
+@pytest.mark.parametrize("H,T", ONE_SPARSE + ONE_DOT)
 def test_every_step_is_as_close_to_64_bits_as_its_sums_allow(ops, H, T, bidir):
     """h of every step against float64 arithmetic on the previous h the kernel itself made, with the cell state carried in float64.
     A pre-activation of K = I + H products is off by at most (K / 8 + 8) * 2^-24 of the sum of their magnitudes (eight and more
@@ -60,7 +63,7 @@ def test_every_step_is_as_close_to_64_bits_as_its_sums_allow(ops, H, T, bidir):
 
 
 @pytest.mark.parametrize("layers,res", [(2, None), (3, 1), (4, None)])
-@pytest.mark.parametrize("H,T", STACK)
+@pytest.mark.parametrize("H,T", STACK_SPARSE)
 def test_stacks_match_libtorch(ops, H, T, layers, res):
     params, x, h0, c0 = workloads.lstm_inputs(H + T, H if res is not None else 40, H, layers, False, T)
     plan = plan_of(ops, params, layers, False, T, res)
@@ -78,9 +81,13 @@ def test_stacks_match_libtorch(ops, H, T, layers, res):
         assert float((got.float().cpu().reshape(-1) - w.float().cpu().reshape(-1)).abs().max()) <= 5e-3
 
 
-@pytest.mark.parametrize("H,T,layers,bidir,res", [(128, 12, 2, False, None), (128, 12, 3, False, 1), (256, 12, 1, True, None), (392, 32, 1, False, None),
-                                                  (904, 16, 1, True, None), (136, 12, 2, False, None), (520, 24, 3, False, 1)])
-def test_waits_that_give_up_and_nans_in_both_kinds(ops, H, T, layers, bidir, res):
+@pytest.mark.parametrize("H,T,layers,bidir,res,dot", [
+    (128, 12, 2, False, None, False), (128, 12, 3, False, 1, False), (256, 12, 1, True, None, False), (392, 32, 1, False, None, False),
+    (904, 16, 1, True, None, False), (136, 12, 2, False, None, False), (520, 24, 3, False, 1, False),
+    (392, 6, 1, True, None, True), (520, 10, 1, True, None, True), (640, 10, 1, False, None, True), (1024, 6, 1, False, None, True),
+    (56, 12, 2, False, None, True), (16, 12, 3, False, None, True), (640, 6, 2, False, None, True), (1024, 3, 2, False, None, True)])
+def test_waits_that_give_up_and_nans_in_both_kinds(ops, H, T, layers, bidir, res, dot):
+    assert dot == (res is None and on_dot(H, T, 1 if bidir else layers))
     params, x, h0, c0 = workloads.lstm_inputs(H, H, H, layers, bidir, T)
     plan = plan_of(ops, params, layers, bidir, T, res)
     args = (x.reshape(T, H).to(DEV), h0.to(DEV), c0.to(DEV))
@@ -108,9 +115,11 @@ def test_waits_that_give_up_and_nans_in_both_kinds(ops, H, T, layers, bidir, res
         assert bool(torch.isnan(y[at:]).all()) and torch.equal(y[:at], want[0][:at])
 
 
-@pytest.mark.parametrize("H,layers,bidir,short,long", [(512, 1, True, 31, 32), (1024, 1, False, 15, 16), (256, 3, False, 9, 10), (640, 2, False, 23, 24)])
+@pytest.mark.parametrize("H,layers,bidir,short,long", [(512, 1, True, 6, 7), (1024, 1, False, 6, 7), (64, 1, False, 23, 24), (264, 2, False, 3, 4), (640, 2, False, 6, 7)])
 def test_one_plan_runs_both_kinds_in_turn(ops, H, layers, bidir, short, long):
     """The two kinds share the exchange, its counters and its slots: sequences on either side of a line in turn, eager and replayed."""
+    chained = 1 if bidir else layers
+    assert on_dot(H, short, chained) and not on_dot(H, long, chained)
     params, x, h0, c0 = workloads.lstm_inputs(H, 40, H, layers, bidir, long)
     xd, h0, c0 = x.reshape(long, 40).to(DEV), h0.to(DEV), c0.to(DEV)
     want = {T: plan_of(ops, params, layers, bidir, T).forward(xd[:T], h0, c0) for T in (short, long)}
