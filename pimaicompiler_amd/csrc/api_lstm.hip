@@ -3,7 +3,6 @@
 #include "api_common.h"
 #include "../../include/pimhip_probe.h"
 #include "lstm_kernels.h"
-#include "lstm_plan.h"
 #include "lstm_xcd_kernels.h"
 
 using namespace pimhip;

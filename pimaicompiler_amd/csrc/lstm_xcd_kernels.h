@@ -53,6 +53,7 @@
 #include <type_traits>
 
 #include "lstm_kernels.h"
+#include "lstm_plan.h"
 #include "lstm_solo.h"
 
 namespace pimhip
@@ -231,16 +232,10 @@ static constexpr int kXcdFrags = kXcdMaxH / 64;  // 64-column weight fragments o
 // the weight matrix the 64 are is free as long as both operands agree.  A lane of B takes two whole 16-byte pieces of its gate
 // row, 8 m + (l >> 4) and four pieces further; halves 0..3 of a piece then meet the even row of A, halves 4..7 the odd one.
 
-// Where the 16-byte piece p of h lies in LDS.  A read of 8 bytes per lane takes from eight rows of 128 bytes (the row pairs of A) two
-// of four pieces; in their own order four of the rows share their banks, and the eight wavefronts' reads of a step took 512 cycles of
-// the LDS where 128 do.  Rows 2 q, 2 q + 1 have their pieces exchanged by 0, 1, 4 or 5 instead: every half wavefront reads all banks
-// once.  Two layers of 1024, 341 steps 480.6 -> 428.8 us, two directions, 50 steps 82.4 -> 75.0.
-__device__ __forceinline__ int xcd_h_place(int p) { return p ^ ((p >> 4 & 1) | (p >> 5 & 1) << 2); }
-
 // Lane l's eight values of h in register set s of A: two 8-byte halves of neighbouring pieces.
 __device__ __forceinline__ half8_t xcd_h_operand(const half_t* hb, int s, int lane)
 {
-    const int row = 8 * s + ((lane & 15) >> 1), lo = xcd_h_place(8 * row + 2 * (lane >> 4));
+    const int lo = xcd_h_place(xcd_h_operand_piece(s, lane));
     return __builtin_shufflevector(*reinterpret_cast<const half4_t*>(hb + lo * 8 + 4 * (lane & 1)),
                                    *reinterpret_cast<const half4_t*>(hb + (lo ^ 1) * 8 + 4 * (lane & 1)), 0, 1, 2, 3, 4, 5, 6, 7);
 }
