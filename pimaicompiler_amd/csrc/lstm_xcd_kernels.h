@@ -97,6 +97,7 @@ static constexpr unsigned long long kXcdWaitTicks = 100000000ull;  // one second
 // (sums around the upper layers, by wavefront 4 / by this one: three layers of 1024, 50 steps 103 / 99 us, three of 512, 100 steps
 // 148 / 135, two of 136, 100 steps 123 / 118).
 static constexpr int kXcdSumWave = 2;
+static_assert(kXcdSumWave >= 2 && kXcdSumWave < kXcdWaves, "wavefronts 0 and 1 poll for h");
 static constexpr int kXcdLag = 2;       // steps a recurrence fed by a P group lets that group get ahead before it starts
 
 struct LstmXcdArgs {
@@ -435,7 +436,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     const int uc = units_ok ? my_unit : H - 1;
     // All lanes of the first two wavefronts fetch one piece of an h vector each: 8 fp16 = columns 8 q .. 8 q + 7.  Spread over eight
     // wavefronts of 16 lanes a step of 1024 units took 1.42 us, over four of 32 1.32, over two 1.31.  (The wavefronts that talk
-    // to other XCDs, 4 .. 7, never poll: a wavefront's loads come back in order.)
+    // to other XCDs, 4 .. 7 and the one that makes the residual sums, never poll for h: a wavefront's loads come back in order.)
     const int piece = wave * 64 + lane;
     const bool polls = wave < 2 && piece * 8 < H;
 

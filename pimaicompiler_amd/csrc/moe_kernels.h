@@ -54,7 +54,7 @@ constexpr int kMoeWaves = kMoeThreads / 64;
 constexpr int kMoeMaxBlocks = 256;
 constexpr int kMoeMaxExperts = 64;
 constexpr int kMoeMaxModel = 2048;                    // d_model: at most four 16-byte pieces of a row per lane
-constexpr int kMoeMaxFf = 4096;                       // d_ff: at most 512 words of eight hidden values, one per thread
+constexpr int kMoeMaxFf = 4096;                       // d_ff: at most 512 words of eight hidden values
 constexpr int kMoeXC = kMoeMaxModel / 8 / 64;         // 16-byte pieces of a W1 row per lane
 constexpr int kMoeFC = kMoeMaxFf / 8 / 64;            // 16-byte pieces of a W2 row per lane
 constexpr int kMoeMaxWordsPerBlock = 2;               // wpb
@@ -62,7 +62,14 @@ constexpr int kMoeMaxRows2 = kMoeWaves;               // W2 rows per block: one 
 constexpr int kMoeEntryWords = 8;                     // 8-byte words per entry (64 bytes); the first 2 * wpb carry values
 constexpr unsigned long long kMoeEmpty = ~0ull;
 constexpr int kMoeCounterStride = 16;                // 32-bit words between the blocks' copies of the launch count: a 64-byte line each
-static_assert(kMoeMaxFf / 8 <= kMoeThreads, "thread t of a block polls word t");
+// Threads [moe_first_poller(rows, words), kMoeThreads) of a block poll up to two words each: the wavefronts without a row of W2, and as
+// many more as two words to a thread need.
+__host__ __device__ constexpr int moe_first_poller(int rows2, int words)
+{
+    const int needed = (words + 127) / 128, without_row = kMoeWaves - rows2;
+    return 64 * (kMoeWaves - (without_row > needed ? without_row : needed));
+}
+static_assert(2 * (kMoeThreads - moe_first_poller(kMoeMaxRows2, kMoeMaxFf / 8)) >= kMoeMaxFf / 8, "every word is polled");
 static_assert(kMoeMaxWordsPerBlock * kMoeMaxBlocks * 8 >= kMoeMaxFf, "every hidden value has a producer");
 static_assert(2 * kMoeMaxWordsPerBlock <= kMoeEntryWords, "a block's words fit its entry");
 
@@ -287,7 +294,7 @@ __global__ __launch_bounds__(kMoeThreads) void moe_ffn_step_f16_kernel(const hal
         report_choice();
         ask_for_w2();
         // ---- everybody's hidden values: word t and word t + n_poll by the threads behind the wavefronts that wait for a row of W2 ----
-        const int poll0 = 64 * min(min(p.rpb2, kMoeWaves), kMoeWaves - (nf + 127) / 128);
+        const int poll0 = moe_first_poller(p.rpb2, nf);
         const int n_poll = kMoeThreads - poll0, t0 = tid - poll0;
         if (t0 >= 0 && t0 < nf) {
             const bool two = t0 + n_poll < nf;

@@ -109,8 +109,10 @@ struct RnntGreedyArgs {
     int* symbols;              // [max_symbols]
     int* result;               // [8]: symbols emitted, frames consumed, steps taken, 1 if one workgroup decoded alone, whether the
                                // last symbol is still to be fed to the prediction network, the last symbol (-1: none), 0, 0
-    unsigned long long* hx;    // [kRnntGreedySets][blocks][kRnntEntryWords], all ones at the start
-    unsigned int* seen;        // [blocks][kRnntSeenStride], zero at the start
+    // Entries of kRnntEntryWords words, all ones at the start: h [kRnntGreedyVersions][the layers' blocks], hidden vectors
+    // [kRnntGreedyRing][joint blocks], logits [kRnntGreedyLogitRing][symbol blocks of one team] (h_entry, hid_entry, lg_entry).
+    unsigned long long* hx;
+    unsigned int* seen;        // [gridDim.x][kRnntSeenStride], the blocks of all teams, zero at the start
     unsigned int* solo_owner;  // zero at the start
     unsigned int* abort_flag;
     unsigned int* abort_host;
