@@ -31,10 +31,10 @@
 //   * the joint blocks publish the step that everybody waits for alone and then four steps behind each barrier.
 //
 // Measured on MI355X (one team and two steps a publish before; us per blank / per symbol / an utterance of 341 frames and 121
-// symbols, 2 x 320 units, 512 joint units, 29 symbols): 1.42 / 6.8 / 1395 before, 0.81 / 7.05 / 1056 now; 200 frames and 33 symbols
-// of a 400-word vocabulary (2 x 256 units) 881 -> 450 us.  What bounds it now: a symbol's four hand-overs of 1.0 - 1.3 us, which
-// the traffic of the steps published ahead made 0.1 us longer each, and in a run of blanks the eight steps ahead over the two
-// hand-overs and three roles' rounds that they travel (12 steps ahead: 5 % less per blank, and 2 % more with one layer).
+// symbols, 2 x 320 units, 512 joint units, 29 symbols): 1.42 / 6.8 - 6.9 / 1405 before, 0.80 / 6.8 - 7.05 (by machine) / 1054 now;
+// 200 frames and 33 symbols of a 400-word vocabulary (2 x 256 units) 881 -> 447 us.  What bounds it now: a symbol's four hand-overs of
+// 1.0 - 1.3 us, and in a run of blanks the eight steps ahead over the two hand-overs and three roles' rounds that they
+// travel (12 steps ahead: 5 % less per blank, and 2 % more with one layer).
 //
 // Exchange: 8-byte words of three fp16 values and a 16-bit tag, three words per producing block in a 128-byte entry of its
 // own, written and read with device-scope accesses.  The tag says what the word belongs to: h of a layer carries the

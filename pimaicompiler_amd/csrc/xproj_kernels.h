@@ -360,8 +360,9 @@ __global__ __launch_bounds__(64 * KS) void input_projection_packed_f16_kernel(co
 // wavefronts per SIMD, and a chain of sums half as long): 4 + MT fragments read for 4 * MT matrix instructions.
 //   - Loads go from memory straight into LDS, four slabs deep, and are counted, not drained (vmcnt): a slab has the time of two
 //     others to arrive.  Staged through registers one slab ahead (two blocks per CU) a slab took 1.0 us, this way 0.53.
-//   - The fragments of the next slab are read while this one is multiplied: 0.43 us.  What is left is LDS (64 KB read and 32 KB
-//     written per slab and CU) and the 0.21 us of matrix instructions taking turns within a barrier's reach.
+//   - The fragments of the next slab are asked for while this one is multiplied: 0.43 us.  What is left is the 0.21 us of matrix
+//     instructions and the latency of the reads: nothing holds their order, and as compiled most of a slab's products stand in front of
+//     the next slab's reads (matrix cores busy 30 %, LDS reads 18 % of a busy CU's time).
 //   - An LDS row is 128 bytes, its 16-byte piece c in place c ^ (row & 7), so that eight rows of one piece fall on all banks.  The
 //     weights are the first operand: a lane's four results are neighbours in a row of out (one 16-byte store).
 //   - PACKED: the weights' fragments (pack_w_fragments_kernel) pass through LDS as they are; the same products in the same order.
