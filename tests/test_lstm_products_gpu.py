@@ -93,11 +93,14 @@ def test_waits_that_give_up_and_nans_in_both_kinds(ops, H, T, layers, bidir, res
     args = (x.reshape(T, H).to(DEV), h0.to(DEV), c0.to(DEV))
     want = plan.forward(*args)
     plan.set_spin_limit(0)
-    got = plan.forward(*args)                              # every workgroup makes its units by itself
-    plan.status()
-    assert plan.fallbacks()[0] >= 1
-    for a, b in zip(got, want):
-        assert float((a.float() - b.float()).abs().max()) <= 2e-3
+    for _ in range(20):                                    # (two directions of 256: in a forward of 20 every first look finds its word)
+        got = plan.forward(*args)
+        plan.status()
+        for a, b in zip(got, want):                        # right whether or not a wait gave up in it
+            assert float((a.float() - b.float()).abs().max()) <= 2e-3
+        if plan.fallbacks()[0]:
+            break                                          # every workgroup made its units by itself
+    assert plan.fallbacks()[0] == 1
     plan.set_spin_limit(1 << 22)
     again = plan.forward(*args)
     assert all(torch.equal(a, b) for a, b in zip(again, want))
