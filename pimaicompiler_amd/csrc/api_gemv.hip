@@ -479,7 +479,7 @@ void launch_group(int count, void* const* outs, const void* const* ins, const vo
         const int rows_per_block = gemv_group_rows_per_block((int)in_ws[i]);
         blocks += ((int)out_ws[i] + rows_per_block - 1) / rows_per_block;
     }
-    g.count = count;
+    for (int i = count; i < MAX; ++i) g.block_begin[i] = INT32_MAX;
     launch_kernel(weight_bytes <= kKeepCachedBytes ? gemv_mv_f16_group_kernel<true, MAX> : gemv_mv_f16_group_kernel<false, MAX>,
                   dim3((unsigned)blocks), kGemvGroupThreads, s, g);
 }
@@ -509,7 +509,7 @@ extern "C" int pimhip_execute_gemv_group(int count, void* const* outs, const voi
             const int a = acts ? acts[i] : PIMHIP_ACT_NONE;
             if (a != PIMHIP_ACT_NONE && a != PIMHIP_ACT_RELU) return fail(PIMHIP_ERR_INVALID_ARGUMENT, "entry %d: unknown activation %d", i, a);
         }
-        (n <= 4 ? launch_group<4> : n <= 8 ? launch_group<8> : launch_group<kGemvGroupMax>)(
+        (n <= 4 ? launch_group<4> : n <= 8 ? launch_group<8> : n <= 16 ? launch_group<16> : launch_group<kGemvGroupMax>)(
             n, outs + done, ins + done, weights + done, biases ? biases + done : nullptr, in_ws + done, out_ws + done, acts ? acts + done : nullptr, s);
         PIMHIP_HIP_CHECK(hipGetLastError());
         done += n;

@@ -1,4 +1,4 @@
-"""execute_gemv_group at the counts where the size of a launch's arguments changes (4, 8, 32 products) and beyond one launch, with
+"""execute_gemv_group at the counts where the size of a launch's arguments changes (4, 8, 16, 32 products) and beyond one launch, with
 activations and biases that differ from product to product.  A row of the sums is fp32, the result one rounding to fp16: against the
 product in 64 bits at most half a unit in the last place (2^-11 relative) plus the sums' own error, below 1e-4 at 264 columns of
 products of at most 1."""
@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("count", [1, 4, 5, 8, 9, 32, 33, 64])
+@pytest.mark.parametrize("count", [1, 4, 5, 8, 9, 16, 17, 32, 33, 64])
 def test_every_product_of_a_group_is_its_own(ops, count):
     g = torch.Generator().manual_seed(count)
     xs = [(torch.rand(1, 264, generator=g) * 2 - 1).half() for _ in range(count)]
