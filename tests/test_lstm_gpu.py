@@ -481,12 +481,14 @@ def test_a_forward_whose_waits_give_up_still_gives_the_right_result(ops, mode, l
     assert plan.fallbacks() == (0, True)
     plan.set_spin_limit(0)
     events = 0
-    for _ in range(5):
+    for i in range(50):
         check()                               # right whether or not a wait gave up in it
         now, exchanging = plan.fallbacks()
         assert now >= events and exchanging == (now < 3)
         events = now
-    assert events >= 3                        # some first look fails in every such forward
+        if events >= 3 and i >= 4:
+            break
+    assert events >= 3                        # (some first look fails in nearly every such forward, in two of three with one layer per XCD)
     plan.set_spin_limit(1 << 22)
     check()
     assert plan.fallbacks() == (events, False)   # one launch per step: nothing waits any more
