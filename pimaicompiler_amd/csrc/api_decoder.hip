@@ -113,7 +113,8 @@ extern "C" int pimhip_decoder_plan_create(PimHipDecoderPlan** plan_out, const vo
     if (classifier_w && !aligned16(classifier_w)) return fail(PIMHIP_ERR_UNSUPPORTED, "the classifier weight is not 16-byte aligned");
 
     const int blocks = (int)((H + kDecUnits - 1) / kDecUnits);
-    for (auto kernel : {decoder_step_f16_kernel<kDecMaxLayers, true, true>, decoder_step_f16_kernel<kDecMaxLayers, true, false>}) {
+    for (auto kernel : {decoder_step_f16_kernel<kDecMaxLayers, true, true, true>, decoder_step_f16_kernel<kDecMaxLayers, true, false, true>,
+                        decoder_step_f16_kernel<kDecMaxLayers, true, true, false>}) {
         int per_cu = 0;
         PIMHIP_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kDecThreads, 0));
         if ((int64_t)per_cu * st->num_cus < blocks)
@@ -351,11 +352,12 @@ extern "C" int pimhip_decoder_step(PimHipDecoderPlan* plan, const void* x, const
         if (rc != PIMHIP_OK) return rc;
     }
     const dim3 grid(plan->blocks), block(kDecThreads);
-    const bool keep = dec_rows_stay(L, H, plan->input_size, L - 1 + plan->first_takes_context, ctx_in != nullptr, plan->enc_len, plan->vocab);
+    const DecPlain plain = dec_plain_loads(L, H, plan->input_size, L - 1 + plan->first_takes_context, ctx_in != nullptr, plan->enc_len, plan->vocab);
     auto launch = [&](auto layers) {
         constexpr int kL = decltype(layers)::value;
-        auto kernel = plan->cls_w ? (keep ? decoder_step_f16_kernel<kL, true, true> : decoder_step_f16_kernel<kL, true, false>)
-                                  : (keep ? decoder_step_f16_kernel<kL, false, true> : decoder_step_f16_kernel<kL, false, false>);
+        auto kernel = !plan->cls_w          ? (plain.layers ? decoder_step_f16_kernel<kL, false, true, true> : decoder_step_f16_kernel<kL, false, false, true>)
+                      : !plain.classifier ? decoder_step_f16_kernel<kL, true, true, false>
+                                          : (plain.layers ? decoder_step_f16_kernel<kL, true, true, true> : decoder_step_f16_kernel<kL, true, false, true>);
         kernel<<<grid, block, 0, s>>>(a);
     };
     switch (L) {

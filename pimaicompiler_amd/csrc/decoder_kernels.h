@@ -283,8 +283,8 @@ __device__ constexpr int cls_groups_after(int k)
     return k <= 2 ? 1 : 0;
 }
 
-// KEEP: how the layers' rows are read (load_weight; dec_rows_stay chooses); classifier rows are read with plain loads.
-template <int L, bool CLS, bool KEEP>
+// KEEP, CLS_KEEP: how the layers' rows and the classifier's are read (load_weight; dec_plain_loads chooses).
+template <int L, bool CLS, bool KEEP, bool CLS_KEEP>
 __global__ __launch_bounds__(kDecThreads) void decoder_step_f16_kernel(DecoderStepArgs p)
 {
     static_assert(L >= 1 && L <= kDecMaxLayers, "layers per step");
@@ -387,7 +387,7 @@ __global__ __launch_bounds__(kDecThreads) void decoder_step_f16_kernel(DecoderSt
                     const long row = min(r0 + v, (long)V - 1);
                     const half8_t* wp = reinterpret_cast<const half8_t*>(p.cls_w + row * H);
 #pragma unroll
-                    for (int c = 0; c < CH; ++c) dst[v][c] = load_weight<true>(wp + min(c * 64 + lane, nchunks - 1));
+                    for (int c = 0; c < CH; ++c) dst[v][c] = load_weight<CLS_KEEP>(wp + min(c * 64 + lane, nchunks - 1));
                 }
             }
         };

@@ -65,3 +65,36 @@ def test_a_wide_first_layer_past_the_caches(ops, vocab):
         bound = 4 * off + 2.0 ** -20   # c collects three gates' errors, h one more; the activations are a few ulps of fp32 off
         assert float((cn.double() - want_c).abs().max()) <= bound + 2.0 ** -11 * float(want_c.abs().max())
         assert float((hn.double() - want).abs().max()) <= bound + 2.0 ** -12
+
+
+@pytest.mark.parametrize("L,vocabs", [(1, (8000, 13000, 20000, 40000)), (2, (1000, 13000)), (3, (0, 1000)), (4, (1000, 9000, 40000))])
+def test_every_way_to_read_the_rows_gives_the_same_bits(ops, L, vocabs):
+    """1024 units with all rows plain, the layers' or the classifier's past the L2s, and all plain again (dec_plain_loads): the same state, and
+    the same logits of the rows they share."""
+    H = 1024
+    g = torch.Generator(device=DEV).manual_seed(7 + L)
+    rnd = lambda *shape: ((2 * torch.rand(*shape, generator=g, device=DEV) - 1) / 32).half()  # noqa: E731
+    params = []
+    for l in range(L):
+        params += [rnd(4 * H, H if l == 0 else 2 * H), rnd(4 * H, H), rnd(4 * H), rnd(4 * H)]
+    w, b, enc = rnd(max(vocabs), H), rnd(max(vocabs)), rnd(9, H)
+    x, h, c = rnd(H) * 32, list(rnd(L, H).unbind(0)), list(rnd(L, H).unbind(0))
+    att = torch.softmax(torch.randn(9, generator=g, device=DEV), -1).half()
+    got = []
+    for rows in vocabs:
+        plan = ops.DecoderPlan(params, True, L, first_takes_context=False, classifier=(w[:rows].contiguous(), b[:rows].contiguous()) if rows else None)
+        plan.set_encoder(enc)
+        hn, cn = [torch.empty_like(t) for t in h], [torch.empty_like(t) for t in c]
+        logits = torch.empty(rows, dtype=torch.float16, device=DEV)
+        step = plan.bind(x, h, c, att=att, hn=hn, cn=cn, logits=logits if rows else None)
+        for _ in range(3):
+            step()
+        torch.cuda.synchronize()
+        got.append((hn + cn, logits))
+    for state, logits in got[1:]:
+        assert all(torch.equal(p, q) for p, q in zip(state, got[0][0]))
+        shared = min(len(logits), len(got[0][1]))
+        assert torch.equal(logits[:shared], got[0][1][:shared])
+    top = got[-1][0][L - 1].float()
+    if L < 3:   # (no sums around the top layer: the classifier takes h)
+        assert float((got[-1][1].float() - (w[:len(got[-1][1])].float() @ top + b[:len(got[-1][1])].float())).abs().max()) <= 1e-3
