@@ -22,7 +22,8 @@ struct PimHipRnntPlan {
     unsigned long long* hx = nullptr;      // [2][blocks][kRnntEntryWords], all ones = empty
     unsigned int* g_counter = nullptr;     // [blocks][kRnntCounterStride]
     unsigned int* greedy = nullptr;        // what the loop kernel exchanges through, refilled before every launch of it:
-                                           // entries of kRnntEntryWords 8-byte words (all ones), then
+                                           // entries of kRnntEntryWords 8-byte words and those of every
+                                           // symbol (all ones), then
                                            // seen [greedy_blocks][kRnntSeenStride] and solo_owner (zero)
     int greedy_teams = 1;                  // teams of symbol blocks in the loop kernel
     bool greedy_resident = false;          // all workgroups of the loop kernel fit on the device together
@@ -41,21 +42,26 @@ std::vector<PimHipRnntPlan*> g_rnnt_plans;
 
 constexpr unsigned long long kRnntEventsBeforeAlone = 3;  // waits given up before a plan stops exchanging for good
 
-auto greedy_kernel(int64_t vocab)
+auto greedy_kernel(int64_t vocab, int64_t layers)
 {
+    const bool every = rnnt_greedy_every(vocab, layers);
     switch (rnnt_greedy_lane_words(vocab)) {
-        case 0: return rnnt_greedy_f16_kernel<0>;
-        case 1: return rnnt_greedy_f16_kernel<1>;
-        case 2: return rnnt_greedy_f16_kernel<2>;
-        default: return rnnt_greedy_f16_kernel<kRnntGreedyLaneWords>;
+        case 0: return every ? rnnt_greedy_f16_kernel<0, true> : rnnt_greedy_f16_kernel<0, false>;
+        case 1: return every ? rnnt_greedy_f16_kernel<1, true> : rnnt_greedy_f16_kernel<1, false>;
+        case 2: return rnnt_greedy_f16_kernel<2, false>;
+        default: return rnnt_greedy_f16_kernel<kRnntGreedyLaneWords, false>;
     }
 }
 
 size_t exchange_words32(const PimHipRnntPlan* plan) { return (size_t)2 * plan->blocks * kRnntEntryWords * 2; }
+size_t greedy_every_words32(const PimHipRnntPlan* plan)
+{
+    return rnnt_greedy_every(plan->vocab, plan->num_layers) ? (size_t)kRnntGreedyVersions * (plan->hidden / 8) * rnnt_every_words((int)plan->vocab) * 2 : 0;
+}
 size_t greedy_exchange_words32(const PimHipRnntPlan* plan)
 {
     const size_t n_lstm = (size_t)plan->num_layers * (plan->hidden / 8), n_joint = plan->joint_size / 8, n_vocab = (plan->vocab + 7) / 8;
-    return (kRnntGreedyVersions * n_lstm + kRnntGreedyRing * n_joint + kRnntGreedyLogitRing * n_vocab) * kRnntEntryWords * 2;
+    return (kRnntGreedyVersions * n_lstm + kRnntGreedyRing * n_joint + kRnntGreedyLogitRing * n_vocab) * kRnntEntryWords * 2 + greedy_every_words32(plan);
 }
 // Workgroups of the loop kernel: those of a step, and the symbol blocks once for each further team.
 int greedy_blocks(const PimHipRnntPlan* plan) { return plan->blocks + (plan->greedy_teams - 1) * (int)((plan->vocab + 7) / 8); }
@@ -182,7 +188,7 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
         const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
         plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);
         int greedy_per_cu = 0;
-        RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, greedy_kernel(vocab), kRnntThreads, 0));
+        RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, greedy_kernel(vocab, num_layers), kRnntThreads, 0));
         plan->greedy_resident = (int64_t)greedy_per_cu * st->num_cus >= greedy_blocks(plan);
     }
     RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->greedy), sizeof(unsigned int) * (greedy_exchange_words32(plan) + greedy_count_words32(plan))));
@@ -375,6 +381,7 @@ extern "C" int pimhip_rnnt_greedy_decode(PimHipRnntPlan* plan, const void* enc, 
     a.symbols = symbols;
     a.result = result;
     a.hx = reinterpret_cast<unsigned long long*>(plan->greedy);
+    a.every = a.hx + (greedy_exchange_words32(plan) - greedy_every_words32(plan)) / 2;
     a.seen = plan->greedy + greedy_exchange_words32(plan);
     a.solo_owner = a.seen + (size_t)greedy_blocks(plan) * kRnntSeenStride;
     a.teams = plan->greedy_teams;
@@ -401,7 +408,7 @@ extern "C" int pimhip_rnnt_greedy_decode(PimHipRnntPlan* plan, const void* enc, 
     // fill kernels, not memsets: the call can be recorded into a HIP graph
     launch_fill_u32(plan->greedy, greedy_exchange_words32(plan), ~0u, s);
     launch_fill_u32(plan->greedy + greedy_exchange_words32(plan), greedy_count_words32(plan), 0u, s);
-    greedy_kernel(plan->vocab)<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
+    greedy_kernel(plan->vocab, plan->num_layers)<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
     PIMHIP_HIP_CHECK(hipGetLastError());
     return PIMHIP_OK;
 }

@@ -19,6 +19,10 @@
 //     travels with the hand-over that ends the step and every workgroup keeps the same loop state (t, symbols so far, ..);
 //   * a layer's blocks also collect their own layer's h (what W_hh multiplies at the next symbol) and sum W_hh . h right
 //     then, long before the next symbol is known;
+//   * the first layer does not wait for the decision either (up to kRnntGreedyEveryVocab symbols): its blocks keep the gates' sums over
+//     every symbol's embedding row, make h for every symbol as soon as the h before it is known, a symbol to a lane, and publish them
+//     all; who needs the first layer's h reads the decided symbol's words, which are there already.  A symbol's chain loses a cell (0.7 us) and
+//     the way of a store (0.4 us);
 //   * most steps of a real utterance are blanks, after which only the frame changes: the joint blocks do not wait for the
 //     decision but publish the hidden vectors of the next steps as well, up to eight ahead, as if every decision in
 //     between were a blank (the frames' columns are asked for a round earlier and their sums kept), and the symbol blocks
@@ -38,7 +42,7 @@
 //
 // Exchange: 8-byte words of three fp16 values and a 16-bit tag, three words per producing block in a 128-byte entry of its
 // own, written and read with device-scope accesses.  The tag says what the word belongs to: h of a layer carries the
-// version of g (the count of the prediction network's runs), hidden vectors and logits carry the step and the version they
+// version of g (the count of the prediction network's runs), so do its words for every symbol, in entries of their own; hidden vectors and logits carry the step and the version they
 // were computed under; a word with another tag is "not there yet", so nothing is ever cleared and a stale word cannot be
 // taken for a fresh one.  h lives in four sets by version, hidden vectors in a ring of sixteen by step, logits in one of 64.  A
 // producer may overwrite what is a ring old: for the joint blocks' entries that follows from the order of things
@@ -91,6 +95,15 @@ inline int rnnt_greedy_lane_words(int64_t vocab)
     return blocks <= kRnntGreedyRowVocab ? 0 : (int)((3 * blocks + 63) / 64);
 }
 constexpr int kRnntGreedyEmbHalfs = 16384;         // embedding rows kept in LDS by the first layer's blocks (32 KB)
+// Whether the first layer runs for every symbol ahead of the decision.  It takes the layer's cell and the store's way off a symbol's
+// chain (start -> now, us an utterance; 512 joint units, 200 frames unless said): two layers of 320, 29 symbols, 341 frames with 74 and 114
+// symbols emitted 739 -> 667 and 996 -> 905; 64 symbols 536 -> 491; 100 symbols 533 -> 491 and, with 34 emitted, 395 -> 387.  With one
+// layer the chain is too short for the cells of more than a symbol a lane: 29 symbols 406 -> 377, one layer of 512 and 128
+// symbols 458 -> 449 and, with 27 emitted, 316 -> 325.
+constexpr int kRnntGreedyEveryVocab = 128;
+inline bool rnnt_greedy_every(int64_t vocab, int64_t layers) { return vocab <= (layers == 1 ? 64 : kRnntGreedyEveryVocab); }
+// 8-byte words that a block of the first layer publishes its units' h after every symbol in: three a symbol, whole 128-byte lines.
+__host__ __device__ inline int rnnt_every_words(int vocab) { return (3 * vocab + 15) & ~15; }
 constexpr int kRnntSeenStride = 16;                // 32-bit words between the blocks' `seen` counts
 
 struct RnntGreedyArgs {
@@ -112,6 +125,7 @@ struct RnntGreedyArgs {
     // Entries of kRnntEntryWords words, all ones at the start: h [kRnntGreedyVersions][the layers' blocks], hidden vectors
     // [kRnntGreedyRing][joint blocks], logits [kRnntGreedyLogitRing][symbol blocks of one team] (h_entry, hid_entry, lg_entry).
     unsigned long long* hx;
+    unsigned long long* every; // [kRnntGreedyVersions][blocks of the first layer][rnnt_every_words]: h of the first layer after every symbol (EVERY)
     unsigned int* seen;        // [gridDim.x][kRnntSeenStride], the blocks of all teams, zero at the start
     unsigned int* solo_owner;  // zero at the start
     unsigned int* abort_flag;
@@ -262,16 +276,17 @@ __device__ __forceinline__ void rnnt_greedy_solo(const RnntGreedyArgs& p, half_t
                 const half8_t* in = reinterpret_cast<const half8_t*>(l == 0 ? x : hs + (long)(l - 1) * H);
                 const half8_t* hv = reinterpret_cast<const half8_t*>(hs + (long)l * H);
                 for (int u = wave; u < H; u += kRnntWaves) {
-                    float a[4];
+                    float a[4], ah[4];
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const long r = (long)g * H + u;
-                        a[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_hh + r * H), hv, nhp, lane, 0.0f);
-                        a[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_ih + r * ly.in_w), in, nxp, lane, a[g]);
+                        ah[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_hh + r * H), hv, nhp, lane, 0.0f);
+                        a[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_ih + r * ly.in_w), in, nxp, lane, 0.0f);
                     }
                     float c_new;
                     half_t h_new;
-                    rnnt_unit(a, ly.bsum ? ly.bsum[(long)(lane & 3) * H + u] : 0.0f, (float)cs[(long)l * H + u], lane, c_new, h_new);
+                    const float hidden = rnnt_gate_sum(ah, lane) + (ly.bsum ? ly.bsum[(long)(lane & 3) * H + u] : 0.0f);
+                    rnnt_unit(rnnt_gate_sum(a, lane) + hidden, (float)cs[(long)l * H + u], lane, c_new, h_new);
                     if (lane == 0) {
                         tmp[u] = __builtin_bit_cast(half_t, rnnt_bits((float)h_new));
                         cs[(long)l * H + u] = rnnt_round(c_new);
@@ -322,7 +337,8 @@ __device__ __forceinline__ void rnnt_greedy_solo(const RnntGreedyArgs& p, half_t
 // number of words and nothing else: with three for every vocabulary past 40 symbols and a branch between it and the row's, a
 // transcript of symbols alone took (2 x 320 units, 512 joint units, us a step) 7.29 with 41, 7.54 with 100, 7.58 with 169 and 7.74 with 512
 // symbols, 6.95, 7.21, 7.49 and 7.71 as it is; a run of blanks 1.07, 1.09, 1.11 and 1.28, now 0.94, 0.96, 1.02 and 1.27.
-template <int LANE_WORDS>
+// EVERY: rnnt_greedy_every.
+template <int LANE_WORDS, bool EVERY>
 __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const RnntGreedyArgs p)
 {
     typedef unsigned long long u64;
@@ -331,6 +347,8 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     __shared__ unsigned int keys[2][kRnntGreedyLook];                               // per pass (alternating): the best key of the next steps' logits, 0: not there
     __shared__ __align__(16) half_t emb[kRnntGreedyEmbHalfs];                       // first layer: the embedding rows and x0 behind them
     __shared__ __align__(16) unsigned short mine[2][kRnntGreedyBatch][12];          // this block's eight values (a joint block's of several steps), alternating per publish
+    __shared__ __align__(16) float4_t ih_of[EVERY ? kRnntWaves : 1][EVERY ? kRnntGreedyEveryVocab : 1];  // first layer: a unit's gate sums over every symbol's row
+    __shared__ __align__(16) unsigned short every_mine[EVERY ? kRnntGreedyEveryVocab : 1][12];           // ... and this block's values of h after it
     __shared__ int missing[3][3];                                                   // per pass (rotating): something of the vector is not there yet; a
                                                                                     // wait has given up; something of a second vector is not there
     __shared__ int someone_gave_up;
@@ -353,6 +371,8 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     }
     if (tid < 9) (&missing[0][0])[tid] = 0;
     if (tid < 2 * kRnntGreedyBatch * 12) (&mine[0][0][0])[tid] = 0;
+    if constexpr (EVERY)
+        for (int i = tid; i < kRnntGreedyEveryVocab * 12; i += kRnntThreads) (&every_mine[0][0])[i] = 0;
     __syncthreads();
 
     RnntGreedyState s = {0, 0, 0, -1, p.run_pred_first};
@@ -431,7 +451,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     unsigned int my_key = 0u;
     int n_there = 0;
     constexpr bool row_per_step = LANE_WORDS == 0;
-    auto pass = [&](const u64* vec, int n_vec, unsigned int vec_tag, half_t* vec_dst, bool vec_blocks, int look_waves, bool step_blocks,
+    auto pass = [&](const u64* vec, int n_vec, unsigned int vec_tag, half_t* vec_dst, bool vec_blocks, int look_waves, bool step_blocks, int vec_stride = kRnntEntryWords,
                     const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr) __attribute__((always_inline)) -> int {
         int* miss = missing[n_pass % 3u];
         u64 w;
@@ -447,7 +467,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     const int i2 = second ? i - 3 * n_vec : i;
                     const int prod = i2 / 3, part = i2 - 3 * prod;
                     if (!second) {
-                        if (fetch(vec + (long)prod * kRnntEntryWords + part, vec_tag, vec_blocks, miss, w))
+                        if (fetch(vec + (long)prod * vec_stride + part, vec_tag, vec_blocks, miss, w))
                             unpack(w, vec_dst, prod, part);
                         else
                             miss[0] = 1;
@@ -588,8 +608,8 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         return taken;
     };
     // Waits for a vector.  Returns false when the block has to leave the loop.
-    auto wait_for_vector = [&](const u64* vec, int n_vec, unsigned int tag, half_t* dst) __attribute__((always_inline)) {
-        pass(vec, n_vec, tag, dst, true, 0, false);
+    auto wait_for_vector = [&](const u64* vec, int n_vec, unsigned int tag, half_t* dst, int stride = kRnntEntryWords) __attribute__((always_inline)) {
+        pass(vec, n_vec, tag, dst, true, 0, false, stride);
         return !dead;
     };
     // Waits until the decision of `step` can be taken, and takes those behind it too if their logits are there already.
@@ -599,6 +619,15 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         if (dead) return false;
         take_decisions();
         return true;
+    };
+
+    const int every_words = rnnt_every_words(p.V);
+    auto every_entry = [&](int version, int block) __attribute__((always_inline)) { return p.every + ((long)(version & (kRnntGreedyVersions - 1)) * nwh + block) * every_words; };
+    // Waits for the first layer's h of a version whose symbol has been decided.  With EVERY it was published for all symbols before the
+    // decision (but for a first run with x0): the words of that symbol are picked out.
+    auto wait_for_first_layer = [&](int version, half_t* dst) __attribute__((always_inline)) {
+        if (EVERY && s.label >= 0) return wait_for_vector(every_entry(version, 0) + 3 * s.label, nwh, h_tag(version), dst, every_words);
+        return wait_for_vector(h_entry(version, 0), nwh, h_tag(version), dst);
     };
 
     if (someone_gave_up == 0 && b < n_lstm) {
@@ -640,10 +669,11 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 for (int i = tid; i < nxp; i += kRnntThreads) d8[n8 + i] = x8[i];
         }
         __syncthreads();
-        // W_hh . h of the layer, summed as soon as h is known
-        float a_hh[4];
-        auto sum_hh = [&]() __attribute__((always_inline)) {
-            const half8_t* hv = reinterpret_cast<const half8_t*>(own);
+        // W_hh . h of the layer and the bias, summed as soon as h is known
+        float hidden = 0.0f;
+        auto sum_hh = [&](const half_t* h) __attribute__((always_inline)) {
+            const half8_t* hv = reinterpret_cast<const half8_t*>(h);
+            float a_hh[4];
 #pragma unroll
             for (int gt = 0; gt < 4; ++gt) {
                 a_hh[gt] = 0.0f;
@@ -651,11 +681,118 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 for (int k = 0; k < kRnntHC; ++k)
                     if (lane + 64 * k < nhp) a_hh[gt] = dot8(whh[gt][k], hv[lane + 64 * k], a_hh[gt]);
             }
+            hidden = rnnt_gate_sum(a_hh, lane) + bias;
         };
-        sum_hh();
+        auto sum_ih = [&](const half8_t* in, float (&a)[4]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int gt = 0; gt < 4; ++gt) {
+                a[gt] = 0.0f;
+#pragma unroll
+                for (int k = 0; k < kRnntXC; ++k)
+                    if (lane + 64 * k < nxp) a[gt] = dot8(wih[gt][k], in[lane + 64 * k], a[gt]);
+            }
+        };
+        // The first layer ahead of the decision: W_ih . embedding[k] once for every symbol (four symbols to a fold), then, whenever h is
+        // known, this block's units of the next h after every symbol, a symbol or two to a lane.
+        constexpr int kEach = EVERY ? kRnntGreedyEveryVocab / 64 : 1;
+        half_t c_every[kEach];
+        unsigned short h_every[kEach];
+        auto sum_every_ih = [&]() __attribute__((always_inline)) {
+            const half8_t* rows = p.emb_in_lds ? reinterpret_cast<const half8_t*>(emb) : reinterpret_cast<const half8_t*>(p.embedding);
+            constexpr int kRows = 8;   // asked for together: where they lie in memory the trips there are most of this
+            for (int k0 = 0; k0 < p.V; k0 += kRows) {
+                half8_t in[kRows][kRnntXC];
+#pragma unroll
+                for (int q = 0; q < kRows; ++q) {
+                    const half8_t* row = rows + (long)min(k0 + q, p.V - 1) * nxp;
+#pragma unroll
+                    for (int k = 0; k < kRnntXC; ++k) {
+                        if (64 * k >= nxp) break;
+                        in[q][k] = row[min(lane + 64 * k, nxp - 1)];
+                    }
+                }
+                float x[kRows];
+#pragma unroll
+                for (int q = 0; q < kRows; ++q) {
+                    float a[4];
+#pragma unroll
+                    for (int gt = 0; gt < 4; ++gt) {
+                        a[gt] = 0.0f;
+#pragma unroll
+                        for (int k = 0; k < kRnntXC; ++k)
+                            if (lane + 64 * k < nxp) a[gt] = dot8(wih[gt][k], in[q][k], a[gt]);
+                    }
+                    x[q] = rnnt_fold4(a, lane);
+                }
+#pragma unroll
+                for (int q = 0; q < kRows; q += 4) {
+                    const float sum = rnnt_join32(rnnt_join16(x[q], x[q + 1]), rnnt_join16(x[q + 2], x[q + 3]));
+                    if ((lane & 12) == 0) reinterpret_cast<float*>(&ih_of[wave][k0 + q + (lane >> 4)])[lane & 3] = sum;
+                }
+            }
+        };
+        static_assert(kRnntGreedyEveryVocab % 8 == 0, "eight symbols a round");
+        auto publish_every = [&](int version) __attribute__((always_inline)) {
+            float hidden_of[4];
+#pragma unroll
+            for (int gt = 0; gt < 4; ++gt) hidden_of[gt] = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, hidden), gt));
+            const float c_prev = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, (float)c_half)));
+#pragma unroll
+            for (int n = 0; n < kEach; ++n) {
+                if (64 * n >= p.V) break;
+                const float4_t ih = ih_of[wave][min(lane + 64 * n, p.V - 1)];
+                float act[4];   // as rnnt_unit does it
+#pragma unroll
+                for (int gt = 0; gt < 4; ++gt) {
+                    const float a = ih[gt] + hidden_of[gt];
+                    const float sg = fast_sigmoid_f32(gt == 2 ? 2.0f * a : a);
+                    act[gt] = gt == 2 ? 2.0f * sg - 1.0f : sg;
+                }
+                const float c_new = __builtin_fmaf(act[1], c_prev, act[0] * act[2]);
+                const half_t h_new = rnnt_round(act[3] * (2.0f * fast_sigmoid_f32(2.0f * c_new) - 1.0f));
+                c_every[n] = rnnt_round(c_new);
+                h_every[n] = rnnt_bits((float)h_new);
+                if (lane + 64 * n < p.V) every_mine[lane + 64 * n][wave] = h_every[n];
+            }
+            rnnt_barrier();
+            if (tid < 3 * p.V) {
+                const int k = tid / 3, part = tid - 3 * k;
+                const unsigned short* m = every_mine[k] + 3 * part;
+                const u64 w = (u64)m[0] | ((u64)m[1] << 16) | ((u64)m[2] << 32) | ((u64)h_tag(version) << 48);
+                __hip_atomic_store(every_entry(version, b) + tid, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+        };
+        static_assert(3 * kRnntGreedyEveryVocab <= kRnntThreads, "a thread per word");
+        sum_hh(own);
+        if constexpr (EVERY) {
+            if (l == 0 && !s.run_pred) {  // (a first step with x0 stands in front of the first decision otherwise)
+                sum_every_ih();
+                publish_every(0);
+            }
+        }
         bool ok = true;
         while (ok && running()) {
-            if (s.run_pred) {
+            if (EVERY && l == 0 && s.run_pred && s.label >= 0) {
+                // this version's h is one of those made ahead
+                const int version = n_pred;
+                const int from = s.label & 63;
+                unsigned int c_bits = (unsigned int)__builtin_amdgcn_readlane((int)__builtin_bit_cast(unsigned short, c_every[0]), from);
+                unsigned int h_bits = (unsigned int)__builtin_amdgcn_readlane((int)h_every[0], from);
+                if constexpr (kEach > 1) {
+                    if (s.label >= 64) {
+                        c_bits = (unsigned int)__builtin_amdgcn_readlane((int)__builtin_bit_cast(unsigned short, c_every[kEach - 1]), from);
+                        h_bits = (unsigned int)__builtin_amdgcn_readlane((int)h_every[kEach - 1], from);
+                    }
+                }
+                c_half = __builtin_bit_cast(half_t, (unsigned short)c_bits);
+                h_last = __builtin_bit_cast(half_t, (unsigned short)h_bits);
+                if (!wait_for_first_layer(version, own)) {
+                    ok = false;
+                    break;
+                }
+                sum_hh(own);
+                publish_every(version + 1);
+            } else if (s.run_pred) {
                 const int version = n_pred;
                 const half8_t* in;
                 if (l == 0) {
@@ -663,23 +800,17 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     in = p.emb_in_lds ? reinterpret_cast<const half8_t*>(emb) + (long)row * nxp
                                       : reinterpret_cast<const half8_t*>(s.label < 0 ? p.x0 : p.embedding + (long)s.label * ly.in_w);
                 } else {
-                    if (!wait_for_vector(h_entry(version, (l - 1) * nwh), nwh, h_tag(version), buf0)) {
+                    if (!(l == 1 ? wait_for_first_layer(version, buf0) : wait_for_vector(h_entry(version, (l - 1) * nwh), nwh, h_tag(version), buf0))) {
                         ok = false;
                         break;
                     }
                     in = reinterpret_cast<const half8_t*>(buf0);
                 }
                 float a[4];
-#pragma unroll
-                for (int gt = 0; gt < 4; ++gt) {
-                    a[gt] = a_hh[gt];
-#pragma unroll
-                    for (int k = 0; k < kRnntXC; ++k)
-                        if (lane + 64 * k < nxp) a[gt] = dot8(wih[gt][k], in[lane + 64 * k], a[gt]);
-                }
+                sum_ih(in, a);
                 float c_new;
                 half_t h_new;
-                rnnt_unit(a, bias, (float)c_half, lane, c_new, h_new);
+                rnnt_unit(rnnt_gate_sum(a, lane) + hidden, (float)c_half, lane, c_new, h_new);
                 c_half = rnnt_round(c_new);
                 const unsigned short bits = rnnt_bits((float)h_new);
                 h_last = __builtin_bit_cast(half_t, bits);
@@ -692,7 +823,13 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     ok = false;
                     break;
                 }
-                sum_hh();
+                sum_hh(own);
+                if constexpr (EVERY) {
+                    if (l == 0) {  // (the first run, with x0)
+                        sum_every_ih();
+                        publish_every(version + 1);
+                    }
+                }
             }
             ok = wait_for_decisions();
         }
@@ -780,6 +917,13 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         };
         int have_g = -1;          // the version of g in `own`
         int pub = 0;              // the next step to publish a hidden vector for
+        half8_t gk[kRnntHC];      // this lane's pieces of g
+        auto take_g = [&](const half_t* g) __attribute__((always_inline)) {
+            const half8_t* gv = reinterpret_cast<const half8_t*>(g);
+#pragma unroll
+            for (int k = 0; k < kRnntHC; ++k) gk[k] = gv[min(lane + 64 * k, nhp - 1)];
+        };
+        take_g(own);
         ask();
         keep();
         bool ok = true;
@@ -788,19 +932,16 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             const int end = min(step + kRnntGreedyAhead + 1, step + (p.T - s.t));
             while (af_hi < s.t + (end - step)) frame_keep(sum_f(af_hi));  // (what was not asked for in time)
             if (version != have_g) {
-                if (!wait_for_vector(h_entry(version, (p.L - 1) * nwh), nwh, h_tag(version), own)) {
+                if (!(p.L == 1 ? wait_for_first_layer(version, own) : wait_for_vector(h_entry(version, (p.L - 1) * nwh), nwh, h_tag(version), own))) {
                     ok = false;
                     break;
                 }
+                take_g(own);
                 have_g = version;
                 pub = step;
             }
             if (pub < step) pub = step;
             // the current step and up to kRnntGreedyAhead behind it: the first alone behind its barrier, then batches
-            const half8_t* gv = reinterpret_cast<const half8_t*>(own);
-            half8_t gk[kRnntHC];
-#pragma unroll
-            for (int k = 0; k < kRnntHC; ++k) gk[k] = gv[min(lane + 64 * k, nhp - 1)];
             auto publish_some = [&](auto how_many, int n) __attribute__((always_inline)) {
                 constexpr int kB = decltype(how_many)::value;
                 float a[kB];
@@ -868,7 +1009,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             // and the team's next one is taken along (to the LDS that the first layer's blocks use for the embedding rows)
             const int pub2 = pub + p.teams;
             const bool want2 = want && frame + p.teams < p.T && pub2 <= step + kRnntGreedyAhead && pub2 - kRnntGreedyLogitRing < min_seen;
-            const int r = pass(hid_entry(pub, 0), want ? nwj : 0, step_tag(pub, version), buf0, pub == step, kRnntWaves - 6, false,
+            const int r = pass(hid_entry(pub, 0), want ? nwj : 0, step_tag(pub, version), buf0, pub == step, kRnntWaves - 6, false, kRnntEntryWords,
                                hid_entry(pub2, 0), want2 ? nwj : 0, step_tag(pub2, version), emb);
             if (dead) {
                 ok = false;

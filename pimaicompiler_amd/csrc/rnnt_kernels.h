@@ -28,7 +28,7 @@
 // the joint network reads g = h_prev of the last layer where it lies.
 //
 // Sums run in one fixed order whoever computes them (per row: lane c takes 16-byte pieces c, c + 64, .. in ascending
-// order, the hidden-state columns before the input columns, f before g; then one reduction tree), so a vector that a
+// order, f before g, then one reduction tree; a cell's rows over the hidden state and over the input each by themselves), so a vector that a
 // workgroup had to make for itself has the bits it would have had from its producers.
 //
 // A wait that gives up does not leave the result undefined.  Every wait is bounded (`spin_limit` polls, one second); a block
@@ -163,19 +163,47 @@ __device__ __forceinline__ float rnnt_sum(float v)
     return rnnt_sum_mod4(v);
 }
 
-// One hidden unit's step from this lane's partial sums of its four gate rows (i, f, g, o).  The four sums are folded
-// into one reduction (after two halving exchanges lane l holds gate l & 3 summed over its quad), lanes 0..3 of every quad
-// activate one gate each (sigmoid and tanh(a) = 2 sigmoid(2a) - 1 on the hardware exp2 and reciprocal: absolute error
-// below 1e-6), quad broadcasts hand the four gates to everybody.  Every lane returns the same c_new, h_new.  `bias` is
-// the bias of gate lane & 3; c_prev the same in every lane.
-__device__ __forceinline__ void rnnt_unit(const float acc[4], float bias, float c_prev, int lane, float& c_new, half_t& h_new)
+// Four values per lane to one: lane l gets value l & 3 summed over its row of 16 lanes, in the order of rnnt_sum (two halving
+// exchanges leave value l & 3 in lane l, summed over its quad, then row rotations).
+__device__ __forceinline__ float rnnt_fold4(const float (&v)[4], int lane)
 {
     const bool b0 = lane & 1, b1 = lane & 2;
-    const float s0 = acc[0], s1 = acc[2], s2 = acc[1], s3 = acc[3];  // slots {i, g, f, o}
-    const float a0 = (b0 ? s2 : s0) + rnnt_dpp<kDppQuadXor1>(b0 ? s0 : s2);
-    const float a1 = (b0 ? s3 : s1) + rnnt_dpp<kDppQuadXor1>(b0 ? s1 : s3);
+    const float a0 = (b0 ? v[1] : v[0]) + rnnt_dpp<kDppQuadXor1>(b0 ? v[0] : v[1]);
+    const float a1 = (b0 ? v[3] : v[2]) + rnnt_dpp<kDppQuadXor1>(b0 ? v[2] : v[3]);
     float a = (b1 ? a1 : a0) + rnnt_dpp<kDppQuadXor2>(b1 ? a0 : a1);
-    a = rnnt_sum_mod4(a) + bias;
+    a += rnnt_dpp<0x124>(a);  // row_ror:4
+    return a + rnnt_dpp<0x128>(a);  // row_ror:8
+}
+
+// Rows 0 and 2 of 16 lanes get x summed over rows 0 and 1, 2 and 3; rows 1 and 3 get y.
+__device__ __forceinline__ float rnnt_join16(float x, float y)
+{
+    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+    return x + y;
+}
+
+// The lower 32 lanes get the sum of x's halves, the upper ones y's.
+__device__ __forceinline__ float rnnt_join32(float x, float y)
+{
+    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(x), "+v"(y));
+    return x + y;
+}
+
+// This lane's partial sums of a hidden unit's four gate rows (i, f, g, o) to the sum of gate lane & 3.
+__device__ __forceinline__ float rnnt_gate_sum(const float (&acc)[4], int lane)
+{
+    const float a = rnnt_fold4(acc, lane);
+    const float b = rnnt_join16(a, a);
+    return rnnt_join32(b, b);
+}
+
+// One hidden unit's step from the sums of its gates, bias included: lane l has gate l & 3.  Lanes 0..3 of every quad
+// activate one gate each (sigmoid and tanh(a) = 2 sigmoid(2a) - 1 on the hardware exp2 and reciprocal: absolute error
+// below 1e-6), quad broadcasts hand the four gates to everybody.  Every lane returns the same c_new, h_new; c_prev is
+// the same in every lane.  The gates' sums over the hidden state and over the input are made apart (the first is known long before
+// the second; the loop kernel makes the second for every symbol) and added as input + (hidden + bias).
+__device__ __forceinline__ void rnnt_unit(float a, float c_prev, int lane, float& c_new, half_t& h_new)
+{
     const bool is_g = (lane & 3) == 2;
     const float sg = fast_sigmoid_f32(is_g ? 2.0f * a : a);
     const float act = is_g ? 2.0f * sg - 1.0f : sg;
@@ -204,16 +232,17 @@ __device__ __forceinline__ const half_t* rnnt_solo(const RnntStepIo& io, const R
             const half8_t* in = reinterpret_cast<const half8_t*>(l == 0 ? io.x : cur);
             const half8_t* hv = reinterpret_cast<const half8_t*>(io.h_prev + (long)l * H);
             for (int u = wave; u < H; u += kRnntWaves) {
-                float a[4];
+                float a[4], ah[4];
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
                     const long r = (long)g * H + u;
-                    a[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_hh + r * H), hv, nhp, lane, 0.0f);
-                    a[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_ih + r * ly.in_w), in, nxp, lane, a[g]);
+                    ah[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_hh + r * H), hv, nhp, lane, 0.0f);
+                    a[g] = rnnt_row_dot(reinterpret_cast<const half8_t*>(ly.w_ih + r * ly.in_w), in, nxp, lane, 0.0f);
                 }
                 float c_new;
                 half_t h_new;
-                rnnt_unit(a, ly.bsum ? ly.bsum[(long)(lane & 3) * H + u] : 0.0f, (float)io.c_prev[(long)l * H + u], lane, c_new, h_new);
+                const float hidden = rnnt_gate_sum(ah, lane) + (ly.bsum ? ly.bsum[(long)(lane & 3) * H + u] : 0.0f);
+                rnnt_unit(rnnt_gate_sum(a, lane) + hidden, (float)io.c_prev[(long)l * H + u], lane, c_new, h_new);
                 if (lane == 0) nxt[u] = __builtin_bit_cast(half_t, rnnt_bits((float)h_new));
             }
             __syncthreads();
@@ -380,6 +409,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_step_f16_kernel(const half_
             for (int k = 0; k < kRnntHC; ++k)
                 if (lane + 64 * k < nhp) a[gt] = dot8(whh[gt][k], hv[k], a[gt]);
         }
+        const float hidden = rnnt_gate_sum(a, lane) + bias;
         const unsigned int set = g & 1u;
         if (l > 0) {
             const half8_t* in = reinterpret_cast<const half8_t*>(vector_of(l - 1, (l - 1) * nwh, nwh, set));
@@ -388,13 +418,14 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_step_f16_kernel(const half_
         }
 #pragma unroll
         for (int gt = 0; gt < 4; ++gt) {
+            a[gt] = 0.0f;
 #pragma unroll
             for (int k = 0; k < kRnntXC; ++k)
                 if (lane + 64 * k < nxp) a[gt] = dot8(wih[gt][k], xin[k], a[gt]);
         }
         float c_new;
         half_t h_new;
-        rnnt_unit(a, bias, c_prev, lane, c_new, h_new);
+        rnnt_unit(rnnt_gate_sum(a, lane) + hidden, c_prev, lane, c_new, h_new);
         if (lane == 0) mine[wave] = rnnt_bits((float)h_new);
         publish(set);
         if (lane == 0) {  // (behind the word the next role waits for)

@@ -1,0 +1,28 @@
+"""The greedy decoding loop where its first layer runs for every symbol ahead of the decision: vocabularies on both sides of the rule
+(64 symbols with one layer, 128 with more) and of a lane's symbols, odd and single ones, embedding rows of one and two pieces a lane in LDS
+and in memory, a first step with and without the prediction network.  Against the loop of single steps: same bits."""
+import pytest
+import torch
+
+from test_rnnt_gpu import DEV, dev
+from test_rnnt_greedy_gpu import check, loop_driven_from_the_host, model
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("run_prediction_first", [True, False])
+@pytest.mark.parametrize("L,I,H,V", [
+    (1, 64, 32, 1), (1, 64, 64, 2), (1, 320, 72, 64), (1, 320, 72, 65),
+    (2, 64, 64, 63), (2, 520, 64, 29), (2, 1024, 72, 64), (2, 64, 136, 65), (2, 320, 320, 127), (2, 320, 64, 128), (2, 64, 64, 129),
+    (3, 64, 64, 29), (4, 72, 64, 100),
+])
+def test_the_first_layer_ahead_of_the_decision(ops, L, I, H, V, run_prediction_first):
+    F, J, T, blank = 128, 64, 40, V // 2
+    params, joint, enc, embedding, x0 = model(31 * V + H + L, L, I, H, F, J, V, T, blank, 0.1 if V > 2 else -0.3)
+    plan = ops.RnntPlan(dev(params), True, L, tuple(dev(joint)))
+    g = torch.Generator().manual_seed(V)
+    h0 = (0.3 * torch.randn(L, H, generator=g)).half().to(DEV)
+    c0 = torch.randn(L, H, generator=g).half().to(DEV)
+    want = loop_driven_from_the_host(plan, enc, embedding, x0, blank, 3, 3 * T, h0, c0, run_prediction_first)
+    r = check(plan.greedy_decode(enc, embedding, x0, blank, 3, h0=h0, c0=c0, run_prediction_first=run_prediction_first), want)
+    assert r[3] == 0 and (V == 1 or r[0] > 0)
