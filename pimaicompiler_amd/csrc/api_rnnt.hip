@@ -42,14 +42,19 @@ std::vector<PimHipRnntPlan*> g_rnnt_plans;
 
 constexpr unsigned long long kRnntEventsBeforeAlone = 3;  // waits given up before a plan stops exchanging for good
 
-auto greedy_kernel(int64_t vocab, int64_t layers)
+auto greedy_kernel(int64_t vocab, int64_t layers, int64_t joint)
 {
     const bool every = rnnt_greedy_every(vocab, layers);
+    switch (rnnt_greedy_own_rows(vocab, joint, layers)) {
+        case 4: return joint <= 512 ? rnnt_greedy_f16_kernel<0, true, 4, 1> : rnnt_greedy_f16_kernel<0, true, 4, 2>;
+        case 8: return rnnt_greedy_f16_kernel<1, true, 8, 1>;
+        default: break;
+    }
     switch (rnnt_greedy_lane_words(vocab)) {
-        case 0: return every ? rnnt_greedy_f16_kernel<0, true> : rnnt_greedy_f16_kernel<0, false>;
-        case 1: return every ? rnnt_greedy_f16_kernel<1, true> : rnnt_greedy_f16_kernel<1, false>;
-        case 2: return rnnt_greedy_f16_kernel<2, false>;
-        default: return rnnt_greedy_f16_kernel<kRnntGreedyLaneWords, false>;
+        case 0: return every ? rnnt_greedy_f16_kernel<0, true, 0, 0> : rnnt_greedy_f16_kernel<0, false, 0, 0>;
+        case 1: return every ? rnnt_greedy_f16_kernel<1, true, 0, 0> : rnnt_greedy_f16_kernel<1, false, 0, 0>;
+        case 2: return rnnt_greedy_f16_kernel<2, false, 0, 0>;
+        default: return rnnt_greedy_f16_kernel<kRnntGreedyLaneWords, false, 0, 0>;
     }
 }
 
@@ -188,7 +193,7 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
         const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
         plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);
         int greedy_per_cu = 0;
-        RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, greedy_kernel(vocab, num_layers), kRnntThreads, 0));
+        RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, greedy_kernel(vocab, num_layers, joint_size), kRnntThreads, 0));
         plan->greedy_resident = (int64_t)greedy_per_cu * st->num_cus >= greedy_blocks(plan);
     }
     RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->greedy), sizeof(unsigned int) * (greedy_exchange_words32(plan) + greedy_count_words32(plan))));
@@ -408,7 +413,7 @@ extern "C" int pimhip_rnnt_greedy_decode(PimHipRnntPlan* plan, const void* enc, 
     // fill kernels, not memsets: the call can be recorded into a HIP graph
     launch_fill_u32(plan->greedy, greedy_exchange_words32(plan), ~0u, s);
     launch_fill_u32(plan->greedy + greedy_exchange_words32(plan), greedy_count_words32(plan), 0u, s);
-    greedy_kernel(plan->vocab, plan->num_layers)<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
+    greedy_kernel(plan->vocab, plan->num_layers, plan->joint_size)<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
     PIMHIP_HIP_CHECK(hipGetLastError());
     return PIMHIP_OK;
 }

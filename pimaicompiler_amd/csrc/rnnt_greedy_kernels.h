@@ -32,13 +32,18 @@
 //     publish) takes 2 us however few rows it has, so one set of blocks handles a run of blanks one or two steps a round.  The
 //     CUs that no other role needs hold up to seven further copies of W2's rows, team q takes the steps that are q modulo the
 //     number of teams, and the steps published ahead become logits side by side;
-//   * the joint blocks publish the step that everybody waits for alone and then four steps behind each barrier.
+//   * the joint blocks publish the step that everybody waits for alone and then four steps behind each barrier;
+//   * the decision behind a symbol, which everybody waits for while nothing else is there, is not waited for from the symbol blocks: with
+//     up to 64 symbols the blocks of layers and joint network read the hidden vector and make it themselves (decided_alone).
 //
-// Measured on MI355X (one team and two steps a publish before; us per blank / per symbol / an utterance of 341 frames and 121
-// symbols, 2 x 320 units, 512 joint units, 29 symbols): 1.42 / 6.8 - 6.9 / 1405 before, 0.80 / 6.8 - 7.05 (by machine) / 1054 now;
-// 200 frames and 33 symbols of a 400-word vocabulary (2 x 256 units) 881 -> 447 us.  What bounds it now: a symbol's four hand-overs of
-// 1.0 - 1.3 us, and in a run of blanks the eight steps ahead over the two hand-overs and three roles' rounds that they
-// travel (12 steps ahead: 5 % less per blank, and 2 % more with one layer).
+// Measured on MI355X, us an utterance of 341 frames (2 x 320 units, 512 joint units, 29 symbols) with 74 / 114 symbols emitted: 739 /
+// 996 with a hand-over of the first layer's h and of the logits per symbol, 667 / 905 without the first, 618 / 814 without both;
+// about 0.6 per blank and 5.2 per symbol now.  What bounds it now: of a symbol's 5.2 us two hand-overs of 1.1 and the look at the first
+// layer's words of 0.95, then the cell 0.5, a joint row 0.4, logits and decision 0.9; in a run of blanks the joint blocks' rounds of 2.5 us for
+// four steps (frames' sums 0.4, a batch of four 0.66, asking for frames 0.6, the look and the decisions 0.7).  (12 steps ahead: 5 %
+// less per blank, and 2 % more with one layer.)  Not kept: all logits made by every block, without symbol blocks (a run of blanks
+// 0.6 -> 0.85 us a step, eight steps' logits take every block 1.9 us); the first layer's words of all symbols collected ahead of
+// the decision (28 KB a block and symbol, 2.8 us).
 //
 // Exchange: 8-byte words of three fp16 values and a 16-bit tag, three words per producing block in a 128-byte entry of its
 // own, written and read with device-scope accesses.  The tag says what the word belongs to: h of a layer carries the
@@ -102,6 +107,15 @@ constexpr int kRnntGreedyEmbHalfs = 16384;         // embedding rows kept in LDS
 // symbols 458 -> 449 and, with 27 emitted, 316 -> 325.
 constexpr int kRnntGreedyEveryVocab = 128;
 inline bool rnnt_greedy_every(int64_t vocab, int64_t layers) { return vocab <= (layers == 1 ? 64 : kRnntGreedyEveryVocab); }
+// Rows of W2 that a wavefront of every block holds, for the decision behind a symbol; 0: that decision waits for the symbol blocks.  (us
+// an utterance, without -> with: two layers of 320, 512 joint units, 29 symbols, 341 frames with 74 and 114 symbols emitted 660 -> 618
+// and 905 -> 814, 200 frames with 64 symbols 480 -> 462.  One layer 347 -> 354: there the decision is not what the next symbol waits
+// for.  640 joint units and 64 symbols, 64 more registers: 449 -> 442 with 47 symbols emitted and 283 -> 292 with 20.)
+inline int rnnt_greedy_own_rows(int64_t vocab, int64_t joint, int64_t layers)
+{
+    if (layers < 2) return 0;
+    return vocab <= 32 && joint <= 1024 ? 4 : vocab <= 64 && joint <= 512 ? 8 : 0;
+}
 // 8-byte words that a block of the first layer publishes its units' h after every symbol in: three a symbol, whole 128-byte lines.
 __host__ __device__ inline int rnnt_every_words(int vocab) { return (3 * vocab + 15) & ~15; }
 constexpr int kRnntSeenStride = 16;                // 32-bit words between the blocks' `seen` counts
@@ -228,32 +242,6 @@ __device__ __forceinline__ unsigned int rnnt_max_row(unsigned int v)
     return max(v, rnnt_dpp_u32<0x128>(v));
 }
 
-// rnnt_sum of several values at once, stage by stage, in the same order each.
-template <int N>
-__device__ __forceinline__ void rnnt_sums(float (&v)[N])
-{
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<kDppQuadXor1>(v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<kDppQuadXor2>(v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<0x124>(v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) v[q] += rnnt_dpp<0x128>(v[q]);
-#pragma unroll
-    for (int q = 0; q < N; ++q) {
-        float a = v[q], b = v[q];
-        asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-        v[q] = a + b;
-    }
-#pragma unroll
-    for (int q = 0; q < N; ++q) {
-        float a = v[q], b = v[q];
-        asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1\n\ts_nop 1" : "+v"(a), "+v"(b));
-        v[q] = a + b;
-    }
-}
-
 // The whole loop by one workgroup.  LDS: hs [L * H] (h of every layer), cs [L * H], tmp [max(H, J)], lg [V].
 __device__ __forceinline__ void rnnt_greedy_solo(const RnntGreedyArgs& p, half_t* hs, half_t* cs, half_t* tmp, half_t* lg)
 {
@@ -337,8 +325,8 @@ __device__ __forceinline__ void rnnt_greedy_solo(const RnntGreedyArgs& p, half_t
 // number of words and nothing else: with three for every vocabulary past 40 symbols and a branch between it and the row's, a
 // transcript of symbols alone took (2 x 320 units, 512 joint units, us a step) 7.29 with 41, 7.54 with 100, 7.58 with 169 and 7.74 with 512
 // symbols, 6.95, 7.21, 7.49 and 7.71 as it is; a run of blanks 1.07, 1.09, 1.11 and 1.28, now 0.94, 0.96, 1.02 and 1.27.
-// EVERY: rnnt_greedy_every.
-template <int LANE_WORDS, bool EVERY>
+// EVERY: rnnt_greedy_every.  OWN_ROWS: rnnt_greedy_own_rows, of OWN_PIECES 16-byte pieces a lane (512 joint units each).
+template <int LANE_WORDS, bool EVERY, int OWN_ROWS, int OWN_PIECES>
 __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const RnntGreedyArgs p)
 {
     typedef unsigned long long u64;
@@ -349,6 +337,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     __shared__ __align__(16) unsigned short mine[2][kRnntGreedyBatch][12];          // this block's eight values (a joint block's of several steps), alternating per publish
     __shared__ __align__(16) float4_t ih_of[EVERY ? kRnntWaves : 1][EVERY ? kRnntGreedyEveryVocab : 1];  // first layer: a unit's gate sums over every symbol's row
     __shared__ __align__(16) unsigned short every_mine[EVERY ? kRnntGreedyEveryVocab : 1][12];           // ... and this block's values of h after it
+    __shared__ unsigned int own_keys[OWN_ROWS ? kRnntWaves * OWN_ROWS / 4 : 1];     // the best key among a wavefront's rows of W2
     __shared__ int missing[3][3];                                                   // per pass (rotating): something of the vector is not there yet; a
                                                                                     // wait has given up; something of a second vector is not there
     __shared__ int someone_gave_up;
@@ -407,13 +396,14 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
 
     // One 8-byte word: looked at once, or (blocks) polled until it carries `tag` or the wait's limits are reached, in which
     // case the thread raises the abort words and this pass's "gave up" flag.  Returns whether the tag is there.
-    auto fetch = [&](const u64* slot, unsigned int tag, bool blocks, int* miss, u64& w) __attribute__((always_inline)) {
+    // With `patience` it is polled that many times and then taken as not there.
+    auto fetch = [&](const u64* slot, unsigned int tag, bool blocks, int* miss, u64& w, unsigned int patience = 0u) __attribute__((always_inline)) {
         unsigned int spins = 0;
         unsigned long long first = 0ull;
         while (true) {
             w = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if ((unsigned int)(w >> 48) == tag) return true;
-            if (!blocks) return false;
+            if (!blocks && spins >= patience) return false;
             bool give_up = false;
             if (spins > 0u && (spins & 255u) == 0u) {
                 if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
@@ -452,14 +442,15 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     int n_there = 0;
     constexpr bool row_per_step = LANE_WORDS == 0;
     auto pass = [&](const u64* vec, int n_vec, unsigned int vec_tag, half_t* vec_dst, bool vec_blocks, int look_waves, bool step_blocks, int vec_stride = kRnntEntryWords,
-                    const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr) __attribute__((always_inline)) -> int {
+                    const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr,
+                    unsigned int patience = 0u) __attribute__((always_inline)) -> int {
         int* miss = missing[n_pass % 3u];
         u64 w;
         const int look = kRnntWaves - 1 - wave;
         if (look >= look_waves) {
             if (tid < 384) {
                 // Where a symbol is on its way and this team's hidden vector is not the next one, one word of it is looked at first.
-                const bool there_yet = !s.run_pred || vec_blocks || n_vec == 0 ||
+                const bool there_yet = !s.run_pred || vec_blocks || patience > 0u || n_vec == 0 ||
                                        (unsigned int)(__hip_atomic_load(vec, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 48) == vec_tag;
                 if (!there_yet) miss[0] = miss[2] = 1;
                 for (int i = tid; there_yet && i < 3 * (n_vec + n_vec2); i += 384) {
@@ -467,7 +458,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     const int i2 = second ? i - 3 * n_vec : i;
                     const int prod = i2 / 3, part = i2 - 3 * prod;
                     if (!second) {
-                        if (fetch(vec + (long)prod * vec_stride + part, vec_tag, vec_blocks, miss, w))
+                        if (fetch(vec + (long)prod * vec_stride + part, vec_tag, vec_blocks, miss, w, patience))
                             unpack(w, vec_dst, prod, part);
                         else
                             miss[0] = 1;
@@ -612,9 +603,71 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         pass(vec, n_vec, tag, dst, true, 0, false, stride);
         return !dead;
     };
+    // ---- the decision behind a symbol, by every block of a layer or of the joint network for itself ----
+    // The first decision under a new g is waited for by everybody and nothing else is there yet, so those blocks do not wait for the
+    // symbol blocks' round and the logits' way (1.9 us): they read the hidden vector too, multiply it by W2 (rows wave,
+    // wave + 8, .. in each wavefront's registers) and take the argmax, 1.1 us from the vector's arrival.  The sums are in rnnt_sum's order:
+    // the symbol blocks' logits have the same bits.  The steps ahead come from the symbol blocks: eight steps' logits by every block
+    // would take it 1.9 us a round.
+    constexpr int kSets = OWN_ROWS ? OWN_ROWS / 4 : 1;          // of four rows
+    constexpr int kOwnPieces = OWN_ROWS ? OWN_PIECES : 1;
+    half8_t w2[4 * kSets][kOwnPieces];
+    float own_bias = 0.0f;
+    // Rows of 16 lanes take the sets in turn, the lanes of a quad the rows of a set.
+    const int own_row = kRnntWaves * (4 * ((lane >> 4) & (kSets - 1)) + (lane & 3)) + wave;
+    auto ask_for_w2 = [&]() __attribute__((always_inline)) {
+        if constexpr (OWN_ROWS > 0) {
+#pragma unroll
+            for (int q = 0; q < OWN_ROWS; ++q) {
+                const half8_t* row = reinterpret_cast<const half8_t*>(p.w2 + (long)min(kRnntWaves * q + wave, p.V - 1) * p.J);
+#pragma unroll
+                for (int k = 0; k < kOwnPieces; ++k) w2[q][k] = row[min(lane + 64 * k, nwj - 1)];
+            }
+            own_bias = p.b2 ? (float)p.b2[min(own_row, p.V - 1)] : 0.0f;
+        }
+    };
+    // Takes the decision of `step`.  False where the hidden vector did not come in time: a block that has fallen behind may find the
+    // entry used again (nobody waits for it before that), and the logits, which are kept until everybody has seen them, are there then.
+    auto decided_alone = [&]() __attribute__((always_inline)) {
+        if constexpr (OWN_ROWS > 0) {
+            constexpr unsigned int kPatience = 64u;   // looks, 40 us or more
+            if (!(pass(hid_entry(step, 0), nwj, step_tag(step, g_version()), buf0, false, 0, false, kRnntEntryWords, nullptr, 0, 0u, nullptr, kPatience) & 1) || dead) return false;
+            const half8_t* in = reinterpret_cast<const half8_t*>(buf0);
+            float x[4];
+#pragma unroll
+            for (int set = 0; set < kSets; ++set) {
+                float a[4];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    a[q] = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < kOwnPieces; ++k)
+                        if (lane + 64 * k < nwj) a[q] = dot8(w2[4 * set + q][k], in[lane + 64 * k], a[q]);
+                }
+                x[set] = rnnt_fold4(a, lane);
+            }
+            static_assert(kSets <= 2, "up to 64 symbols");
+            const float pair = rnnt_join16(x[0], x[kSets - 1]);
+            const float sum = rnnt_join32(pair, pair);
+            unsigned int key = rnnt_key(own_row < p.V ? rnnt_bits(sum + own_bias) : (unsigned short)0xfc00u, own_row);   // (-inf past the last symbol)
+            key = max(key, rnnt_dpp_u32<kDppQuadXor1>(key));
+            key = max(key, rnnt_dpp_u32<kDppQuadXor2>(key));
+            // (a row of 16 lanes has its sums in lanes 0 .. 3)
+            if ((lane & 15) == 0 && lane < 16 * kSets) own_keys[wave + kRnntWaves * (lane >> 4)] = key;
+            rnnt_barrier();
+            my_key = rnnt_max_u32(own_keys[lane & (kRnntWaves * kSets - 1)]);
+            n_there = 1;
+            take_decisions();
+            return true;
+        } else {
+            return false;
+        }
+    };
     // Waits until the decision of `step` can be taken, and takes those behind it too if their logits are there already.
     // Returns false when the block has to leave the loop.
     auto wait_for_decisions = [&]() __attribute__((always_inline)) {
+        if (s.run_pred && decided_alone()) return true;
+        if (dead) return false;
         pass(nullptr, 0, 0u, nullptr, false, kRnntWaves, true);
         if (dead) return false;
         take_decisions();
@@ -654,6 +707,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 wih[gt][k] = row[min(lane + 64 * k, nxp - 1)];
             }
         }
+        ask_for_w2();
         const float bias = ly.bsum ? ly.bsum[(long)(lane & 3) * H + u] : 0.0f;
         half_t c_half = p.c0 ? p.c0[(long)l * H + u] : (half_t)0.0f;
         half_t h_last = p.h0 ? p.h0[(long)l * H + u] : (half_t)0.0f;
@@ -697,19 +751,17 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         constexpr int kEach = EVERY ? kRnntGreedyEveryVocab / 64 : 1;
         half_t c_every[kEach];
         unsigned short h_every[kEach];
-        auto sum_every_ih = [&]() __attribute__((always_inline)) {
+        auto sum_every_rows = [&](auto pieces, auto how_many) __attribute__((always_inline)) {
+            constexpr int kP = decltype(pieces)::value, kRows = decltype(how_many)::value;   // rows asked for together: the trips to them are most of this
             const half8_t* rows = p.emb_in_lds ? reinterpret_cast<const half8_t*>(emb) : reinterpret_cast<const half8_t*>(p.embedding);
-            constexpr int kRows = 8;   // asked for together: where they lie in memory the trips there are most of this
+#pragma unroll 1
             for (int k0 = 0; k0 < p.V; k0 += kRows) {
-                half8_t in[kRows][kRnntXC];
+                half8_t in[kRows][kP];
 #pragma unroll
                 for (int q = 0; q < kRows; ++q) {
                     const half8_t* row = rows + (long)min(k0 + q, p.V - 1) * nxp;
 #pragma unroll
-                    for (int k = 0; k < kRnntXC; ++k) {
-                        if (64 * k >= nxp) break;
-                        in[q][k] = row[min(lane + 64 * k, nxp - 1)];
-                    }
+                    for (int k = 0; k < kP; ++k) in[q][k] = row[min(lane + 64 * k, nxp - 1)];
                 }
                 float x[kRows];
 #pragma unroll
@@ -719,7 +771,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     for (int gt = 0; gt < 4; ++gt) {
                         a[gt] = 0.0f;
 #pragma unroll
-                        for (int k = 0; k < kRnntXC; ++k)
+                        for (int k = 0; k < kP; ++k)
                             if (lane + 64 * k < nxp) a[gt] = dot8(wih[gt][k], in[q][k], a[gt]);
                     }
                     x[q] = rnnt_fold4(a, lane);
@@ -730,6 +782,11 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     if ((lane & 12) == 0) reinterpret_cast<float*>(&ih_of[wave][k0 + q + (lane >> 4)])[lane & 3] = sum;
                 }
             }
+        };
+        auto sum_every_ih = [&]() __attribute__((always_inline)) {
+            static_assert(kRnntXC == 2, "rows of one piece to a lane or of two");
+            if (nxp <= 64) sum_every_rows(std::integral_constant<int, 1>{}, std::integral_constant<int, 8>{});
+            else sum_every_rows(std::integral_constant<int, 2>{}, std::integral_constant<int, 4>{});
         };
         static_assert(kRnntGreedyEveryVocab % 8 == 0, "eight symbols a round");
         auto publish_every = [&](int version) __attribute__((always_inline)) {
@@ -854,7 +911,8 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             if (64 * k >= nhp) break;
             wg[k] = row[nfp + min(lane + 64 * k, nhp - 1)];
         }
-        const float bias = (lane == 0 && p.b1) ? (float)p.b1[r] : 0.0f;
+        ask_for_w2();
+        const float bias = p.b1 ? (float)p.b1[r] : 0.0f;
         for (int i = tid; i < H; i += kRnntThreads) own[i] = p.h0 ? p.h0[(long)(p.L - 1) * H + i] : (half_t)0.0f;  // g before the first run
         __syncthreads();
         // this lane's part of the row's sum over a frame (nothing is read for a frame the utterance does not have)
@@ -882,16 +940,23 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         static_assert(16 <= kPieces && kPieces % kRnntFC == 0, "eight frames of two pieces, or four of four");
         const bool short_frames = nfp <= 128;
         half8_t col[kPieces];
+        int piece_at[kRnntFC];
+#pragma unroll
+        for (int k = 0; k < kRnntFC; ++k) piece_at[k] = min(lane + 64 * k, nfp - 1);
         int f_first = 0, n_ask = 0;
         auto ask_frames = [&](auto pieces) __attribute__((always_inline)) {
             constexpr int kP = decltype(pieces)::value;
             f_first = af_hi;
             n_ask = max(0, min(min(kPieces / kP, p.T - f_first), s.t + kRnntGreedyRing - f_first));  // (what the ring still needs stays in it)
+            const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)f_first * p.F);
+#pragma unroll
+            for (int i = 0; i < kPieces; ++i) asm volatile("" : "=v"(col[i]));  // (a piece not asked for now is not one to keep from before)
 #pragma unroll
             for (int q = 0; q < kPieces / kP; ++q) {
+                if (q >= n_ask) break;
 #pragma unroll
-                for (int k = 0; k < kP; ++k)
-                    col[q * kP + k] = (q < n_ask && lane + 64 * k < nfp) ? reinterpret_cast<const half8_t*>(p.enc + (long)(f_first + q) * p.F)[lane + 64 * k] : wf[k];
+                for (int k = 0; k < kP; ++k) col[q * kP + k] = f8[piece_at[k]];   // (a lane past the frame's end reads its last piece and keeps nothing of it)
+                f8 += nfp;
             }
         };
         auto keep_frames = [&](auto pieces) __attribute__((always_inline)) {
@@ -953,10 +1018,16 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     for (int k = 0; k < kRnntHC; ++k)
                         if (lane + 64 * k < nhp) a[q] = dot8(wg[k], gk[k], a[q]);
                 }
-                rnnt_sums(a);
-#pragma unroll
-                for (int q = 0; q < kB; ++q)
-                    if (lane == 0) my_value(q) = rnnt_bits(relu_f32(a[q] + bias));
+                if constexpr (kB == 1) {
+                    const float sum = rnnt_sum(a[0]);
+                    if (lane == 0) my_value(0) = rnnt_bits(relu_f32(sum + bias));
+                } else {
+                    static_assert(kB == 4, "a batch is folded to one step a lane");
+                    float sum = rnnt_fold4(a, lane);
+                    sum = rnnt_join16(sum, sum);
+                    sum = rnnt_join32(sum, sum);
+                    if (lane < kB) my_value(lane) = rnnt_bits(relu_f32(sum + bias));
+                }
                 rnnt_barrier();
                 if (wave < n) store_words(wave, hid_entry(pub + wave, jb), step_tag(pub + wave, version));
                 ++n_publish;

@@ -26,3 +26,15 @@ def test_the_first_layer_ahead_of_the_decision(ops, L, I, H, V, run_prediction_f
     want = loop_driven_from_the_host(plan, enc, embedding, x0, blank, 3, 3 * T, h0, c0, run_prediction_first)
     r = check(plan.greedy_decode(enc, embedding, x0, blank, 3, h0=h0, c0=c0, run_prediction_first=run_prediction_first), want)
     assert r[3] == 0 and (V == 1 or r[0] > 0)
+
+
+@pytest.mark.parametrize("L,J,V", [(2, 512, 32), (2, 520, 32), (2, 1024, 31), (2, 1032, 29), (2, 512, 33), (2, 8, 40), (2, 512, 64), (3, 504, 41),
+                                   (2, 520, 64), (1, 512, 29)])
+def test_the_decision_behind_a_symbol(ops, L, J, V):
+    """Where every block makes it (four or eight rows of W2 a wavefront, one or two pieces of them a lane) and on the other side of that rule."""
+    I, H, F, T, blank = 64, 64, 128, 40, 0
+    params, joint, enc, embedding, x0 = model(7 * V + J, L, I, H, F, J, V, T, blank, 0.0)
+    plan = ops.RnntPlan(dev(params), True, L, tuple(dev(joint)))
+    want = loop_driven_from_the_host(plan, enc, embedding, x0, blank, 3, 3 * T)
+    r = check(plan.greedy_decode(enc, embedding, x0, blank, 3), want)
+    assert r[3] == 0 and r[0] > 0
