@@ -73,6 +73,15 @@ struct PimHipLstmPlan {
 
 namespace
 {
+// The per-XCD kernels on sparse matrix instructions for a hidden size.
+auto xcd_sparse_kernel(bool pipeline, int64_t hidden)
+{
+    constexpr int kFew = kXcdFewUnits / 64;
+    if (hidden <= kXcdFewUnits) return pipeline ? lstm_xcd_f16_kernel<true, kFew> : lstm_xcd_f16_kernel<false, kFew>;
+    return pipeline ? lstm_xcd_f16_kernel<true, kXcdFrags> : lstm_xcd_f16_kernel<false, kXcdFrags>;
+}
+auto xcd_res_kernel(int64_t hidden) { return hidden <= kXcdFewUnits ? lstm_xcd_res_f16_kernel<kXcdFewUnits / 64> : lstm_xcd_res_f16_kernel<kXcdFrags>; }
+
 constexpr unsigned long long kLstmEventsBeforeSafe = 3;
 }
 
@@ -301,7 +310,7 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
             return e;
         };
         plan->xcd_ok = true;
-        PLAN_HIP_CHECK(resident(pipeline ? lstm_xcd_f16_kernel<true> : lstm_xcd_f16_kernel<false>, &plan->xcd_ok));
+        PLAN_HIP_CHECK(resident(xcd_sparse_kernel(pipeline, hidden_size), &plan->xcd_ok));
         PLAN_HIP_CHECK(resident(pipeline ? lstm_xcd_dot_f16_kernel<true> : lstm_xcd_dot_f16_kernel<false>, &plan->xcd_ok));
         if (plan->xcd_ok) {
             bool rotation = false;
@@ -310,7 +319,7 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
             plan->xcd_ok = rotation;
         }
         plan->xcd_res_ok = plan->xcd_ok && pipeline;
-        if (pipeline) PLAN_HIP_CHECK(resident(lstm_xcd_res_f16_kernel, &plan->xcd_res_ok));
+        if (pipeline) PLAN_HIP_CHECK(resident(xcd_res_kernel(hidden_size), &plan->xcd_res_ok));
     }
     if (plan->xcd_ok) {
         const size_t words = (size_t)kXcdRegionWords * kXcdMaxChains;
@@ -632,7 +641,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             a.H = (int)H;
             a.T = (int)T;
             a.spin_limit = plan->spin_limit;
-            auto kernel = any_res ? lstm_xcd_res_f16_kernel : xcd_on_dot(H, T, n) ? lstm_xcd_dot_f16_kernel<true> : lstm_xcd_f16_kernel<true>;
+            auto kernel = any_res ? xcd_res_kernel(H) : xcd_on_dot(H, T, n) ? lstm_xcd_dot_f16_kernel<true> : xcd_sparse_kernel(true, H);
             kernel<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
             PIMHIP_HIP_CHECK(hipGetLastError());
             layer_in = group_out;
@@ -677,7 +686,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             a.H = (int)H;
             a.T = (int)T;
             a.spin_limit = plan->spin_limit;
-            (xcd_on_dot(H, T, 1) ? lstm_xcd_dot_f16_kernel<false> : lstm_xcd_f16_kernel<false>)<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
+            (xcd_on_dot(H, T, 1) ? lstm_xcd_dot_f16_kernel<false> : xcd_sparse_kernel(false, H))<<<dim3((unsigned)(kXcdCount * members)), dim3(kXcdThreads), 0, s>>>(a);
             if (residual(l)) add_input(layer_out, layer_in);
             PIMHIP_HIP_CHECK(hipGetLastError());
             layer_in = layer_out;

@@ -166,8 +166,13 @@ struct XcdDot {
         __device__ __forceinline__ void clear() {}
     };
 
+    // What is read of h as soon as it is there: nothing (pieces are read as they are used).
+    struct Operands {
+    };
+    static __device__ __forceinline__ Operands operands(const half_t*, int) { return {}; }
+
     // In every lane: the dot product of its unit's gate row gate(lane) with hb[0 .. H).
-    __device__ __forceinline__ float matvec(const half_t* hb, Sums&, int H, int lane) const
+    __device__ __forceinline__ float matvec(const half_t* hb, const Operands&, Sums&, int H, int lane) const
     {
         float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -241,8 +246,14 @@ __device__ __forceinline__ half8_t xcd_h_operand(const half_t* hb, int s, int la
                                    *reinterpret_cast<const half4_t*>(hb + (lo ^ 1) * 8 + 4 * (lane & 1)), 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
+// FRAGS: four (up to 256 units) or sixteen of them.  Four have a kernel of their own: half the sums and no second operand, and with both in one
+// kernel the accumulators were copied on a step's path.
+static constexpr int kXcdFewUnits = 256;
+template <int FRAGS>
 struct XcdSparse {
-    half16_t w[kXcdFrags];
+    static_assert(FRAGS == kXcdFewUnits / 64 || FRAGS == kXcdFrags, "up to 256 units, or any number");
+    static constexpr bool kFew = FRAGS < kXcdFrags;
+    half16_t w[FRAGS];
 
     // Lane l holds gate l & 3 of unit (l >> 2) & 3, in all four rows of 16 lanes.
     static __device__ __forceinline__ int unit(int lane) { return (lane >> 2) & 3; }
@@ -261,9 +272,9 @@ struct XcdSparse {
         half8_t zero;
 #pragma unroll
         for (int e = 0; e < 8; ++e) zero[e] = (half_t)0.0f;
-        half8_t raw[kXcdFrags / 2][4];
+        half8_t raw[FRAGS / 2][4];
 #pragma unroll
-        for (int i = 0; i < kXcdFrags / 2; ++i) {
+        for (int i = 0; i < FRAGS / 2; ++i) {
             if (128 * i >= H) break;  // (uniform)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
@@ -273,7 +284,7 @@ struct XcdSparse {
         }
         const int n = lane & 15, g = lane >> 4;
 #pragma unroll
-        for (int i = 0; i < kXcdFrags / 2; ++i) {
+        for (int i = 0; i < FRAGS / 2; ++i) {
             if (128 * i >= H) {  // (uniform) nothing but zeros: 64 KB per CU and i that need not pass through LDS
 #pragma unroll
                 for (int m = 0; m < 2; ++m) w[2 * i + m] = __builtin_shufflevector(zero, zero, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
@@ -297,34 +308,45 @@ struct XcdSparse {
 
     // The accumulators of a step, cleared where the wavefront has nothing else to do (in front of its wait for h).
     struct Sums {
-        float4_t d[8];
+        float4_t d[kFew ? 4 : 8];
         __device__ __forceinline__ void clear()
         {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) {
+            for (int j = 0; j < (kFew ? 4 : 8); ++j) {
                 d[j] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
                 asm volatile("" : "+v"(d[j]));
             }
         }
     };
 
+    // Both register sets of h, asked for together right behind the step's barrier (past the hidden state hb holds zeros).  Asked for
+    // behind the first set's instructions, the second came 100 cycles after the last of them.
+    struct Operands {
+        half8_t h0, h1;
+    };
+    static __device__ __forceinline__ Operands operands(const half_t* hb, int lane)
+    {
+        Operands o;
+        o.h0 = xcd_h_operand(hb, 0, lane);
+        o.h1 = kFew ? o.h0 : xcd_h_operand(hb, 1, lane);
+        return o;
+    }
+
     // In every lane l: the dot product of gate row l & 15 of the wavefront with hb[0 .. H).
-    __device__ __forceinline__ float matvec(const half_t* hb, Sums& acc, int H, int lane) const
+    __device__ __forceinline__ float matvec(const half_t*, const Operands& h, Sums& acc, int H, int lane) const
     {
         const int index = (lane & 1) ? 0xeeeeeeee : 0x44444444;  // columns 2, 3 / 0, 1 of every four
-        const half8_t h0 = xcd_h_operand(hb, 0, lane);
-        if (H <= 256) {  // (uniform) four fragments: half the sums and no second operand; the chain is all a step of few units has
+        if constexpr (kFew) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m) acc.d[m] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(h0, w[m], acc.d[m], index, 0, 0);
+            for (int m = 0; m < 4; ++m) acc.d[m] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(h.h0, w[m], acc.d[m], index, 0, 0);
             const float f0 = (acc.d[0][0] + acc.d[0][1]) + (acc.d[1][2] + acc.d[1][3]);
             const float f1 = (acc.d[2][0] + acc.d[2][1]) + (acc.d[3][2] + acc.d[3][3]);
             return wave_sum_rows((lane & 32) ? 0.0f : (lane & 16) ? f1 : f0);
-        }
-        const half8_t h1 = xcd_h_operand(hb, 1, lane);
+        } else {
 #pragma unroll
-        for (int m = 0; m < kXcdFrags; ++m) {
-            if ((m & 3) == 0 && m * 64 >= H) break;  // (uniform) whole fragments past the hidden state are zeros
-            acc.d[m & 7] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(m < 8 ? h0 : h1, w[m], acc.d[m & 7], index, 0, 0);
+        for (int m = 0; m < FRAGS; ++m) {
+            if (m >= 8 && (m & 3) == 0 && m * 64 >= H) break;  // (uniform) whole fragments past the hidden state are zeros
+            acc.d[m & 7] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(m < 8 ? h.h0 : h.h1, w[m], acc.d[m & 7], index, 0, 0);
         }
         // Row r of D lies in register r & 3 of lanes 16 (r >> 2) .. + 15: row group q keeps pairs 2 q (registers 0, 1) and 2 q + 1.
         float f[4];
@@ -332,6 +354,7 @@ struct XcdSparse {
         for (int q = 0; q < 4; ++q) f[q] = (acc.d[2 * q][0] + acc.d[2 * q][1]) + (acc.d[2 * q + 1][2] + acc.d[2 * q + 1][3]);
         const float lo = (lane & 16) ? f[1] : f[0], hi = (lane & 16) ? f[3] : f[2];
         return wave_sum_rows((lane & 32) ? hi : lo);
+        }
     }
 
     // The activated gates of a unit: the quad's four lanes share them.
@@ -502,7 +525,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
                 lo = __hip_atomic_load(nxt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 hi = __hip_atomic_load(nxt + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            const float v = weights.matvec(hb, acc, H, lane) + bias;
+            const float v = weights.matvec(hb, Product::operands(hb, lane), acc, H, lane) + bias;
             if (dead) return;  // rows made from a stale h must not reach the recurrence: it will make its own
             if (units_ok && Product::first_of_gate(lane))
                 __hip_atomic_store(reinterpret_cast<unsigned int*>(dst + (long)t * 4 * H), __builtin_bit_cast(unsigned int, v), __ATOMIC_RELAXED,
@@ -594,10 +617,24 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         reinterpret_cast<unsigned int&>(xring[wave][1][my_gate][unit]) = wait_xp(min(1, T - 1));
     }
 
+    // Where this wavefront publishes its four values, alternating by the count; what stands between a step's gates and that store is
+    // waited for by the whole group, so nothing of it is computed there.
+    unsigned char* publish_at = reinterpret_cast<unsigned char*>(region + ((long)(g_base & 1u) * kXcdMembers + rank) * kXcdEntryWords) + wave * 8;
+    long publish_step = (g_base & 1u) ? -(long)sizeof(unsigned int) * kXcdMembers * kXcdEntryWords : (long)sizeof(unsigned int) * kXcdMembers * kXcdEntryWords;
+    unsigned int published32 = units_ok ? 0xffffffffu : 0u;
+    asm volatile("" : "+v"(published32));
+    const unsigned long long published = ((unsigned long long)published32 << 32) | published32;
+    const bool publishes = lane == 0;
+    half_t* const y = ch.y;
+    const long y_stride = p.y_stride;
+
     for (int s = 0; s < T; ++s) {
         half_t* hb = hbuf[s & 1];
         typename Product::Sums acc;
         acc.clear();
+        unsigned int flag32 = (((g_base + (unsigned int)s) >> 1) & 1u) ? 0x40004000u : 0u;
+        asm volatile("" : "+v"(flag32));  // (made here, not in front of the store)
+        const unsigned long long flag = ((unsigned long long)flag32 << 32) | flag32;
         if (!polled) {
             // steps s + 16 .. s + 31 are fetched when step s starts a half, and written over the half that has just been
             // used up one step later (this wavefront's poll in between has waited for them)
@@ -635,7 +672,12 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         lds_barrier();
         // (the same value in every thread: it is written in front of barriers only.  Asked for here, with the reads of h,
         // and looked at where values would leave the workgroup: the step's arithmetic does not wait for it)
-        const int dead = __builtin_amdgcn_readfirstlane(block_gave_up);
+        // The operands of the product and the projection terms are asked for here too, in front of everything that is not on
+        // the step's path: the terms behind the sums came an LDS round trip (100 cycles) later.
+        const int dead_lds = block_gave_up;
+        const typename Product::Operands operands = Product::operands(hb, lane);
+        unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][unit]);
+        const int dead = __builtin_amdgcn_readfirstlane(dead_lds);
         if (polled && fetcher && s + 2 < T) {
             xp_ahead = xp_bits_at(s + 2);
             xp_ahead_other = __hip_atomic_load(xp_other + (long)(s + 2) * 4 * H, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -649,10 +691,16 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             if (s > 0 && !dead) emit_sum(s - 1);
         }
 
+        // (a wavefront one of whose waits gave up after this step's barrier makes its h from stale values: it keeps them
+        // to itself, and the group's other members stop at their next wait)
+        bool stop = dead || __builtin_amdgcn_ballot_w64(gave_up) != 0ull;
+
         // ---- 2. the wavefront's 16 gate rows
-        const float dot = weights.matvec(hb, acc, H, lane);
-        unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][unit]);
-        if (polled && xp_bits == 0xffffffffu) xp_bits = wait_xp(s);  // the P group had not got there when it was fetched
+        const float dot = weights.matvec(hb, operands, acc, H, lane);
+        if (polled && __builtin_amdgcn_ballot_w64(xp_bits == 0xffffffffu) != 0ull) {  // the P group had not got there when it was fetched
+            if (xp_bits == 0xffffffffu) xp_bits = wait_xp(s);
+            stop = stop || __builtin_amdgcn_ballot_w64(gave_up) != 0ull;
+        }
         const float a = dot + __builtin_bit_cast(float, xp_bits);
         const int t = rev ? (T - 1 - s) : s;
 
@@ -667,23 +715,20 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         const half_t h = (half_t)(g_o * (2.0f * fast_sigmoid_f32(2.0f * c_new) - 1.0f));
         c_reg = c_new;
 
-        // ---- 3. the wavefront's four h values: lane 0 stores y and publishes
+        // ---- 3. the wavefront's four h values: lane 0 publishes, then stores y (whose place in front of the publishing store
+        // nothing may take: everybody waits for that one)
         const unsigned int hb16 = (unsigned int)__builtin_bit_cast(unsigned short, h);
         const unsigned int pb16 = h_is_number ? hb16 : 0u;       // a NaN cannot carry the flag: it is exchanged as 0, y keeps it
         const unsigned int sb16 = h_is_number ? hb16 : 0x7e00u;  // and goes to the layer above in its canonical form
         const unsigned long long pw = Product::pack(pb16);
+        // units past H publish zeros with the flag, so that every piece of a member's entry validates
+        if (publishes && !stop) store8_plain(publish_at, (pw & published) | flag);
+        publish_at += publish_step;
+        publish_step = -publish_step;
         const unsigned long long yw = Product::pack(hb16);
         const unsigned long long sw = emits ? Product::pack(sb16) : 0ull;
-        // (a wavefront one of whose waits gave up after this step's barrier has made its h from stale values: it keeps them
-        // to itself, and the group's other members stop at their next wait)
-        const bool wave_gave_up = __builtin_amdgcn_ballot_w64(gave_up) != 0ull;
         if (lane == 0) {
-            const unsigned int g = g_base + (unsigned int)s;
-            const unsigned long long flag = ((g >> 1) & 1u) ? 0x4000400040004000ull : 0ull;
-            // units past H publish zeros with the flag, so that every piece of a member's entry validates
-            unsigned char* dst = reinterpret_cast<unsigned char*>(region + ((long)(g & 1u) * kXcdMembers + rank) * kXcdEntryWords) + wave * 8;
-            if (!wave_gave_up && !dead) store8_plain(dst, (units_ok ? pw : 0ull) | flag);
-            if (!res && units_ok && ch.y) *reinterpret_cast<unsigned long long*>(ch.y + (long)t * p.y_stride + u0) = yw;
+            if (!res && units_ok && y) *reinterpret_cast<unsigned long long*>(y + (long)t * y_stride + u0) = yw;
             if (emits) hout[s & 1][wave] = sw;
         }
         if (s == T - 1 && units_ok && Product::first_of_unit(lane)) {
@@ -755,10 +800,11 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         __hip_atomic_store(p.g_counter + k, g_base + (unsigned int)T, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <bool PIPE>
+// FRAGS: four up to kXcdFewUnits, otherwise sixteen.
+template <bool PIPE, int FRAGS>
 __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_f16_kernel(LstmXcdArgs p)
 {
-    lstm_xcd_body<PIPE, false, XcdSparse>(p);
+    lstm_xcd_body<PIPE, false, XcdSparse<FRAGS>>(p);
 }
 
 template <bool PIPE>
@@ -768,9 +814,10 @@ __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_dot_f16_kernel(LstmXcdAr
 }
 
 // The pipeline for stacks that have layers with a residual sum.
+template <int FRAGS>
 __global__ __launch_bounds__(kXcdThreads) void lstm_xcd_res_f16_kernel(LstmXcdArgs p)
 {
-    lstm_xcd_body<true, true, XcdSparse>(p);
+    lstm_xcd_body<true, true, XcdSparse<FRAGS>>(p);
 }
 
 }  // namespace pimhip
