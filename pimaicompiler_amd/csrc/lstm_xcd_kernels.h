@@ -98,6 +98,7 @@ static constexpr unsigned long long kXcdWaitTicks = 100000000ull;  // one second
 // 148 / 135, two of 136, 100 steps 123 / 118).
 static constexpr int kXcdSumWave = 2;
 static_assert(kXcdSumWave >= 2 && kXcdSumWave < kXcdWaves, "wavefronts 0 and 1 poll for h");
+static constexpr float kXcdLog2 = -1.4426950408889634f;  // exp(-v) = exp2(kXcdLog2 v)
 static constexpr int kXcdLag = 2;       // steps a recurrence fed by a P group lets that group get ahead before it starts
 
 struct LstmXcdArgs {
@@ -120,13 +121,12 @@ struct LstmXcdArgs {
 // to another XCD and back; nothing that passes between the wavefronts of a workgroup here goes through global memory.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
-__device__ __forceinline__ void load16_nt(const void* p, unsigned long long& lo, unsigned long long& hi)
+typedef unsigned int xcd_u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ xcd_u32x4 load16_nt(const void* p)
 {
-    typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-    u32x4 v;
+    xcd_u32x4 v;
     asm volatile("global_load_dwordx4 %0, %1, off nt\n\ts_waitcnt vmcnt(0)" : "=v"(v) : "v"(p) : "memory");
-    lo = (unsigned long long)v[0] | ((unsigned long long)v[1] << 32);
-    hi = (unsigned long long)v[2] | ((unsigned long long)v[3] << 32);
+    return v;
 }
 
 __device__ __forceinline__ void store8_plain(void* p, unsigned long long v)
@@ -347,6 +347,7 @@ struct XcdSparse {
         for (int m = 0; m < FRAGS; ++m) {
             if (m >= 8 && (m & 3) == 0 && m * 64 >= H) break;  // (uniform) whole fragments past the hidden state are zeros
             acc.d[m & 7] = __builtin_amdgcn_smfmac_f32_16x16x64_f16(m < 8 ? h.h0 : h.h1, w[m], acc.d[m & 7], index, 0, 0);
+            if (m == 7) asm volatile("" : : "v"(h.h1));  // (read for it behind the barrier, not behind the next line's branch)
         }
         // Row r of D lies in register r & 3 of lanes 16 (r >> 2) .. + 15: row group q keeps pairs 2 q (registers 0, 1) and 2 q + 1.
         float f[4];
@@ -396,7 +397,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
-    const int wave = tid >> 6;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // (in a scalar register: what goes by it is a branch, not a mask)
     const int xcd = (int)hw_xcc_id();  // the XCD this workgroup runs on
     const int rank = blockIdx.x >> 3;
     if (xcd >= kXcdCount) {
@@ -460,19 +461,24 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     // All lanes of the first two wavefronts fetch one piece of an h vector each: 8 fp16 = columns 8 q .. 8 q + 7.  Spread over eight
     // wavefronts of 16 lanes a step of 1024 units took 1.42 us, over four of 32 1.32, over two 1.31.  (The wavefronts that talk
     // to other XCDs, 4 .. 7 and the one that makes the residual sums, never poll for h: a wavefront's loads come back in order.)
-    const int piece = wave * 64 + lane;
-    const bool polls = wave < 2 && piece * 8 < H;
+    // Whole wavefronts poll: a lane past the hidden state looks at the last piece beside the others and keeps nothing.
+    const bool polls = wave < 2 && wave * 64 * 8 < H;
+    const bool in_range = (wave * 64 + lane) * 8 < H;
+    const int piece = min(wave * 64 + lane, H / 8 - 1);
 
-    // One bounded wait: `again` loads and tests; gives up like every wait of this kernel, after spin_limit polls, and
-    // also after kXcdWaitTicks of the constant 100 MHz clock, however long a poll takes in the environment the kernel
-    // finds itself in (a wait that succeeds does so within microseconds).
-    auto bounded_wait = [&](auto again) __attribute__((always_inline)) {
+    // One bounded wait of the wavefront's active lanes: `again` loads and tests, a lane each; gives up like every wait of this kernel,
+    // after spin_limit polls, and also after kXcdWaitTicks of the constant 100 MHz clock, however long a poll takes in the
+    // environment the kernel finds itself in (a wait that succeeds does so within microseconds).  The lanes leave together: with lanes
+    // that leave by themselves the way out of the loop was ten instructions of mask arithmetic, on every step's path.
+    auto bounded_wait = [&](bool& gave_up_here, auto again) __attribute__((always_inline)) {
         unsigned int spins = 0;
         unsigned long long t_first = 0ull;
-        while (!again() && !gave_up) {
+        while (true) {
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(!again()) == 0ull, 1)) return;
+            if (gave_up_here) return;
             ++spins;
             if ((spins & 255u) == 0u) {
-                if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) gave_up = true;
+                if (__builtin_amdgcn_readfirstlane(__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u) gave_up_here = true;
                 const unsigned long long now = __builtin_amdgcn_s_memrealtime();
                 if (spins == 256u) t_first = now;
                 else if (now - t_first > kXcdWaitTicks) spins = 0xffffffffu;  // gives up below
@@ -480,7 +486,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             if (spins >= p.spin_limit) {
                 __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                gave_up = true;
+                gave_up_here = true;
             }
         }
     };
@@ -506,15 +512,15 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
             acc.clear();
             if (polls) {
                 const unsigned long long* src = reinterpret_cast<const unsigned long long*>(pj.seq_in + (long)t * H + piece * 8);
-                if (!(filled16(lo) && filled16(hi))) {
-                    bounded_wait([&]() {
+                if (__builtin_amdgcn_ballot_w64(!(filled16(lo) && filled16(hi))) != 0ull) {
+                    bounded_wait(gave_up, [&]() {
                         load16_device_scope(src, lo, hi);
                         return filled16(lo) && filled16(hi);
                     });
                 }
                 typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
                 const u64x2 both = {lo, hi};
-                *reinterpret_cast<half8_t*>(hb + Product::place(piece) * 8) = __builtin_bit_cast(half8_t, both);
+                if (in_range) *reinterpret_cast<half8_t*>(hb + Product::place(piece) * 8) = __builtin_bit_cast(half8_t, both);
             }
             if (gave_up) block_gave_up = 1;
             lds_barrier();
@@ -556,11 +562,12 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     // that step's barrier.  Every wavefront drains its loads once per step, so what matters is that the load leaves
     // early in the step: issued behind the sum of the step before, it cost 0.23 us per step.
     unsigned short in_ahead = 0xffffu;
+    bool sum_gave_up = false;  // (a lane's: not every lane makes sums)
     auto emit_sum = [&](int se) __attribute__((always_inline)) {
         unsigned short in_bits = in_ring[se & 1][lane & 31];
         if (ch.res_polled && in_bits == 0xffffu) {
             const unsigned short* rin = reinterpret_cast<const unsigned short*>(ch.res_in) + (long)se * H + eu;
-            bounded_wait([&]() {
+            bounded_wait(sum_gave_up, [&]() {
                 in_bits = __hip_atomic_load(rin, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 return in_bits != 0xffffu;
             });
@@ -597,10 +604,9 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     const unsigned int* xp_other =
         reinterpret_cast<const unsigned int*>(ch.xproj + (long)my_gate * H + min(max(u0 - 16, 0) + unit, H - 1));  // wavefront w - 4's
     auto xp_bits_at = [&](int t) { return __hip_atomic_load(xp_mine + (long)t * 4 * H, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-    auto wait_xp = [&](int t) {
-        unsigned int bits = 0xffffffffu;
-        bounded_wait([&]() {
-            bits = xp_bits_at(t);
+    auto wait_xp = [&](int t, unsigned int bits = 0xffffffffu) {
+        bounded_wait(gave_up, [&]() {
+            if (bits == 0xffffffffu) bits = xp_bits_at(t);
             return bits != 0xffffffffu;
         });
         return bits;
@@ -625,8 +631,10 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     asm volatile("" : "+v"(published32));
     const unsigned long long published = ((unsigned long long)published32 << 32) | published32;
     const bool publishes = lane == 0;
-    half_t* const y = ch.y;
-    const long y_stride = p.y_stride;
+    const bool stores_y = lane == 0 && !res && units_ok && ch.y != nullptr;
+    unsigned char* y_at = reinterpret_cast<unsigned char*>(ch.y + (rev ? (long)(T - 1) * p.y_stride : 0l) + u0);
+    const long y_step = (long)sizeof(half_t) * (rev ? -p.y_stride : p.y_stride);
+    const float gate_scale = my_gate == 2 ? 2.0f * kXcdLog2 : kXcdLog2, gate_mul = my_gate == 2 ? 2.0f : 1.0f, gate_add = my_gate == 2 ? -1.0f : 0.0f;
 
     for (int s = 0; s < T; ++s) {
         half_t* hb = hbuf[s & 1];
@@ -650,23 +658,19 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         if (polls) {
             half8_t hv;
             if (s == 0) {
-                hv = *reinterpret_cast<const half8_t*>(ch.h0 + piece * 8);
+                hv = __builtin_bit_cast(half8_t, load16_nt(ch.h0 + piece * 8));  // (waited for here: left to the compiler it is a wait for all memory in every step)
             } else {
                 const unsigned int gp = g_base + (unsigned int)s - 1u;
-                const unsigned long long want = ((gp >> 1) & 1u) ? 0x4000400040004000ull : 0ull;
+                const unsigned int want = ((gp >> 1) & 1u) ? 0x40004000u : 0u;
                 const unsigned char* src = reinterpret_cast<const unsigned char*>(region + (long)(gp & 1u) * kXcdMembers * kXcdEntryWords) + piece * 16;
-                unsigned long long lo = 0ull, hi = 0ull;
-                bounded_wait([&]() {
-                    load16_nt(src, lo, hi);
-                    return (lo & 0x4000400040004000ull) == want && (hi & 0x4000400040004000ull) == want;
+                xcd_u32x4 v;
+                bounded_wait(gave_up, [&]() {
+                    v = load16_nt(src) ^ want;   // what has its flags is h, without them, by that
+                    return ((v[0] | v[1] | v[2] | v[3]) & 0x40004000u) == 0u;
                 });
-                lo &= 0xbfffbfffbfffbfffull;
-                hi &= 0xbfffbfffbfffbfffull;
-                typedef unsigned long long u64x2 __attribute__((ext_vector_type(2)));
-                const u64x2 both = {lo, hi};
-                hv = __builtin_bit_cast(half8_t, both);
+                hv = __builtin_bit_cast(half8_t, v);
             }
-            *reinterpret_cast<half8_t*>(hb + Product::place(piece) * 8) = hv;
+            if (in_range) *reinterpret_cast<half8_t*>(hb + Product::place(piece) * 8) = hv;
         }
         if (gave_up) block_gave_up = 1;
         lds_barrier();
@@ -677,6 +681,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         const int dead_lds = block_gave_up;
         const typename Product::Operands operands = Product::operands(hb, lane);
         unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][unit]);
+        __builtin_amdgcn_sched_barrier(0);
         const int dead = __builtin_amdgcn_readfirstlane(dead_lds);
         if (polled && fetcher && s + 2 < T) {
             xp_ahead = xp_bits_at(s + 2);
@@ -690,29 +695,28 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
                                          __HIP_MEMORY_SCOPE_AGENT);
             if (s > 0 && !dead) emit_sum(s - 1);
         }
+        if (res) gave_up = gave_up || __builtin_amdgcn_ballot_w64(sum_gave_up) != 0ull;
 
         // (a wavefront one of whose waits gave up after this step's barrier makes its h from stale values: it keeps them
         // to itself, and the group's other members stop at their next wait)
-        bool stop = dead || __builtin_amdgcn_ballot_w64(gave_up) != 0ull;
+        bool stop = dead || gave_up;
 
         // ---- 2. the wavefront's 16 gate rows
         const float dot = weights.matvec(hb, operands, acc, H, lane);
         if (polled && __builtin_amdgcn_ballot_w64(xp_bits == 0xffffffffu) != 0ull) {  // the P group had not got there when it was fetched
-            if (xp_bits == 0xffffffffu) xp_bits = wait_xp(s);
-            stop = stop || __builtin_amdgcn_ballot_w64(gave_up) != 0ull;
+            xp_bits = wait_xp(s, xp_bits);
+            stop = stop || gave_up;
         }
         const float a = dot + __builtin_bit_cast(float, xp_bits);
-        const int t = rev ? (T - 1 - s) : s;
-
         // Every lane activates its own gate; the lanes of a unit then share them.
-        const bool is_g = my_gate == 2;
-        const float sg = fast_sigmoid_f32(is_g ? 2.0f * a : a);
-        const float act = is_g ? 2.0f * sg - 1.0f : sg;
+        // sigmoid(a), or tanh(a) = 2 sigmoid(2a) - 1 for g: the factors are the lane's (exact: powers of two, one and zero).
+        const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gate_scale * a));
+        const float act = __builtin_fmaf(sg, gate_mul, gate_add);
         float g_i, g_f, g_g, g_o;
         Product::share(act, g_i, g_f, g_g, g_o);
         const float c_new = g_f * c_reg + g_i * g_g;
         const bool h_is_number = (c_new == c_new) && (g_o == g_o);
-        const half_t h = (half_t)(g_o * (2.0f * fast_sigmoid_f32(2.0f * c_new) - 1.0f));
+        const half_t h = (half_t)(g_o * __builtin_fmaf(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.0f * kXcdLog2 * c_new)), 2.0f, -1.0f));
         c_reg = c_new;
 
         // ---- 3. the wavefront's four h values: lane 0 publishes, then stores y (whose place in front of the publishing store
@@ -727,10 +731,9 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         publish_step = -publish_step;
         const unsigned long long yw = Product::pack(hb16);
         const unsigned long long sw = emits ? Product::pack(sb16) : 0ull;
-        if (lane == 0) {
-            if (!res && units_ok && y) *reinterpret_cast<unsigned long long*>(y + (long)t * y_stride + u0) = yw;
-            if (emits) hout[s & 1][wave] = sw;
-        }
+        if (stores_y) *reinterpret_cast<unsigned long long*>(y_at) = yw;
+        y_at += y_step;
+        if (emits && lane == 0) hout[s & 1][wave] = sw;
         if (s == T - 1 && units_ok && Product::first_of_unit(lane)) {
             ch.hn[my_unit] = h;
             ch.cn[my_unit] = (half_t)c_new;
@@ -743,7 +746,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     if (emits && !block_gave_up) {
         if (!res && wave == 4 && lane < 4 && rank * kXcdUnitsPerBlock + lane * 8 < H) emit(T - 1);
         if (sums) emit_sum(T - 1);
-        if (gave_up) block_gave_up = 1;  // (the last sum's own wait)
+        if (res && __builtin_amdgcn_ballot_w64(sum_gave_up) != 0ull) block_gave_up = 1;  // (the last sum's own wait)
     }
     lds_barrier();
     };
