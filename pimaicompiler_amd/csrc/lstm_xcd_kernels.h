@@ -169,7 +169,11 @@ struct XcdDot {
     // What is read of h as soon as it is there: nothing (pieces are read as they are used).
     struct Operands {
     };
-    static __device__ __forceinline__ Operands operands(const half_t*, int) { return {}; }
+    struct At {
+    };
+    static __device__ __forceinline__ At operands_at(const half_t*, int) { return {}; }
+    static __device__ __forceinline__ void keep(At&) {}
+    static __device__ __forceinline__ Operands operands(At) { return {}; }
 
     // In every lane: the dot product of its unit's gate row gate(lane) with hb[0 .. H).
     __device__ __forceinline__ float matvec(const half_t* hb, const Operands&, Sums&, int H, int lane) const
@@ -238,12 +242,25 @@ static constexpr int kXcdFrags = kXcdMaxH / 64;  // 64-column weight fragments o
 // the weight matrix the 64 are is free as long as both operands agree.  A lane of B takes two whole 16-byte pieces of its gate
 // row, 8 m + (l >> 4) and four pieces further; halves 0..3 of a piece then meet the even row of A, halves 4..7 the odd one.
 
-// Lane l's eight values of h in register set s of A: two 8-byte halves of neighbouring pieces.
-__device__ __forceinline__ half8_t xcd_h_operand(const half_t* hb, int s, int lane)
+// Lane l's eight values of h in a register set of A: two 8-byte halves of neighbouring pieces, at these two LDS addresses for the first set
+// and 1 KB further for the second.  Addresses, because a lane has them ready in front of the barrier that it reads behind.
+struct XcdOperandAt {
+    unsigned int lo, hi;
+};
+typedef __attribute__((address_space(3))) const half4_t* xcd_lds_half4;
+__device__ __forceinline__ unsigned int xcd_lds_address(const void* p)
 {
-    const int lo = xcd_h_place(xcd_h_operand_piece(s, lane));
-    return __builtin_shufflevector(*reinterpret_cast<const half4_t*>(hb + lo * 8 + 4 * (lane & 1)),
-                                   *reinterpret_cast<const half4_t*>(hb + (lo ^ 1) * 8 + 4 * (lane & 1)), 0, 1, 2, 3, 4, 5, 6, 7);
+    return (unsigned int)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
+}
+__device__ __forceinline__ XcdOperandAt xcd_h_operand_at(const half_t* hb, int lane)
+{
+    const int lo = xcd_h_place(xcd_h_operand_piece(0, lane));
+    return {xcd_lds_address(hb + lo * 8 + 4 * (lane & 1)), xcd_lds_address(hb + (lo ^ 1) * 8 + 4 * (lane & 1))};
+}
+static constexpr unsigned int kXcdSecondOperand = 64 * 16;   // bytes
+__device__ __forceinline__ half8_t xcd_h_operand(XcdOperandAt at)
+{
+    return __builtin_shufflevector(*(xcd_lds_half4)(uintptr_t)at.lo, *(xcd_lds_half4)(uintptr_t)at.hi, 0, 1, 2, 3, 4, 5, 6, 7);
 }
 
 // FRAGS: four (up to 256 units) or sixteen of them.  Four have a kernel of their own: half the sums and no second operand, and with both in one
@@ -324,11 +341,25 @@ struct XcdSparse {
     struct Operands {
         half8_t h0, h1;
     };
-    static __device__ __forceinline__ Operands operands(const half_t* hb, int lane)
+    struct At {
+        XcdOperandAt h0, h1;
+    };
+    static __device__ __forceinline__ At operands_at(const half_t* hb, int lane)
+    {
+        const XcdOperandAt h0 = xcd_h_operand_at(hb, lane);
+        return {h0, {h0.lo + kXcdSecondOperand, h0.hi + kXcdSecondOperand}};
+    }
+    // (all four addresses: with an offset for the second set the reads become two of 16 bytes, whose halves then have to change places)
+    static __device__ __forceinline__ void keep(At& at)
+    {
+        asm volatile("" : "+v"(at.h0.lo), "+v"(at.h0.hi));
+        if constexpr (!kFew) asm volatile("" : "+v"(at.h1.lo), "+v"(at.h1.hi));
+    }
+    static __device__ __forceinline__ Operands operands(At at)
     {
         Operands o;
-        o.h0 = xcd_h_operand(hb, 0, lane);
-        o.h1 = kFew ? o.h0 : xcd_h_operand(hb, 1, lane);
+        o.h0 = xcd_h_operand(at.h0);
+        o.h1 = kFew ? o.h0 : xcd_h_operand(at.h1);
         return o;
     }
 
@@ -508,6 +539,8 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         }
         for (int t = 0; t < T; ++t) {
             half_t* hb = hbuf[t & 1];
+            typename Product::At operands_at = Product::operands_at(hb, lane);
+            Product::keep(operands_at);
             typename Product::Sums acc;
             acc.clear();
             if (polls) {
@@ -531,7 +564,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
                 lo = __hip_atomic_load(nxt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 hi = __hip_atomic_load(nxt + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
-            const float v = weights.matvec(hb, Product::operands(hb, lane), acc, H, lane) + bias;
+            const float v = weights.matvec(hb, Product::operands(operands_at), acc, H, lane) + bias;
             if (dead) return;  // rows made from a stale h must not reach the recurrence: it will make its own
             if (units_ok && Product::first_of_gate(lane))
                 __hip_atomic_store(reinterpret_cast<unsigned int*>(dst + (long)t * 4 * H), __builtin_bit_cast(unsigned int, v), __ATOMIC_RELAXED,
@@ -638,6 +671,10 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
 
     for (int s = 0; s < T; ++s) {
         half_t* hb = hbuf[s & 1];
+        typename Product::At operands_at = Product::operands_at(hb, lane);
+        unsigned int xp_at = xcd_lds_address(&xring[wave][s & 31][my_gate][unit]);
+        Product::keep(operands_at);
+        asm volatile("" : "+v"(xp_at));  // (made here, not behind the barrier)
         typename Product::Sums acc;
         acc.clear();
         unsigned int flag32 = (((g_base + (unsigned int)s) >> 1) & 1u) ? 0x40004000u : 0u;
@@ -679,8 +716,8 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         // The operands of the product and the projection terms are asked for here too, in front of everything that is not on
         // the step's path: the terms behind the sums came an LDS round trip (100 cycles) later.
         const int dead_lds = block_gave_up;
-        const typename Product::Operands operands = Product::operands(hb, lane);
-        unsigned int xp_bits = reinterpret_cast<const unsigned int&>(xring[wave][s & 31][my_gate][unit]);
+        const typename Product::Operands operands = Product::operands(operands_at);
+        unsigned int xp_bits = *(__attribute__((address_space(3))) const unsigned int*)(uintptr_t)xp_at;
         __builtin_amdgcn_sched_barrier(0);
         const int dead = __builtin_amdgcn_readfirstlane(dead_lds);
         if (polled && fetcher && s + 2 < T) {
