@@ -121,6 +121,18 @@ __device__ __forceinline__ float wave_sum(float v)
 static constexpr unsigned int kXccIdMask = 15u;
 __device__ __forceinline__ unsigned int hw_xcc_id() { return __builtin_amdgcn_s_getreg((3 << 11) | (0 << 6) | 20) & kXccIdMask; }
 
+// A barrier that waits for this wavefront's LDS traffic only: __syncthreads() would wait for its global loads and stores too.
+// Builtins, not inline assembly: behind a wait that the compiler does not know of it takes earlier scalar loads for pending, and the
+// first use of an LDS read behind the barrier then waits for all reads in flight.
+static constexpr int kWaitLdsOnly = 0xc07f;  // s_waitcnt: lgkmcnt(0), nothing of vmcnt and expcnt
+__device__ __forceinline__ void lds_only_barrier()
+{
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(kWaitLdsOnly);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+
 // Every bounded wait of the kernels here also ends after kWaitTicks of the constant 100 MHz clock, whatever its poll
 // count: where a poll takes far longer than usual (counter collection serialising the memory system, a tool stepping the
 // device), the poll limit alone bounds nothing useful.  Called every 256 unsuccessful polls; `t_first` keeps the time of

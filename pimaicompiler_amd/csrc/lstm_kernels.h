@@ -448,7 +448,7 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
                 }
             }
         }
-        __syncthreads();
+        lds_only_barrier();  // (nothing that passes between the wavefronts here goes through memory)
         // Written only in front of this barrier: every thread reads the same value, and the block leaves together.  Asked
         // for here, with the reads of h, and looked at where the block would publish: the step's arithmetic does not wait
         // for it (a step that should not have been made is made on stale values and dropped).
@@ -543,6 +543,19 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
                 const unsigned int hbits = (unit_ok && h_is_number[k]) ? (unsigned int)__builtin_bit_cast(unsigned short, h_new[k]) : 0u;
                 pub[k][wave] = (unsigned short)(hbits | flag);
             }
+        }
+        lds_only_barrier();  // (not for the projection terms asked for above: 0.5 to 1 us of every step)
+        alone = gave_up_in_this_step != 0;
+        if (tid == 0 && !alone) {
+            const unsigned int g = g_base + (unsigned int)tau;
+            unsigned long long* dst = reinterpret_cast<unsigned long long*>(p.hx + ((long)(g & 1u) * nb + blockIdx.x) * kSeqEntryWords);
+            const unsigned long long* src = reinterpret_cast<const unsigned long long*>(&pub[0][0]);
+#pragma unroll
+            for (int k = 0; k + 1 < NW; k += 2) store16_device_scope(dst + k, src[k], src[k + 1]);
+            if (NW & 1) __hip_atomic_store(dst + (NW - 1), src[NW - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        // The outputs behind the word that everybody waits for (a block that goes on by itself makes them again).
+        if (lane == 0 && !alone) {
             if (unit_ok) {
 #pragma unroll
                 for (int k = 0; k < NC; ++k) {
@@ -556,16 +569,6 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
                     }
                 }
             }
-        }
-        __syncthreads();
-        alone = gave_up_in_this_step != 0;
-        if (tid == 0 && !alone) {
-            const unsigned int g = g_base + (unsigned int)tau;
-            unsigned long long* dst = reinterpret_cast<unsigned long long*>(p.hx + ((long)(g & 1u) * nb + blockIdx.x) * kSeqEntryWords);
-            const unsigned long long* src = reinterpret_cast<const unsigned long long*>(&pub[0][0]);
-#pragma unroll
-            for (int k = 0; k + 1 < NW; k += 2) store16_device_scope(dst + k, src[k], src[k + 1]);
-            if (NW & 1) __hip_atomic_store(dst + (NW - 1), src[NW - 1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
 

@@ -119,16 +119,7 @@ struct LstmXcdArgs {
 // The barrier of a step: LDS traffic of this wavefront done, then s_barrier.  __syncthreads() would also wait for every
 // global store and load the wavefront has in flight (its release semantics cover global memory), and some of those cross
 // to another XCD and back; nothing that passes between the wavefronts of a workgroup here goes through global memory.
-// (Builtins, not inline assembly: behind a wait that the compiler does not know of, it takes scalar loads for pending, and the first use of
-// the reads behind the barrier waits for all of them.)
-static constexpr int kWaitLdsOnly = 0xc07f;  // s_waitcnt: lgkmcnt(0), nothing of vmcnt and expcnt
-__device__ __forceinline__ void lds_barrier()
-{
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(kWaitLdsOnly);
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
+__device__ __forceinline__ void lds_barrier() { lds_only_barrier(); }
 
 typedef unsigned int xcd_u32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ xcd_u32x4 load16_nt(const void* p)
