@@ -185,10 +185,9 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
     launch_fill_u32(plan->g_counter, (size_t)plan->blocks * kRnntCounterStride, 0u, s);
     {
         // As many teams of symbol blocks as the CUs that are left take, one workgroup to a CU, up to one for each step that the joint
-        // blocks run ahead (2 x 320 units, 29 symbols, us per blank: 1.01 with one team, 0.82 with four, 0.81 with eight; 341 frames with 121
-        // symbols 1180 and 1053).  Products of another stream share CUs with them: beside such a decode a projection of 341 frames
-        // onto 4096 takes 12.1 us instead of 11.5 with one team, beside one of 400 symbols, whose teams take 244 CUs, 14.3 instead of 11.1
-        // (8.6 alone), and the decode 1095 instead of 1254 us, 442 instead of 530.
+        // blocks run ahead (2 x 320 units, 29 symbols, 341 frames with 74 and 114 symbols emitted, us: six teams 594 and 798, twelve 581 and 784).
+        // Products of another stream share CUs with them (measured with eight: beside such a decode a projection of 341 frames onto 4096 takes
+        // 12.1 us instead of 11.5 with one team, beside one of 400 symbols, whose teams take 244 CUs, 14.3 instead of 11.1; 8.6 alone).
         const int n_vocab = (int)((vocab + 7) / 8);
         const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
         plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);

@@ -24,36 +24,38 @@
 //     all; who needs the first layer's h reads the decided symbol's words, which are there already.  A symbol's chain loses a cell (0.7 us) and
 //     the way of a store (0.4 us);
 //   * most steps of a real utterance are blanks, after which only the frame changes: the joint blocks do not wait for the
-//     decision but publish the hidden vectors of the next steps as well, up to eight ahead, as if every decision in
-//     between were a blank (the frames' columns are asked for a round earlier and their sums kept), and the symbol blocks
-//     turn every hidden vector that arrives into logits.  When a symbol is emitted, g gets a new version
-//     and what was computed ahead under the old one is simply never looked at;
+//     decision but publish the hidden vectors of the next steps as well, up to twelve ahead, as if every decision in
+//     between were a blank, and the symbol blocks turn every hidden vector that arrives into logits.  When a symbol is emitted, g gets
+//     a new version and what was computed ahead under the old one is simply never looked at.  A row's sum over the frame and its
+//     sum over g are made apart: the frames' ahead of their turn, a frame to a wavefront with all of the block's rows, and g's once per version, so
+//     that the words of all steps ahead are sums of two values each and one store;
 //   * the symbol blocks exist several times over, as TEAMS: a symbol block's round (a look at 64 entries, a barrier, its sums, the
 //     publish) takes 2 us however few rows it has, so one set of blocks handles a run of blanks one or two steps a round.  The
-//     CUs that no other role needs hold up to seven further copies of W2's rows, team q takes the steps that are q modulo the
+//     CUs that no other role needs hold up to eleven further copies of W2's rows, team q takes the steps that are q modulo the
 //     number of teams, and the steps published ahead become logits side by side;
-//   * the joint blocks publish the step that everybody waits for alone and then four steps behind each barrier;
 //   * the decision behind a symbol, which everybody waits for while nothing else is there, is not waited for from the symbol blocks: with
 //     up to 64 symbols the blocks of layers and joint network read the hidden vector and make it themselves (decided_alone).
 //
 // Measured on MI355X, us an utterance of 341 frames (2 x 320 units, 512 joint units, 29 symbols) with 74 / 114 symbols emitted: 739 /
-// 996 with a hand-over of the first layer's h and of the logits per symbol, 667 / 905 without the first, 618 / 814 without both;
-// about 0.6 per blank and 5.2 per symbol now.  What bounds it now: of a symbol's 5.2 us two hand-overs of 1.1 and the look at the first
-// layer's words of 0.95, then the cell 0.5, a joint row 0.4, logits and decision 0.9; in a run of blanks the joint blocks' rounds of 2.5 us for
-// four steps (frames' sums 0.4, a batch of four 0.66, asking for frames 0.6, the look and the decisions 0.7).  (12 steps ahead: 5 %
-// less per blank, and 2 % more with one layer.)  Not kept: all logits made by every block, without symbol blocks (a run of blanks
-// 0.6 -> 0.85 us a step, eight steps' logits take every block 1.9 us); the first layer's words of all symbols collected ahead of
-// the decision (28 KB a block and symbol, 2.8 us).
+// 996 with a hand-over of the first layer's h and of the logits per symbol, 667 / 905 without the first, 618 / 814 without both, 581 / 784
+// with the sums over frames and g apart; 200 frames of 100 symbols with 34 emitted 395 / 387 / 382 / 344, of 300 symbols with 44 emitted 510 -> 481.  What bounds it
+// now: of a symbol's 5 us two hand-overs of 1.1 and the look at the first layer's words of 0.95, then the cell 0.5, a joint row 0.4,
+// logits and decision 0.9; in a run of blanks the steps ahead over the two hand-overs and the symbol blocks' rounds (steps ahead / teams: 8 / 8
+// 605 and 366, 12 / 8 595 and 343, 16 / 8 605 and 339, 12 / 12 581 and 344 in the first and the 100-symbol case).  Not kept: all logits made by
+// every block, without symbol blocks (a run of blanks 0.6 -> 0.85 us a step, eight steps' logits take every block 1.9 us); the first layer's words of
+// all symbols collected ahead of the decision (28 KB a block and symbol, 2.8 us); fewer steps ahead behind a symbol (0, 2, 4 instead of 8: 705, 669, 632
+// against 606).
 //
 // Exchange: 8-byte words of three fp16 values and a 16-bit tag, three words per producing block in a 128-byte entry of its
 // own, written and read with device-scope accesses.  The tag says what the word belongs to: h of a layer carries the
 // version of g (the count of the prediction network's runs), so do its words for every symbol, in entries of their own; hidden vectors and logits carry the step and the version they
 // were computed under; a word with another tag is "not there yet", so nothing is ever cleared and a stale word cannot be
-// taken for a fresh one.  h lives in four sets by version, hidden vectors in a ring of sixteen by step, logits in one of 64.  A
-// producer may overwrite what is a ring old: for the joint blocks' entries that follows from the order of things
-// (they run at most eight steps ahead of decisions that the symbol blocks have already published); the symbol blocks, whom
-// a slow reader could fall a ring behind (nobody waits for the layers' blocks during a run of blanks), look at a
-// count that every block keeps of the decisions it has taken in (`seen`) before they reuse an entry.
+// taken for a fresh one.  h lives in four sets by version, hidden vectors in a ring of 32 by step, logits in one of 64.  A
+// producer may overwrite what is a ring old: for the joint blocks' entries that follows from the order of things where all decisions
+// come from the symbol blocks (they run at most twelve steps ahead of decisions that the symbol blocks have already published); where
+// blocks decide for themselves, and for the symbol blocks' entries, a slow reader could fall a ring behind (nobody waits for the symbol blocks
+// during a run of symbols, nor for the layers' blocks during a run of blanks): the producers look at a count that every block keeps of the
+// decisions it has taken in (`seen`) before they reuse an entry.
 //
 // Waiting: a block looks at everything it waits for in one round ("pass"): the words of a vector by the first six
 // wavefronts, the logits of the next steps by the last ones (of four steps by one wavefront with up to 40 symbols, one step by
@@ -77,12 +79,16 @@ namespace pimhip
 {
 
 constexpr int kRnntGreedyVersions = 4;             // h of a layer: one entry per block and version of g, modulo this
-constexpr int kRnntGreedyRing = 16;                // hidden vectors: one entry per block and step, modulo this
+constexpr int kRnntGreedyRing = 32;                // hidden vectors: one entry per block and step, modulo this
 constexpr int kRnntGreedyLogitRing = 64;           // logits: the same
-constexpr int kRnntGreedyAhead = 8;                // steps the joint network runs ahead of the decisions
+constexpr int kRnntGreedyAhead = 12;                // steps the joint network runs ahead of the decisions
 constexpr int kRnntGreedyLook = 8;                 // steps whose logits one pass looks at, at most
-constexpr int kRnntGreedyTeams = 8;                // at most this many teams of symbol blocks, each with the steps of one residue
-constexpr int kRnntGreedyBatch = 4;                // hidden vectors a joint block publishes behind one barrier
+constexpr int kRnntGreedyTeams = 12;               // at most this many teams of symbol blocks, each with the steps of one residue
+constexpr int kRnntGreedyBatch = 2;                // steps' logits a symbol block publishes behind one barrier
+constexpr int kRnntGreedyFrames = 64;              // frames whose sums a joint block keeps, by frame modulo this
+constexpr int kRnntGreedyFramesAhead = 48;         // frames ahead of the current one that it sums at most
+static_assert(kRnntGreedyAhead + 1 + kRnntWaves <= kRnntGreedyFramesAhead && kRnntGreedyFramesAhead <= kRnntGreedyFrames, "what a publish needs is kept, and nothing it needs is overwritten");
+static_assert(3 * (kRnntGreedyAhead + 1) <= 64, "a joint block's words of all steps it publishes are one store of a wavefront");
 static_assert(kRnntGreedyAhead < kRnntGreedyRing && (kRnntGreedyRing & (kRnntGreedyRing - 1)) == 0, "ring");
 static_assert((kRnntGreedyLogitRing & (kRnntGreedyLogitRing - 1)) == 0 && kRnntGreedyLogitRing <= 128, "a ring's steps differ in their 8-bit tags");
 static_assert(kRnntGreedyLook + kRnntGreedyAhead < kRnntGreedyLogitRing, "a look and what is published ahead of it lie in one ring");
@@ -289,10 +295,9 @@ __device__ __forceinline__ void rnnt_greedy_solo(const RnntGreedyArgs& p, half_t
         const half8_t* gv = reinterpret_cast<const half8_t*>(hs + (long)(p.L - 1) * H);
         for (int r = wave; r < p.J; r += kRnntWaves) {
             const half8_t* row = reinterpret_cast<const half8_t*>(p.w1 + (long)r * (p.F + H));
-            float a = rnnt_row_dot(row, fv, nfp, lane, 0.0f);
-            a = rnnt_row_dot(row + nfp, gv, nhp, lane, a);
-            a = rnnt_sum(a);
-            if (lane == 0) tmp[r] = __builtin_bit_cast(half_t, rnnt_bits(relu_f32(a + (p.b1 ? (float)p.b1[r] : 0.0f))));
+            const float f = rnnt_sum(rnnt_row_dot(row, fv, nfp, lane, 0.0f));
+            const float g = rnnt_sum(rnnt_row_dot(row + nfp, gv, nhp, lane, 0.0f));
+            if (lane == 0) tmp[r] = __builtin_bit_cast(half_t, rnnt_bits(relu_f32(f + (g + (p.b1 ? (float)p.b1[r] : 0.0f)))));
         }
         __syncthreads();
         for (int v = wave; v < p.V; v += kRnntWaves) {
@@ -334,7 +339,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     __shared__ __align__(16) half_t own[kRnntMaxH];                                 // a layer's blocks: h of their layer; joint blocks: g
     __shared__ unsigned int keys[2][kRnntGreedyLook];                               // per pass (alternating): the best key of the next steps' logits, 0: not there
     __shared__ __align__(16) half_t emb[kRnntGreedyEmbHalfs];                       // first layer: the embedding rows and x0 behind them
-    __shared__ __align__(16) unsigned short mine[2][kRnntGreedyBatch][12];          // this block's eight values (a joint block's of several steps), alternating per publish
+    __shared__ __align__(16) unsigned short mine[2][kRnntGreedyBatch][12];          // this block's eight values (a symbol block's of two steps), alternating per publish
     __shared__ __align__(16) float4_t ih_of[EVERY ? kRnntWaves : 1][EVERY ? kRnntGreedyEveryVocab : 1];  // first layer: a unit's gate sums over every symbol's row
     __shared__ __align__(16) unsigned short every_mine[EVERY ? kRnntGreedyEveryVocab : 1][12];           // ... and this block's values of h after it
     __shared__ unsigned int own_keys[OWN_ROWS ? kRnntWaves * OWN_ROWS / 4 : 1];     // the best key among a wavefront's rows of W2
@@ -343,6 +348,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     __shared__ int someone_gave_up;
     __shared__ int i_decode_alone;
     __shared__ int min_seen_lds;
+    __shared__ int seen_lds[2];                                                     // joint blocks: the same, made beside their rounds (alternating)
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nb = gridDim.x, b = blockIdx.x;
@@ -396,14 +402,13 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
 
     // One 8-byte word: looked at once, or (blocks) polled until it carries `tag` or the wait's limits are reached, in which
     // case the thread raises the abort words and this pass's "gave up" flag.  Returns whether the tag is there.
-    // With `patience` it is polled that many times and then taken as not there.
-    auto fetch = [&](const u64* slot, unsigned int tag, bool blocks, int* miss, u64& w, unsigned int patience = 0u) __attribute__((always_inline)) {
+    auto fetch = [&](const u64* slot, unsigned int tag, bool blocks, int* miss, u64& w) __attribute__((always_inline)) {
         unsigned int spins = 0;
         unsigned long long first = 0ull;
         while (true) {
             w = __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if ((unsigned int)(w >> 48) == tag) return true;
-            if (!blocks && spins >= patience) return false;
+            if (!blocks) return false;
             bool give_up = false;
             if (spins > 0u && (spins & 255u) == 0u) {
                 if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
@@ -442,15 +447,14 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     int n_there = 0;
     constexpr bool row_per_step = LANE_WORDS == 0;
     auto pass = [&](const u64* vec, int n_vec, unsigned int vec_tag, half_t* vec_dst, bool vec_blocks, int look_waves, bool step_blocks, int vec_stride = kRnntEntryWords,
-                    const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr,
-                    unsigned int patience = 0u) __attribute__((always_inline)) -> int {
+                    const u64* vec2 = nullptr, int n_vec2 = 0, unsigned int vec2_tag = 0u, half_t* vec2_dst = nullptr) __attribute__((always_inline)) -> int {
         int* miss = missing[n_pass % 3u];
         u64 w;
         const int look = kRnntWaves - 1 - wave;
         if (look >= look_waves) {
             if (tid < 384) {
                 // Where a symbol is on its way and this team's hidden vector is not the next one, one word of it is looked at first.
-                const bool there_yet = !s.run_pred || vec_blocks || patience > 0u || n_vec == 0 ||
+                const bool there_yet = !s.run_pred || vec_blocks || n_vec == 0 ||
                                        (unsigned int)(__hip_atomic_load(vec, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >> 48) == vec_tag;
                 if (!there_yet) miss[0] = miss[2] = 1;
                 for (int i = tid; there_yet && i < 3 * (n_vec + n_vec2); i += 384) {
@@ -458,7 +462,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                     const int i2 = second ? i - 3 * n_vec : i;
                     const int prod = i2 / 3, part = i2 - 3 * prod;
                     if (!second) {
-                        if (fetch(vec + (long)prod * vec_stride + part, vec_tag, vec_blocks, miss, w, patience))
+                        if (fetch(vec + (long)prod * vec_stride + part, vec_tag, vec_blocks, miss, w))
                             unpack(w, vec_dst, prod, part);
                         else
                             miss[0] = 1;
@@ -626,12 +630,11 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             own_bias = p.b2 ? (float)p.b2[min(own_row, p.V - 1)] : 0.0f;
         }
     };
-    // Takes the decision of `step`.  False where the hidden vector did not come in time: a block that has fallen behind may find the
-    // entry used again (nobody waits for it before that), and the logits, which are kept until everybody has seen them, are there then.
+    // (The joint blocks do not use its entry again before every block has counted that decision: `seen`.)
     auto decided_alone = [&]() __attribute__((always_inline)) {
         if constexpr (OWN_ROWS > 0) {
-            constexpr unsigned int kPatience = 64u;   // looks, 40 us or more
-            if (!(pass(hid_entry(step, 0), nwj, step_tag(step, g_version()), buf0, false, 0, false, kRnntEntryWords, nullptr, 0, 0u, nullptr, kPatience) & 1) || dead) return false;
+            pass(hid_entry(step, 0), nwj, step_tag(step, g_version()), buf0, true, 0, false);
+            if (dead) return false;
             const half8_t* in = reinterpret_cast<const half8_t*>(buf0);
             float x[4];
 #pragma unroll
@@ -666,8 +669,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
     // Waits until the decision of `step` can be taken, and takes those behind it too if their logits are there already.
     // Returns false when the block has to leave the loop.
     auto wait_for_decisions = [&]() __attribute__((always_inline)) {
-        if (s.run_pred && decided_alone()) return true;
-        if (dead) return false;
+        if (OWN_ROWS > 0 && s.run_pred) return decided_alone();
         pass(nullptr, 0, 0u, nullptr, false, kRnntWaves, true);
         if (dead) return false;
         take_decisions();
@@ -895,148 +897,217 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             if (p.cn) p.cn[(long)l * H + u] = c_half;
         }
     } else if (someone_gave_up == 0 && b < n_lstm + nwj) {
-        // ---- the joint network's first layer: row r of W1 over cat(f, g), for the current step and, while nothing else
-        // is to do, for the steps behind it should they all be blanks ----
-        const int jb = b - n_lstm, r = 8 * jb + wave;
+        // ---- the joint network's first layer: rows 8 jb .. + 7 of W1 over cat(f, g), for the current step and the steps behind it should
+        // they all be blanks.  The sums over f and over g are made apart: the frames' sums are made ahead, eight a round, and kept, and g's
+        // once per version, so that a step's eight values are a sum of two each and all steps' words leave in one store ----
+        const int jb = b - n_lstm;
         const int nfp = p.F >> 3;
-        const half8_t* row = reinterpret_cast<const half8_t*>(p.w1 + (long)r * (p.F + H));
-        half8_t wf[kRnntFC], wg[kRnntHC];
+        const half8_t* rows = reinterpret_cast<const half8_t*>(p.w1 + (long)8 * jb * (p.F + H));
+        const long row_step = (long)(nfp + nhp);
+        // Frames of up to two pieces a lane (1024 wide): a wavefront takes a frame, with all eight rows in registers (every wavefront
+        // reading every frame for a row of its own is 128 KB a round through the CU's 64 bytes a clock).  Longer ones: a row each.
+        constexpr int kShort = 2;
+        const bool short_frames = nfp <= 64 * kShort;
+        // One array for both kinds: eight short rows and a short frame's pieces behind them, or a long row and four long frames'.
+        constexpr int kColShort = 8 * kShort, kColLong = kRnntFC, kRegs = 5 * kRnntFC;
+        static_assert(kColShort + kShort <= kRegs, "both fit");
+        half8_t reg[kRegs], wg[kRnntHC];
+        if (short_frames) {
 #pragma unroll
-        for (int k = 0; k < kRnntFC; ++k) {
-            if (64 * k >= nfp) break;
-            wf[k] = row[min(lane + 64 * k, nfp - 1)];
+            for (int r = 0; r < 8; ++r) {
+#pragma unroll
+                for (int k = 0; k < kShort; ++k) reg[r * kShort + k] = rows[r * row_step + min(lane + 64 * k, nfp - 1)];
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < kRnntFC; ++k) reg[k] = rows[wave * row_step + min(lane + 64 * k, nfp - 1)];
         }
 #pragma unroll
         for (int k = 0; k < kRnntHC; ++k) {
             if (64 * k >= nhp) break;
-            wg[k] = row[nfp + min(lane + 64 * k, nhp - 1)];
+            wg[k] = rows[wave * row_step + nfp + min(lane + 64 * k, nhp - 1)];
         }
         ask_for_w2();
-        const float bias = p.b1 ? (float)p.b1[r] : 0.0f;
+        const float bias = p.b1 ? (float)p.b1[8 * jb + wave] : 0.0f;
         for (int i = tid; i < H; i += kRnntThreads) own[i] = p.h0 ? p.h0[(long)(p.L - 1) * H + i] : (half_t)0.0f;  // g before the first run
         __syncthreads();
-        // this lane's part of the row's sum over a frame (nothing is read for a frame the utterance does not have)
-        auto sum_f = [&](int frame) __attribute__((always_inline)) {
-            float a = 0.0f;
-            if (frame >= 0 && frame < p.T) {
-                const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)frame * p.F);
+        float* const over_f = reinterpret_cast<float*>(emb);           // [kRnntGreedyFrames][8]: sums over frames f_lo .. af_hi (where the first layer's blocks have the embedding rows)
+        float* const over_g = over_f + kRnntGreedyFrames * 8;          // [8]: over g, with the bias
+        int af_hi = 0, af_seen = 0;                                    // frames summed so far; those whose sums every wavefront sees
+        // The next frames are asked for in front of a wait and summed behind it (their columns travel while the symbol blocks work).
+        int n_ask = 0;
+        auto ask = [&]() __attribute__((always_inline)) {
+            n_ask = max(0, min(min(short_frames ? kRnntWaves : 4, p.T - af_hi), s.t + kRnntGreedyFramesAhead - af_hi));
+            if (n_ask == 0) return;
+            if (short_frames) {
+                const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)(af_hi + min(wave, n_ask - 1)) * p.F);
 #pragma unroll
-                for (int k = 0; k < kRnntFC; ++k)
-                    if (lane + 64 * k < nfp) a = dot8(wf[k], f8[lane + 64 * k], a);
-            }
-            return a;
-        };
-        // The sums over the frames around the current one are kept (per thread, in the LDS that the first layer's blocks
-        // use for the embedding rows): frame f in slot f mod 16, those up to af_hi.  A frame is summed once, ahead of its
-        // turn, whatever the number of symbols it then emits.
-        float* af_ring = reinterpret_cast<float*>(emb) + tid;
-        static_assert(kRnntGreedyRing * kRnntThreads * sizeof(float) <= kRnntGreedyEmbHalfs * sizeof(half_t), "the ring of frame sums fits");
-        static_assert(kRnntGreedyAhead + 1 <= kRnntGreedyRing, "and holds what a round publishes");
-        int af_hi = 0;
-        auto frame_keep = [&](float a) __attribute__((always_inline)) { af_ring[(af_hi++ & (kRnntGreedyRing - 1)) * kRnntThreads] = a; };
-        // The next frames the ring does not hold yet are asked for in front of a wait and summed behind it (their columns travel
-        // while the symbol blocks work): as many as sixteen pieces per lane hold, the eight that two looks can consume.
-        constexpr int kPieces = 16;
-        static_assert(16 <= kPieces && kPieces % kRnntFC == 0, "eight frames of two pieces, or four of four");
-        const bool short_frames = nfp <= 128;
-        half8_t col[kPieces];
-        int piece_at[kRnntFC];
+                for (int k = 0; k < kShort; ++k) reg[kColShort + k] = f8[min(lane + 64 * k, nfp - 1)];   // (a lane past the frame's end keeps nothing of it)
+            } else {
 #pragma unroll
-        for (int k = 0; k < kRnntFC; ++k) piece_at[k] = min(lane + 64 * k, nfp - 1);
-        int f_first = 0, n_ask = 0;
-        auto ask_frames = [&](auto pieces) __attribute__((always_inline)) {
-            constexpr int kP = decltype(pieces)::value;
-            f_first = af_hi;
-            n_ask = max(0, min(min(kPieces / kP, p.T - f_first), s.t + kRnntGreedyRing - f_first));  // (what the ring still needs stays in it)
-            const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)f_first * p.F);
+                for (int q = 0; q < 4; ++q) {
+                    const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)(af_hi + min(q, n_ask - 1)) * p.F);
 #pragma unroll
-            for (int i = 0; i < kPieces; ++i) asm volatile("" : "=v"(col[i]));  // (a piece not asked for now is not one to keep from before)
-#pragma unroll
-            for (int q = 0; q < kPieces / kP; ++q) {
-                if (q >= n_ask) break;
-#pragma unroll
-                for (int k = 0; k < kP; ++k) col[q * kP + k] = f8[piece_at[k]];   // (a lane past the frame's end reads its last piece and keeps nothing of it)
-                f8 += nfp;
-            }
-        };
-        auto keep_frames = [&](auto pieces) __attribute__((always_inline)) {
-            constexpr int kP = decltype(pieces)::value;
-#pragma unroll
-            for (int q = 0; q < kPieces / kP; ++q) {
-                if (q < n_ask) {
-                    float a = 0.0f;
-#pragma unroll
-                    for (int k = 0; k < kP; ++k)
-                        if (lane + 64 * k < nfp) a = dot8(wf[k], col[q * kP + k], a);
-                    frame_keep(a);
+                    for (int k = 0; k < kRnntFC; ++k) reg[kColLong + q * kRnntFC + k] = f8[min(lane + 64 * k, nfp - 1)];
                 }
             }
         };
-        auto ask = [&]() __attribute__((always_inline)) {
-            if (short_frames) ask_frames(std::integral_constant<int, 2>{});
-            else ask_frames(std::integral_constant<int, 4>{});
-        };
         auto keep = [&]() __attribute__((always_inline)) {
-            if (short_frames) keep_frames(std::integral_constant<int, 2>{});
-            else keep_frames(std::integral_constant<int, 4>{});
-        };
-        int have_g = -1;          // the version of g in `own`
-        int pub = 0;              // the next step to publish a hidden vector for
-        half8_t gk[kRnntHC];      // this lane's pieces of g
-        auto take_g = [&](const half_t* g) __attribute__((always_inline)) {
-            const half8_t* gv = reinterpret_cast<const half8_t*>(g);
+            if (n_ask == 0) return;
+            float lo[4], hi[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+            if (short_frames) {
 #pragma unroll
-            for (int k = 0; k < kRnntHC; ++k) gk[k] = gv[min(lane + 64 * k, nhp - 1)];
+                for (int r = 0; r < 4; ++r) {
+                    lo[r] = hi[r] = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < kShort; ++k)
+                        if (lane + 64 * k < nfp) {
+                            lo[r] = dot8(reg[r * kShort + k], reg[kColShort + k], lo[r]);
+                            hi[r] = dot8(reg[(r + 4) * kShort + k], reg[kColShort + k], hi[r]);
+                        }
+                }
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    lo[q] = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < kRnntFC; ++k)
+                        if (lane + 64 * k < nfp) lo[q] = dot8(reg[k], reg[kColLong + q * kRnntFC + k], lo[q]);
+                }
+            }
+            // lane 16 i + j, j < 4, of the first 32: the sum of lo[j], or of hi[j]
+            const float both = rnnt_join16(rnnt_fold4(lo, lane), rnnt_fold4(hi, lane));
+            const float sum = rnnt_join32(both, both);
+            const int i = 4 * (lane >> 4) + (lane & 3);
+            if ((lane & 12) == 0 && lane < 32) {
+                if (short_frames) {
+                    if (wave < n_ask) over_f[((af_hi + wave) & (kRnntGreedyFrames - 1)) * 8 + i] = sum;
+                } else {
+                    if (i < n_ask) over_f[((af_hi + i) & (kRnntGreedyFrames - 1)) * 8 + wave] = sum;
+                }
+            }
+            af_hi += n_ask;
+            n_ask = 0;
         };
-        take_g(own);
-        ask();
-        keep();
+        int have_g = -1;          // the version of g whose sums are in over_g
+        int pub = 0;              // the next step to publish a hidden vector for
+        // (barriers between the sums' writers and their readers: this one, and those of the waits)
+        auto sum_g = [&]() __attribute__((always_inline)) {
+            const half8_t* gv = reinterpret_cast<const half8_t*>(own);
+            float a = 0.0f;
+#pragma unroll
+            for (int k = 0; k < kRnntHC; ++k)
+                if (lane + 64 * k < nhp) a = dot8(wg[k], gv[lane + 64 * k], a);
+            a = rnnt_sum(a);
+            if (lane == 0) over_g[wave] = a + bias;
+            rnnt_barrier();
+            af_seen = af_hi;
+        };
+        sum_g();
+        // With decisions that the symbol blocks have no part in (a run of symbols), nothing else keeps the joint blocks from running a ring
+        // ahead of them or of a layer's block: they look at everybody's count until the entry of `step` may be used again.  What the
+        // slowest block needs is there, so the wait ends.
+        int min_seen = 0;         // no block has taken in fewer decisions than this
+        int seen_stage = 0, seen_slot = 0, seen_here = 0x7fffffff;
+        auto wait_for_the_slowest = [&]() __attribute__((always_inline)) {
+            unsigned int spins = 0;
+            unsigned long long first = 0ull;
+            do {
+                int* miss = missing[n_pass % 3u];
+                if (tid == 0) min_seen_lds = 0x7fffffff;
+                rnnt_barrier();
+                if (tid < nb)
+                    atomicMin(&min_seen_lds, (int)__hip_atomic_load(p.seen + (long)kRnntSeenStride * tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+                rnnt_barrier();
+                min_seen = min_seen_lds;
+                if (tid == 0 && step - kRnntGreedyRing >= min_seen) {
+                    bool give_up = false;
+                    if (spins > 0u && (spins & 255u) == 0u) {
+                        if (__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) give_up = true;
+                        if (wait_clock_expired(spins, first)) spins = 0xffffffffu;
+                    }
+                    if (spins >= p.spin_limit) {
+                        __hip_atomic_store(p.abort_flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                        __hip_atomic_store(p.abort_host, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        give_up = true;
+                    }
+                    if (give_up) {
+                        miss[1] = 1;
+                        someone_gave_up = 1;
+                    }
+                    if (spins != 0xffffffffu) ++spins;
+                }
+                rnnt_barrier();
+                if (miss[1] != 0) dead = true;
+                if (tid < 3) missing[(n_pass + 2u) % 3u][tid] = 0;
+                ++n_pass;
+            } while (!dead && step - kRnntGreedyRing >= min_seen);
+            return !dead;
+        };
+        const int word_step = lane / 3, word_part = lane - 3 * word_step;   // a lane's word when all steps are published
         bool ok = true;
         while (ok && running()) {
             const int version = g_version();
-            const int end = min(step + kRnntGreedyAhead + 1, step + (p.T - s.t));
-            while (af_hi < s.t + (end - step)) frame_keep(sum_f(af_hi));  // (what was not asked for in time)
+            int end = min(step + kRnntGreedyAhead + 1, step + (p.T - s.t));
+            while (af_hi < s.t + (end - step)) {  // (the first frames, and what was not asked for in time)
+                ask();
+                keep();
+            }
             if (version != have_g) {
                 if (!(p.L == 1 ? wait_for_first_layer(version, own) : wait_for_vector(h_entry(version, (p.L - 1) * nwh), nwh, h_tag(version), own))) {
                     ok = false;
                     break;
                 }
-                take_g(own);
+                sum_g();
                 have_g = version;
                 pub = step;
             }
             if (pub < step) pub = step;
-            // the current step and up to kRnntGreedyAhead behind it: the first alone behind its barrier, then batches
-            auto publish_some = [&](auto how_many, int n) __attribute__((always_inline)) {
-                constexpr int kB = decltype(how_many)::value;
-                float a[kB];
-#pragma unroll
-                for (int q = 0; q < kB; ++q) a[q] = af_ring[((s.t + (pub + q - step)) & (kRnntGreedyRing - 1)) * kRnntThreads];
-#pragma unroll
-                for (int q = 0; q < kB; ++q) {
-#pragma unroll
-                    for (int k = 0; k < kRnntHC; ++k)
-                        if (lane + 64 * k < nhp) a[q] = dot8(wg[k], gk[k], a[q]);
+            if (OWN_ROWS > 0 && end - 1 - kRnntGreedyRing >= min_seen) {
+                if (!wait_for_the_slowest()) {
+                    ok = false;
+                    break;
                 }
-                if constexpr (kB == 1) {
-                    const float sum = rnnt_sum(a[0]);
-                    if (lane == 0) my_value(0) = rnnt_bits(relu_f32(sum + bias));
-                } else {
-                    static_assert(kB == 4, "a batch is folded to one step a lane");
-                    float sum = rnnt_fold4(a, lane);
-                    sum = rnnt_join16(sum, sum);
-                    sum = rnnt_join32(sum, sum);
-                    if (lane < kB) my_value(lane) = rnnt_bits(relu_f32(sum + bias));
-                }
+                end = min(end, min_seen + kRnntGreedyRing);
+            }
+            // the current step and up to kRnntGreedyAhead behind it
+            if (af_seen < s.t + (end - step)) {
                 rnnt_barrier();
-                if (wave < n) store_words(wave, hid_entry(pub + wave, jb), step_tag(pub + wave, version));
-                ++n_publish;
-                pub += n;
-            };
-            if (pub == step) publish_some(std::integral_constant<int, 1>{}, 1);
-            while (pub < end) publish_some(std::integral_constant<int, kRnntGreedyBatch>{}, min(kRnntGreedyBatch, end - pub));
+                af_seen = af_hi;
+            }
+            if (wave == 6 && pub < end) {
+                auto store = [&]() __attribute__((always_inline)) {
+                    const float* f = over_f + ((s.t + (pub + word_step - step)) & (kRnntGreedyFrames - 1)) * 8 + 3 * word_part;
+                    const float* g = over_g + 3 * word_part;
+                    const u64 w0 = rnnt_bits(relu_f32(f[0] + g[0])), w1 = rnnt_bits(relu_f32(f[1] + g[1])), w2 = word_part < 2 ? rnnt_bits(relu_f32(f[2] + g[2])) : (unsigned short)0;
+                    return w0 | (w1 << 16) | (w2 << 32) | ((u64)step_tag(pub + word_step, version) << 48);
+                };
+                if (lane < 3 * (end - pub)) {
+                    const u64 w = store();
+                    u64* const entry = hid_entry(pub + word_step, jb) + word_part;
+                    if (pub == step && lane < 3) __hip_atomic_store(entry, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // (everybody waits for this one)
+                    if (pub != step || lane >= 3) __hip_atomic_store(entry, w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+            }
+            pub = max(pub, end);
+            // Everybody's count of decisions, asked for when half the ring has been used: it is there two rounds later.
+            const bool look_now = OWN_ROWS > 0 && seen_stage == 0 && end - 1 - kRnntGreedyRing / 2 >= min_seen;
+            if (look_now) {
+                if (tid == 0) seen_lds[seen_slot] = 0x7fffffff;
+                if (tid < nb) seen_here = (int)__hip_atomic_load(p.seen + (long)kRnntSeenStride * tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
             ask();
+            const int summed = af_hi;
             ok = wait_for_decisions();
+            af_seen = summed;
+            if (seen_stage == 2) {
+                min_seen = max(min_seen, seen_lds[seen_slot]);
+                seen_slot ^= 1;
+                seen_stage = 0;
+            } else if (look_now) {
+                if (tid < nb) atomicMin(&seen_lds[seen_slot], seen_here);
+                seen_stage = 2;
+            }
             keep();
         }
     } else if (someone_gave_up == 0) {

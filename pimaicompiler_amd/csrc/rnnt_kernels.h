@@ -28,7 +28,7 @@
 // the joint network reads g = h_prev of the last layer where it lies.
 //
 // Sums run in one fixed order whoever computes them (per row: lane c takes 16-byte pieces c, c + 64, .. in ascending
-// order, f before g, then one reduction tree; a cell's rows over the hidden state and over the input each by themselves), so a vector that a
+// order, then one reduction tree; a cell's rows over the hidden state and over the input each by themselves, and W1's over f and over g), so a vector that a
 // workgroup had to make for itself has the bits it would have had from its producers.
 //
 // A wait that gives up does not leave the result undefined.  Every wait is bounded (`spin_limit` polls, one second); a block
@@ -257,13 +257,9 @@ __device__ __forceinline__ const half_t* rnnt_solo(const RnntStepIo& io, const R
         const int nfp = p.F >> 3;
         for (int r = wave; r < io.J; r += kRnntWaves) {
             const half8_t* row = reinterpret_cast<const half8_t*>(p.w1 + (long)r * (p.F + H));
-            float a = rnnt_row_dot(row, fv, nfp, lane, 0.0f);
-            a = rnnt_row_dot(row + nfp, gv, nhp, lane, a);
-            a = rnnt_sum(a);
-            if (lane == 0) {
-                if (p.b1) a += (float)p.b1[r];
-                nxt[r] = __builtin_bit_cast(half_t, rnnt_bits(relu_f32(a)));
-            }
+            const float f = rnnt_sum(rnnt_row_dot(row, fv, nfp, lane, 0.0f));
+            const float g = rnnt_sum(rnnt_row_dot(row + nfp, gv, nhp, lane, 0.0f));
+            if (lane == 0) nxt[r] = __builtin_bit_cast(half_t, rnnt_bits(relu_f32(f + (g + (p.b1 ? (float)p.b1[r] : 0.0f)))));
         }
         __syncthreads();
         cur = nxt;
@@ -462,6 +458,8 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_step_f16_kernel(const half_
 #pragma unroll
         for (int k = 0; k < kRnntFC; ++k)
             if (lane + 64 * k < nfp) a = dot8(wf[k], fv[k], a);
+        const float over_f = rnnt_sum(a);
+        a = 0.0f;
         const unsigned int set = g & 1u;
         if (io.run_prediction) {
             const half8_t* in = reinterpret_cast<const half8_t*>(vector_of(io.L - 1, (io.L - 1) * nwh, nwh, set));
@@ -473,7 +471,7 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_step_f16_kernel(const half_
             if (lane + 64 * k < nhp) a = dot8(wg[k], gv[k], a);
         a = rnnt_sum(a);
         if (lane == 0) {
-            const unsigned short bits = rnnt_bits(relu_f32(a + bias));
+            const unsigned short bits = rnnt_bits(relu_f32(over_f + (a + bias)));
             mine[wave] = bits;
             if (p.joint_hidden) p.joint_hidden[r] = __builtin_bit_cast(half_t, bits);
         }

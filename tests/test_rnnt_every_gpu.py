@@ -38,3 +38,21 @@ def test_the_decision_behind_a_symbol(ops, L, J, V):
     want = loop_driven_from_the_host(plan, enc, embedding, x0, blank, 3, 3 * T)
     r = check(plan.greedy_decode(enc, embedding, x0, blank, 3), want)
     assert r[3] == 0 and r[0] > 0
+
+
+@pytest.mark.parametrize("L,F,J,V,T,blank_bias", [
+    (2, 128, 64, 29, 120, -30.0),    # symbols alone, more of them than the rings hold: nobody waits for the symbol blocks
+    (2, 1024, 64, 29, 140, 0.0),     # frames of two pieces a lane, a mix
+    (2, 1032, 64, 40, 70, 0.0),      # of three
+    (1, 2048, 72, 29, 70, 9.0),      # of four, blanks alone: frames across the ring of their sums
+    (2, 8, 64, 64, 130, 9.0),
+    (2, 200, 64, 129, 70, 0.0),
+])
+def test_rings_and_frames(ops, L, F, J, V, T, blank_bias):
+    """Frames of every number of pieces, summed ahead in a ring, and hidden vectors' entries used again after runs of one kind of decision."""
+    I, H, blank = 64, 64, V - 1
+    params, joint, enc, embedding, x0 = model(3 * V + F, L, I, H, F, J, V, T, blank, blank_bias)
+    plan = ops.RnntPlan(dev(params), True, L, tuple(dev(joint)))
+    want = loop_driven_from_the_host(plan, enc, embedding, x0, blank, 2, 2 * T)
+    r = check(plan.greedy_decode(enc, embedding, x0, blank, 2), want)
+    assert r[3] == 0 and (r[0] == 2 * T if blank_bias < 0 else r[0] == 0 if blank_bias > 5 else r[0] > 0)
