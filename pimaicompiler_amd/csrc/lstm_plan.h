@@ -21,6 +21,11 @@ namespace pimhip
 //     0.97, 64 1.01 / 1.02 / 1.03
 //   three layers, at 2 / 3 / 4: 512 1.01 / 1.01 / 1.02, 640 0.97 / 1.00 / 1.00, 1024 1.00 / 1.02 / 1.03; at 24 / 80 / 200: 16 0.97 / 0.98 / 0.98, 32 1.06 / 1.13 / 1.15;
 //     four layers, at 2 / 4 / 8: 16 0.98 .. 1.00, 640 1.00 / 1.01 / 1.03
+// Since what stands around the products on a step's path was shortened for both (same layout as above): one layer, at 2 / 4 / 6 / 8 / 10 / 16 / 80 steps:
+//     8 1.05 / 1.02 / 1.01 / 1.04 / 1.04 / 1.02 / 1.01, 64 1.02 / 1.02 / 1.03 / 1.02 / 1.04 / 1.04 / 1.05, 128 1.00 / 1.01 / 1.01 / 1.02 / 1.04 / 1.06 / 1.09, 512 0.91 / 0.96 / 1.00 /
+//     1.03 / 1.05 / 1.12 / 1.26, 640 0.89 / 0.92 / 1.00 / 1.04 / 1.06 / 1.10 / 1.26, 1024 0.93 / 0.97 / 1.01 / 1.05 / 1.09 / 1.16 / 1.38; two layers at 2 / 3 / 4 / 80: 48 1.04 / 1.03 /
+//     1.04 / 1.05, 512 0.98 / 1.01 / 1.02 / 1.28, 1024 0.98 / 1.01 / 1.03 / 1.41.  The lines stay: between them and these figures lie a few percent of calls of few
+//     steps or few units.
 inline bool xcd_on_dot(int64_t H, int64_t T, int chained)
 {
     const bool half_empty = H > 512 && H <= 656;

@@ -39,10 +39,14 @@
 // registers per lane for the whole sequence.  Per step: the first wavefronts fetch the group's entries into LDS (16 bytes per lane),
 // one barrier, the 16 rows' products with h, the gate arithmetic, and one 8-byte store of the wavefront's four new h values into the
 // workgroup's entry.  What bounds a step: the store becoming visible in the L2 and the poll that finds it, 0.43 us at best
-// for such a round, and a chain of dependent instructions between two rounds.
+// for such a round, and a chain of dependent instructions between two rounds.  Everybody waits for the slowest wavefront's way from the
+// barrier to its store, so nothing stands on it that can be done before or after: the reads behind the barrier are all issued at once from
+// addresses made in front of it, the store's place and flag are known, y is packed and stored behind it, and no wait on it covers memory
+// operations (two layers of 1024, 341 steps, MI355X: 432 us -> 338; two directions, 50 steps 75.6 -> 63.4; one layer of 256, 200 steps
+// 173 -> 144).
 // The products come in two kinds:
-//   XcdSparse  16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16: 0.21 us of matrix instructions at H = 1024; a step 1.16 us
-//              for a single layer, 1.18 in pipelines (v_dot2 1.43, 1.64)
+//   XcdSparse  16 fragments of 64 columns for v_smfmac_f32_16x16x64_f16: 0.21 us of matrix instructions at H = 1024 (4 up to 256
+//              units); a step 0.93 us for a single layer, 0.95 in pipelines (v_dot2 1.3, 1.4)
 //   XcdDot     v_dot2 and a transposing reduction over 16 lanes: nothing passes through LDS at the start of a launch, which short
 //              sequences notice, and few units leave less of it idle (xcd_on_dot in lstm_plan.h has the lines and the figures)
 // Against 64 bits the sums are equally far off (rms error over the sum of the products' magnitudes, 64 .. 1024 columns, MI355X): signs
