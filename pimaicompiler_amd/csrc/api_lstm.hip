@@ -49,7 +49,7 @@ struct PimHipLstmPlan {
     int seq_blocks = 0;
     bool reset_exchange = false;     // the next forward starts from a cleared exchange buffer (layout change)
     bool seq_units8_ok = false;      // a single chain may run with 8 hidden units per block (half as many blocks)
-    bool seq_wide = false;           // 1024 < H <= 2048: 32 columns per lane, eight units per block, one layer per launch
+    bool seq_wide = false;           // 1024 < H <= 2048: 24 or 32 columns per lane, eight units per block, two layers per launch
     // Mode 4: every recurrence on one XCD (lstm_xcd_f16_kernel).
     bool xcd_ok = false;             // H fits one XCD's registers and the device has the eight XCDs of 32 CUs the kernel assumes
     unsigned int* xcd_hx = nullptr;  // [kXcdMaxChains] regions of kXcdRegionWords, zero when the chain's counter is 2
@@ -81,6 +81,15 @@ auto xcd_sparse_kernel(bool pipeline, int64_t hidden)
     return pipeline ? lstm_xcd_f16_kernel<true, kXcdFrags> : lstm_xcd_f16_kernel<false, kXcdFrags>;
 }
 auto xcd_res_kernel(int64_t hidden) { return hidden <= kXcdFewUnits ? lstm_xcd_res_f16_kernel<kXcdFewUnits / 64> : lstm_xcd_res_f16_kernel<kXcdFrags>; }
+
+// The all-CU kernel for more than kSeqMaxH units: two directions, two layers as a wavefront or one chain, with as few columns a lane as hold a row
+// (us, 32 / 24: two directions of 1424, 98 steps 291 / 278; one layer of 1200, 60 steps 116 / 113).
+auto seq_wide_kernel(int dirs, int chains, int64_t hidden)
+{
+    if (hidden <= kSeqMaxHMiddle)
+        return dirs == 2 ? lstm_seq_f16_kernel<2, false, 8, 24> : chains == 2 ? lstm_seq_f16_kernel<2, true, 8, 24> : lstm_seq_f16_kernel<1, true, 8, 24>;
+    return dirs == 2 ? lstm_seq_f16_kernel<2, false, 8, 32> : chains == 2 ? lstm_seq_f16_kernel<2, true, 8, 32> : lstm_seq_f16_kernel<1, true, 8, 32>;
+}
 
 constexpr unsigned long long kLstmEventsBeforeSafe = 3;
 }
@@ -222,7 +231,10 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
     } while (0)
 
     plan->seq_wide = H > kSeqMaxH && H <= kSeqMaxHWide;
-    if (plan->seq_wide) plan->max_wavefront = 1;  // W_hh and W_ih of a second layer would not fit a wavefront's registers
+    // Of two layers W_hh and the upper one's W_ih are 192 registers a lane at 32 columns, 144 at 24.  A second layer in the same launch takes a
+    // step from two exchanges to one (us, a launch per layer / both in one: two layers of 1136, 31 steps 130 / 99 and 4 steps 34 /
+    // 25; of 1704, 44 steps 200 / 154; of 2048, 50 steps 236 / 171, where 26 registers of a lane are spilled; three of 1280, 40 steps 254 / 212).
+    if (plan->seq_wide) plan->max_wavefront = 2;
     PLAN_HIP_CHECK(hipMalloc(&plan->bsum_all, sizeof(float) * 4 * H * plan->cells.size()));
     for (int l = 0; l < num_layers; ++l) {
         for (int d = 0; d < D; ++d) {
@@ -242,9 +254,10 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
     }
     PLAN_HIP_CHECK(hipGetLastError());
     // Cells whose input projection runs as a batch over the sequence (every layer of a bidirectional stack, the first
-    // layer of every wavefront group of a unidirectional one) get a copy of w_ih in MFMA fragment order.
+    // layer of every wavefront group of a unidirectional one, any layer above kSeqMaxH units, where one with a residual sum runs alone)
+    // get a copy of w_ih in MFMA fragment order.
     for (int l = 0; l < num_layers; ++l) {
-        if (D == 1 && l % plan->max_wavefront != 0) continue;
+        if (D == 1 && !plan->seq_wide && l % plan->max_wavefront != 0) continue;
         for (int d = 0; d < D; ++d) {
             PimHipLstmPlan::Cell& c = plan->cells[(size_t)l * D + d];
             int ntiles = 0;
@@ -280,7 +293,7 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
         plan->seq_kernel_ok = (int64_t)per_cu * plan->num_cus >= plan->seq_blocks;
     } else if (plan->seq_wide) {
         int per_cu = 0;
-        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, lstm_seq_f16_kernel<2, false, 8, 32>, 512, 0));
+        PLAN_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, seq_wide_kernel(D, D == 1 && num_layers >= 2 ? 2 : D, H), 512, 0));
         plan->seq_kernel_ok = (int64_t)per_cu * plan->num_cus >= (plan->seq_blocks + 1) / 2;
     }
     if (plan->seq_kernel_ok && !plan->seq_wide) {
@@ -758,11 +771,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             a.spin_limit = plan->spin_limit;
             const dim3 grid(plan->seq_blocks), block(256);
             if (plan->seq_wide) {
-                const dim3 grid8((unsigned)((H + 7) / 8)), block8(512);
-                if (D == 2)
-                    lstm_seq_f16_kernel<2, false, 8, 32><<<grid8, block8, 0, s>>>(a);
-                else
-                    lstm_seq_f16_kernel<1, true, 8, 32><<<grid8, block8, 0, s>>>(a);  // max_wavefront == 1
+                seq_wide_kernel(D, nc, H)<<<dim3((unsigned)((H + 7) / 8)), dim3(512), 0, s>>>(a);
             } else if (D == 2) {
                 lstm_seq_f16_kernel<2, false><<<grid, block, 0, s>>>(a);
             } else {

@@ -259,7 +259,8 @@ __global__ __launch_bounds__(WAVES * 64) void lstm_step_pair_f16_kernel(LstmStep
 // ---------------------------------------------------------------------------------------------
 static constexpr int kSeqUnits = 4;        // hidden units per block, one per wavefront
 static constexpr int kSeqMaxH = 1024;      // 64 lanes x 16 columns
-static constexpr int kSeqMaxHWide = 2048;  // 64 lanes x 32 columns (eight units per block; one layer, or the two directions of one)
+static constexpr int kSeqMaxHWide = 2048;  // 64 lanes x 32 columns (eight units per block; two layers, or the two directions of one)
+static constexpr int kSeqMaxHMiddle = 1536; // 64 lanes x 24 columns (the same)
 static constexpr int kSeqEntryWords = 16;  // 32-bit words between the entries of consecutive blocks (64 bytes)
 static constexpr int kSeqMaxT = 1 << 30;    // super-steps per launch (the counters are 32-bit)
 static constexpr int kSeqMaxChains = 4;
@@ -293,7 +294,7 @@ template <int NC, bool WAVEFRONT, int UNITS = kSeqUnits, int COLS = 16>
 __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
 {
     static_assert(UNITS == 4 || UNITS == 8, "one or two 8-byte words per chain and block");
-    static_assert(COLS == 16 || COLS == 32, "columns of a weight row per lane");
+    static_assert(COLS == 16 || COLS == 24 || COLS == 32, "columns of a weight row per lane");
     constexpr int MAXH = 64 * COLS;  // widest hidden state this instantiation takes
     constexpr int CH = COLS / 8;     // 16-byte pieces of a weight row per lane
     static_assert(MAXH <= 64 * UNITS * UNITS, "lane t of a block fetches the entry of block t");
@@ -323,10 +324,10 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
     const bool poisoned = __builtin_amdgcn_readfirstlane(__hip_atomic_load(p.abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) != 0u;
     if (tid == 0) block_gave_up = poisoned ? 1 : 0;
 
-    // The 16-byte pieces of a row that a lane has: with 32 columns neighbouring lanes take neighbouring pieces (in one run per lane the
+    // The 16-byte pieces of a row that a lane has: with 24 or 32 columns neighbouring lanes take neighbouring pieces (in one run per lane the
     // reads of h from LDS met four to a bank: 1424 units, two directions, 98 steps 351 -> 341 us, one layer of 1688, 100 steps 230.5 ->
     // 228.7), with 16 one run (two to a bank; the other way 2 to 5 % faster with two chains and 1.5 % slower with four).
-    auto piece_of = [&](int c) { return COLS == 32 ? 64 * c + lane : lane * CH + c; };
+    auto piece_of = [&](int c) { return COLS != 16 ? 64 * c + lane : lane * CH + c; };
     // ---- weights into registers: per chain the four gate rows of unit j ----
     // Accumulator slot v holds gate {i, g, f, o}[v]: the transpose-sum below then leaves gate k in lane k.
     half8_t w_hh[NC][4][CH];

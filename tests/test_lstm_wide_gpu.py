@@ -1,0 +1,56 @@
+"""Layers of 1025 to 2048 units by the all-CU kernel: two of a stack in one launch as a wavefront, with 24 and 32 columns of
+a row to a lane, at the edges of both; a layer left over, few steps, sums around a layer, two directions; and every wait
+giving up.  Against the recurrence in 64 bits with h rounded to fp16 after every step, as the kernels hand it on: they
+differ where a rounding turns, 2^-11 of |h| <= 1 each, which the steps and layers that follow carry along (c adds up at
+most T of them); 4e-3 is eight of them.
+"""
+import pytest
+import torch
+
+from pimaicompiler_amd import workloads
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def in_64_bits(params, x, h0, c0, L, D, res):
+    seq, hn, cn = x.double(), [], []
+    for l in range(L):
+        outs = []
+        for d in range(D):
+            w_ih, w_hh, b_ih, b_hh = (p.to(DEV).double() for p in params[4 * (l * D + d):4 * (l * D + d) + 4])
+            h, c, ys = h0[l * D + d].double(), c0[l * D + d].double(), []
+            gates_in = seq @ w_ih.t() + b_ih + b_hh
+            for t in (range(seq.size(0)) if d == 0 else range(seq.size(0) - 1, -1, -1)):
+                i, f, g, o = (gates_in[t] + w_hh @ h).chunk(4)
+                c = torch.sigmoid(f) * c + torch.sigmoid(i) * torch.tanh(g)
+                h = (torch.sigmoid(o) * torch.tanh(c)).half().double()
+                ys.append(h)
+            outs.append(torch.stack(ys if d == 0 else ys[::-1]))
+            hn.append(h)
+            cn.append(c)
+        y = torch.cat(outs, 1)
+        seq = (y + seq).half().double() if res is not None and l >= res else y
+    return seq, torch.stack(hn), torch.stack(cn)
+
+
+@pytest.mark.parametrize("H,L,D,T,res", [(1032, 2, 1, 2, None), (1032, 3, 1, 7, None), (1536, 2, 1, 9, None), (1544, 2, 1, 9, None), (2048, 2, 1, 5, None), (1136, 4, 1, 3, None),
+                                             (1536, 4, 1, 5, 2), (1136, 3, 1, 4, 1), (1040, 1, 1, 9, None), (1536, 1, 2, 6, None), (1544, 2, 2, 3, None)])
+@pytest.mark.parametrize("gives_up", [False, True])
+def test_wide_layers(ops, H, L, D, T, res, gives_up):
+    if gives_up and (H * T > 10000 or L > 3):
+        pytest.skip("a workgroup computes the stack by itself: milliseconds per step")
+    params, x, h0, c0 = workloads.lstm_inputs(H + L, 64, H, L, D == 2, T)
+    g = torch.Generator().manual_seed(H)
+    x, h0, c0 = (v.half().to(DEV) for v in (x.reshape(T, 64), 0.3 * torch.randn(L * D, H, generator=g), torch.randn(L * D, H, generator=g)))
+    plan = ops.LstmPlan([p.to(DEV) for p in params], True, L, D == 2, T)
+    plan.set_mode(2)
+    if res is not None:
+        plan.set_residual(res)
+    if gives_up:
+        plan.set_spin_limit(0)
+    want = in_64_bits(params, x, h0, c0, L, D, res)
+    for _ in range(1 if gives_up else 3):
+        for got, w in zip(plan.forward(x, h0, c0), want):
+            assert float((got.double().reshape(w.shape) - w).abs().max()) <= 4e-3
+        plan.status()
