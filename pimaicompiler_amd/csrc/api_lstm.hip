@@ -814,6 +814,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
             const unsigned grid = (unsigned)((H + 3) / 4);
             // what a step's launch reads: W_hh, and W_ih when the projection is made in the same kernel
             const int keep = (unsigned long long)D * (unsigned long long)(4 * H) * (unsigned long long)(H + (fuse_xproj ? in_w : 0)) * sizeof(half_t) <= kKeepCachedBytes;
+            const bool sum_in_step = residual(l) && T == 1;
             LstmStepPair p2;
             memset(&p2, 0, sizeof(p2));
             for (int64_t step = 0; step < T; ++step) {
@@ -844,11 +845,11 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
                     const LstmStepDir& sd = p2.dir[0];
                     launch_kernel(
                         keep ? lstm_step_f16_kernel<4, true> : lstm_step_f16_kernel<4, false>, dim3(grid), 256, s, sd.w_ih, sd.w_hh, sd.bsum, sd.xproj,
-                        sd.x, sd.h_prev, sd.c_in_f16, sd.c_state, sd.h_out, sd.hn_f16, sd.cn_f16, (int)in_w, (int)H);
+                        sd.x, sd.h_prev, sd.c_in_f16, sd.c_state, sd.h_out, sd.hn_f16, sd.cn_f16, sum_in_step ? sd.x : (const half_t*)nullptr, (int)in_w, (int)H);
                 }
             }
             PIMHIP_HIP_CHECK(hipGetLastError());
-            if (residual(l)) {
+            if (residual(l) && !sum_in_step) {
                 add_input(layer_out, layer_in);
                 PIMHIP_HIP_CHECK(hipGetLastError());
             }

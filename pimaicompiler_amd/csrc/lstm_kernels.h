@@ -117,12 +117,14 @@ __device__ __forceinline__ void lstm_step_sums(float (&acc)[4], const half_t* __
     }
 }
 
-// One step of one direction: hidden unit j per wavefront.
+// One step of one direction: hidden unit j per wavefront.  residual (or null): the layer's input, where its output is h plus that.  Only for a
+// call's single step, as a next one would read h from h_out (MI355X, us a call of one step, with a launch for each sum -> in here: two layers
+// of 512, one sum 12.6 -> 8.1; four of 768, three sums 26.2 -> 19.0; three of 1024, two 19.8 -> 15.1; three of 1600, two 30.2 -> 26.7).
 template <int WAVES, bool KEEP>
 __device__ __forceinline__ void lstm_step_body(const half_t* __restrict__ w_ih, const half_t* __restrict__ w_hh, const float* __restrict__ bsum,
                                                const float* __restrict__ xproj, const half_t* __restrict__ x, const half_t* __restrict__ h_prev,
                                                const half_t* __restrict__ c_in_f16, float* __restrict__ c_state, half_t* __restrict__ h_out,
-                                               half_t* __restrict__ hn_f16, half_t* __restrict__ cn_f16, int I, int H)
+                                               half_t* __restrict__ hn_f16, half_t* __restrict__ cn_f16, const half_t* __restrict__ residual, int I, int H)
 {
     const int lane = threadIdx.x & 63;
     const int j = blockIdx.x * WAVES + (threadIdx.x >> 6);
@@ -137,6 +139,7 @@ __device__ __forceinline__ void lstm_step_body(const half_t* __restrict__ w_ih, 
     else if (bsum)
         addend = bsum[(long)gate * H + j];
     const float c_prev = c_in_f16 ? (float)c_in_f16[j] : c_state[j];
+    const half_t below = residual ? residual[j] : (half_t)0.0f;
 
     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     lstm_step_sums<KEEP>(acc, w_ih, w_hh, xproj, x, h_prev, I, H, j, lane);
@@ -162,7 +165,7 @@ __device__ __forceinline__ void lstm_step_body(const half_t* __restrict__ w_ih, 
     const half_t h_new = (half_t)(g_o * (2.0f * fast_sigmoid_f32(2.0f * c_new) - 1.0f));
     if (lane == 0) {
         c_state[j] = c_new;
-        h_out[j] = h_new;
+        h_out[j] = residual ? (half_t)((float)h_new + (float)below) : h_new;
         if (hn_f16) hn_f16[j] = h_new;
         if (cn_f16) cn_f16[j] = (half_t)c_new;
     }
@@ -174,9 +177,9 @@ __global__ __launch_bounds__(WAVES * 64) void lstm_step_f16_kernel(
     const half_t* __restrict__ w_ih, const half_t* __restrict__ w_hh, const float* __restrict__ bsum,
     const float* __restrict__ xproj, const half_t* __restrict__ x, const half_t* __restrict__ h_prev,
     const half_t* __restrict__ c_in_f16, float* __restrict__ c_state, half_t* __restrict__ h_out,
-    half_t* __restrict__ hn_f16, half_t* __restrict__ cn_f16, int I, int H)
+    half_t* __restrict__ hn_f16, half_t* __restrict__ cn_f16, const half_t* __restrict__ residual, int I, int H)
 {
-    lstm_step_body<WAVES, KEEP>(w_ih, w_hh, bsum, xproj, x, h_prev, c_in_f16, c_state, h_out, hn_f16, cn_f16, I, H);
+    lstm_step_body<WAVES, KEEP>(w_ih, w_hh, bsum, xproj, x, h_prev, c_in_f16, c_state, h_out, hn_f16, cn_f16, residual, I, H);
 }
 
 // The same step of both directions of a bidirectional layer (blockIdx.y), which depend on nothing of each other: a short step is
@@ -203,7 +206,7 @@ template <int WAVES, bool KEEP>
 __global__ __launch_bounds__(WAVES * 64) void lstm_step_pair_f16_kernel(LstmStepPair p, int I, int H)
 {
     const LstmStepDir& d = p.dir[blockIdx.y];
-    lstm_step_body<WAVES, KEEP>(d.w_ih, d.w_hh, d.bsum, d.xproj, d.x, d.h_prev, d.c_in_f16, d.c_state, d.h_out, d.hn_f16, d.cn_f16, I, H);
+    lstm_step_body<WAVES, KEEP>(d.w_ih, d.w_hh, d.bsum, d.xproj, d.x, d.h_prev, d.c_in_f16, d.c_state, d.h_out, d.hn_f16, d.cn_f16, nullptr, I, H);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -221,7 +224,7 @@ __global__ __launch_bounds__(WAVES * 64) void lstm_step_pair_f16_kernel(LstmStep
 // Grid: NB = ceil(H / UNITS) blocks of UNITS wavefronts (H <= 1024, H % 8 == 0; UNITS = 4, or 8 for a single chain,
 // whose entry then still is one 16-byte store and load and whose exchange among half as many blocks is about 0.4 us
 // shorter), all resident at once.  Hidden sizes up to 2048 run with COLS = 32 columns of a weight row per lane and eight
-// units per block (256 blocks at most), for one layer or the two directions of one (a second layer's W_ih would spill).  The text below is written for UNITS = 4.  Block b owns
+// units per block (256 blocks at most; 24 columns up to 1536), for up to two layers or the two directions of one.  The text below is written for UNITS = 4.  Block b owns
 // hidden units 4b .. 4b+3 of every chain, one unit per wavefront: wavefront w keeps, per chain, the four W_hh
 // gate rows of unit 4b+w (and the four W_ih rows for wavefront chains k > 0) in registers for the whole
 // launch (lane l holds columns 16l .. 16l+15 of each row) and the cell states in registers.
