@@ -243,7 +243,8 @@ int pimhip_lstm_plan_set_mode(PimHipLstmPlan* plan, int mode);
 
 /* No counterpart in the reference beyond the above.  enabled == 0: automatic mode stops measuring and forgets what it
  * measured (thresholds choose); != 0 (the default): it measures as described.  pimhip_lstm_plan_measured_mode: the mode
- * automatic mode uses for sequences of seq_len (>= 2) steps, 0 if that range of lengths has not been measured yet. */
+ * automatic mode uses for sequences of seq_len (>= 2) steps, 0 if that range of lengths (two; three; four to seven; ...)
+ * has not been measured yet. */
 int pimhip_lstm_plan_set_measure(PimHipLstmPlan* plan, int enabled);
 int pimhip_lstm_plan_measured_mode(PimHipLstmPlan* plan, int64_t seq_len, int* mode);
 

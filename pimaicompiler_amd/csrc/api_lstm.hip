@@ -64,8 +64,9 @@ struct PimHipLstmPlan {
     // kernels whose workgroups wait for one another.
     unsigned long long gave_up_events = 0;
     bool safe_only = false;
-    // Automatic mode: the kernel family measured fastest on this plan for sequence lengths in [2^b, 2^(b+1)), 0 = not
-    // measured yet (pimhip_lstm_forward measures on the first eager call of a bucket; see measured_mode below).
+    // Automatic mode: the kernel family measured fastest on this plan for sequence lengths in [2^b, 2^(b+1)), for b = 0 of two
+    // steps (which a launch per step makes without one for the projection; b = 1 is three), 0 = not measured yet
+    // (pimhip_lstm_forward measures on the first eager call of a bucket; see measured_mode below).
     unsigned char measured_mode[32] = {};
     bool measure = true;             // pimhip_lstm_plan_set_measure
     hipEvent_t tune_event[2] = {nullptr, nullptr};
@@ -92,6 +93,14 @@ auto seq_wide_kernel(int dirs, int chains, int64_t hidden)
 }
 
 constexpr unsigned long long kLstmEventsBeforeSafe = 3;
+
+// The entry of PimHipLstmPlan::measured_mode for T >= 2 steps.
+int measured_bucket(int64_t T)
+{
+    int bucket = 0;
+    while (T > 2 && (T >> (bucket + 1)) != 0 && bucket < 31) ++bucket;
+    return bucket;
+}
 }
 
 namespace
@@ -531,8 +540,7 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
     if (mode == 0 && T >= 2) {
         // Automatic: what was measured fastest on this plan for sequences of about this length; failing that (nothing
         // measured yet and no way to measure now) the thresholds above.
-        int bucket = 0;
-        while ((T >> (bucket + 1)) != 0 && bucket < 31) ++bucket;
+        const int bucket = measured_bucket(T);
         if (plan->measured_mode[bucket] == 0 && plan->measure && !capturing && forced_mode < 0 && (xcd_takes_it || seq_takes_it)) {
             rc = measure_modes(plan, x, h0, c0, y, hn, cn, seq_len, stream, bucket, xcd_takes_it, seq_takes_it);
             if (rc != PIMHIP_OK) return rc;
@@ -565,8 +573,12 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
         PIMHIP_HIP_CHECK(hipGetLastError());
         plan->reset_exchange = false;
     }
-    // seq_len == 1: fuse the input projection into the step (one launch per layer and direction).
-    const bool fuse_xproj = !use_seq && T == 1;
+    // One step, and two of a layer or of both directions: each step's launch makes its projection too.  Two steps then read W_ih
+    // twice, but the projection's launch is saved (us, automatic mode, before / after: one layer of 1024 11.4 / 9.5, over 2048
+    // inputs 15.5 / 11.4, of 128 unchanged; two directions of 512 12.0 / 8.9, of 1024 14.4 / 11.0, two layers of both directions of
+    // 512 24.0 / 15.0).  Of three steps one layer of 512 is slower so, 11.7 / 13.3 (one launch for all of them is the faster
+    // mode), and of two a stack of one direction, two layers of 1024 15.3 / 16.7.
+    const bool fuse_xproj = !use_seq && (T == 1 || (T == 2 && (D == 2 || L == 1)));
 
     const half_t* layer_in = (const half_t*)x;
     const long y_stride = (long)D * H;
@@ -918,8 +930,6 @@ extern "C" int pimhip_lstm_plan_measured_mode(PimHipLstmPlan* plan, int64_t seq_
 {
     if (!plan || !mode) return fail(PIMHIP_ERR_INVALID_ARGUMENT, "plan and mode must be non-null");
     if (seq_len < 2) return fail(PIMHIP_ERR_INVALID_ARGUMENT, "seq_len=%lld: one step has one kernel", (long long)seq_len);
-    int bucket = 0;
-    while ((seq_len >> (bucket + 1)) != 0 && bucket < 31) ++bucket;
-    *mode = plan->measured_mode[bucket];
+    *mode = plan->measured_mode[measured_bucket(seq_len)];
     return PIMHIP_OK;
 }
