@@ -42,10 +42,10 @@ std::vector<PimHipRnntPlan*> g_rnnt_plans;
 
 constexpr unsigned long long kRnntEventsBeforeAlone = 3;  // waits given up before a plan stops exchanging for good
 
-auto greedy_kernel(int64_t vocab, int64_t layers, int64_t joint)
+auto greedy_kernel(int64_t vocab, int64_t layers, int64_t joint, int64_t frames)
 {
-    const bool every = rnnt_greedy_every(vocab, layers);
-    switch (rnnt_greedy_own_rows(vocab, joint, layers)) {
+    const bool every = rnnt_greedy_every(vocab, layers, frames);
+    switch (rnnt_greedy_own_rows(vocab, joint, layers, frames)) {
         case 4: return joint <= 512 ? rnnt_greedy_f16_kernel<0, true, 4, 1> : rnnt_greedy_f16_kernel<0, true, 4, 2>;
         case 8: return rnnt_greedy_f16_kernel<1, true, 8, 1>;
         default: break;
@@ -61,7 +61,7 @@ auto greedy_kernel(int64_t vocab, int64_t layers, int64_t joint)
 size_t exchange_words32(const PimHipRnntPlan* plan) { return (size_t)2 * plan->blocks * kRnntEntryWords * 2; }
 size_t greedy_every_words32(const PimHipRnntPlan* plan)
 {
-    return rnnt_greedy_every(plan->vocab, plan->num_layers) ? (size_t)kRnntGreedyVersions * (plan->hidden / 8) * rnnt_every_words((int)plan->vocab) * 2 : 0;
+    return rnnt_greedy_every_fits(plan->vocab, plan->num_layers) ? (size_t)kRnntGreedyVersions * (plan->hidden / 8) * rnnt_every_words((int)plan->vocab) * 2 : 0;
 }
 size_t greedy_exchange_words32(const PimHipRnntPlan* plan)
 {
@@ -191,9 +191,12 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
         const int n_vocab = (int)((vocab + 7) / 8);
         const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
         plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);
-        int greedy_per_cu = 0;
-        RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, greedy_kernel(vocab, num_layers, joint_size), kRnntThreads, 0));
-        plan->greedy_resident = (int64_t)greedy_per_cu * st->num_cus >= greedy_blocks(plan);
+        plan->greedy_resident = true;
+        for (const int64_t frames : {(int64_t)1, (int64_t)INT32_MAX}) {  // the kernels for few and for many
+            int greedy_per_cu = 0;
+            RNNT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&greedy_per_cu, greedy_kernel(vocab, num_layers, joint_size, frames), kRnntThreads, 0));
+            plan->greedy_resident = plan->greedy_resident && (int64_t)greedy_per_cu * st->num_cus >= greedy_blocks(plan);
+        }
     }
     RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->greedy), sizeof(unsigned int) * (greedy_exchange_words32(plan) + greedy_count_words32(plan))));
     RNNT_HIP_CHECK(hipMalloc(reinterpret_cast<void**>(&plan->abort_flag), sizeof(unsigned int)));
@@ -410,9 +413,11 @@ extern "C" int pimhip_rnnt_greedy_decode(PimHipRnntPlan* plan, const void* enc, 
         if (rc != PIMHIP_OK) return rc;
     }
     // fill kernels, not memsets: the call can be recorded into a HIP graph
-    launch_fill_u32(plan->greedy, greedy_exchange_words32(plan), ~0u, s);
+    // (the words of every symbol, the last of them, only for a kernel that has them)
+    const size_t unused = rnnt_greedy_every(plan->vocab, plan->num_layers, n_frames) ? 0 : greedy_every_words32(plan);
+    launch_fill_u32(plan->greedy, greedy_exchange_words32(plan) - unused, ~0u, s);
     launch_fill_u32(plan->greedy + greedy_exchange_words32(plan), greedy_count_words32(plan), 0u, s);
-    greedy_kernel(plan->vocab, plan->num_layers, plan->joint_size)<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
+    greedy_kernel(plan->vocab, plan->num_layers, plan->joint_size, n_frames)<<<dim3(a.alone ? 1u : (unsigned)greedy_blocks(plan)), dim3(kRnntThreads), 0, s>>>(a);
     PIMHIP_HIP_CHECK(hipGetLastError());
     return PIMHIP_OK;
 }

@@ -19,7 +19,7 @@
 //     travels with the hand-over that ends the step and every workgroup keeps the same loop state (t, symbols so far, ..);
 //   * a layer's blocks also collect their own layer's h (what W_hh multiplies at the next symbol) and sum W_hh . h right
 //     then, long before the next symbol is known;
-//   * the first layer does not wait for the decision either (up to kRnntGreedyEveryVocab symbols): its blocks keep the gates' sums over
+//   * the first layer does not wait for the decision either (rnnt_greedy_every in rnnt_plan.h): its blocks keep the gates' sums over
 //     every symbol's embedding row, make h for every symbol as soon as the h before it is known, a symbol to a lane, and publish them
 //     all; who needs the first layer's h reads the decided symbol's words, which are there already.  A symbol's chain loses a cell (0.7 us) and
 //     the way of a store (0.4 us);
@@ -34,7 +34,7 @@
 //     CUs that no other role needs hold up to eleven further copies of W2's rows, team q takes the steps that are q modulo the
 //     number of teams, and the steps published ahead become logits side by side;
 //   * the decision behind a symbol, which everybody waits for while nothing else is there, is not waited for from the symbol blocks: with
-//     up to 64 symbols the blocks of layers and joint network read the hidden vector and make it themselves (decided_alone).
+//     up to 64 symbols (rnnt_greedy_own_rows) the blocks of layers and joint network read the hidden vector and make it themselves (decided_alone).
 //
 // Measured on MI355X, us an utterance of 341 frames (2 x 320 units, 512 joint units, 29 symbols) with 74 / 114 symbols emitted: 739 /
 // 996 with a hand-over of the first layer's h and of the logits per symbol, 667 / 905 without the first, 618 / 814 without both, 581 / 784
@@ -74,6 +74,7 @@
 #include <type_traits>
 
 #include "rnnt_kernels.h"
+#include "rnnt_plan.h"
 
 namespace pimhip
 {
@@ -95,33 +96,10 @@ static_assert(kRnntGreedyLook + kRnntGreedyAhead < kRnntGreedyLogitRing, "a look
 static_assert(kRnntGreedyLook == kRnntWaves && kRnntGreedyLook == 8, "a wavefront per step");
 static_assert(kRnntGreedyBatch <= kRnntWaves, "a wavefront stores one step's word of a batch");
 constexpr int kRnntGreedyMaxVocab = 512;           // symbols
-constexpr int kRnntGreedyRowVocab = 5;             // up to this many symbol blocks to a team (15 words) a step's logits are a row of 16 lanes'
-constexpr int kRnntGreedyRows = 4;                 // ... and a pass looks at as many steps
+constexpr int kRnntGreedyRows = 4;                 // steps that a pass looks at where a step's logits are a row of 16 lanes'
 constexpr int kRnntGreedyLaneWords = 3;            // at most this many words of a step's logits to a lane where a wavefront takes them
 static_assert(3 * (kRnntGreedyMaxVocab / 8) <= 64 * kRnntGreedyLaneWords, "a wavefront takes a step's logits");
-// The kernel for a vocabulary: 0 where a step's words fit a row of 16 lanes, else how many of them a lane of a wavefront takes.
-inline int rnnt_greedy_lane_words(int64_t vocab)
-{
-    const int64_t blocks = (vocab + 7) / 8;
-    return blocks <= kRnntGreedyRowVocab ? 0 : (int)((3 * blocks + 63) / 64);
-}
 constexpr int kRnntGreedyEmbHalfs = 16384;         // embedding rows kept in LDS by the first layer's blocks (32 KB)
-// Whether the first layer runs for every symbol ahead of the decision.  It takes the layer's cell and the store's way off a symbol's
-// chain (start -> now, us an utterance; 512 joint units, 200 frames unless said): two layers of 320, 29 symbols, 341 frames with 74 and 114
-// symbols emitted 739 -> 667 and 996 -> 905; 64 symbols 536 -> 491; 100 symbols 533 -> 491 and, with 34 emitted, 395 -> 387.  With one
-// layer the chain is too short for the cells of more than a symbol a lane: 29 symbols 406 -> 377, one layer of 512 and 128
-// symbols 458 -> 449 and, with 27 emitted, 316 -> 325.
-constexpr int kRnntGreedyEveryVocab = 128;
-inline bool rnnt_greedy_every(int64_t vocab, int64_t layers) { return vocab <= (layers == 1 ? 64 : kRnntGreedyEveryVocab); }
-// Rows of W2 that a wavefront of every block holds, for the decision behind a symbol; 0: that decision waits for the symbol blocks.  (us
-// an utterance, without -> with: two layers of 320, 512 joint units, 29 symbols, 341 frames with 74 and 114 symbols emitted 660 -> 618
-// and 905 -> 814, 200 frames with 64 symbols 480 -> 462.  One layer 347 -> 354: there the decision is not what the next symbol waits
-// for.  640 joint units and 64 symbols, 64 more registers: 449 -> 442 with 47 symbols emitted and 283 -> 292 with 20.)
-inline int rnnt_greedy_own_rows(int64_t vocab, int64_t joint, int64_t layers)
-{
-    if (layers < 2) return 0;
-    return vocab <= 32 && joint <= 1024 ? 4 : vocab <= 64 && joint <= 512 ? 8 : 0;
-}
 // 8-byte words that a block of the first layer publishes its units' h after every symbol in: three a symbol, whole 128-byte lines.
 __host__ __device__ inline int rnnt_every_words(int vocab) { return (3 * vocab + 15) & ~15; }
 constexpr int kRnntSeenStride = 16;                // 32-bit words between the blocks' `seen` counts

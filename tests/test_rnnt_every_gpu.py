@@ -17,7 +17,7 @@ pytestmark = pytest.mark.gpu
     (3, 64, 64, 29), (4, 72, 64, 100),
 ])
 def test_the_first_layer_ahead_of_the_decision(ops, L, I, H, V, run_prediction_first):
-    F, J, T, blank = 128, 64, 40, V // 2
+    F, J, T, blank = 128, 64, 64, V // 2   # (frames enough for every one of these vocabularies)
     params, joint, enc, embedding, x0 = model(31 * V + H + L, L, I, H, F, J, V, T, blank, 0.1 if V > 2 else -0.3)
     plan = ops.RnntPlan(dev(params), True, L, tuple(dev(joint)))
     g = torch.Generator().manual_seed(V)
