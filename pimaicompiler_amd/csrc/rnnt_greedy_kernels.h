@@ -883,11 +883,13 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         const half8_t* rows = reinterpret_cast<const half8_t*>(p.w1 + (long)8 * jb * (p.F + H));
         const long row_step = (long)(nfp + nhp);
         // Frames of up to two pieces a lane (1024 wide): a wavefront takes a frame, with all eight rows in registers (every wavefront
-        // reading every frame for a row of its own is 128 KB a round through the CU's 64 bytes a clock).  Longer ones: a row each.
-        constexpr int kShort = 2;
-        const bool short_frames = nfp <= 64 * kShort;
+        // reading every frame for a row of its own is 128 KB a round through the CU's 64 bytes a clock).  Longer ones: a row each, and so
+        // where there are no more frames than such a round asks for, and the eight rows to a wavefront would be the 128 KB (us a call of
+        // 1 / 2 / 3 frames, two layers of 320, 29 symbols, no first run, a frame / a row each: 13.4 / 12.4, 14.0 / 13.8, 14.1 / 13.5; at six 15.1 / 16.0).
+        constexpr int kShort = 2, kLongAsk = 4;
+        const bool short_frames = nfp <= 64 * kShort && p.T > kLongAsk;
         // One array for both kinds: eight short rows and a short frame's pieces behind them, or a long row and four long frames'.
-        constexpr int kColShort = 8 * kShort, kColLong = kRnntFC, kRegs = 5 * kRnntFC;
+        constexpr int kColShort = 8 * kShort, kColLong = kRnntFC, kRegs = (1 + kLongAsk) * kRnntFC;
         static_assert(kColShort + kShort <= kRegs, "both fit");
         half8_t reg[kRegs], wg[kRnntHC];
         if (short_frames) {
@@ -898,7 +900,10 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             }
         } else {
 #pragma unroll
-            for (int k = 0; k < kRnntFC; ++k) reg[k] = rows[wave * row_step + min(lane + 64 * k, nfp - 1)];
+            for (int k = 0; k < kRnntFC; ++k) {
+                if (64 * k >= nfp) break;
+                reg[k] = rows[wave * row_step + min(lane + 64 * k, nfp - 1)];
+            }
         }
 #pragma unroll
         for (int k = 0; k < kRnntHC; ++k) {
@@ -907,15 +912,13 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
         }
         ask_for_w2();
         const float bias = p.b1 ? (float)p.b1[8 * jb + wave] : 0.0f;
-        for (int i = tid; i < H; i += kRnntThreads) own[i] = p.h0 ? p.h0[(long)(p.L - 1) * H + i] : (half_t)0.0f;  // g before the first run
-        __syncthreads();
         float* const over_f = reinterpret_cast<float*>(emb);           // [kRnntGreedyFrames][8]: sums over frames f_lo .. af_hi (where the first layer's blocks have the embedding rows)
         float* const over_g = over_f + kRnntGreedyFrames * 8;          // [8]: over g, with the bias
         int af_hi = 0, af_seen = 0;                                    // frames summed so far; those whose sums every wavefront sees
         // The next frames are asked for in front of a wait and summed behind it (their columns travel while the symbol blocks work).
         int n_ask = 0;
         auto ask = [&]() __attribute__((always_inline)) {
-            n_ask = max(0, min(min(short_frames ? kRnntWaves : 4, p.T - af_hi), s.t + kRnntGreedyFramesAhead - af_hi));
+            n_ask = max(0, min(min(short_frames ? kRnntWaves : kLongAsk, p.T - af_hi), s.t + kRnntGreedyFramesAhead - af_hi));
             if (n_ask == 0) return;
             if (short_frames) {
                 const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)(af_hi + min(wave, n_ask - 1)) * p.F);
@@ -923,10 +926,14 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 for (int k = 0; k < kShort; ++k) reg[kColShort + k] = f8[min(lane + 64 * k, nfp - 1)];   // (a lane past the frame's end keeps nothing of it)
             } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)(af_hi + min(q, n_ask - 1)) * p.F);
+                for (int q = 0; q < kLongAsk; ++q) {
+                    if (q >= n_ask) break;
+                    const half8_t* f8 = reinterpret_cast<const half8_t*>(p.enc + (long)(af_hi + q) * p.F);
 #pragma unroll
-                    for (int k = 0; k < kRnntFC; ++k) reg[kColLong + q * kRnntFC + k] = f8[min(lane + 64 * k, nfp - 1)];
+                    for (int k = 0; k < kRnntFC; ++k) {
+                        if (64 * k >= nfp) break;
+                        reg[kColLong + q * kRnntFC + k] = f8[min(lane + 64 * k, nfp - 1)];
+                    }
                 }
             }
         };
@@ -946,8 +953,9 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
                 }
             } else {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
+                for (int q = 0; q < kLongAsk; ++q) {
                     lo[q] = 0.0f;
+                    if (q >= n_ask) continue;
 #pragma unroll
                     for (int k = 0; k < kRnntFC; ++k)
                         if (lane + 64 * k < nfp) lo[q] = dot8(reg[k], reg[kColLong + q * kRnntFC + k], lo[q]);
@@ -967,6 +975,10 @@ __global__ __launch_bounds__(kRnntThreads) void rnnt_greedy_f16_kernel(const Rnn
             af_hi += n_ask;
             n_ask = 0;
         };
+        ask();                    // (the first frames travel with the weights)
+        for (int i = tid; i < H; i += kRnntThreads) own[i] = p.h0 ? p.h0[(long)(p.L - 1) * H + i] : (half_t)0.0f;  // g before the first run
+        __syncthreads();
+        keep();
         int have_g = -1;          // the version of g whose sums are in over_g
         int pub = 0;              // the next step to publish a hidden vector for
         // (barriers between the sums' writers and their readers: this one, and those of the waits)

@@ -47,3 +47,18 @@ def test_chunks_on_both_sides_of_the_line(ops, L, I, H, J, V, chunks):
         if r[3]:
             break
     assert r[3] == 1 and plan.fallbacks()[0] >= 1
+
+
+@pytest.mark.parametrize("first", [True, False])
+@pytest.mark.parametrize("F", [8, 512, 520, 1024, 1032, 1536, 1544, 2048])
+@pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 9])
+def test_frames_summed_by_rows_and_by_frames(ops, F, T, first):
+    """No more frames than a round asks for and more of them, of every number of 16-byte pieces to a lane, the last of them whole and not."""
+    L, H, J, V, blank = 1, 64, 64, 29, 3
+    params, joint, enc, embedding, x0 = model(F + T, L, H, H, F, J, V, T, blank, 0.1)
+    plan = ops.RnntPlan(dev(params), True, L, tuple(dev(joint)))
+    g = torch.Generator().manual_seed(T)
+    h, c = (0.3 * torch.randn(L, H, generator=g)).half().to(DEV), torch.randn(L, H, generator=g).half().to(DEV)
+    want = loop_driven_from_the_host(plan, enc, embedding, x0, blank, 3, 3 * T, h, c, first)
+    for _ in range(2):
+        check(plan.greedy_decode(enc, embedding, x0, blank, 3, h0=h, c0=c, run_prediction_first=first), want)
