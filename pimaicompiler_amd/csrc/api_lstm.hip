@@ -573,13 +573,6 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
         PIMHIP_HIP_CHECK(hipGetLastError());
         plan->reset_exchange = false;
     }
-    // One step, and two of a layer or of both directions: each step's launch makes its projection too.  Two steps then read W_ih
-    // twice, but the projection's launch is saved (us, automatic mode, before / after: one layer of 1024 11.4 / 9.5, over 2048
-    // inputs 15.5 / 11.4, of 128 unchanged; two directions of 512 12.0 / 8.9, of 1024 14.4 / 11.0, two layers of both directions of
-    // 512 24.0 / 15.0).  Of three steps one layer of 512 is slower so, 11.7 / 13.3 (one launch for all of them is the faster
-    // mode), and of two a stack of one direction, two layers of 1024 15.3 / 16.7.
-    const bool fuse_xproj = !use_seq && (T == 1 || (T == 2 && (D == 2 || L == 1)));
-
     const half_t* layer_in = (const half_t*)x;
     const long y_stride = (long)D * H;
     auto residual = [&](int l) { return D == 1 && l >= plan->first_residual_layer; };
@@ -810,6 +803,9 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
         for (int l = 0; l < L; ++l) {
             half_t* layer_out = (l == L - 1) ? (half_t*)y : plan->ybuf[l & 1];
             const int64_t in_w = plan->cells[(size_t)l * D].in_w;
+            // One step, and two where it pays: each step's launch makes its projection too.  (Of three steps one layer of 512 is slower
+            // so, 11.7 / 13.3 us, one launch for all of them being the faster mode.)
+            const bool fuse_xproj = T == 1 || (T == 2 && lstm_two_steps_project(D, L, H, in_w, st->num_cus));
             if (!fuse_xproj) {
                 float* outs2[2];
                 const half_t* ws2[2];

@@ -4,8 +4,30 @@
 
 #include <stdint.h>
 
+#include "xproj_plan.h"
+
 namespace pimhip
 {
+// Whether the launches of a layer's two steps make its projection too, in place of a launch for both rows (a launch per step, the layer
+// alone or in both directions; a stack of one direction stays with the projection's launch, two layers of 1024 15.3 / 16.7 us).  W_ih is
+// then read twice and a launch saved.  What that is worth depends on the kernel that makes the projection of two rows otherwise: the
+// split-K kernel, for up to 127 tiles of 128 gate rows, costs nearly always more than a second read, the tiles' kernel of more rows streams
+// W_ih as fast as the steps do (us a call, the projection's launch / in the steps, with the same weights again and with plans in turn that
+// do not fit the caches; megabytes of W_ih).
+//   split-K: one layer of 1024 over 2048 18.9 / 10.0 and 22.7 / 12.8, over 16384 (134) 86 / 46 and 114 / 50; of 1536 over 8192 (101) 54 / 43 and 68 / 46; of 2056 over 2056
+//     32.0 / 27.1 and 35.5 / 31.2, over 8192 (135) 64 / 63 and 77 / 67; of 3072 over 3072 (75) 48.1 / 45.9 and 54.4 / 49.5, over 6144 (151) 65.1 / 71.2 and 79.5 / 74.7; two
+//     directions of 1024 over 1024 15.5 / 12.5 and 19.0 / 14.9, of 1536 over 4096 (101) 43.3 / 42.7 and 51.4 / 46.4, over 6144 (151) 55.2 / 59.7 and 68.6 / 63.1
+//   tiles: one layer of 4096 over 256 (8) 52.9 / 50.3 and 56.1 / 55.6, over 1024 (34) 59.4 / 55.9 and 59.6 / 60.7, over 4096 (134) 72.6 / 92.8 and 86.7 / 97.9; two directions of
+//     2056 over 256 (8) 31.8 / 28.1 and 34.6 / 32.6, over 1024 (34) 37.7 / 35.1 and 38.4 / 39.7, over 2056 (68) 43.1 / 47.2 and 50.4 / 51.7, over 4096 (135) 52.9 / 73.5
+//     and 62.9 / 77.8
+inline bool lstm_two_steps_project(int dirs, int layers, int64_t H, int64_t in_w, int num_cus)
+{
+    if (dirs == 1 && layers > 1) return false;
+    const bool tiles = xproj_tile_rows(2, 4 * H, dirs, false, num_cus) != 0;
+    const double megabytes = 8.0 * (double)dirs * (double)H * (double)in_w / (1 << 20);  // of W_ih, 2^20 bytes each
+    return tiles ? megabytes <= 32.0 : megabytes <= 96.0 || 4 * H * dirs < 10240;
+}
+
 // v_dot2 instead of sparse matrix instructions.  The latter's weights pass through LDS first (1 to 1.6 us per launch), and they take
 // whole fragments of 64 columns in groups of four: v_dot2 is better for short sequences, for fewer than 64 units at any length, and
 // longest for 513 to 656 units, of whose second and third group the sparse fragments are half empty.  From 65 to 256 units one

@@ -35,3 +35,9 @@ def test_two_steps_are_measured_by_themselves(ops):
     assert plan.measured_mode(2) != 0 and plan.measured_mode(3) == 0 and plan.measured_mode(4) == 0
     plan.forward(x[:3], h0, c0)
     assert plan.measured_mode(3) != 0 and plan.measured_mode(4) == 0
+
+
+@pytest.mark.parametrize("I,H,L,bidir", [(2056, 2056, 1, True), (64, 2056, 2, True), (6600, 2560, 1, False)])
+def test_two_steps_with_a_projection_of_their_own(ops, I, H, L, bidir):
+    """W_ih too large to be read by each step: of the only layer, of the second of two, and by the kernel for fewer rows."""
+    test_two_steps_by_launches(ops, I, H, L, bidir)
