@@ -253,7 +253,9 @@ int pimhip_lstm_plan_measured_mode(PimHipLstmPlan* plan, int64_t seq_len, int* m
  * encoder and decoder, which the reference runs as one executeAtenLSTM1 and one executeAtenAdd per layer
  * (aten_ops_executor.cpp:2135-2307, :43-179).  hn / cn stay the layers' own h and c.  Such a layer's input width must equal
  * hidden_size.  first_residual_layer >= num_layers switches it off (the default).  A stack then still runs as one
- * pipeline launch where pimhip_lstm_forward would use one without the sums. */
+ * pipeline launch where pimhip_lstm_forward would use one without the sums.  From 1025 to 2048 units, where a layer with a sum runs alone, the
+ * first call that gives a layer one also makes the plan's own copy of that layer's w_ih (4 hidden_size^2 fp16) and waits for it,
+ * on a stream of its own and beside a capture; without memory for it the layer reads w_ih as it lies. */
 int pimhip_lstm_plan_set_residual(PimHipLstmPlan* plan, int first_residual_layer);
 
 /* The dense input projection of one LSTM layer over all time steps, the only MFMA kernel of the path:

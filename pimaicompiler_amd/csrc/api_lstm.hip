@@ -177,6 +177,48 @@ int xcd_dispatch_is_a_rotation(int blocks, hipStream_t s, bool* ok)
     *ok = rotation;
     return PIMHIP_OK;
 }
+
+// The cell's copy of w_ih in MFMA fragment order.
+hipError_t pack_input_weight(PimHipLstmPlan* plan, PimHipLstmPlan::Cell& c, hipStream_t s)
+{
+    int ntiles = 0, ksteps = 0;
+    packed_geometry(c.in_w, 4 * plan->hidden, &ntiles, &ksteps);
+    half_t* packed = nullptr;
+    hipError_t e = hipMalloc(&packed, (size_t)ntiles * ksteps * 64 * 16);
+    if (e != hipSuccess) return e;
+    plan->packed.push_back(packed);
+    launch_pack_w_fragments(c.w_ih, packed, 4 * plan->hidden, c.in_w, ntiles, ksteps, s);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    c.w_ih_packed = packed;
+    c.ksteps = ksteps;
+    return hipSuccess;
+}
+
+// The copies that layers from `first` on lack.  The caller may be recording a graph and has given no stream: this happens beside it, on a
+// stream of its own, and is over on return.  Without memory for them such a layer reads w_ih as it is.
+void pack_missing_input_weights(PimHipLstmPlan* plan, int first)
+{
+    bool missing = false;
+    for (int l = first; l < plan->num_layers; ++l) missing = missing || !plan->cells[(size_t)l].w_ih_packed;
+    if (!missing) return;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return;
+    int prev = -1;
+    hipStream_t s = nullptr;
+    hipError_t e = hipGetDevice(&prev);
+    if (e == hipSuccess) e = hipSetDevice(plan->device);
+    if (e == hipSuccess) e = hipStreamCreateWithFlags(&s, hipStreamNonBlocking);
+    for (int l = first; e == hipSuccess && l < plan->num_layers; ++l)
+        if (!plan->cells[(size_t)l].w_ih_packed) e = pack_input_weight(plan, plan->cells[(size_t)l], s);
+    if (s) {
+        (void)hipStreamSynchronize(s);
+        (void)hipStreamDestroy(s);
+    }
+    if (prev >= 0) (void)hipSetDevice(prev);
+    if (e != hipSuccess) (void)hipGetLastError();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+}
 }  // namespace
 
 extern "C" int pimhip_probe_xcc_map(void* out, int blocks, int threads, void* stream)
@@ -263,19 +305,11 @@ extern "C" int pimhip_lstm_plan_create(PimHipLstmPlan** plan_out, const void* co
     }
     PLAN_HIP_CHECK(hipGetLastError());
     // Cells whose input projection runs as a batch over the sequence (every layer of a bidirectional stack, the first
-    // layer of every wavefront group of a unidirectional one, any layer above kSeqMaxH units, where one with a residual sum runs alone)
-    // get a copy of w_ih in MFMA fragment order.
+    // layer of every wavefront group of a unidirectional one) get a copy of w_ih in MFMA fragment order.  From 1025 to 2048 units a
+    // layer with a residual sum runs alone: pimhip_lstm_plan_set_residual makes the copies that only such a layer reads.
     for (int l = 0; l < num_layers; ++l) {
-        if (D == 1 && !plan->seq_wide && l % plan->max_wavefront != 0) continue;
-        for (int d = 0; d < D; ++d) {
-            PimHipLstmPlan::Cell& c = plan->cells[(size_t)l * D + d];
-            int ntiles = 0;
-            packed_geometry(c.in_w, 4 * H, &ntiles, &c.ksteps);
-            const size_t chunks = (size_t)ntiles * c.ksteps * 64;
-            PLAN_HIP_CHECK(hipMalloc(&c.w_ih_packed, chunks * 16));
-            plan->packed.push_back(c.w_ih_packed);
-            launch_pack_w_fragments(c.w_ih, c.w_ih_packed, 4 * H, c.in_w, ntiles, c.ksteps, s);
-        }
+        if (D == 1 && l % plan->max_wavefront != 0) continue;
+        for (int d = 0; d < D; ++d) PLAN_HIP_CHECK(pack_input_weight(plan, plan->cells[(size_t)l * D + d], s));
     }
     PLAN_HIP_CHECK(hipGetLastError());
     PLAN_HIP_CHECK(hipMalloc(&plan->xproj, sizeof(float) * (size_t)D * max_seq_len * 4 * H));
@@ -419,6 +453,7 @@ extern "C" int pimhip_lstm_plan_set_residual(PimHipLstmPlan* plan, int first_res
                 return fail(PIMHIP_ERR_INVALID_ARGUMENT, "layer %d has input width %lld and hidden size %lld: its input cannot be added to its output",
                             l, (long long)plan->cells[(size_t)l].in_w, (long long)plan->hidden);
     }
+    if (plan->seq_wide && plan->num_dirs == 1) pack_missing_input_weights(plan, first_residual_layer);
     if (plan->first_residual_layer != first_residual_layer) memset(plan->measured_mode, 0, sizeof(plan->measured_mode));
     plan->first_residual_layer = first_residual_layer;
     return PIMHIP_OK;

@@ -54,3 +54,43 @@ def test_wide_layers(ops, H, L, D, T, res, gives_up):
         for got, w in zip(plan.forward(x, h0, c0), want):
             assert float((got.double().reshape(w.shape) - w).abs().max()) <= 4e-3
         plan.status()
+
+
+def test_a_layer_has_a_copy_of_its_input_weights_only_where_it_runs_alone(ops):
+    """The upper one of two layers in a launch multiplies by w_ih as it lies; the copy for a launch of its own, 4 H^2 values, is made when
+    residual sums are switched on, in the middle of a graph's capture too, and once."""
+    H, L, T = 2048, 2, 4
+    copy = 4 * H * H * 2
+    params, x, h0, c0 = workloads.lstm_inputs(H, H, H, L, False, T)
+    params, (x, h0, c0) = [p.to(DEV) for p in params], (v.half().to(DEV) for v in (x.reshape(T, H), h0.reshape(L, H), c0.reshape(L, H)))
+
+    def used_by(f):
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        f()
+        torch.cuda.synchronize()
+        return before - torch.cuda.mem_get_info()[0]
+    plans = []
+
+    def plan_of():
+        plans.append(ops.LstmPlan(params, True, L, False, T))
+        plans[-1].set_mode(2)
+    plan_of()   # (whatever the device loads once)
+    assert copy <= used_by(plan_of) < 1.5 * copy
+    plan = plans[-1]
+    assert copy <= used_by(lambda: plan.set_residual(1)) < 1.5 * copy
+    want = in_64_bits(params, x, h0, c0, L, 1, 1)
+    eager = plan.forward(x, h0, c0)
+    assert all(float((got.double().reshape(w.shape) - w).abs().max()) <= 4e-3 for got, w in zip(eager, want))
+    assert used_by(lambda: (plan.set_residual(L), plan.set_residual(0))) == 0   # (both copies are there)
+
+    other = plans[0]
+    other.forward(x, h0, c0)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        other.set_residual(1)
+        got = other.forward(x, h0, c0)
+    for _ in range(3):
+        graph.replay()
+        assert all(torch.equal(a, b) for a, b in zip(got, eager))
+        assert all(torch.equal(a, b) for a, b in zip(other.forward(x, h0, c0), eager))
