@@ -231,8 +231,8 @@ int pimhip_lstm_plan_set_spin_limit(PimHipLstmPlan* plan, unsigned int spin_limi
  * (layer and direction) on one XCD of the part, the two directions of a layer side by side on two, the layers of a
  * unidirectional stack as a pipeline (hidden_size up to 1024 on a device of 8 XCDs x 32 CUs; PIMHIP_ERR_UNSUPPORTED
  * otherwise).  A call with seq_len 1 runs the fused step launch in every mode.
- * Automatic mode measures: the first pimhip_lstm_forward of a plan with a sequence length in [2^b, 2^(b+1)) that is issued
- * outside a graph capture runs the call under every mode that takes it (a few runs each, timed with HIP events: that
+ * Automatic mode measures: the first pimhip_lstm_forward of a plan with a sequence length of a range (two; three; four to seven;
+ * eight to fifteen; ...) that is issued outside a graph capture runs the call under every mode that takes it (a few runs each, timed with HIP events: that
  * call synchronises its stream and costs a few times its usual duration), and the plan keeps the fastest for that range of
  * lengths; as the reference does with its two libraries on the first inference
  * (runtime/source/executor/stream_executor.cpp:312-339).  Until then (calls inside a capture, or after

@@ -558,10 +558,10 @@ int lstm_forward_impl(PimHipLstmPlan* plan, const void* x, const void* h0, const
     // (Its 32 CUs per group take longer to load the weights and a pipeline has to fill, which few steps do not win back.  Plans that
     // have measured do not come here.  For the others the lines lie on the safe side: the per-XCD kernel is faster at all of these lengths,
     // and from fewer steps on for most sizes.  Measured on MI355X, time over all CUs over time per XCD, graph replays: two
-    // directions at 4 / 8 / 16 / 64 steps 256 units 1.19 / 1.41 / 1.61 / 1.99, 1024 units 0.86 / 1.02 / 1.24 / 1.61; one layer at 8 / 16 / 24 / 64
-    // steps 256 1.30 / 1.51 / 1.65 / 1.87, 512 1.11 / 1.30 / 1.42 / 1.62, 1024 0.79 / 0.95 / 1.05 / 1.24; two layers at 8 / 16 / 32 256 1.07 / 1.28 / 1.56, 1024
-    // 0.86 / 1.08 / 1.32; three at 6 / 8 / 16 256 1.07 / 1.20 / 1.50, 1024 0.93 / 1.02 / 1.30; stacks with residual sums at 2 / 16 two layers
-    // of 1024 1.03 / 1.66, three 1.29 / 2.07.)
+    // directions at 4 / 8 / 16 / 64 steps 256 units 1.23 / 1.49 / 1.75 / 2.14, 1024 units 0.83 / 1.01 / 1.28 / 1.78; one layer at 8 / 16 / 24 / 64
+    // steps 256 1.42 / 1.66 / 1.80 / 2.10, 512 1.21 / 1.46 / 1.61 / 1.82, 1024 0.82 / 1.02 / 1.16 / 1.44; two layers at 8 / 16 / 32 256 1.13 / 1.46 / 1.80, 1024
+    // 0.85 / 1.12 / 1.41; three at 6 / 8 / 16 256 1.08 / 1.19 / 1.52, 1024 0.91 / 0.99 / 1.29; stacks with residual sums at 2 / 16 two layers
+    // of 1024 1.03 / 1.77, three 1.31 / 2.20.)
     const bool xcd_pays = (D == 2 && T >= 16) || (D == 1 && L == 1 && T >= (H > 512 ? 64 : 16)) ||
                           (D == 1 && L >= 2 && T >= (L >= 3 ? 16 : 32));
     // (a stack with residual sums needs the pipeline kernel that makes them; where that one is not resident the stack runs

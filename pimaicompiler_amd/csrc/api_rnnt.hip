@@ -186,8 +186,9 @@ extern "C" int pimhip_rnnt_plan_create(PimHipRnntPlan** plan_out, const void* co
     {
         // As many teams of symbol blocks as the CUs that are left take, one workgroup to a CU, up to one for each step that the joint
         // blocks run ahead (2 x 320 units, 29 symbols, 341 frames with 74 and 114 symbols emitted, us: six teams 594 and 798, twelve 581 and 784).
-        // Products of another stream share CUs with them (measured with eight: beside such a decode a projection of 341 frames onto 4096 takes
-        // 12.1 us instead of 11.5 with one team, beside one of 400 symbols, whose teams take 244 CUs, 14.3 instead of 11.1; 8.6 alone).
+        // Products of another stream share CUs with them: beside such a decode (192 workgroups) a projection of 341 frames onto 4096 takes
+        // 23.3 us, beside eight teams it took 23.1 (9.6 alone); beside one of 400 symbols, whose two teams take 244 CUs, it hardly advances
+        // before the loop's end.
         const int n_vocab = (int)((vocab + 7) / 8);
         const int spare = std::min(st->num_cus, kRnntMaxBlocks) - plan->blocks;
         plan->greedy_teams = std::min(kRnntGreedyTeams, 1 + std::max(0, spare) / n_vocab);

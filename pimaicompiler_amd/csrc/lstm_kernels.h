@@ -235,8 +235,9 @@ __global__ __launch_bounds__(WAVES * 64) void lstm_step_pair_f16_kernel(LstmStep
 //   2. per chain: 4 rows x 16 columns of dot products per lane (twice that with W_ih), a transpose-sum over
 //      the 64 lanes (6 exchanges) that leaves gate k in lane k, the four activations in parallel in lanes 0..3,
 //      the cell update;
-//   3. lane 0 of each wavefront stores y and hands its h values to LDS; one barrier; one lane publishes the block's
-//      entry with one store per 16 bytes.
+//   3. lane 0 of each wavefront hands its h values to LDS; one barrier; one lane publishes the block's entry with one
+//      store per 16 bytes; behind that lane 0 of each wavefront stores y (and hn, cn at the end), unless the block goes
+//      on by itself and makes them again.  Neither barrier of a step waits for memory operations.
 //
 // Exchange buffer: hx[2][NB] entries of 64 bytes (entries of different blocks do not share a 64-byte segment,
 // which measurably shortens the exchange); chain k of block b uses the 8-byte word k of the entry, one fp16 per
@@ -515,7 +516,7 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
                 a[k] += xp_slot[k];
                 // The term fetched two steps ago has been consumed: refill the same register for two steps ahead.
                 // (Issued only now so that the old and the new value never live at once, which would cost a copy,
-                // and with it a wait for this load and for the stores below, at the loop's back edge.)
+                // and with it a wait for this load, at the loop's back edge.)
                 xp_slot[k] = xp_ptr[k][(long)max(0, min(s_k + 2, T - 1)) * xp_step[k]];
             }
             // Each of lanes 0..3 activates its own gate: sigmoid for i, f, o and tanh(a) = 2 * sigmoid(2a) - 1 for g.
@@ -534,7 +535,7 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
             c_out[k] = c_new;
         }
 
-        // ---- 3. outputs, then publish ----
+        // ---- 3. publish, then outputs ----
         // The block's values are gathered in LDS and published by ONE lane with ONE store per 16 bytes: the time
         // until every block has seen a super-step grows by about 0.3 us with every further store per block.
         if (lane == 0) {
@@ -542,7 +543,7 @@ __global__ __launch_bounds__(64 * UNITS) void lstm_seq_f16_kernel(LstmSeqArgs p)
 #pragma unroll
             for (int k = 0; k < NC; ++k) {
                 // A NaN (from non-finite inputs or weights) has bit 14 set and cannot travel with the flag: y, hn and
-                // cn below still receive it, the exchange carries 0 for this unit instead of making every reader wait
+                // cn, stored behind the publish, still receive it, the exchange carries 0 for this unit instead of making every reader wait
                 // for a flag that never matches.
                 const unsigned int hbits = (unit_ok && h_is_number[k]) ? (unsigned int)__builtin_bit_cast(unsigned short, h_new[k]) : 0u;
                 pub[k][wave] = (unsigned short)(hbits | flag);

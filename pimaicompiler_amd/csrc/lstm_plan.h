@@ -29,11 +29,12 @@ inline bool lstm_two_steps_project(int dirs, int layers, int64_t H, int64_t in_w
 }
 
 // v_dot2 instead of sparse matrix instructions.  The latter's weights pass through LDS first (1 to 1.6 us per launch), and they take
-// whole fragments of 64 columns in groups of four: v_dot2 is better for short sequences, for fewer than 64 units at any length, and
-// longest for 513 to 656 units, of whose second and third group the sparse fragments are half empty.  From 65 to 256 units one
-// group holds the row and there is nothing to win.  `chained`: the layers a launch runs as a pipeline, 1 for recurrences that are fed by
-// none other; the more there are, the more steps the launch has beside its sequence's.
-// Measured on MI355X (graph replays, time on v_dot2 over time on sparse instructions):
+// whole fragments of 64 columns in groups of four: v_dot2 is better for a few steps of more than 256 units, and longest for 513 to 656, of
+// whose second and third group the sparse fragments are half empty.  From 65 to 256 units one group holds the row and there is nothing to
+// win.  `chained`: the layers a launch runs as a pipeline, 1 for recurrences that are fed by none other; the more there are, the more steps
+// the launch has beside its sequence's.
+// The lines were drawn at these figures (MI355X, graph replays, time on v_dot2 over time on sparse instructions), which had v_dot2 ahead
+// for fewer than 64 units at any length too:
 //   one layer, at 2 / 4 / 6 / 8 / 10 / 16 steps: 64 units 1.00 / 0.95 / 0.99 / 0.99 / 1.01 / 1.01, 128 0.95 / 0.97 / 1.00 / 1.00 / 1.02 / 1.02, 192 1.01 / 1.01 /
 //     1.06 / 1.04 / 1.07 / 1.08, 320 0.97 / 0.97 / 0.99 / 1.02 / 1.04 / 1.06, 512 0.94 / 0.97 / 0.99 / 1.02 / 1.04 / 1.07, 640 0.90 / 0.93 / 0.95 / 0.97 / 0.98 / 1.01,
 //     768 0.94 / 0.97 / 0.99 / 1.02 / 1.02 / 1.05, 1024 0.95 / 0.98 / 1.00 / 1.02 / 1.04 / 1.08; two directions within 0.02 of these
@@ -43,11 +44,13 @@ inline bool lstm_two_steps_project(int dirs, int layers, int64_t H, int64_t in_w
 //     0.97, 64 1.01 / 1.02 / 1.03
 //   three layers, at 2 / 3 / 4: 512 1.01 / 1.01 / 1.02, 640 0.97 / 1.00 / 1.00, 1024 1.00 / 1.02 / 1.03; at 24 / 80 / 200: 16 0.97 / 0.98 / 0.98, 32 1.06 / 1.13 / 1.15;
 //     four layers, at 2 / 4 / 8: 16 0.98 .. 1.00, 640 1.00 / 1.01 / 1.03
-// Since what stands around the products on a step's path was shortened for both (same layout as above): one layer, at 2 / 4 / 6 / 8 / 10 / 16 / 80 steps:
+// What stands around the products on a step's path has been shortened since, for the sparse kind by more (same layout as above): one layer, at 2 / 4 / 6 / 8 / 10 / 16 / 80 steps:
 //     8 1.05 / 1.02 / 1.01 / 1.04 / 1.04 / 1.02 / 1.01, 64 1.02 / 1.02 / 1.03 / 1.02 / 1.04 / 1.04 / 1.05, 128 1.00 / 1.01 / 1.01 / 1.02 / 1.04 / 1.06 / 1.09, 512 0.91 / 0.96 / 1.00 /
 //     1.03 / 1.05 / 1.12 / 1.26, 640 0.89 / 0.92 / 1.00 / 1.04 / 1.06 / 1.10 / 1.26, 1024 0.93 / 0.97 / 1.01 / 1.05 / 1.09 / 1.16 / 1.38; two layers at 2 / 3 / 4 / 80: 48 1.04 / 1.03 /
-//     1.04 / 1.05, 512 0.98 / 1.01 / 1.02 / 1.28, 1024 0.98 / 1.01 / 1.03 / 1.41.  The lines stay: between them and these figures lie a few percent of calls of few
-//     steps or few units.
+//     1.04 / 1.05, 512 0.98 / 1.01 / 1.02 / 1.28, 1024 0.98 / 1.01 / 1.03 / 1.41.
+// By these v_dot2 is the slower kind now for all of fewer than 64 units (1 to 5 %), for 64 and 128 (0 to 4 %) and in the last steps in front of the other
+// lines (up to 6 %), though no call is slower than it was when the lines were drawn.  A move of the lines changes which sums such calls make,
+// and with them last bits of their results.
 inline bool xcd_on_dot(int64_t H, int64_t T, int chained)
 {
     const bool half_empty = H > 512 && H <= 656;

@@ -596,8 +596,8 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
     const bool sums = res && wave == kXcdSumWave && lane < 32 && eu < H;
     // The input of step s is asked for right after that step's barrier, together with the projection rows two steps ahead
     // (it exists: the projection row made from it is in use), parked in LDS at the top of step s + 1 and added after
-    // that step's barrier.  Every wavefront drains its loads once per step, so what matters is that the load leaves
-    // early in the step: issued behind the sum of the step before, it cost 0.23 us per step.
+    // that step's barrier.  Parking it waits for the load, so what matters is that the load leaves early in the step: issued
+    // behind the sum of the step before, it cost 0.23 us per step.
     unsigned short in_ahead = 0xffffu;
     bool sum_gave_up = false;  // (a lane's: not every lane makes sums)
     auto emit_sum = [&](int se) __attribute__((always_inline)) {
@@ -686,7 +686,7 @@ __device__ __forceinline__ void lstm_xcd_body(const LstmXcdArgs& p)
         const unsigned long long flag = ((unsigned long long)flag32 << 32) | flag32;
         if (!polled) {
             // steps s + 16 .. s + 31 are fetched when step s starts a half, and written over the half that has just been
-            // used up one step later (this wavefront's poll in between has waited for them)
+            // used up one step later (in a polling wavefront the poll in between has waited for them)
             if ((s & 15) == 0 && s > 0) xp_next = fetch_xp(s + 16);
             if ((s & 15) == 1 && s > 1) deposit_xp(((s >> 4) & 1) ^ 1, xp_next);
         } else if (fetcher && s >= 1 && s + 1 < T) {
